@@ -1,4 +1,5 @@
-"""ctypes binding of libggml_mmq_gfx950.so (the C ABI declared in include/ggml_mmq_gfx950.h).
+"""Bindings of libggml_mmq_gfx950.so (the C ABI declared in include/ggml_mmq_gfx950.h): ``load()`` gives every entry point
+through ctypes, ``host()`` the native module that runs the layers' own calls (``csrc/host.cpp``).
 
 The library is the only implementation of the hot path: there is no CPU or framework fallback, and
 loading fails loudly when the shared object has not been built (``python -c "import __graft_entry__
@@ -8,13 +9,17 @@ as g; g.build()"`` or ``make -C <package>/csrc``).
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p
 from pathlib import Path
 
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libggml_mmq_gfx950.so"
+HOST_PATH = LIB_PATH.with_name("_host.so")
 _lib: ctypes.CDLL | None = None
+_host = None
 
 _P, _I, _L, _F = c_void_p, c_int, c_int64, c_float
 
@@ -82,6 +87,20 @@ def load() -> ctypes.CDLL:
             fn.argtypes = argtypes
         _lib = lib
     return _lib
+
+
+def host():
+    """The native host module, loaded once; like the library itself it has no fallback."""
+    global _host
+    if _host is None:
+        load()
+        if not HOST_PATH.exists():
+            raise RuntimeError(f"{HOST_PATH} is missing: run __graft_entry__.build() (or make -C transformers5-qwen3.5-recipe_amd/csrc).")
+        loader = importlib.machinery.ExtensionFileLoader("_host", str(HOST_PATH))
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_host", loader))
+        loader.exec_module(module)
+        _host = module
+    return _host
 
 
 def check(rc: int, exc: type[Exception] = RuntimeError) -> None:

@@ -65,26 +65,10 @@ def mmq_grad_input(grad_output: torch.Tensor, payload: torch.Tensor, quant_type:
     return dx.reshape(*grad_output.shape[:-1], in_features)
 
 
-class _Mmq(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, payload, quant_type, out_features):
-        ctx.save_for_backward(payload)
-        ctx.quant_type, ctx.in_features = quant_type, x.shape[-1]
-        return _mmq_forward(x, payload, quant_type, out_features)
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        if torch.is_grad_enabled():
-            raise RuntimeError("packed MMQ does not support higher-order gradients")
-        (payload,) = ctx.saved_tensors
-        dx = mmq_grad_input(grad_output.contiguous(), payload, ctx.quant_type, ctx.in_features) if ctx.needs_input_grad[0] else None
-        return dx, None, None, None
-
-
 def mmq(x: torch.Tensor, payload: torch.Tensor, quant_type: int, out_features: int) -> torch.Tensor:
     """Y = X . W^T over packed rows (the reference's ``torch_ggml_ops.mmq``, fast_lora.py:155-160)."""
-    payload = payload.as_subclass(torch.Tensor)
-    return _Mmq.apply(x, payload, int(quant_type), int(out_features))
+    y = _lib.host().linear(x, payload, int(quant_type), int(out_features), None, None, 0.0)
+    return y if y is not None else _rejected_linear(x, payload, int(quant_type), int(out_features), None, None, "mmq")
 
 
 class _FixedGroupedMmq(torch.autograd.Function):
@@ -141,58 +125,22 @@ def fixed_grouped_mmq_grad_input(grad_output: torch.Tensor, packed_groups: torch
     return dx
 
 
-def _workspace(device, rows: int, groups: int, experts: int, n_total: int, k: int, r: int) -> torch.Tensor:
-    nbytes = _lib.load().ggq_lora_workspace_bytes(rows, groups, experts, n_total, k, r)
-    return torch.empty(nbytes, dtype=torch.uint8, device=device)
-
-
-class _LoraMmq(torch.autograd.Function):
-    """Base matmul + LoRA residual in one forward call; dX, dA, dB in one backward call."""
-
-    @staticmethod
-    def forward(ctx, x, payload, quant_type, out_features, lora_a, lora_b, scaling):
-        x2 = _flat_bf16(x, "LoRA linear input")
-        m, k = x2.shape
-        _check_packed(payload, quant_type, out_features, k, "LoRA linear")
+def _rejected_linear(x, payload, quant_type, out_features, lora_a, lora_b, what):
+    """Raises the error that says why the native call did not take its operands."""
+    x2 = _flat_bf16(x, f"{what} input")
+    k = x2.shape[1]
+    _check_packed(payload.as_subclass(torch.Tensor), quant_type, out_features, k, what)
+    if lora_a is not None:
         _lib.require_device_tensor(lora_a, "lora_A", torch.bfloat16)
         _lib.require_device_tensor(lora_b, "lora_B", torch.bfloat16)
-        r = lora_a.shape[0]
-        if tuple(lora_a.shape) != (r, k) or tuple(lora_b.shape) != (out_features, r):
-            raise ValueError(f"LoRA factors must be A [r,{k}] and B [{out_features},r], got {tuple(lora_a.shape)} and {tuple(lora_b.shape)}")
-        r_pad = (r + 15) // 16 * 16
-        xa = torch.empty(m, r_pad, dtype=torch.bfloat16, device=x.device)
-        y = torch.empty(m, out_features, dtype=torch.bfloat16, device=x.device)
-        if m:
-            ws = _workspace(x.device, m, 0, 1, out_features, k, r)
-            _lib.check(_lib.load().ggq_lora_mmq_forward(
-                x2.data_ptr(), payload.data_ptr(), quant_type, m, out_features, k, lora_a.data_ptr(), lora_b.data_ptr(), r,
-                float(scaling), xa.data_ptr(), y.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_handle(x.device)))
-        ctx.save_for_backward(x2, xa, payload, lora_a, lora_b)
-        ctx.meta = (quant_type, out_features, float(scaling), x.shape)
-        return y.reshape(*x.shape[:-1], out_features)
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        if torch.is_grad_enabled():
-            raise RuntimeError("packed MMQ LoRA linear does not support higher-order gradients")
-        x2, xa, payload, lora_a, lora_b = ctx.saved_tensors
-        quant_type, n, scaling, x_shape = ctx.meta
-        g2 = _flat_bf16(grad_output.contiguous(), "LoRA linear cotangent")
-        m, k = x2.shape
-        r = lora_a.shape[0]
-        dx = torch.empty_like(x2)
-        da = torch.empty_like(lora_a) if ctx.needs_input_grad[4] else None
-        db = torch.empty_like(lora_b) if ctx.needs_input_grad[5] else None
-        ws = _workspace(x2.device, m, 0, 1, n, k, r)
-        _lib.check(_lib.load().ggq_lora_mmq_backward(
-            g2.data_ptr(), payload.data_ptr(), quant_type, m, n, k, x2.data_ptr(), xa.data_ptr(), lora_a.data_ptr(),
-            lora_b.data_ptr(), r, scaling, dx.data_ptr(), _lib.ptr(da), _lib.ptr(db), ws.data_ptr(), ws.numel(),
-            _lib.stream_handle(x2.device)))
-        return (dx.reshape(x_shape) if ctx.needs_input_grad[0] else None), None, None, None, da, db, None
+        raise ValueError(f"LoRA factors must be A [r,{k}] and B [{out_features},r], got {tuple(lora_a.shape)} and {tuple(lora_b.shape)}")
+    raise ValueError(f"{what}: operands do not describe a packed linear on one device")
 
 
 def lora_mmq(x, payload, quant_type, out_features, lora_a, lora_b, scaling) -> torch.Tensor:
-    return _LoraMmq.apply(x, payload.as_subclass(torch.Tensor), int(quant_type), int(out_features), lora_a, lora_b, float(scaling))
+    """Base matmul + LoRA residual in one forward call; dX, dA, dB in one backward call."""
+    y = _lib.host().linear(x, payload, int(quant_type), int(out_features), lora_a, lora_b, float(scaling))
+    return y if y is not None else _rejected_linear(x, payload, int(quant_type), int(out_features), lora_a, lora_b, "LoRA linear")
 
 
 def _fused_lora_add(result, x, lora_A: torch.nn.Linear, lora_B: torch.nn.Linear, dropout: torch.nn.Module, scaling: float):

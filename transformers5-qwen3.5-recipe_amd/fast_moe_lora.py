@@ -21,7 +21,7 @@ from typing import Any
 
 import torch
 
-from . import _lib
+from . import _lib, fast_moe_routing
 from .fast_lora import _NATIVE_MMQ_QUANT_TYPES, supports_native_mmq
 from .fast_moe_routing import ExpertRoutingPlan, finalize_expert_routing, prepare_expert_routing
 from .gguf import GGUFQuantizedTensor, dequantize_gguf_tensor, row_bytes
@@ -444,6 +444,8 @@ class GGUFExperts(torch.nn.Module):
         self._all_experts = torch.arange(e, dtype=torch.int64, device=gate_proj.device)
 
     def _prepare_expert_hidden_states(self, hidden_states: torch.Tensor) -> torch.Tensor:
+        if hidden_states.ndim == 2 and hidden_states.dtype == self.compute_dtype and hidden_states.is_contiguous():
+            return hidden_states
         return hidden_states.reshape(-1, self.hidden_dim).to(self.compute_dtype).contiguous()
 
     def _prepare_expert_execution(self, routing_plan: ExpertRoutingPlan, mode: str) -> _ExpertExecutionPlan:
@@ -461,6 +463,14 @@ class GGUFExperts(torch.nn.Module):
         if fn is None:
             raise RuntimeError(f"experts implementation {self.experts_implementation!r} is not registered")
         return fn(self, hidden_states, top_k_index, top_k_weights, lora_weights)
+
+
+def _runs_as_one_node(experts: GGUFExperts) -> bool:
+    """Whether nothing asks for the layer's pieces: the switches above are at their defaults, ids need not be validated, and
+    the module's plan and activation are this class's own."""
+    cls = type(experts)
+    return (FUSE_GATED_DOWN_COMBINE and SHARE_GROUP_TABLES and not fast_moe_routing.VALIDATE_EXPERT_IDS
+            and cls._apply_split_gate is GGUFExperts._apply_split_gate and cls._prepare_expert_execution is GGUFExperts._prepare_expert_execution)
 
 
 def qwen3_5_moe_gguf_mmq_lora_forward(self: GGUFExperts, hidden_states: torch.Tensor, top_k_index: torch.Tensor,
@@ -483,6 +493,15 @@ def qwen3_5_moe_gguf_mmq_lora_forward(self: GGUFExperts, hidden_states: torch.Te
         raise RuntimeError("Paired grouped GGUF MMQ requires one quantization type.")
 
     compute_hidden_states = self._prepare_expert_hidden_states(hidden_states)
+    if _runs_as_one_node(self):
+        # the whole layer as one native call and one autograd node; operands it does not take go through the nodes below,
+        # whose checks name what is wrong
+        factors = (lora_weights.gate_up_a, lora_weights.gate_up_b, lora_weights.down_a, lora_weights.down_b) if lora_weights is not None else (None,) * 4
+        out = _lib.host().experts(compute_hidden_states, top_k_index, top_k_weights, self.gate_proj, self.up_proj, self.down_proj, *factors,
+                                  self._all_experts, self.gate_proj.quant_type, self.down_proj.quant_type,
+                                  lora_weights.scaling if lora_weights is not None else 0.0, self.swiglu_limit or 0.0)
+        if out is not None:
+            return out if out.dtype == hidden_states.dtype and out.shape == hidden_states.shape else out.to(hidden_states.dtype).reshape(hidden_states.shape)
     tokens, top_k = top_k_index.shape[0], top_k_index.shape[1]
     # The gate/up launch reads the token rows in place where it can; the routed copy is made otherwise.
     in_place = (compute_hidden_states.ndim == 2 and compute_hidden_states.is_contiguous()

@@ -66,7 +66,10 @@ def qwen_router_forward(weight: torch.Tensor, hidden_states: torch.Tensor, top_k
     scores come from one kernel when nothing differentiates through the logits; under autograd the scores are recomputed
     from the selected logits with framework operators, as the reference does, so that the gradient reaches the router's
     input (and its weight, when that trains)."""
-    flat = hidden_states.reshape(-1, weight.shape[1])
+    flat = hidden_states if hidden_states.ndim == 2 else hidden_states.reshape(-1, weight.shape[1])
+    done = _lib.host().router(weight, flat, int(top_k))
+    if done is not None:
+        return done
     router_logits = F.linear(flat, weight)
     if router_logits.requires_grad and torch.is_grad_enabled():
         indices = _select(router_logits.detach(), top_k, None, "identity", 0, 1.0)[0]
