@@ -133,6 +133,12 @@ int ggq_debug_force_grouped_shape(int shape) {
     return GGQ_OK;
 }
 
+int ggq_debug_force_dense_shape(int shape, int splits) {
+    if (shape < -1 || shape > 3 || splits < 0 || splits > 8) return set_error(GGQ_ERR_SHAPE, "debug_force_dense_shape: unknown shape %d or %d splits", shape, splits);
+    dense_force_shape(shape, splits);
+    return GGQ_OK;
+}
+
 int ggq_set_factor_gradient_overlap(int enabled) {
     g_overlap_enabled.store(enabled ? 1 : 0, std::memory_order_relaxed);
     return GGQ_OK;
@@ -200,7 +206,7 @@ int64_t ggq_lora_workspace_bytes(int64_t rows, int64_t groups, int64_t experts, 
     const int64_t tiles = rows / 64 + groups + 2;
     return 5 * align256(tiles * (int64_t)sizeof(TileDesc)) + align256(16) + align256(experts * 2 * 4) +
            align256(experts * n_total * rp * 2) * 2 + align256(experts * k * rp * 2) + align256(rows * rp * 2) + 4096 +
-           (groups == 0 ? align256(kDenseFactorSplits * std::max(n_total, k) * rp * 4) : 0);
+           (groups == 0 ? align256(kDenseFactorSplits * std::max(n_total, k) * rp * 4) + dense_workspace_bytes(rows, n_total, k) + 256 : 0);
 }
 
 int ggq_lora_mmq_forward(const void* x, const void* packed, int qt, int64_t m, int64_t n, int64_t k, const void* lora_a,
@@ -405,6 +411,13 @@ static int grouped_forward(const char* what, const void* x, RowIndex x_index, co
         }
         p.la = (const bf16_t*)xa_out, p.lb = lb, p.lb_expert_elems = (int64_t)nseg * n * rp, p.r_pad = rp, p.lora_scale = scale;
     }
+    if (groups == 0 && dense_takes(kModeNT, rows, n, k, x, k)) {
+        DenseCall q{};
+        q.qt = qt, q.mode = kModeNT, q.m = rows, q.n = n, q.k = k, q.a = x, q.lda = k, q.w = packed1, q.c = y1, q.ldc = n;
+        if (lora_a) q.la = p.la, q.lb = p.lb, q.r_pad = rp, q.rank = r, q.lora_scale = scale;
+        const int64_t need = dense_workspace_bytes(rows, n, k);
+        if (void* panels = ws ? bump.take(need) : nullptr) return dense_mmq(q, panels, need, s);  // (callers without a workspace keep the tile kernel)
+    }
     if (t_small) {
         MmqParams ps = p;
         ps.tiles = t_small, ps.num_tiles = n_small, ps.max_row_tiles = (int)groups, ps.shape = kShapeSmall;
@@ -536,6 +549,13 @@ static int grouped_backward(const char* what, const void* dy1, const void* dy2, 
     }
     auto grad_input = [&]() -> int {
         if (rows == 0) return GGQ_OK;
+        if (groups == 0 && dense_takes(kModeNN, rows, n, k, dy1, n)) {
+            DenseCall q{};
+            q.qt = qt, q.mode = kModeNN, q.m = rows, q.n = n, q.k = k, q.a = dy1, q.lda = n, q.w = packed1, q.c = dx, q.ldc = k;
+            if (lora_a) q.la = p.la, q.lb = p.lb, q.r_pad = rp, q.rank = r, q.lora_scale = scale;
+            const int64_t need = dense_workspace_bytes(rows, n, k);
+            if (void* panels = ws ? bump.take(need) : nullptr) return dense_mmq(q, panels, need, s);
+        }
         if (t_tall) return launch_wide_and_tall(qt, kModeNN, p, (int)rows, (int)n, (int)k, nseg, t_tall, n_tall, max_tall, s);
         return launch_mmq(qt, kModeNN, kEpiStore, p, s);
     };

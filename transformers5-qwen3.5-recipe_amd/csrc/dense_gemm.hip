@@ -1,0 +1,579 @@
+// Dense launches (one row range, one weight matrix) as two passes: the packed weights are decoded once into a bf16 scratch
+// laid out for the matrix cores, and a plain bf16 tile kernel multiplies with it.
+//
+// The kernels of mmq_tile.h decode every weight once per 256-row tile inside the matmul's step, where the decoding waves and
+// the barrier per 64-wide step set the pace: 0.80-0.85 PFLOP/s at 4096 rows whatever the block format.  Decoding ahead costs
+// one write and a few reads of 2 bytes per weight, which stay in the memory-side cache, and leaves a loop whose only work
+// per step is LDS reads and MFMAs.
+//
+// Scratch layout ("panels"): the output columns in groups of eight, each group holding its contraction in steps of 64:
+//   panel[column / 8][step][8 columns][64 contraction elements], the eight 16-byte chunks of a column XOR-swizzled (a_slot),
+// so that one 1 KB request moves one group's step to LDS as it is, and the operand reads meet no bank conflict.  The forward
+// panel's columns are weight rows; the grad-input panel's columns are the weights' k and its contraction the weight rows
+// (the decoder transposes through LDS), so both directions run the same kernel.
+#include <algorithm>
+#include <atomic>
+#include <type_traits>
+
+#include "blocks.h"
+#include "iq2xxs_grid.h"
+#include "launch.h"
+#include "mmq_host.h"
+
+namespace ggq {
+
+static __device__ const uint64_t d_iq2xxs_grid_dense[256] = GGQ_IQ2XXS_GRID_INIT;
+static __device__ const uint4 d_zero16 = {0, 0, 0, 0};  // what a lane loads past the end of a contraction
+
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+
+// ------------------------------------------------------------------------------------------------
+// Decoding passes.  HBM-bound: packed bytes in, two bytes per weight out.
+
+template <int QT>
+__device__ __forceinline__ const uint2* stage_tables(uint32_t* lds, int tid, int threads) {
+    if constexpr (QT == kIQ2_XXS) {
+        for (int i = tid; i < Fmt<kIQ2_XXS>::kTableWords; i += threads) lds[i] = Fmt<kIQ2_XXS>::table_word(i, i < 1024 ? d_iq2xxs_grid_dense[i >> 2] : 0ull);
+        __syncthreads();
+    }
+    return (const uint2*)lds;
+}
+
+// Forward panel.  One wave per (group of eight weight rows, 256 elements of k): lane (row lane / 8, run lane % 8) decodes one
+// 32-element run; the eight lanes of a row read adjacent bytes.  The wave's 4 KB go through LDS and leave in whole 1 KB pieces.
+template <int QT>
+__global__ __launch_bounds__(256) void decode_panel_nt_kernel(const uint8_t* w, int64_t row_bytes, int n, int k, uint8_t* panel) {
+    __shared__ __attribute__((aligned(16))) uint8_t out_lds[4][4096];
+    __shared__ uint32_t tables[QT == kIQ2_XXS ? Fmt<kIQ2_XXS>::kTableWords : 1];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint2* tab = stage_tables<QT>(tables, threadIdx.x, 256);
+    const int kblocks = (k + 255) >> 8, steps = k >> 6;
+    const int64_t unit = (int64_t)blockIdx.x * 4 + wave;
+    const int group = (int)(unit / kblocks), kb = (int)(unit - (int64_t)group * kblocks);
+    if (group * 8 >= n) return;
+    const int row = min(group * 8 + (lane >> 3), n - 1), ksub = kb * 8 + (lane & 7);
+    const int live_steps = min(4, steps - kb * 4);
+    typename Fmt<QT>::Raw raw;
+    uint32_t v[16];
+    Fmt<QT>::load(raw, w + (int64_t)row * row_bytes, min(ksub, (k >> 5) - 1));
+    Fmt<QT>::decode(raw, ksub, v, tab);
+    const int r8 = lane >> 3, sw = ((group * 8 + r8) >> 1) & 7, st = (lane & 7) >> 1, c0 = (lane & 1) * 4;
+    uint8_t* mine = out_lds[wave] + st * 1024 + r8 * 128;
+#pragma unroll
+    for (int i = 0; i < 4; i++) *(uint4*)(mine + ((c0 + i) ^ sw) * 16) = make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+    // (LDS serves a wave in order; each wave reads back only what it wrote)
+    uint8_t* dst = panel + ((int64_t)group * steps + kb * 4) * 1024 + lane * 16;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint4 piece = *(const uint4*)(out_lds[wave] + i * 1024 + lane * 16);
+        if (i < live_steps) *(uint4*)(dst + i * 1024) = piece;
+    }
+}
+
+// Grad-input panel of the columns [k0, k0 + kcols).  One workgroup per (64 weight rows, 256 elements of k): a lane decodes
+// two 32-element runs of one weight row (lanes = consecutive rows); neighbouring rows trade halves through a data-parallel
+// move so that every LDS write carries two adjacent contraction elements of one column; the 32 KB block then is the panel's
+// image and leaves in 1 KB pieces.  Weight rows past n count as zero (a contraction runs to the next multiple of 64).
+template <int QT>
+__global__ __launch_bounds__(256) void decode_panel_nn_kernel(const uint8_t* w, int64_t row_bytes, int n, int k, int k0, int kcols, uint8_t* panel) {
+    __shared__ __attribute__((aligned(16))) uint32_t image[256 * 32];
+    __shared__ uint32_t tables[QT == kIQ2_XXS ? Fmt<kIQ2_XXS>::kTableWords : 1];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint2* tab = stage_tables<QT>(tables, threadIdx.x, 256);
+    const int kblocks = (kcols + 255) >> 8, steps = (n + 63) >> 6;
+    const int step = blockIdx.x / kblocks, kb = blockIdx.x - step * kblocks;
+    const int row = step * 64 + lane;
+    const uint8_t* src = w + (int64_t)min(row, n - 1) * row_bytes;
+    const int kk0 = k0 + kb * 256;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int run = wave * 2 + u;  // of the block's eight
+        const int ksub = min((kk0 >> 5) + run, (k >> 5) - 1);
+        typename Fmt<QT>::Raw raw;
+        uint32_t v[16];
+        Fmt<QT>::load(raw, src, ksub);
+        Fmt<QT>::decode(raw, ksub, v, tab);
+        const uint32_t sel = (lane & 1) ? 0x03020706u : 0x05040100u;  // odd rows: {mine.hi : theirs.hi}, even rows: {theirs.lo : mine.lo}
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const uint32_t mine = row < n ? v[i] : 0u;
+            const uint32_t theirs = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, 0xB1, 0xF, 0xF, true);  // the neighbouring lane's
+            // v_perm selects bytes of {first argument : second}: bytes 4..7 are `theirs`, 0..3 are `mine`
+            const uint32_t pair = __builtin_amdgcn_perm(theirs, mine, sel);
+            const int col = run * 32 + 2 * i + (lane & 1), d = lane >> 1;  // column of the block, dword of its 64 elements
+            image[col * 32 + ((((d >> 2) ^ i) & 7) << 2) + (d & 3)] = pair;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < 8; g++) {
+        const int grp = wave * 8 + g;  // eight columns = 1 KB
+        if (kb * 256 + grp * 8 < kcols)
+            *(uint4*)(panel + (((int64_t)kb * 32 + grp) * steps + step) * 1024 + lane * 16) = *(const uint4*)((const uint8_t*)image + grp * 1024 + lane * 16);
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
+// The tile kernel: C[m, col] = sum_t A[m, t] * panel[col][t], plus scale * LA . LB when a LoRA term comes along.
+struct DenseParams {
+    const bf16_t* a;
+    int64_t lda;
+    int contraction;       // real length; steps = ceil / 64; past it A counts as zero
+    const uint8_t* panel;
+    int m, cols;           // cols: columns of this launch
+    void* c;               // bf16 [m][ldc], or fp32
+    int64_t ldc;
+    const float* row_scale;  // accumulate epilogue
+    int splits;            // contraction dealt to this many workgroups (partial epilogue)
+    int64_t split_stride;  // floats between two splits' partial sums
+    // LoRA: la [m, r_pad]; lb [cols][r_pad], or (lb_k_major) [rank][lb_ld] with the columns contiguous
+    const bf16_t *la, *lb;
+    int r_pad, rank, lb_k_major;
+    int64_t lb_ld;
+    float lora_scale;
+};
+enum : int { kDenseStore = 0, kDenseAccum = 1, kDensePartial = 2 };
+
+// Waves form a WM x WN grid, each owning RB x CB blocks of 32 x 32; NS stages of 64 contraction elements in LDS.
+template <int WM, int WN, int RB, int CB, int NS>
+struct DenseTile {
+    static constexpr int kBM = WM * RB * 32, kBN = WN * CB * 32, kWaves = WM * WN, kThreadsWG = 64 * kWaves;
+    static constexpr int kLoadsA = kBM / 8 / kWaves, kLoadsB = kBN / 8 / kWaves, kLoads = kLoadsA + kLoadsB;
+    static constexpr int kStageA = kBM * 128, kStage = (kBM + kBN) * 128;
+    static constexpr int kLdsBytes = NS * kStage;
+    static constexpr int kOutPitch = CB * 64 + 16;  // bytes of a staged output row
+    static_assert(kWaves * 32 * kOutPitch <= kLdsBytes, "output staging");
+};
+
+__device__ __forceinline__ void wait_loads(int n) {  // at most n of this wave's requests outstanding (n known at compile time after inlining)
+    switch (n) {
+        case 0: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
+        case 4: asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); break;
+        case 6: asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); break;
+        case 8: asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); break;
+        case 12: asm volatile("s_waitcnt vmcnt(12)" ::: "memory"); break;
+        default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
+    }
+}
+
+template <class T, int WM, int WN, int RB, int CB, int NS, int EPI>
+__device__ __forceinline__ void dense_body(const DenseParams& p, uint8_t* lds) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave % WM, wn = wave / WM;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+    // tile: every XCD takes a contiguous run of the tiles, ordered in stripes of four row tiles, so that the workgroups
+    // running together on one XCD share row and column operands in its L2
+    const int row_tiles = (p.m + T::kBM - 1) / T::kBM, col_tiles = (p.cols + T::kBN - 1) / T::kBN;
+    const int total = row_tiles * col_tiles * p.splits, per_xcd = (total + 7) >> 3;
+    int t = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || t >= total) return;
+    const int split = t % p.splits;
+    t /= p.splits;
+    constexpr int kStripe = 4;
+    const int stripe = t / (kStripe * col_tiles), in_stripe = t - stripe * kStripe * col_tiles;
+    const int stripe_rows = min(kStripe, row_tiles - stripe * kStripe);
+    const int row0 = (stripe * kStripe + in_stripe % stripe_rows) * T::kBM, col0 = (in_stripe / stripe_rows) * T::kBN;
+    const int rows_valid = min(T::kBM, p.m - row0);
+
+    const int all_steps = (p.contraction + 63) >> 6;
+    const int per_split = (all_steps + p.splits - 1) / p.splits;
+    const int s_begin = split * per_split, s_end = min(all_steps, s_begin + per_split), steps = s_end - s_begin;
+
+    uint32_t a_off[T::kLoadsA];
+    int a_chunk[T::kLoadsA];
+#pragma unroll
+    for (int j = 0; j < T::kLoadsA; j++) {
+        const int r = 8 * (wave + T::kWaves * j) + (lane >> 3);
+        a_chunk[j] = a_slot(r, lane & 7);
+        a_off[j] = ((uint32_t)min(r, rows_valid - 1) * (uint32_t)p.lda + (uint32_t)a_chunk[j] * 8u) * 2u;  // rows past the end repeat the last: never stored
+    }
+    const bf16_t* a_base = p.a + (int64_t)row0 * p.lda + (int64_t)s_begin * 64;
+    const uint8_t* b_base = p.panel + ((int64_t)(col0 / 8 + wave) * all_steps + s_begin) * 1024;
+    const int64_t b_stride = (int64_t)T::kWaves * all_steps * 1024;
+    const int tail = p.contraction & 63;  // live elements of the last step, 0: all
+    // request q of step s into its stage; whole: the step is known not to be the one the contraction ends in
+    auto request = [&](int s, uint32_t stage_off, int q, bool whole) __attribute__((always_inline)) {
+        const uint32_t dst = lds0 + stage_off + (q < T::kLoadsA ? (wave + T::kWaves * q) * 1024 : T::kStageA + (wave + T::kWaves * (q - T::kLoadsA)) * 1024);
+        if (q >= T::kLoadsA) {
+            load16_to_lds(dst, (uint32_t)lane * 16u, b_base + (int64_t)(q - T::kLoadsA) * b_stride + (int64_t)s * 1024);
+        } else if (!whole && tail != 0 && s_begin + s == all_steps - 1) {
+            const void* src = a_chunk[q] * 8 < tail ? (const void*)((const uint8_t*)(a_base + (int64_t)s * 64) + a_off[q]) : (const void*)&d_zero16;
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(dst), "v"(src) : "memory");
+        } else {
+            load16_to_lds(dst, a_off[q], a_base + (int64_t)s * 64);
+        }
+    };
+
+    f32x16_t acc[RB][CB];
+#pragma unroll
+    for (int i = 0; i < RB; i++)
+#pragma unroll
+        for (int j = 0; j < CB; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+
+    const int l32 = lane & 31, half = lane >> 5;
+    if (p.la && split == 0) {  // scale * LA . LB first (operands straight from memory: one to four MFMAs per block and tile)
+        for (int r0 = 0; r0 < p.r_pad; r0 += 16) {
+            bf16x8_t lbv[CB];
+#pragma unroll
+            for (int j = 0; j < CB; j++) {
+                const int col = min(col0 + (wn * CB + j) * 32 + l32, p.cols - 1);
+                if (!p.lb_k_major) {
+                    lbv[j] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(p.lb + (int64_t)col * p.r_pad + r0 + 8 * half));
+                } else {
+                    uint32_t e[8];
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        const int r = r0 + 8 * half + i;
+                        const uint32_t x = p.lb[(int64_t)min(r, p.rank - 1) * p.lb_ld + col];
+                        e[i] = r < p.rank ? x : 0u;
+                    }
+                    lbv[j] = __builtin_bit_cast(bf16x8_t, make_uint4(e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)));
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < RB; i++) {
+                const int row = row0 + min((wm * RB + i) * 32 + l32, rows_valid - 1);
+                const bf16x8_t lav = __builtin_bit_cast(bf16x8_t, *(const uint4*)(p.la + (int64_t)row * p.r_pad + r0 + 8 * half));
+#pragma unroll
+                for (int j = 0; j < CB; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lbv[j], lav, acc[i][j], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < RB; i++)
+#pragma unroll
+            for (int j = 0; j < CB; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[i][j][v] *= p.lora_scale;
+    }
+
+    // Main loop.  A step is four sub-steps of 16 contraction elements; a sub-step's operands are read from LDS during the one
+    // before it.  In front of the last sub-step every wave has the whole stage in registers: there the step's one barrier
+    // stands, behind it the stage is refilled with step s + NS and the next stage's first operands are read, both under
+    // the MFMAs of the last sub-step, so no wave meets the barrier with an idle matrix pipe behind it.
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+        if (s < steps)
+#pragma unroll
+            for (int q = 0; q < T::kLoads; q++) request(s, s * T::kStage, q, false);
+    uint32_t ra[4], rb[4];  // LDS offset of this lane's operand chunk per sub-step
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++) {
+        const uint32_t slot = (uint32_t)(((2 * kk + half) ^ (l32 >> 1)) & 7) * 16u;
+        ra[kk] = (uint32_t)(wm * RB * 32 + l32) * 128u + slot;
+        rb[kk] = (uint32_t)T::kStageA + (uint32_t)(wn * CB * 32 + l32) * 128u + slot;
+    }
+    bf16x8_t fa[2][RB], fb[2][CB];
+    auto read_a = [&](int set, int i, uint32_t stage_off, int kk) __attribute__((always_inline)) {
+        fa[set][i] = *(const bf16x8_t*)(lds + stage_off + ra[kk] + i * 4096);
+    };
+    auto read_b = [&](int set, int j, uint32_t stage_off, int kk) __attribute__((always_inline)) {
+        fb[set][j] = *(const bf16x8_t*)(lds + stage_off + rb[kk] + j * 4096);
+    };
+    if (steps > 0) {
+        if (steps >= NS) wait_loads((NS - 1) * T::kLoads);
+        else wait_loads(0);
+        lds_barrier();
+#pragma unroll
+        for (int j = 0; j < CB; j++) read_b(0, j, 0, 0);
+#pragma unroll
+        for (int i = 0; i < RB; i++) read_a(0, i, 0, 0);
+        uint32_t cur = 0;
+        constexpr int kM = RB * CB, kReads = RB + CB;
+        // one step; WHOLE: step s + NS exists and is not the contraction's last
+        auto step = [&](int s, auto whole_tag) __attribute__((always_inline)) {
+            constexpr bool WHOLE = decltype(whole_tag)::value;
+            const uint32_t nxt = cur == (NS - 1) * T::kStage ? 0u : cur + T::kStage;
+#pragma unroll
+            for (int kk = 0; kk < 4; kk++) {
+                const int set = kk & 1;
+                if (kk == 3) {
+                    // step s + 1 has landed when only the requests of the steps after it are outstanding
+                    if (WHOLE || s + NS - 1 < steps) wait_loads((NS - 2) * T::kLoads);
+                    else wait_loads(0);
+                    lds_barrier();
+                }
+                const uint32_t from = kk == 3 ? nxt : cur;
+#pragma unroll
+                for (int x = 0; x < kM; x++) {
+                    // reads of the next sub-step, ahead of the MFMAs as far as they go: column operands first, in the order
+                    // the MFMAs take them
+                    constexpr int kPer = (kReads + kM - 1) / kM;
+#pragma unroll
+                    for (int q = x * kPer; q < (x + 1) * kPer && q < kReads; q++) {
+                        if (q < CB) read_b(set ^ 1, q, from, (kk + 1) & 3);
+                        else read_a(set ^ 1, q - CB, from, (kk + 1) & 3);
+                    }
+                    if (kk == 3 && (WHOLE || s + NS < steps)) {
+#pragma unroll
+                        for (int q = x * T::kLoads / kM; q < (x + 1) * T::kLoads / kM; q++) request(s + NS, cur, q, WHOLE);
+                    }
+                    acc[x / CB][x % CB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[set][x % CB], fa[set][x / CB], acc[x / CB][x % CB], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            cur = nxt;
+        };
+        int s = 0;
+        for (; s + NS < steps - 1; s++) step(s, std::true_type{});
+        for (; s < steps; s++) step(s, std::false_type{});
+    }
+
+    // acc[i][j][v]: row 32 (wm RB + i) + lane % 32, column 32 (wn CB + j) + 8 (v / 4) + 4 (lane / 32) + v % 4
+    if constexpr (EPI == kDenseStore) {
+        __syncthreads();  // every wave is done with the stages; the (surplus) operand reads have returned
+        uint8_t* stage = lds + wave * 32 * T::kOutPitch;
+        constexpr int kLanesPerRow = CB * 4, kRowsPerStore = 64 / kLanesPerRow;
+        const int cw = col0 + wn * CB * 32;
+        const bool whole = (p.ldc & 7) == 0 && (((uintptr_t)p.c) & 15) == 0;
+#pragma unroll
+        for (int i = 0; i < RB; i++) {
+#pragma unroll
+            for (int j = 0; j < CB; j++)
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    *(uint2*)(stage + l32 * T::kOutPitch + j * 64 + g * 16 + half * 8) =
+                        make_uint2(pack_bf16(acc[i][j][4 * g], acc[i][j][4 * g + 1]), pack_bf16(acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]));
+            const int ch = lane % kLanesPerRow;
+#pragma unroll
+            for (int u = 0; u < 32 / kRowsPerStore; u++) {
+                const int rl = u * kRowsPerStore + lane / kLanesPerRow;
+                const uint4 piece = *(const uint4*)(stage + rl * T::kOutPitch + ch * 16);
+                const int row = (wm * RB + i) * 32 + rl, col = cw + ch * 8;
+                if (row < rows_valid) {
+                    bf16_t* dst = (bf16_t*)p.c + (int64_t)(row0 + row) * p.ldc + col;
+                    if (whole && col + 8 <= p.cols) {
+                        *(uint4*)dst = piece;
+                    } else {
+                        const uint32_t wds[4] = {piece.x, piece.y, piece.z, piece.w};
+#pragma unroll
+                        for (int e = 0; e < 8; e++)
+                            if (col + e < p.cols) dst[e] = (bf16_t)((e & 1) ? wds[e >> 1] >> 16 : wds[e >> 1] & 0xFFFFu);
+                    }
+                }
+            }
+        }
+    } else {
+        float* c = (float*)p.c + (EPI == kDensePartial ? (int64_t)split * p.split_stride : 0);
+#pragma unroll
+        for (int i = 0; i < RB; i++) {
+            const int row = (wm * RB + i) * 32 + l32;
+            if (row >= rows_valid) continue;
+            const float rs = EPI == kDenseAccum && p.row_scale ? p.row_scale[row0 + row] : 1.0f;
+            float* dst_row = c + (int64_t)(row0 + row) * p.ldc;
+#pragma unroll
+            for (int j = 0; j < CB; j++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const int col = col0 + (wn * CB + j) * 32 + g * 8 + half * 4;
+                    if (col >= p.cols) continue;  // (fp32 outputs have a multiple of four columns)
+                    float4* dst = (float4*)(dst_row + col);
+                    float4 o = make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
+                    if (EPI == kDenseAccum) {
+                        const float4 old = *dst;
+                        o.x = fmaf(old.x, rs, o.x), o.y = fmaf(old.y, rs, o.y), o.z = fmaf(old.z, rs, o.z), o.w = fmaf(old.w, rs, o.w);
+                    }
+                    *dst = o;
+                }
+        }
+    }
+}
+
+template <int WM, int WN, int RB, int CB, int NS, int EPI>
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2, 2))) void dense_gemm_kernel(DenseParams p) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t dense_lds[];
+    dense_body<DenseTile<WM, WN, RB, CB, NS>, WM, WN, RB, CB, NS, EPI>(p, dense_lds);
+}
+
+// Split partial sums, added in split order, into an fp32 accumulator: c = c * row_scale + sum (replace: c = sum).
+__global__ __launch_bounds__(256) void dense_reduce_accum_kernel(const float* partial, int64_t split_stride, int splits, int64_t m, int64_t cols, float* c, int64_t ldc,
+                                                                 const float* row_scale, int replace) {
+    const int64_t quads = cols / 4, total = m * quads;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
+        const int64_t row = i / quads, q = i - row * quads;
+        float4 s = ((const float4*)(partial + row * cols))[q];
+        for (int k = 1; k < splits; k++) {
+            const float4 t = ((const float4*)(partial + k * split_stride + row * cols))[q];
+            s.x += t.x, s.y += t.y, s.z += t.z, s.w += t.w;
+        }
+        float4* dst = (float4*)(c + row * ldc) + q;
+        if (!replace) {
+            const float rs = row_scale ? row_scale[row] : 1.0f;
+            const float4 old = *dst;
+            s.x = fmaf(old.x, rs, s.x), s.y = fmaf(old.y, rs, s.y), s.z = fmaf(old.z, rs, s.z), s.w = fmaf(old.w, rs, s.w);
+        }
+        *dst = s;
+    }
+}
+
+// bf16 result of split partial sums, added in split order.
+__global__ __launch_bounds__(256) void dense_reduce_kernel(const float* partial, int64_t split_stride, int splits, int64_t m, int64_t cols, bf16_t* c, int64_t ldc) {
+    const int64_t quads = cols / 4, total = m * quads;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
+        const int64_t row = i / quads, q = i - row * quads;
+        float4 s = ((const float4*)(partial + row * cols))[q];
+        for (int k = 1; k < splits; k++) {
+            const float4 t = ((const float4*)(partial + k * split_stride + row * cols))[q];
+            s.x += t.x, s.y += t.y, s.z += t.z, s.w += t.w;
+        }
+        *(uint2*)(c + row * ldc + q * 4) = make_uint2(pack_bf16(s.x, s.y), pack_bf16(s.z, s.w));
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
+template <int WM, int WN, int RB, int CB, int NS, int EPI>
+static int launch_tile(const DenseParams& p, hipStream_t s) {
+    using T = DenseTile<WM, WN, RB, CB, NS>;
+    const int64_t tiles = (int64_t)((p.m + T::kBM - 1) / T::kBM) * ((p.cols + T::kBN - 1) / T::kBN) * p.splits;
+    const int64_t grid = (tiles + 7) / 8 * 8;
+    if (grid > 0x7FFFFFF0) return set_error(GGQ_ERR_SHAPE, "dense_gemm: too many tiles for one launch");
+    static LdsLimit lim;
+    if (int rc = raise_lds_limit(lim, (const void*)dense_gemm_kernel<WM, WN, RB, CB, NS, EPI>, T::kLdsBytes, "dense_gemm")) return rc;
+    hipLaunchKernelGGL((dense_gemm_kernel<WM, WN, RB, CB, NS, EPI>), dim3((unsigned)grid), dim3(T::kThreadsWG), T::kLdsBytes, s, p);
+    return check_launch("dense_gemm");
+}
+template <int EPI>
+static int launch_shape(int shape, const DenseParams& p, hipStream_t s) {
+    switch (shape) {
+        case 0: return launch_tile<2, 4, 4, 2, 2, EPI>(p, s);   // 256 x 256
+        case 1: return launch_tile<4, 2, 2, 2, 3, EPI>(p, s);   // 256 x 128
+        case 2: return launch_tile<2, 2, 2, 2, 2, EPI>(p, s);   // 128 x 128, two workgroups per compute unit
+        case 3: return launch_tile<2, 2, 1, 1, 4, EPI>(p, s);   // 64 x 64, two workgroups per compute unit
+    }
+    return set_error(GGQ_ERR_SHAPE, "dense_gemm: unknown tile shape");
+}
+static void shape_size(int shape, int& bm, int& bn) {
+    bm = shape <= 1 ? 256 : shape == 2 ? 128 : 64;
+    bn = shape == 0 ? 256 : shape <= 2 ? 128 : 64;
+}
+
+template <int QT>
+static int decode_panel(int mode, const uint8_t* w, int64_t row_bytes, int n, int k, int k0, int kcols, uint8_t* panel, hipStream_t s) {
+    if (mode == kModeNT) {
+        const int64_t units = (int64_t)((n + 7) / 8) * ((k + 255) / 256);
+        hipLaunchKernelGGL(decode_panel_nt_kernel<QT>, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, w, row_bytes, n, k, panel);
+    } else {
+        const int64_t units = (int64_t)((n + 63) / 64) * ((kcols + 255) / 256);
+        hipLaunchKernelGGL(decode_panel_nn_kernel<QT>, dim3((unsigned)units), dim3(256), 0, s, w, row_bytes, n, k, k0, kcols, panel);
+    }
+    return check_launch("decode_panel");
+}
+static int decode_panel_qt(int qt, int mode, const uint8_t* w, int64_t row_bytes, int n, int k, int k0, int kcols, uint8_t* panel, hipStream_t s) {
+    switch (qt) {
+        case kQ8_0: return decode_panel<kQ8_0>(mode, w, row_bytes, n, k, k0, kcols, panel, s);
+        case kQ2_K: return decode_panel<kQ2_K>(mode, w, row_bytes, n, k, k0, kcols, panel, s);
+        case kQ3_K: return decode_panel<kQ3_K>(mode, w, row_bytes, n, k, k0, kcols, panel, s);
+        case kQ4_K: return decode_panel<kQ4_K>(mode, w, row_bytes, n, k, k0, kcols, panel, s);
+        case kQ5_K: return decode_panel<kQ5_K>(mode, w, row_bytes, n, k, k0, kcols, panel, s);
+        case kQ6_K: return decode_panel<kQ6_K>(mode, w, row_bytes, n, k, k0, kcols, panel, s);
+        case kIQ2_XXS: return decode_panel<kIQ2_XXS>(mode, w, row_bytes, n, k, k0, kcols, panel, s);
+    }
+    return set_error(GGQ_ERR_QTYPE, "unsupported GGML type id %d", qt);
+}
+
+// ------------------------------------------------------------------------------------------------
+// Panels of at most this many bytes are decoded at a time: small enough to be read back out of the 256 MB memory-side cache,
+// large enough that a slab's launch fills the chip.  Larger matrices go in slabs of output columns.
+constexpr int64_t kPanelBytes = 64ll << 20;
+constexpr int kMaxSplits = 8;
+
+static int64_t slab_columns(int64_t cols, int64_t contraction) {
+    const int64_t steps = (contraction + 63) / 64, fit = kPanelBytes / (steps * 128) / 256 * 256;
+    const int64_t padded = (cols + 255) / 256 * 256;
+    return std::min(padded, std::max<int64_t>(fit, 256));
+}
+
+// Tile shape and number of contraction splits for an [m, cols] output: the smallest estimate of
+// rounds of workgroups x (steps x time per step + fixed cost), plus the pass that adds split partial sums.
+static std::atomic<int> g_force_shape{-1}, g_force_splits{0};
+void dense_force_shape(int shape, int splits) { g_force_shape.store(shape), g_force_splits.store(splits); }
+
+static void pick_tile(int64_t m, int64_t cols, int64_t steps, bool can_split, int& shape, int& splits) {
+    // microseconds per 64-wide step with every slot of the chip busy, workgroups per chip, and cost of a tile's start and end
+    static const struct { double step, fixed; int slots; } kShape[4] = {{1.15, 6.0, 256}, {0.65, 4.5, 256}, {0.60, 4.0, 512}, {0.25, 3.0, 512}};
+    double best = 1e30;
+    shape = 0, splits = 1;
+    const int forced = g_force_shape.load();
+    for (int sh = 0; sh < 4; sh++) {
+        if (forced >= 0 && sh != forced) continue;
+        int bm, bn;
+        shape_size(sh, bm, bn);
+        const int64_t tiles = ((m + bm - 1) / bm) * ((cols + bn - 1) / bn);
+        for (int sp = 1; sp <= kMaxSplits; sp *= 2) {
+            if (sp > 1 && (!can_split || steps < 4 * sp)) break;
+            if (g_force_splits.load() > 0 && sp != g_force_splits.load() && can_split) continue;
+            const double rounds = (double)((tiles * sp + kShape[sh].slots - 1) / kShape[sh].slots);
+            double t = rounds * (((steps + sp - 1) / sp) * kShape[sh].step + kShape[sh].fixed);
+            if (sp > 1) t += 3.0 + (double)m * cols * 4.0 * (2 * sp) / 4.5e6;
+            if (t < best) best = t, shape = sh, splits = sp;
+        }
+    }
+}
+
+int64_t dense_workspace_bytes(int64_t m, int64_t n, int64_t k) {
+    if (m <= 0 || n <= 0 || k <= 0) return 0;
+    const int64_t nt = slab_columns(n, k) * ((k + 63) / 64) * 128, nn = slab_columns(k, n) * ((n + 63) / 64) * 128;
+    int64_t partial = 0;
+    for (int mode = 0; mode < 2; mode++) {
+        const int64_t cols = mode == kModeNT ? n : k, c = mode == kModeNT ? k : n;
+        const int64_t slab = std::min(cols, slab_columns(cols, c));
+        int shape, splits;
+        pick_tile(m, slab, (c + 63) / 64, slab % 4 == 0, shape, splits);
+        if (splits > 1) partial = std::max(partial, (int64_t)splits * m * slab * 4);
+    }
+    return (std::max(nt, nn) + 255) / 256 * 256 + (partial + 255) / 256 * 256;
+}
+
+bool dense_takes(int mode, int64_t m, int64_t n, int64_t k, const void* a, int64_t lda, bool a_zero_padded) {
+    const int64_t cols = mode == kModeNT ? n : k, contraction = mode == kModeNT ? k : n;
+    return m >= kDenseMinRows && ((uintptr_t)a & 15) == 0 && lda % 8 == 0 && (contraction % 8 == 0 || a_zero_padded) && 256 * lda < (1ll << 30) && cols > 0;
+}
+
+int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s) {
+    const int64_t cols = q.mode == kModeNT ? q.n : q.k, contraction = q.mode == kModeNT ? q.k : q.n, steps = (contraction + 63) / 64;
+    const int64_t slab = slab_columns(cols, contraction), panel_bytes = (slab * steps * 128 + 255) / 256 * 256;
+    if (!ws || ws_bytes < panel_bytes) return set_error(GGQ_ERR_WORKSPACE, "dense_gemm: workspace too small");
+    const int64_t row_bytes = packed_row_bytes(q.qt, q.k);
+    uint8_t* panel = (uint8_t*)ws;
+    TimedScope timed(q.qt, q.mode, q.fp32 ? kEpiAccumF32 : kEpiStore, kShapePanels, s);
+    for (int64_t c0 = 0; c0 < cols; c0 += slab) {
+        const int64_t cn = std::min(slab, cols - c0);
+        const uint8_t* w = (const uint8_t*)q.w + (q.mode == kModeNT ? c0 * row_bytes : 0);
+        if (int rc = decode_panel_qt(q.qt, q.mode, w, row_bytes, (int)(q.mode == kModeNT ? cn : q.n), (int)q.k, (int)(q.mode == kModeNT ? 0 : c0), (int)cn, panel, s)) return rc;
+        DenseParams p{};
+        p.a = (const bf16_t*)q.a, p.lda = q.lda, p.contraction = (int)(q.a_zero_padded ? steps * 64 : contraction);
+        p.panel = panel, p.m = (int)q.m, p.cols = (int)cn, p.ldc = q.ldc, p.row_scale = q.row_scale;
+        if (q.la) {
+            p.la = (const bf16_t*)q.la, p.r_pad = q.r_pad, p.rank = q.rank, p.lora_scale = q.lora_scale, p.lb_k_major = q.mode == kModeNN, p.lb_ld = q.k;
+            p.lb = (const bf16_t*)q.lb + (q.mode == kModeNT ? c0 * q.r_pad : c0);
+        }
+        int shape, splits;
+        const bool can_split = cn % 4 == 0 && q.ldc % 4 == 0 && ((uintptr_t)q.c & 7) == 0;
+        pick_tile(q.m, cn, steps, can_split, shape, splits);
+        if (splits > 1 && ws_bytes < panel_bytes + splits * q.m * cn * 4) splits = 1;
+        p.splits = splits;
+        if (splits > 1) {
+            float* partial = (float*)(panel + panel_bytes);
+            p.c = partial, p.ldc = cn, p.split_stride = q.m * cn;
+            if (int rc = launch_shape<kDensePartial>(shape, p, s)) return rc;
+            const int64_t work = q.m * (cn / 4);
+            if (q.fp32)
+                hipLaunchKernelGGL(dense_reduce_accum_kernel, dim3((unsigned)std::min<int64_t>((work + 255) / 256, 4096)), dim3(256), 0, s, partial, p.split_stride, splits, q.m,
+                                   cn, (float*)q.c + c0, q.ldc, q.row_scale, q.accumulate ? 0 : 1);
+            else hipLaunchKernelGGL(dense_reduce_kernel, dim3((unsigned)std::min<int64_t>((work + 255) / 256, 4096)), dim3(256), 0, s, partial, p.split_stride, splits, q.m, cn,
+                               (bf16_t*)q.c + c0, q.ldc);
+            if (int rc = check_launch("dense_reduce")) return rc;
+        } else if (q.fp32) {
+            p.c = (float*)q.c + c0;
+            if (int rc = q.accumulate ? launch_shape<kDenseAccum>(shape, p, s) : launch_shape<kDensePartial>(shape, p, s)) return rc;
+        } else {
+            p.c = (bf16_t*)q.c + c0;
+            if (int rc = launch_shape<kDenseStore>(shape, p, s)) return rc;
+        }
+    }
+    return GGQ_OK;
+}
+
+}  // namespace ggq

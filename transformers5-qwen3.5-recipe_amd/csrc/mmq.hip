@@ -174,6 +174,18 @@ int profile_end(float* ms, int* qt, int* mode, int* epi, int* shape, int capacit
     return n;
 }
 
+TimedScope::TimedScope(int qt, int mode, int epi, int shape, hipStream_t s) : stream_(s) {
+    if (!g_timing || g_timed_count >= kMaxTimedLaunches) return;
+    TimedLaunch* t = &g_timed[g_timed_count];
+    if (hipEventCreate(&t->start) != hipSuccess || hipEventCreate(&t->stop) != hipSuccess) return;
+    t->qt = qt, t->mode = mode, t->epi = epi, t->shape = shape;
+    slot_ = g_timed_count++;
+    (void)hipEventRecord(t->start, s);
+}
+TimedScope::~TimedScope() {
+    if (slot_ >= 0) (void)hipEventRecord(g_timed[slot_].stop, stream_);
+}
+
 template <int QT, int MODE, int EPI, int SH>
 static int launch_one(const MmqParams& p, hipStream_t s) {
     const int col_tiles = (MODE == kModeNT ? p.nseg : 1) * p.col_tiles_per_seg;

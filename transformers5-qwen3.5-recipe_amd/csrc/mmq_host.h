@@ -123,6 +123,41 @@ int launch_mmq_mixed(int qt, int mode, const MmqParams& p, hipStream_t s);  // Q
 int launch_mmq_small(const MmqParams& p, hipStream_t s);  // IQ2_XXS forward, store epilogue, tiles of kSmallBM rows
 int init_params(MmqParams& p, int qt, int mode, int m, int n, int k, int nseg, int shape = kShapeTall);
 
+// Event pair around the launches of its lifetime, when launches are being timed (profile_begin).
+class TimedScope {
+public:
+    TimedScope(int qt, int mode, int epi, int shape, hipStream_t s);
+    ~TimedScope();
+private:
+    int slot_ = -1;
+    hipStream_t stream_;
+};
+
+// Dense launches over decoded panels (dense_gemm.hip).
+constexpr int kShapePanels = 6;  // (profile records only)
+// Below this many rows a decoded panel is read too few times to pay for writing it.
+constexpr int64_t kDenseMinRows = 48;
+struct DenseCall {
+    int qt, mode;
+    int64_t m, n, k;      // W is [n, k]
+    const void* a;        // NT [m, k], NN [m, n]; 16-byte aligned rows
+    int64_t lda;
+    const void* w;
+    void* c;
+    int64_t ldc;
+    bool a_zero_padded;   // rows of a hold zeros from the contraction's end to the next multiple of 64
+    bool fp32;            // c is fp32 (a multiple of four columns)
+    bool accumulate;      // fp32: c = c * row_scale[m] + result instead of c = result
+    const float* row_scale;
+    const void *la, *lb;  // LoRA: la [m, r_pad]; lb NT [n, r_pad], NN the factor A [rank, k]
+    int r_pad, rank;
+    float lora_scale;
+};
+bool dense_takes(int mode, int64_t m, int64_t n, int64_t k, const void* a, int64_t lda, bool a_zero_padded = false);
+int64_t dense_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s);
+void dense_force_shape(int shape, int splits);  // test aid: -1 = the automatic choice
+
 int pad_factor(const bf16_t* src, bf16_t* dst, int64_t experts, int c, int r, int r_pad, bool transpose, hipStream_t s);
 int transpose_factor(const bf16_t* src, bf16_t* dst, int64_t experts, int c, int r, hipStream_t s);
 int skinny_nt(const SkinnyNtParams& p, int r_pad, int grid_tiles, hipStream_t s);
