@@ -6,11 +6,12 @@
 // one write and a few reads of 2 bytes per weight, which stay in the memory-side cache, and leaves a loop whose only work
 // per step is LDS reads and MFMAs.
 //
-// Scratch layout ("panels"): the output columns in groups of eight, each group holding its contraction in steps of 64:
-//   panel[column / 8][step][8 columns][64 contraction elements], the eight 16-byte chunks of a column XOR-swizzled (a_slot),
-// so that one 1 KB request moves one group's step to LDS as it is, and the operand reads meet no bank conflict.  The forward
-// panel's columns are weight rows; the grad-input panel's columns are the weights' k and its contraction the weight rows
-// (the decoder transposes through LDS), so both directions run the same kernel.
+// Scratch layout ("panel"): weight rows in groups of eight, each group holding its k in blocks of 64:
+//   panel[row / 8][k / 64][8 rows][64 elements], the eight 16-byte chunks of a row XOR-swizzled (panel_slot),
+// so that one 1 KB request moves a group's block to LDS as it is.  Forward reads it as [output column][contraction] with
+// 16-byte operand reads; grad-input reads the same panel as [contraction][output column] with transposing 8-byte reads
+// (ds_read_b64_tr_b16).  The swizzle keeps both free of bank conflicts: sixteen consecutive rows at one chunk cover all
+// bank groups, and four consecutive rows at an aligned pair of chunks cover four distinct 32-byte bank runs of each half.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -30,6 +31,12 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 // ------------------------------------------------------------------------------------------------
 // Decoding passes.  HBM-bound: packed bytes in, two bytes per weight out.
 
+typedef short v4i16_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) v4i16_t* lds_v4i16_ptr;
+
+// What chunk index of row r is XOR-ed with (r mod 16 counts).
+__device__ __forceinline__ int panel_swizzle(int r) { return (((r >> 1) & 3) << 1) | ((r >> 3) & 1); }
+
 template <int QT>
 __device__ __forceinline__ const uint2* stage_tables(uint32_t* lds, int tid, int threads) {
     if constexpr (QT == kIQ2_XXS) {
@@ -39,25 +46,31 @@ __device__ __forceinline__ const uint2* stage_tables(uint32_t* lds, int tid, int
     return (const uint2*)lds;
 }
 
-// Forward panel.  One wave per (group of eight weight rows, 256 elements of k): lane (row lane / 8, run lane % 8) decodes one
-// 32-element run; the eight lanes of a row read adjacent bytes.  The wave's 4 KB go through LDS and leave in whole 1 KB pieces.
+// One wave per (group of eight weight rows, 256 elements of k): lane (row lane / 8, run lane % 8) decodes one 32-element run;
+// the eight lanes of a row read adjacent bytes.  The wave's 4 KB go through LDS and leave in whole 1 KB pieces.  The panel
+// holds k0 .. k0 + kcols - 1 of every row; rows from n up to the next multiple of 64 are zeros (a contraction over the rows
+// runs to there).
 template <int QT>
-__global__ __launch_bounds__(256) void decode_panel_nt_kernel(const uint8_t* w, int64_t row_bytes, int n, int k, uint8_t* panel) {
+__global__ __launch_bounds__(256) void decode_panel_kernel(const uint8_t* w, int64_t row_bytes, int n, int k, int k0, int kcols, uint8_t* panel) {
     __shared__ __attribute__((aligned(16))) uint8_t out_lds[4][4096];
     __shared__ uint32_t tables[QT == kIQ2_XXS ? Fmt<kIQ2_XXS>::kTableWords : 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint2* tab = stage_tables<QT>(tables, threadIdx.x, 256);
-    const int kblocks = (k + 255) >> 8, steps = k >> 6;
+    const int kblocks = (kcols + 255) >> 8, steps = kcols >> 6;
     const int64_t unit = (int64_t)blockIdx.x * 4 + wave;
     const int group = (int)(unit / kblocks), kb = (int)(unit - (int64_t)group * kblocks);
-    if (group * 8 >= n) return;
-    const int row = min(group * 8 + (lane >> 3), n - 1), ksub = kb * 8 + (lane & 7);
+    if (group * 8 >= ((n + 63) & ~63)) return;
+    const int row = group * 8 + (lane >> 3), ksub = min((k0 >> 5) + kb * 8 + (lane & 7), (k >> 5) - 1);
     const int live_steps = min(4, steps - kb * 4);
     typename Fmt<QT>::Raw raw;
     uint32_t v[16];
-    Fmt<QT>::load(raw, w + (int64_t)row * row_bytes, min(ksub, (k >> 5) - 1));
+    Fmt<QT>::load(raw, w + (int64_t)min(row, n - 1) * row_bytes, ksub);
     Fmt<QT>::decode(raw, ksub, v, tab);
-    const int r8 = lane >> 3, sw = ((group * 8 + r8) >> 1) & 7, st = (lane & 7) >> 1, c0 = (lane & 1) * 4;
+    if (row >= n) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) v[i] = 0u;
+    }
+    const int r8 = lane >> 3, sw = panel_swizzle(row), st = (lane & 7) >> 1, c0 = (lane & 1) * 4;
     uint8_t* mine = out_lds[wave] + st * 1024 + r8 * 128;
 #pragma unroll
     for (int i = 0; i < 4; i++) *(uint4*)(mine + ((c0 + i) ^ sw) * 16) = make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
@@ -70,56 +83,14 @@ __global__ __launch_bounds__(256) void decode_panel_nt_kernel(const uint8_t* w, 
     }
 }
 
-// Grad-input panel of the columns [k0, k0 + kcols).  One workgroup per (64 weight rows, 256 elements of k): a lane decodes
-// two 32-element runs of one weight row (lanes = consecutive rows); neighbouring rows trade halves through a data-parallel
-// move so that every LDS write carries two adjacent contraction elements of one column; the 32 KB block then is the panel's
-// image and leaves in 1 KB pieces.  Weight rows past n count as zero (a contraction runs to the next multiple of 64).
-template <int QT>
-__global__ __launch_bounds__(256) void decode_panel_nn_kernel(const uint8_t* w, int64_t row_bytes, int n, int k, int k0, int kcols, uint8_t* panel) {
-    __shared__ __attribute__((aligned(16))) uint32_t image[256 * 32];
-    __shared__ uint32_t tables[QT == kIQ2_XXS ? Fmt<kIQ2_XXS>::kTableWords : 1];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint2* tab = stage_tables<QT>(tables, threadIdx.x, 256);
-    const int kblocks = (kcols + 255) >> 8, steps = (n + 63) >> 6;
-    const int step = blockIdx.x / kblocks, kb = blockIdx.x - step * kblocks;
-    const int row = step * 64 + lane;
-    const uint8_t* src = w + (int64_t)min(row, n - 1) * row_bytes;
-    const int kk0 = k0 + kb * 256;
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-        const int run = wave * 2 + u;  // of the block's eight
-        const int ksub = min((kk0 >> 5) + run, (k >> 5) - 1);
-        typename Fmt<QT>::Raw raw;
-        uint32_t v[16];
-        Fmt<QT>::load(raw, src, ksub);
-        Fmt<QT>::decode(raw, ksub, v, tab);
-        const uint32_t sel = (lane & 1) ? 0x03020706u : 0x05040100u;  // odd rows: {mine.hi : theirs.hi}, even rows: {theirs.lo : mine.lo}
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const uint32_t mine = row < n ? v[i] : 0u;
-            const uint32_t theirs = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, 0xB1, 0xF, 0xF, true);  // the neighbouring lane's
-            // v_perm selects bytes of {first argument : second}: bytes 4..7 are `theirs`, 0..3 are `mine`
-            const uint32_t pair = __builtin_amdgcn_perm(theirs, mine, sel);
-            const int col = run * 32 + 2 * i + (lane & 1), d = lane >> 1;  // column of the block, dword of its 64 elements
-            image[col * 32 + ((((d >> 2) ^ i) & 7) << 2) + (d & 3)] = pair;
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int g = 0; g < 8; g++) {
-        const int grp = wave * 8 + g;  // eight columns = 1 KB
-        if (kb * 256 + grp * 8 < kcols)
-            *(uint4*)(panel + (((int64_t)kb * 32 + grp) * steps + step) * 1024 + lane * 16) = *(const uint4*)((const uint8_t*)image + grp * 1024 + lane * 16);
-    }
-}
-
 // ------------------------------------------------------------------------------------------------
-// The tile kernel: C[m, col] = sum_t A[m, t] * panel[col][t], plus scale * LA . LB when a LoRA term comes along.
+// The tile kernel: C[m, col] = sum_t A[m, t] * W(col, t), plus scale * LA . LB when a LoRA term comes along.
 struct DenseParams {
     const bf16_t* a;
     int64_t lda;
     int contraction;       // real length; steps = ceil / 64; past it A counts as zero
     const uint8_t* panel;
+    int panel_steps;       // 64-element blocks of a panel row
     int m, cols;           // cols: columns of this launch
     void* c;               // bf16 [m][ldc], or fp32
     int64_t ldc;
@@ -156,7 +127,7 @@ __device__ __forceinline__ void wait_loads(int n) {  // at most n of this wave's
     }
 }
 
-template <class T, int WM, int WN, int RB, int CB, int NS, int EPI>
+template <class T, int MODE, int WM, int WN, int RB, int CB, int NS, int EPI>
 __device__ __forceinline__ void dense_body(const DenseParams& p, uint8_t* lds) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -185,18 +156,32 @@ __device__ __forceinline__ void dense_body(const DenseParams& p, uint8_t* lds) {
 #pragma unroll
     for (int j = 0; j < T::kLoadsA; j++) {
         const int r = 8 * (wave + T::kWaves * j) + (lane >> 3);
-        a_chunk[j] = a_slot(r, lane & 7);
+        a_chunk[j] = (lane & 7) ^ panel_swizzle(r);
         a_off[j] = ((uint32_t)min(r, rows_valid - 1) * (uint32_t)p.lda + (uint32_t)a_chunk[j] * 8u) * 2u;  // rows past the end repeat the last: never stored
     }
     const bf16_t* a_base = p.a + (int64_t)row0 * p.lda + (int64_t)s_begin * 64;
-    const uint8_t* b_base = p.panel + ((int64_t)(col0 / 8 + wave) * all_steps + s_begin) * 1024;
-    const int64_t b_stride = (int64_t)T::kWaves * all_steps * 1024;
+    // column operand requests: forward, eight columns (a row group) x 64 contraction elements each; grad-input, eight
+    // contraction rows x 64 columns, block b of the tile's columns behind block b - 1 in LDS
+    const uint8_t* b_src[T::kLoadsB];
+    int64_t b_step;
+    if (MODE == kModeNT) {
+        b_step = 1024;
+#pragma unroll
+        for (int j = 0; j < T::kLoadsB; j++) b_src[j] = p.panel + ((int64_t)(col0 / 8 + wave + T::kWaves * j) * all_steps + s_begin) * 1024;
+    } else {
+        b_step = (int64_t)p.panel_steps * 8 * 1024;
+#pragma unroll
+        for (int j = 0; j < T::kLoadsB; j++) {
+            const int u = wave + T::kWaves * j, block = min(col0 / 64 + (u >> 3), p.panel_steps - 1);  // (columns past the end are never stored)
+            b_src[j] = p.panel + ((int64_t)(s_begin * 8 + (u & 7)) * p.panel_steps + block) * 1024;
+        }
+    }
     const int tail = p.contraction & 63;  // live elements of the last step, 0: all
     // request q of step s into its stage; whole: the step is known not to be the one the contraction ends in
     auto request = [&](int s, uint32_t stage_off, int q, bool whole) __attribute__((always_inline)) {
         const uint32_t dst = lds0 + stage_off + (q < T::kLoadsA ? (wave + T::kWaves * q) * 1024 : T::kStageA + (wave + T::kWaves * (q - T::kLoadsA)) * 1024);
         if (q >= T::kLoadsA) {
-            load16_to_lds(dst, (uint32_t)lane * 16u, b_base + (int64_t)(q - T::kLoadsA) * b_stride + (int64_t)s * 1024);
+            load16_to_lds(dst, (uint32_t)lane * 16u, b_src[q - T::kLoadsA] + s * b_step);
         } else if (!whole && tail != 0 && s_begin + s == all_steps - 1) {
             const void* src = a_chunk[q] * 8 < tail ? (const void*)((const uint8_t*)(a_base + (int64_t)s * 64) + a_off[q]) : (const void*)&d_zero16;
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(dst), "v"(src) : "memory");
@@ -258,19 +243,38 @@ __device__ __forceinline__ void dense_body(const DenseParams& p, uint8_t* lds) {
         if (s < steps)
 #pragma unroll
             for (int q = 0; q < T::kLoads; q++) request(s, s * T::kStage, q, false);
-    uint32_t ra[4], rb[4];  // LDS offset of this lane's operand chunk per sub-step
+    // LDS offsets of this lane's operand chunks: rows by sub-step; columns by sub-step (forward), or by half of the eight
+    // contraction rows and column block (grad-input: lane s of sixteen points at row s / 4, columns 4 (s % 4) .. + 3)
+    uint32_t ra[4], rb[MODE == kModeNT ? 4 : 2 * CB];
 #pragma unroll
     for (int kk = 0; kk < 4; kk++) {
-        const uint32_t slot = (uint32_t)(((2 * kk + half) ^ (l32 >> 1)) & 7) * 16u;
+        const uint32_t slot = (uint32_t)((2 * kk + half) ^ panel_swizzle(l32)) * 16u;
         ra[kk] = (uint32_t)(wm * RB * 32 + l32) * 128u + slot;
-        rb[kk] = (uint32_t)T::kStageA + (uint32_t)(wn * CB * 32 + l32) * 128u + slot;
+        if (MODE == kModeNT) rb[kk] = (uint32_t)T::kStageA + (uint32_t)(wn * CB * 32 + l32) * 128u + slot;
+    }
+    if (MODE == kModeNN) {
+        const int src = lane & 15, sub = (lane >> 4) & 1;
+#pragma unroll
+        for (int j = 0; j < CB; j++)
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const int col = (wn * CB + j) * 32 + 16 * sub + 4 * (src & 3), row = 8 * half + 4 * t + (src >> 2);
+                rb[2 * j + t] = (uint32_t)T::kStageA + (uint32_t)(col >> 6) * 8192u + (uint32_t)row * 128u +
+                                (uint32_t)(((col & 63) >> 3) ^ panel_swizzle(row)) * 16u + (uint32_t)(src & 1) * 8u;
+            }
     }
     bf16x8_t fa[2][RB], fb[2][CB];
     auto read_a = [&](int set, int i, uint32_t stage_off, int kk) __attribute__((always_inline)) {
         fa[set][i] = *(const bf16x8_t*)(lds + stage_off + ra[kk] + i * 4096);
     };
     auto read_b = [&](int set, int j, uint32_t stage_off, int kk) __attribute__((always_inline)) {
-        fb[set][j] = *(const bf16x8_t*)(lds + stage_off + rb[kk] + j * 4096);
+        if constexpr (MODE == kModeNT) {
+            fb[set][j] = *(const bf16x8_t*)(lds + stage_off + rb[kk] + j * 4096);
+        } else {
+            const v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)(lds + stage_off + rb[2 * j] + kk * 2048));
+            const v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)(lds + stage_off + rb[2 * j + 1] + kk * 2048));
+            fb[set][j] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
     };
     if (steps > 0) {
         if (steps >= NS) wait_loads((NS - 1) * T::kLoads);
@@ -381,10 +385,10 @@ __device__ __forceinline__ void dense_body(const DenseParams& p, uint8_t* lds) {
     }
 }
 
-template <int WM, int WN, int RB, int CB, int NS, int EPI>
+template <int MODE, int WM, int WN, int RB, int CB, int NS, int EPI>
 __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2, 2))) void dense_gemm_kernel(DenseParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t dense_lds[];
-    dense_body<DenseTile<WM, WN, RB, CB, NS>, WM, WN, RB, CB, NS, EPI>(p, dense_lds);
+    dense_body<DenseTile<WM, WN, RB, CB, NS>, MODE, WM, WN, RB, CB, NS, EPI>(p, dense_lds);
 }
 
 // Split partial sums, added in split order, into an fp32 accumulator: c = c * row_scale + sum (replace: c = sum).
@@ -423,26 +427,30 @@ __global__ __launch_bounds__(256) void dense_reduce_kernel(const float* partial,
 }
 
 // ------------------------------------------------------------------------------------------------
-template <int WM, int WN, int RB, int CB, int NS, int EPI>
+template <int MODE, int WM, int WN, int RB, int CB, int NS, int EPI>
 static int launch_tile(const DenseParams& p, hipStream_t s) {
     using T = DenseTile<WM, WN, RB, CB, NS>;
     const int64_t tiles = (int64_t)((p.m + T::kBM - 1) / T::kBM) * ((p.cols + T::kBN - 1) / T::kBN) * p.splits;
     const int64_t grid = (tiles + 7) / 8 * 8;
     if (grid > 0x7FFFFFF0) return set_error(GGQ_ERR_SHAPE, "dense_gemm: too many tiles for one launch");
     static LdsLimit lim;
-    if (int rc = raise_lds_limit(lim, (const void*)dense_gemm_kernel<WM, WN, RB, CB, NS, EPI>, T::kLdsBytes, "dense_gemm")) return rc;
-    hipLaunchKernelGGL((dense_gemm_kernel<WM, WN, RB, CB, NS, EPI>), dim3((unsigned)grid), dim3(T::kThreadsWG), T::kLdsBytes, s, p);
+    if (int rc = raise_lds_limit(lim, (const void*)dense_gemm_kernel<MODE, WM, WN, RB, CB, NS, EPI>, T::kLdsBytes, "dense_gemm")) return rc;
+    hipLaunchKernelGGL((dense_gemm_kernel<MODE, WM, WN, RB, CB, NS, EPI>), dim3((unsigned)grid), dim3(T::kThreadsWG), T::kLdsBytes, s, p);
     return check_launch("dense_gemm");
 }
-template <int EPI>
-static int launch_shape(int shape, const DenseParams& p, hipStream_t s) {
+template <int MODE, int EPI>
+static int launch_shape_mode(int shape, const DenseParams& p, hipStream_t s) {
     switch (shape) {
-        case 0: return launch_tile<2, 4, 4, 2, 2, EPI>(p, s);   // 256 x 256
-        case 1: return launch_tile<4, 2, 2, 2, 3, EPI>(p, s);   // 256 x 128
-        case 2: return launch_tile<2, 2, 2, 2, 2, EPI>(p, s);   // 128 x 128, two workgroups per compute unit
-        case 3: return launch_tile<2, 2, 1, 1, 4, EPI>(p, s);   // 64 x 64, two workgroups per compute unit
+        case 0: return launch_tile<MODE, 2, 4, 4, 2, 2, EPI>(p, s);   // 256 x 256
+        case 1: return launch_tile<MODE, 4, 2, 2, 2, 3, EPI>(p, s);   // 256 x 128
+        case 2: return launch_tile<MODE, 2, 2, 2, 2, 2, EPI>(p, s);   // 128 x 128, two workgroups per compute unit
+        case 3: return launch_tile<MODE, 2, 2, 1, 1, 4, EPI>(p, s);   // 64 x 64, two workgroups per compute unit
     }
     return set_error(GGQ_ERR_SHAPE, "dense_gemm: unknown tile shape");
+}
+template <int EPI>
+static int launch_shape(int mode, int shape, const DenseParams& p, hipStream_t s) {
+    return mode == kModeNT ? launch_shape_mode<kModeNT, EPI>(shape, p, s) : launch_shape_mode<kModeNN, EPI>(shape, p, s);
 }
 static void shape_size(int shape, int& bm, int& bn) {
     bm = shape <= 1 ? 256 : shape == 2 ? 128 : 64;
@@ -450,25 +458,20 @@ static void shape_size(int shape, int& bm, int& bn) {
 }
 
 template <int QT>
-static int decode_panel(int mode, const uint8_t* w, int64_t row_bytes, int n, int k, int k0, int kcols, uint8_t* panel, hipStream_t s) {
-    if (mode == kModeNT) {
-        const int64_t units = (int64_t)((n + 7) / 8) * ((k + 255) / 256);
-        hipLaunchKernelGGL(decode_panel_nt_kernel<QT>, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, w, row_bytes, n, k, panel);
-    } else {
-        const int64_t units = (int64_t)((n + 63) / 64) * ((kcols + 255) / 256);
-        hipLaunchKernelGGL(decode_panel_nn_kernel<QT>, dim3((unsigned)units), dim3(256), 0, s, w, row_bytes, n, k, k0, kcols, panel);
-    }
+static int launch_decode_panel(const uint8_t* w, int64_t row_bytes, int n, int k, int k0, int kcols, uint8_t* panel, hipStream_t s) {
+    const int64_t units = (int64_t)((n + 63) / 64 * 8) * ((kcols + 255) / 256);
+    hipLaunchKernelGGL(decode_panel_kernel<QT>, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, w, row_bytes, n, k, k0, kcols, panel);
     return check_launch("decode_panel");
 }
-static int decode_panel_qt(int qt, int mode, const uint8_t* w, int64_t row_bytes, int n, int k, int k0, int kcols, uint8_t* panel, hipStream_t s) {
+static int decode_panel(int qt, const uint8_t* w, int64_t row_bytes, int n, int k, int k0, int kcols, uint8_t* panel, hipStream_t s) {
     switch (qt) {
-        case kQ8_0: return decode_panel<kQ8_0>(mode, w, row_bytes, n, k, k0, kcols, panel, s);
-        case kQ2_K: return decode_panel<kQ2_K>(mode, w, row_bytes, n, k, k0, kcols, panel, s);
-        case kQ3_K: return decode_panel<kQ3_K>(mode, w, row_bytes, n, k, k0, kcols, panel, s);
-        case kQ4_K: return decode_panel<kQ4_K>(mode, w, row_bytes, n, k, k0, kcols, panel, s);
-        case kQ5_K: return decode_panel<kQ5_K>(mode, w, row_bytes, n, k, k0, kcols, panel, s);
-        case kQ6_K: return decode_panel<kQ6_K>(mode, w, row_bytes, n, k, k0, kcols, panel, s);
-        case kIQ2_XXS: return decode_panel<kIQ2_XXS>(mode, w, row_bytes, n, k, k0, kcols, panel, s);
+        case kQ8_0: return launch_decode_panel<kQ8_0>(w, row_bytes, n, k, k0, kcols, panel, s);
+        case kQ2_K: return launch_decode_panel<kQ2_K>(w, row_bytes, n, k, k0, kcols, panel, s);
+        case kQ3_K: return launch_decode_panel<kQ3_K>(w, row_bytes, n, k, k0, kcols, panel, s);
+        case kQ4_K: return launch_decode_panel<kQ4_K>(w, row_bytes, n, k, k0, kcols, panel, s);
+        case kQ5_K: return launch_decode_panel<kQ5_K>(w, row_bytes, n, k, k0, kcols, panel, s);
+        case kQ6_K: return launch_decode_panel<kQ6_K>(w, row_bytes, n, k, k0, kcols, panel, s);
+        case kIQ2_XXS: return launch_decode_panel<kIQ2_XXS>(w, row_bytes, n, k, k0, kcols, panel, s);
     }
     return set_error(GGQ_ERR_QTYPE, "unsupported GGML type id %d", qt);
 }
@@ -476,7 +479,7 @@ static int decode_panel_qt(int qt, int mode, const uint8_t* w, int64_t row_bytes
 // ------------------------------------------------------------------------------------------------
 // Panels of at most this many bytes are decoded at a time: small enough to be read back out of the 256 MB memory-side cache,
 // large enough that a slab's launch fills the chip.  Larger matrices go in slabs of output columns.
-constexpr int64_t kPanelBytes = 64ll << 20;
+constexpr int64_t kPanelBytes = 128ll << 20;
 constexpr int kMaxSplits = 8;
 
 static int64_t slab_columns(int64_t cols, int64_t contraction) {
@@ -484,6 +487,9 @@ static int64_t slab_columns(int64_t cols, int64_t contraction) {
     const int64_t padded = (cols + 255) / 256 * 256;
     return std::min(padded, std::max<int64_t>(fit, 256));
 }
+
+// Whether both directions of an [n, k] matrix run over one panel of all of it.
+bool dense_panel_whole(int64_t n, int64_t k) { return slab_columns(n, k) >= n && slab_columns(k, n) >= k; }
 
 // Tile shape and number of contraction splits for an [m, cols] output: the smallest estimate of
 // rounds of workgroups x (steps x time per step + fixed cost), plus the pass that adds split partial sums.
@@ -541,10 +547,12 @@ int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s) {
     for (int64_t c0 = 0; c0 < cols; c0 += slab) {
         const int64_t cn = std::min(slab, cols - c0);
         const uint8_t* w = (const uint8_t*)q.w + (q.mode == kModeNT ? c0 * row_bytes : 0);
-        if (int rc = decode_panel_qt(q.qt, q.mode, w, row_bytes, (int)(q.mode == kModeNT ? cn : q.n), (int)q.k, (int)(q.mode == kModeNT ? 0 : c0), (int)cn, panel, s)) return rc;
+        const int kcols = (int)(q.mode == kModeNT ? q.k : cn);
+        if (!q.panel_ready)
+            if (int rc = decode_panel(q.qt, w, row_bytes, (int)(q.mode == kModeNT ? cn : q.n), (int)q.k, (int)(q.mode == kModeNT ? 0 : c0), kcols, panel, s)) return rc;
         DenseParams p{};
         p.a = (const bf16_t*)q.a, p.lda = q.lda, p.contraction = (int)(q.a_zero_padded ? steps * 64 : contraction);
-        p.panel = panel, p.m = (int)q.m, p.cols = (int)cn, p.ldc = q.ldc, p.row_scale = q.row_scale;
+        p.panel = panel, p.panel_steps = kcols / 64, p.m = (int)q.m, p.cols = (int)cn, p.ldc = q.ldc, p.row_scale = q.row_scale;
         if (q.la) {
             p.la = (const bf16_t*)q.la, p.r_pad = q.r_pad, p.rank = q.rank, p.lora_scale = q.lora_scale, p.lb_k_major = q.mode == kModeNN, p.lb_ld = q.k;
             p.lb = (const bf16_t*)q.lb + (q.mode == kModeNT ? c0 * q.r_pad : c0);
@@ -557,7 +565,7 @@ int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s) {
         if (splits > 1) {
             float* partial = (float*)(panel + panel_bytes);
             p.c = partial, p.ldc = cn, p.split_stride = q.m * cn;
-            if (int rc = launch_shape<kDensePartial>(shape, p, s)) return rc;
+            if (int rc = launch_shape<kDensePartial>(q.mode, shape, p, s)) return rc;
             const int64_t work = q.m * (cn / 4);
             if (q.fp32)
                 hipLaunchKernelGGL(dense_reduce_accum_kernel, dim3((unsigned)std::min<int64_t>((work + 255) / 256, 4096)), dim3(256), 0, s, partial, p.split_stride, splits, q.m,
@@ -567,10 +575,10 @@ int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s) {
             if (int rc = check_launch("dense_reduce")) return rc;
         } else if (q.fp32) {
             p.c = (float*)q.c + c0;
-            if (int rc = q.accumulate ? launch_shape<kDenseAccum>(shape, p, s) : launch_shape<kDensePartial>(shape, p, s)) return rc;
+            if (int rc = q.accumulate ? launch_shape<kDenseAccum>(q.mode, shape, p, s) : launch_shape<kDensePartial>(q.mode, shape, p, s)) return rc;
         } else {
             p.c = (bf16_t*)q.c + c0;
-            if (int rc = launch_shape<kDenseStore>(shape, p, s)) return rc;
+            if (int rc = launch_shape<kDenseStore>(q.mode, shape, p, s)) return rc;
         }
     }
     return GGQ_OK;

@@ -56,10 +56,11 @@ __global__ __launch_bounds__(1024) void ce_row_scale_kernel(const int64_t* label
     if (threadIdx.x == 0 && status) status[0] = n, status[1] = partial_bad[0];
 }
 
-// One workgroup per row.  The row's block of logits is read once and kept in registers (up to four 16-byte pieces per lane);
+// One workgroup per row.  The row's block of logits is read once and kept in registers (four 16-byte pieces per lane);
 // it becomes p = exp(logit - running max) in place (bf16), alpha = exp(old max - new max) rescales what was accumulated so
 // far.  HBM-bound: 27.7 us per 4096 x 8192 block when the block was read twice.
-constexpr int kStreamThreads = 1024, kStreamPieces = kMaxVocabBlock / 8 / kStreamThreads;
+constexpr int kStreamPieces = 4;
+template <int kStreamThreads>
 __global__ __launch_bounds__(kStreamThreads) void ce_stream_block_kernel(bf16_t* slab, int64_t ld, int nb, int64_t v0, const int64_t* labels, float* run_max,
                                                                          float* run_sum, float* target, float* alpha, int64_t* run_arg) {
     constexpr int kWaves = kStreamThreads / 64;
@@ -144,6 +145,17 @@ __global__ void fill_f32_kernel(float* p, int64_t n, float v) {
 static unsigned grid1d(int64_t n) {
     int64_t g = (n + 255) / 256;
     return (unsigned)(g < 1 ? 1 : (g > 16384 ? 16384 : g));
+}
+
+static void launch_stream_block(int rows, bf16_t* slab, int64_t ld, int nb, int64_t v0, const int64_t* labels, float* run_max, float* run_sum, float* target, float* alpha,
+                                int64_t* run_arg, hipStream_t s) {
+    static_assert(1024 * kStreamPieces * 8 >= kMaxVocabBlock, "a block fits the registers of one workgroup");
+    if (nb <= 256 * kStreamPieces * 8)
+        hipLaunchKernelGGL(ce_stream_block_kernel<256>, dim3((unsigned)rows), dim3(256), 0, s, slab, ld, nb, v0, labels, run_max, run_sum, target, alpha, run_arg);
+    else if (nb <= 512 * kStreamPieces * 8)
+        hipLaunchKernelGGL(ce_stream_block_kernel<512>, dim3((unsigned)rows), dim3(512), 0, s, slab, ld, nb, v0, labels, run_max, run_sum, target, alpha, run_arg);
+    else
+        hipLaunchKernelGGL(ce_stream_block_kernel<1024>, dim3((unsigned)rows), dim3(1024), 0, s, slab, ld, nb, v0, labels, run_max, run_sum, target, alpha, run_arg);
 }
 
 // Packed rows of the labels (row 0 for ignored or out-of-range labels: their gradient is zero or undefined anyway).
@@ -240,12 +252,11 @@ int lmhead_ce(int qt, const void* hidden, const void* packed, const int64_t* lab
                 if (int rcode = launch_mmq(qt, kModeNT, kEpiStore, g, s)) return rcode;
             }
             // (2) running statistics; the slab becomes exp(logit - running max)
-            hipLaunchKernelGGL(ce_stream_block_kernel, dim3((unsigned)rc), dim3(kStreamThreads), 0, s, slab, block, nb, v0, labels + r0, run_max + r0, run_sum + r0,
-                               target + r0, alpha + r0, run_arg ? run_arg + r0 : nullptr);
+            launch_stream_block(rc, slab, block, nb, v0, labels + r0, run_max + r0, run_sum + r0, target + r0, alpha + r0, run_arg ? run_arg + r0 : nullptr, s);
             // (3) acc = acc * alpha + p . W_block; the first block starts the accumulator
             if (panel_path) {
                 q.mode = kModeNN, q.a = slab, q.lda = block, q.a_zero_padded = true, q.c = dh32, q.ldc = hidden_dim;
-                q.fp32 = true, q.accumulate = v0 > 0, q.row_scale = alpha + r0;
+                q.panel_ready = dense_panel_whole(nb, hidden_dim), q.fp32 = true, q.accumulate = v0 > 0, q.row_scale = alpha + r0;
                 if (int rcode = dense_mmq(q, panels, panel_bytes, s)) return rcode;
             } else {
                 if (v0 == 0) hipLaunchKernelGGL(fill_f32_kernel, dim3(grid1d((int64_t)rc * hidden_dim)), dim3(256), 0, s, dh32, (int64_t)rc * hidden_dim, 0.f);

@@ -146,6 +146,7 @@ struct DenseCall {
     void* c;
     int64_t ldc;
     bool a_zero_padded;   // rows of a hold zeros from the contraction's end to the next multiple of 64
+    bool panel_ready;     // the workspace holds this matrix's panel from the call before (only where dense_panel_whole)
     bool fp32;            // c is fp32 (a multiple of four columns)
     bool accumulate;      // fp32: c = c * row_scale[m] + result instead of c = result
     const float* row_scale;
@@ -154,6 +155,7 @@ struct DenseCall {
     float lora_scale;
 };
 bool dense_takes(int mode, int64_t m, int64_t n, int64_t k, const void* a, int64_t lda, bool a_zero_padded = false);
+bool dense_panel_whole(int64_t n, int64_t k);
 int64_t dense_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s);
 void dense_force_shape(int shape, int splits);  // test aid: -1 = the automatic choice
