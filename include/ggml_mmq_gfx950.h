@@ -234,6 +234,17 @@ int ggq_swiglu_backward_routed(const void* gate, const void* up, const void* dh_
                                const int64_t* permutation, void* dgate, void* dup, void* grad_weights, int64_t rows, int inter, float limit,
                                void* stream);
 
+/* The routed expert FFN's forward (fast_moe_lora.py:685-770) for a few routes, as while sampling: every route reads its own
+ * expert's weights, so there is no routing plan.  ids int32 or int64 [tokens, top_k] (clamped to [0, experts)); weights fp32 or
+ * bf16 [tokens, top_k]; gate, up [experts, inter, hidden] and down [experts, hidden, inter] packed; the LoRA factors as in the
+ * grouped entries (A NULL: none); limit 0: no clamp.  act is scratch, bf16 [tokens * top_k, inter]; out bf16 [tokens, hidden].
+ * ggq_experts_few_routes_takes says whether these sizes are taken (host-side answer). */
+int ggq_experts_few_routes_takes(int qt_gate_up, int qt_down, int64_t tokens, int top_k, int64_t hidden, int64_t inter);
+int ggq_experts_few_routes_forward(const void* hidden_states, const void* ids, int ids_are_int64, const void* weights, int weights_are_bf16, int64_t tokens, int top_k,
+                                   int64_t experts, int64_t hidden, int64_t inter, int qt_gate_up, int qt_down, const void* gate, const void* up, const void* down,
+                                   const void* a_gate_up, const void* b_gate_up, int r_gate_up, const void* a_down, const void* b_down, int r_down, float scale,
+                                   float limit, void* act, void* out, void* stream);
+
 /* AITER's grouped products as the reference calls them (gmm / ptgmm, fast_moe_lora.py:22, 42-87; _AiterGroupedMM :90-151),
  * for bf16 or fp16 matrices (is_f16; both operands and the output share the type) with no packed weight: the LoRA factors of an expert layer (:674-682) and expert weights without a
  * packed kernel (:230-247).  group_sizes [experts] int32 on the device: consecutive row groups of lhs, group e owning
@@ -280,12 +291,11 @@ int ggq_router_topk(const void* logits, int logits_are_bf16, int64_t tokens, int
  * predicted_tokens int64 [rows] or NULL: the row's argmax over the bf16 logits (the first maximum), -1 for rows that do not
  *   count; token_correct fp32 [rows] or NULL: 1 where the argmax is the label, else 0 (Liger's RETURN_PREDICTED_TOKENS /
  *   RETURN_TOKEN_ACCURACY outputs, gguf_liger_loss.py:92-100, 117-185; the accuracy is sum(token_correct) / status_out[0]).
- * Memory: `chunk` stands for the reference's [chunk, vocab] logits tensor.  From 4096 rows per chunk on, or when one chunk
- * covers all rows, the chunk's bf16 logits are kept in the workspace and rewritten as their gradient.  Below that nothing wider
- * than 8192 vocabulary columns is held (one sweep over the vocabulary with a running max, sum and argmax per row), but the
- * sweep takes min(rows, 4096) rows at a time whatever the chunk: the workspace then holds a [min(rows, 4096), 8192] bf16 slab,
- * an fp32 [min(rows, 4096), hidden] accumulator and two bf16-sized [.., hidden] label-row buffers (about 128 MiB at hidden 2048),
- * for chunk 64 as for chunk 1024.  Two vocabulary-sized GEMMs either way. */
+ * Memory: `chunk` stands for the reference's [chunk, vocab] logits tensor; no logits are kept whatever it is.  The vocabulary is
+ * swept once per min(rows, 4096) rows with a running max, sum and argmax per row: the workspace holds a slab of at most 64 MB of
+ * logits (8192 columns of 4096 rows, up to 32768 of fewer), an fp32 [min(rows, 4096), hidden] accumulator, two bf16-sized
+ * [.., hidden] label-row buffers and the decoded weights of one block of columns (at most 128 MB), with the partial sums of a
+ * split contraction where rows are few.  Two vocabulary-sized GEMMs. */
 int64_t ggq_lmhead_ce_workspace_bytes(int64_t rows, int64_t vocab, int64_t hidden_dim, int64_t chunk);
 int ggq_lmhead_cross_entropy(int qt, const void* hidden, const void* packed, const int64_t* labels, int64_t rows, int64_t vocab,
                              int64_t hidden_dim, int64_t chunk, int64_t ignore_index, int reduction_mean, float* loss_per_row,

@@ -64,6 +64,8 @@ SIGNATURES: dict[str, tuple] = {
     "ggq_swiglu_backward_routed": (_I, [_P, _P, _P, _P, _I, _P, _P, _P, _P, _L, _I, _F, _P]),
     "ggq_grouped_lora_mmq_backward_routed_output": (_I, [_P, _L, _P, _I, _P, _I, _P, _P, _P, _L, _L, _I, _L, _L, _L, _P, _P, _P, _P, _I, _F, _P, _P, _P,
                                                          _P, _P, _L, _P]),
+    "ggq_experts_few_routes_takes": (_I, [_I, _I, _L, _I, _L, _L]),
+    "ggq_experts_few_routes_forward": (_I, [_P, _P, _I, _P, _I, _L, _I, _L, _L, _L, _I, _I, _P, _P, _P, _P, _P, _I, _P, _P, _I, _F, _F, _P, _P, _P]),
     "ggq_gmm_workspace_bytes": (_L, [_L]),
     "ggq_gmm": (_I, [_P, _P, _P, _P, _L, _L, _L, _L, _I, _I, _P, _L, _P]),
     "ggq_ptgmm": (_I, [_P, _P, _P, _P, _L, _L, _L, _L, _I, _P, _L, _P]),

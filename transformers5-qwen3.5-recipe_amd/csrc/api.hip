@@ -345,6 +345,8 @@ static int grouped_forward(const char* what, const void* x, RowIndex x_index, co
     if (int rc = init_params(p, qt, kModeNT, (int)rows, (int)n, (int)k, nseg, pick_shape(qt, rows, groups, direct_ok))) return rc;
     if (x_index.on() && (!forward_reads_indexed_rows(qt, rows, groups, x_index.index_rows, k) || x_index.index_div <= 0))
         return set_error(GGQ_ERR_SHAPE, "%s: this source matrix cannot be read through a row index (ask ggq_grouped_forward_reads_indexed_rows first)", what);
+    if (groups == 0 && !packed2 && !x_index.on() && gemv_takes(qt, rows, n, k, x) && (!lora_a || aligned16(xa_out)))
+        return gemv(qt, x, packed1, rows, n, k, lora_a, lora_b, r, scale, xa_out, y1, s);
     p.a[0] = (const bf16_t*)x, p.lda = k, p.a_rows = x_index;
     p.w[0] = (const uint8_t*)packed1, p.w[1] = (const uint8_t*)packed2;
     p.c[0] = y1, p.c[1] = y2, p.ldc = n;
@@ -720,6 +722,27 @@ int ggq_swiglu_clamped_backward(const void* gate, const void* up, const void* dh
     if (!gate || !up || !dh || !dgate || !dup) return set_error(GGQ_ERR_NULL, "swiglu_clamped_backward: null pointer");
     if (!(limit > 0.0f)) return set_error(GGQ_ERR_SHAPE, "swiglu_clamped_backward: the limit must be positive");
     return swiglu_bwd(gate, up, dh, dgate, dup, elems, limit, as_stream(stream));
+}
+
+int ggq_experts_few_routes_takes(int qt_gate_up, int qt_down, int64_t tokens, int top_k, int64_t hidden, int64_t inter) {
+    return ggq_row_bytes(qt_gate_up, hidden) > 0 && ggq_row_bytes(qt_down, inter) > 0 && hidden % 64 == 0 && inter % 64 == 0 &&
+           few_routes_takes(qt_gate_up, qt_down, tokens, top_k, hidden, inter);
+}
+
+int ggq_experts_few_routes_forward(const void* hidden_states, const void* ids, int ids_are_int64, const void* weights, int weights_are_bf16, int64_t tokens, int top_k,
+                                   int64_t experts, int64_t hidden, int64_t inter, int qt_gate_up, int qt_down, const void* gate, const void* up, const void* down,
+                                   const void* a_gate_up, const void* b_gate_up, int r_gate_up, const void* a_down, const void* b_down, int r_down, float scale,
+                                   float limit, void* act, void* out, void* stream) {
+    const char* what = "experts_few_routes_forward";
+    if (!ggq_experts_few_routes_takes(qt_gate_up, qt_down, tokens, top_k, hidden, inter) || experts < 1) return set_error(GGQ_ERR_SHAPE, "%s: not for these sizes (ask ggq_experts_few_routes_takes)", what);
+    for (const void* w : {gate, up, down})
+        if (int rc = check_weights(what, w == down ? qt_down : qt_gate_up, w, w == down ? inter : hidden)) return rc;
+    if (int rc = check_lora(what, a_gate_up, b_gate_up, r_gate_up)) return rc;
+    if (int rc = check_lora(what, a_down, b_down, r_down)) return rc;
+    if (!hidden_states || !ids || !weights || !act || !out) return set_error(GGQ_ERR_NULL, "%s: null pointer", what);
+    if (!aligned16(hidden_states) || !aligned16(act) || !aligned16(out)) return set_error(GGQ_ERR_ALIGN, "%s: row buffers must be 16-byte aligned", what);
+    return few_routes_forward(hidden_states, ids, ids_are_int64, weights, weights_are_bf16, tokens, top_k, experts, hidden, inter, qt_gate_up, qt_down, gate, up, down,
+                              a_gate_up, b_gate_up, r_gate_up, a_down, b_down, r_down, scale, limit, act, out, as_stream(stream));
 }
 
 int64_t ggq_gmm_workspace_bytes(int64_t experts) { return grouped_gemm_workspace_bytes(experts); }

@@ -1,0 +1,505 @@
+// Products of a few activation rows with packed weights: sampling (one row per sequence) and its expert layers.
+//
+// What bounds them is the packed bytes: every weight is used by 1 to 64 rows.  A tile of mmq_tile.h pads the rows to 256 and
+// gives a 4096-column layer 32 workgroups; here a workgroup takes sixteen weight ROWS (a contiguous run of packed bytes,
+// whatever the block format) at a time, moves them global -> LDS in whole 1 KB requests (a lane-per-row register load costs
+// the vector cache an access per lane), and its waves decode them from LDS straight into 16x16x32 MFMA operands: lane
+// (weight row lane % 16, quarter lane / 16) owns one 32-element run of a 128-element span and feeds its eight-element
+// pieces to four MFMAs whose other operand holds the matching pieces of sixteen activation rows, in registers for the
+// whole kernel.  The matrix pipe, idle otherwise, does the multiplication, so one row costs what sixteen do.
+#include <algorithm>
+
+#include "blocks.h"
+#include "iq2xxs_grid.h"
+#include "launch.h"
+#include "mmq_host.h"
+
+namespace ggq {
+
+static __device__ const uint64_t d_iq2xxs_grid_gemv[256] = GGQ_IQ2XXS_GRID_INIT;
+
+constexpr int kSpan = 128;                 // contraction elements of four runs
+template <int QT>
+constexpr int kTableBytes = QT == kIQ2_XXS ? Fmt<kIQ2_XXS>::kTableWords * 4 : 0;
+
+template <int QT>
+__device__ __forceinline__ void stage_tables(uint8_t* lds, int tid, int threads) {
+    if constexpr (QT == kIQ2_XXS)
+        for (int i = tid; i < Fmt<kIQ2_XXS>::kTableWords; i += threads) ((uint32_t*)lds)[i] = Fmt<kIQ2_XXS>::table_word(i, i < 1024 ? d_iq2xxs_grid_gemv[i >> 2] : 0ull);
+}
+
+__device__ __forceinline__ bf16x8_t as_operand(const uint4& v) { return __builtin_bit_cast(bf16x8_t, v); }
+__device__ __forceinline__ f32x4_t mfma16(const bf16x8_t& a, const bf16x8_t& b, const f32x4_t& c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+
+// A run of packed bytes global -> LDS, dealt to the workgroup's waves in 1 KB requests; both ends 16-byte aligned except for
+// the length, whose odd end (less than 16 bytes) a few lanes carry.  Returns the requests this wave made.
+__device__ __forceinline__ int request_bytes(const uint8_t* src, uint8_t* dst, int bytes, int wave, int waves, int lane) {
+    const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)dst;
+    const int whole = bytes & ~15;
+    int made = 0;
+    for (int c = wave; c * 1024 < whole; c += waves, made++)
+        if (c * 1024 + lane * 16 < whole) load16_to_lds(lds + c * 1024, (uint32_t)lane * 16u, src + c * 1024);
+    if (wave == 0 && lane * 2 < bytes - whole) *(uint16_t*)(dst + whole + lane * 2) = *(const uint16_t*)(src + whole + lane * 2);
+    return made;
+}
+
+// Eight consecutive factor elements p[0..valid) (zeros past it); vec: 16-byte aligned and whole.
+__device__ __forceinline__ uint4 load_factor8(const bf16_t* p, int valid, bool vec) {
+    if (vec && valid >= 8) return *(const uint4*)p;
+    if (valid <= 0) return make_uint4(0, 0, 0, 0);
+    uint32_t e[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) e[i] = i < valid ? (uint32_t)p[i] : 0u;
+    return make_uint4(e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16));
+}
+
+// ------------------------------------------------------------------------------------------------
+// Dense: y [m, n] = x [m, k] . W [n, k]^T (+ scale (x A^T) B^T).
+struct GemvParams {
+    const bf16_t* x;
+    int m, n, k;
+    const uint8_t* w;
+    int row_bytes;
+    bf16_t* y;
+    const bf16_t *lora_a, *lora_b;  // [r][k], [n][r]; null: none
+    bf16_t* xa_out;                 // [m][r_pad]
+    int r, r_pad;
+    float lora_scale;
+    int stage_bytes, buffers;       // LDS bytes of sixteen packed rows, one or two of them
+};
+
+// WAVES waves deal the spans of the contraction out (span s to wave s % WAVES, at most SP each); TB blocks of sixteen rows of x.
+template <int QT, int WAVES, int SP, int TB>
+__global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t gemv_lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, q = lane >> 4;
+    uint8_t* stage = gemv_lds + kTableBytes<QT>;
+    f32x4_t* red = (f32x4_t*)(stage + p.buffers * p.stage_bytes);            // [WAVES][TB][64]
+    bf16_t* xa = (bf16_t*)(red + WAVES * TB * 64);                           // [TB * 16][64]
+    const int blocks = (p.n + 15) / 16, spans = (p.k + kSpan - 1) / kSpan;
+    int block = blockIdx.x;
+    auto request_block = [&](int b, int buf) __attribute__((always_inline)) {
+        return request_bytes(p.w + (int64_t)b * 16 * p.row_bytes, stage + buf * p.stage_bytes, min(16, p.n - b * 16) * p.row_bytes, wave, WAVES, lane);
+    };
+    // (the barriers here order LDS traffic only: __syncthreads would also wait for the block requested ahead)
+    if (block < blocks) request_block(block, 0);
+    stage_tables<QT>(gemv_lds, threadIdx.x, 64 * WAVES);
+
+    uint4 xf[SP][TB][4];
+#pragma unroll
+    for (int sp = 0; sp < SP; sp++)
+#pragma unroll
+        for (int tb = 0; tb < TB; tb++) {
+            const int row = min(tb * 16 + l16, p.m - 1), e0 = (wave + WAVES * sp) * kSpan + 32 * q;
+            const bool live = e0 < p.k;  // (k is a multiple of 32: a run is whole or absent)
+            const uint4* src = (const uint4*)(p.x + (int64_t)row * p.k + (live ? e0 : 0));
+#pragma unroll
+            for (int i = 0; i < 4; i++) xf[sp][tb][i] = live ? src[i] : make_uint4(0, 0, 0, 0);
+        }
+    if (p.lora_a) {  // x A^T over this wave's spans, added over the waves, kept as bf16 rows in LDS
+        for (int r0 = 0; r0 < p.r_pad; r0 += 16) {
+            f32x4_t acc[TB];
+#pragma unroll
+            for (int tb = 0; tb < TB; tb++) acc[tb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+            const bf16_t* arow = p.lora_a + (int64_t)min(r0 + l16, p.r - 1) * p.k;
+#pragma unroll
+            for (int sp = 0; sp < SP; sp++) {
+                const int e0 = (wave + WAVES * sp) * kSpan + 32 * q;
+                const bool live = e0 < p.k && r0 + l16 < p.r;
+                uint4 a[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) a[i] = live ? ((const uint4*)(arow + e0))[i] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int tb = 0; tb < TB; tb++) acc[tb] = mfma16(as_operand(a[i]), as_operand(xf[sp][tb][i]), acc[tb]);
+            }
+#pragma unroll
+            for (int tb = 0; tb < TB; tb++) red[(wave * TB + tb) * 64 + lane] = acc[tb];
+            lds_barrier();
+            for (int tb = wave; tb < TB; tb += WAVES) {
+                f32x4_t sum = red[tb * 64 + lane];
+                for (int w = 1; w < WAVES; w++) sum += red[(w * TB + tb) * 64 + lane];
+                const uint2 v = make_uint2(pack_bf16(sum[0], sum[1]), pack_bf16(sum[2], sum[3]));
+                const int row = tb * 16 + l16;  // factor rows r0 + 4 q .. + 3 of x row `row`
+                *(uint2*)(xa + row * 64 + r0 + 4 * q) = v;
+                if (blockIdx.x == 0 && row < p.m) *(uint2*)(p.xa_out + (int64_t)row * p.r_pad + r0 + 4 * q) = v;
+            }
+            lds_barrier();
+        }
+    }
+    const bool b_vec = (p.r & 7) == 0 && ((uintptr_t)p.lora_b & 15) == 0;
+    for (int buf = 0; block < blocks; block += gridDim.x) {
+        const int next = block + gridDim.x;
+        if (p.buffers == 2 && next < blocks) wait_loads_at_most(request_block(next, buf ^ 1));
+        else wait_loads_at_most(0);
+        lds_barrier();
+        f32x4_t acc[TB];
+#pragma unroll
+        for (int tb = 0; tb < TB; tb++) acc[tb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        const uint8_t* row = stage + buf * p.stage_bytes + min(l16, p.n - block * 16 - 1) * p.row_bytes;
+#pragma unroll
+        for (int sp = 0; sp < SP; sp++) {
+            const int span = wave + WAVES * sp;
+            if (span >= spans) break;  // uniform over the wave
+            const int run = min(span * 4 + q, (p.k >> 5) - 1);
+            typename Fmt<QT>::Raw raw;
+            uint32_t v[16];
+            Fmt<QT>::load(raw, row, run);
+            Fmt<QT>::decode(raw, run, v, (const uint2*)gemv_lds);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int tb = 0; tb < TB; tb++)
+                    acc[tb] = mfma16(as_operand(make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3])), as_operand(xf[sp][tb][i]), acc[tb]);
+        }
+#pragma unroll
+        for (int tb = 0; tb < TB; tb++) red[(wave * TB + tb) * 64 + lane] = acc[tb];
+        lds_barrier();
+        if (p.buffers == 1 && next < blocks) request_block(next, 0);
+        // (a buffer is refilled, and the partial sums rewritten, only behind the next barrier)
+        for (int tb = (wave + block) % WAVES; tb < TB; tb += WAVES) {
+            f32x4_t sum = red[tb * 64 + lane];
+            for (int w = 1; w < WAVES; w++) sum += red[(w * TB + tb) * 64 + lane];
+            const int col = block * 16 + 4 * q, xrow = tb * 16 + l16;
+            if (p.lora_a) {
+                f32x4_t lo = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+                const bf16_t* brow = p.lora_b + (int64_t)min(block * 16 + l16, p.n - 1) * p.r;
+                for (int r0 = 0; r0 < p.r_pad; r0 += 32) {
+                    const int j = r0 + 8 * q;
+                    const uint4 b = load_factor8(brow + j, p.r - j, b_vec);
+                    const uint4 xv = j < p.r_pad ? *(const uint4*)(xa + xrow * 64 + j) : make_uint4(0, 0, 0, 0);
+                    lo = mfma16(as_operand(b), as_operand(xv), lo);
+                }
+                sum += lo * p.lora_scale;
+            }
+            if (xrow < p.m) {
+                bf16_t* dst = p.y + (int64_t)xrow * p.n + col;
+                if ((p.n & 3) == 0 && ((uintptr_t)p.y & 7) == 0) {
+                    if (col < p.n) *(uint2*)dst = make_uint2(pack_bf16(sum[0], sum[1]), pack_bf16(sum[2], sum[3]));
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                        if (col + v < p.n) dst[v] = to_bf16(sum[v]);
+                }
+            }
+        }
+        if (p.buffers == 2) buf ^= 1;
+    }
+}
+
+template <int QT, int WAVES, int SP, int TB>
+static int launch_gemv(const GemvParams& p, hipStream_t s) {
+    const int lds = kTableBytes<QT> + p.buffers * p.stage_bytes + WAVES * TB * 64 * 16 + TB * 16 * 64 * 2;
+    static LdsLimit lim;
+    if (int rc = raise_lds_limit(lim, (const void*)gemv_kernel<QT, WAVES, SP, TB>, 160 * 1024, "gemv")) return rc;
+    const int per_cu = std::max(1, std::min(160 * 1024 / lds, 16 / WAVES));
+    hipLaunchKernelGGL((gemv_kernel<QT, WAVES, SP, TB>), dim3(std::min((p.n + 15) / 16, 256 * per_cu)), dim3(64 * WAVES), lds, s, p);
+    return check_launch("gemv");
+}
+template <int QT>
+static int launch_gemv_qt(const GemvParams& p, hipStream_t s) {
+    const int tb = (p.m + 15) / 16;
+    if (p.k <= 2048) {
+        if (tb == 1) return launch_gemv<QT, 8, 2, 1>(p, s);
+        if (tb == 2) return launch_gemv<QT, 8, 2, 2>(p, s);
+        return launch_gemv<QT, 8, 2, 4>(p, s);
+    }
+    if (p.k <= 4096) return tb == 1 ? launch_gemv<QT, 8, 4, 1>(p, s) : launch_gemv<QT, 8, 4, 2>(p, s);
+    return launch_gemv<QT, 16, 4, 1>(p, s);
+}
+
+// Rows up to which x fits the registers of the waves that share it: 64 of 2048 elements, 32 of 4096, 16 of 8192.
+bool gemv_takes(int qt, int64_t m, int64_t n, int64_t k, const void* x) {
+    if (m < 1 || n < 1 || k > 8192 || ((uintptr_t)x & 15)) return false;
+    if (m > (k <= 2048 ? 64 : k <= 4096 ? 32 : 16)) return false;
+    return 16 * packed_row_bytes(qt, k) <= (k <= 4096 ? 72 : 136) * 1024;
+}
+
+int gemv(int qt, const void* x, const void* w, int64_t m, int64_t n, int64_t k, const void* lora_a, const void* lora_b, int r, float scale, void* xa_out, void* y, hipStream_t s) {
+    GemvParams p{};
+    p.x = (const bf16_t*)x, p.m = (int)m, p.n = (int)n, p.k = (int)k, p.w = (const uint8_t*)w, p.row_bytes = (int)packed_row_bytes(qt, k), p.y = (bf16_t*)y;
+    if (lora_a) p.lora_a = (const bf16_t*)lora_a, p.lora_b = (const bf16_t*)lora_b, p.r = r, p.r_pad = (r + 15) / 16 * 16, p.lora_scale = scale, p.xa_out = (bf16_t*)xa_out;
+    p.stage_bytes = (16 * p.row_bytes + 1023) / 1024 * 1024;
+    p.buffers = (p.n + 15) / 16 > 256 && p.stage_bytes <= 36 * 1024 ? 2 : 1;  // (one block per workgroup needs one buffer)
+    TimedScope timed(qt, kModeNT, kEpiStore, kShapeFewRows, s);
+    switch (qt) {
+        case kQ8_0: return launch_gemv_qt<kQ8_0>(p, s);
+        case kQ2_K: return launch_gemv_qt<kQ2_K>(p, s);
+        case kQ3_K: return launch_gemv_qt<kQ3_K>(p, s);
+        case kQ4_K: return launch_gemv_qt<kQ4_K>(p, s);
+        case kQ5_K: return launch_gemv_qt<kQ5_K>(p, s);
+        case kQ6_K: return launch_gemv_qt<kQ6_K>(p, s);
+        case kIQ2_XXS: return launch_gemv_qt<kIQ2_XXS>(p, s);
+    }
+    return set_error(GGQ_ERR_QTYPE, "unsupported GGML type id %d", qt);
+}
+
+// ------------------------------------------------------------------------------------------------
+// Expert FFN of a few routes, without a routing plan: with a handful of routes hardly two share an expert, so every route
+// reads its own expert's weights and the four launches of plan and tables, the gather by expert and the combine's pass fall
+// away.  Two launches:
+//   act[route] = silu(gate) * up         one workgroup per (route, eight gate rows and the eight up rows of the same columns)
+//   out[token] = sum w[route] * down     one workgroup per (token, sixteen output columns), one wave per route
+// The LoRA products x A^T are formed by every workgroup for itself (64 KB of factor out of the L2 at rank 16 and 2048
+// columns): cheaper than a launch.
+struct FewRoutesParams {
+    const bf16_t* x;       // [tokens, hidden]
+    const void* ids;
+    int ids64;
+    const void* weights;   // [tokens, top_k]
+    int weights_bf16;
+    int tokens, top_k, experts, hidden, inter;
+    const uint8_t *gate, *up, *down;
+    int row_bytes_in, row_bytes_down;
+    const bf16_t *a1, *b1, *a2, *b2;
+    int r1, r2;
+    float scale, limit;
+    bf16_t* act;           // [routes, inter]
+    bf16_t* out;           // [tokens, hidden]
+};
+
+__device__ __forceinline__ int route_expert(const FewRoutesParams& p, int route) {
+    const int64_t e = p.ids64 ? ((const int64_t*)p.ids)[route] : (int64_t)((const int32_t*)p.ids)[route];
+    return (int)(e < 0 ? 0 : e >= p.experts ? p.experts - 1 : e);  // (the routing plan clamps in the same way)
+}
+
+// sum over j of b[j] * xa[j] for the sixteen rows of a block: lane (row lane % 16, quarter) takes every fourth group of eight
+// ranks; every lane of a row returns the row's sum.
+__device__ __forceinline__ float lora_row_dot(const bf16_t* brow, const bf16_t* xa, int r, bool vec, int q) {
+    float s = 0.f;
+    for (int j = 8 * q; j < r; j += 32) {
+        const uint4 b = load_factor8(brow + j, r - j, vec), x = *(const uint4*)(xa + j);
+        const uint32_t bw[4] = {b.x, b.y, b.z, b.w}, xw[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) s = fmaf(bf16_lo(bw[i]), bf16_lo(xw[i]), s), s = fmaf(bf16_hi(bw[i]), bf16_hi(xw[i]), s);
+    }
+    s += __shfl_xor(s, 16, 64);
+    return s + __shfl_xor(s, 32, 64);
+}
+
+template <int QT, int SP>
+__global__ __launch_bounds__(512) void few_routes_gate_up_kernel(FewRoutesParams p) {
+    constexpr int WAVES = 8;
+    extern __shared__ __attribute__((aligned(16))) uint8_t gu_lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, q = lane >> 4;
+    const int half_bytes = 8 * p.row_bytes_in;
+    uint8_t* stage = gu_lds + kTableBytes<QT>;
+    float* red = (float*)(stage + 2 * half_bytes);   // [WAVES][16]
+    float* red_xa = red + WAVES * 16;                // [WAVES][64]
+    bf16_t* xa = (bf16_t*)(red_xa + WAVES * 64);     // [64]
+    const int route = blockIdx.y, i0 = blockIdx.x * 8, k = p.hidden;
+    const int expert = route_expert(p, route);
+    const int64_t row0 = (int64_t)expert * p.inter + i0;
+    request_bytes(p.gate + row0 * p.row_bytes_in, stage, half_bytes, wave, WAVES, lane);
+    request_bytes(p.up + row0 * p.row_bytes_in, stage + half_bytes, half_bytes, (wave + 4) & 7, WAVES, lane);
+    stage_tables<QT>(gu_lds, threadIdx.x, 512);
+    const bf16_t* x = p.x + (int64_t)(route / p.top_k) * k;
+    uint4 xf[SP][4];
+#pragma unroll
+    for (int sp = 0; sp < SP; sp++) {
+        const int e0 = (wave + WAVES * sp) * kSpan + 32 * q;
+#pragma unroll
+        for (int i = 0; i < 4; i++) xf[sp][i] = e0 < k ? ((const uint4*)(x + e0))[i] : make_uint4(0, 0, 0, 0);
+    }
+    const int r_pad = (p.r1 + 15) & ~15;
+    if (p.a1) {
+        const bf16_t* a = p.a1 + (int64_t)expert * p.r1 * k;
+        for (int r0 = 0; r0 < r_pad; r0 += 16) {
+            f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+            const bf16_t* arow = a + (int64_t)min(r0 + l16, p.r1 - 1) * k;
+#pragma unroll
+            for (int sp = 0; sp < SP; sp++) {
+                const int e0 = (wave + WAVES * sp) * kSpan + 32 * q;
+                const bool live = e0 < k && r0 + l16 < p.r1;
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc = mfma16(as_operand(live ? ((const uint4*)(arow + e0))[i] : make_uint4(0, 0, 0, 0)), as_operand(xf[sp][i]), acc);
+            }
+            if (l16 == 0) *(f32x4_t*)(red_xa + wave * 64 + r0 + 4 * q) = acc;
+        }
+    }
+    wait_loads_at_most(0);
+    __syncthreads();
+    f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    const uint8_t* row = stage + l16 * p.row_bytes_in;  // rows 0..7 gate, 8..15 up
+    const int spans = (k + kSpan - 1) / kSpan;
+#pragma unroll
+    for (int sp = 0; sp < SP; sp++) {
+        const int span = wave + WAVES * sp;
+        if (span >= spans) break;
+        const int run = min(span * 4 + q, (k >> 5) - 1);
+        typename Fmt<QT>::Raw raw;
+        uint32_t v[16];
+        Fmt<QT>::load(raw, row, run);
+        Fmt<QT>::decode(raw, run, v, (const uint2*)gu_lds);
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc = mfma16(as_operand(make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3])), as_operand(xf[sp][i]), acc);
+    }
+    if (l16 == 0) *(f32x4_t*)(red + wave * 16 + 4 * q) = acc;
+    if (p.a1 && wave == 0) {  // (red_xa is complete since the barrier above)
+        float s = 0.f;
+        if (lane < r_pad)
+            for (int w = 0; w < WAVES; w++) s += red_xa[w * 64 + lane];
+        xa[lane] = lane < r_pad ? to_bf16(s) : (bf16_t)0;
+    }
+    __syncthreads();
+    if (wave > 0) return;
+    float y = 0.f;  // of row l16, in all four quarters
+    for (int w = 0; w < WAVES; w++) y += red[w * 16 + l16];
+    if (p.a1) {
+        const int64_t brow = (int64_t)expert * 2 * p.inter + (l16 < 8 ? i0 + l16 : p.inter + i0 + l16 - 8);
+        y = fmaf(p.scale, lora_row_dot(p.b1 + brow * p.r1, xa, p.r1, (p.r1 & 7) == 0, q), y);
+    }
+    y = bf16_to_f32(to_bf16(y));
+    const float up = __shfl(y, (lane & 7) + 8, 64), gate = __shfl(y, lane & 7, 64);
+    if (lane < 8) {
+        const float hi = p.limit > 0.0f ? p.limit : INFINITY;
+        const float g = fminf(gate, hi), u = fminf(fmaxf(up, -hi), hi);
+        p.act[(int64_t)route * p.inter + i0 + lane] = to_bf16(g / (1.0f + __expf(-g)) * u);
+    }
+}
+
+template <int QT>
+__global__ __launch_bounds__(512) void few_routes_down_kernel(FewRoutesParams p) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t down_lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, q = lane >> 4;
+    const int stage_bytes = (16 * p.row_bytes_down + 1023) / 1024 * 1024;
+    uint8_t* mine = down_lds + kTableBytes<QT> + wave * stage_bytes;
+    float* red = (float*)(down_lds + kTableBytes<QT> + 8 * stage_bytes);  // [16 routes][16]
+    bf16_t* xa = (bf16_t*)(red + 256) + wave * 64;
+    const int token = blockIdx.y, h0 = blockIdx.x * 16, k = p.inter, spans = (k + kSpan - 1) / kSpan;
+    const int rows = min(16, p.hidden - h0);
+    stage_tables<QT>(down_lds, threadIdx.x, 512);
+    if (kTableBytes<QT>) __syncthreads();
+    for (int rank = wave; rank < p.top_k; rank += 8) {
+        const int route = token * p.top_k + rank, expert = route_expert(p, route);
+        // this wave's own sixteen rows: no other wave touches them, so no barrier stands between their requests and their use
+        request_bytes(p.down + ((int64_t)expert * p.hidden + h0) * p.row_bytes_down, mine, rows * p.row_bytes_down, 0, 1, lane);
+        const bf16_t* x = p.act + (int64_t)route * k;
+        const bf16_t* a = p.a2 ? p.a2 + (int64_t)expert * p.r2 * k : nullptr;
+        f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f}, acc_a[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc_a[j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        const uint8_t* row = mine + min(l16, rows - 1) * p.row_bytes_down;
+        for (int s0 = 0; s0 < spans; s0 += 4) {  // four spans of x in registers at a time, requested together
+            uint4 xf[4][4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int e0 = (s0 + u) * kSpan + 32 * q;
+#pragma unroll
+                for (int i = 0; i < 4; i++) xf[u][i] = e0 < k ? ((const uint4*)(x + e0))[i] : make_uint4(0, 0, 0, 0);
+            }
+            if (a) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if (16 * j >= p.r2) break;
+                    const bf16_t* arow = a + (int64_t)min(16 * j + l16, p.r2 - 1) * k;
+#pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        const int e0 = (s0 + u) * kSpan + 32 * q;
+                        const bool live = e0 < k && 16 * j + l16 < p.r2;
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc_a[j] = mfma16(as_operand(live ? ((const uint4*)(arow + e0))[i] : make_uint4(0, 0, 0, 0)), as_operand(xf[u][i]), acc_a[j]);
+                    }
+                }
+            }
+            if (s0 == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int run = min((s0 + u) * 4 + q, (k >> 5) - 1);  // (past the end x is zero)
+                typename Fmt<QT>::Raw raw;
+                uint32_t v[16];
+                Fmt<QT>::load(raw, row, run);
+                Fmt<QT>::decode(raw, run, v, (const uint2*)down_lds);
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc = mfma16(as_operand(make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3])), as_operand(xf[u][i]), acc);
+            }
+        }
+        if (a && l16 == 0) {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (16 * j < p.r2) *(uint2*)(xa + 16 * j + 4 * q) = make_uint2(pack_bf16(acc_a[j][0], acc_a[j][1]), pack_bf16(acc_a[j][2], acc_a[j][3]));
+        }
+        if (l16 == 0) *(f32x4_t*)(red + rank * 16 + 4 * q) = acc;
+        if (p.a2) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            const float dot = lora_row_dot(p.b2 + ((int64_t)expert * p.hidden + min(h0 + l16, p.hidden - 1)) * p.r2, xa, p.r2, (p.r2 & 7) == 0, q);
+            if (q == 0) red[rank * 16 + l16] = fmaf(p.scale, dot, red[rank * 16 + l16]);
+        }
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < rows) {  // the combine: routes in rank order, weights and rows at bf16 precision
+        float sum = 0.f;
+        for (int rank = 0; rank < p.top_k; rank++) {
+            const int64_t route = (int64_t)token * p.top_k + rank;
+            const float w = p.weights_bf16 ? bf16_to_f32(((const bf16_t*)p.weights)[route]) : bf16_to_f32(to_bf16(((const float*)p.weights)[route]));
+            sum = fmaf(bf16_to_f32(to_bf16(red[rank * 16 + threadIdx.x])), w, sum);
+        }
+        p.out[(int64_t)token * p.hidden + h0 + threadIdx.x] = to_bf16(sum);
+    }
+}
+
+static int gate_up_lds(int qt, int row_bytes) { return (qt == kIQ2_XXS ? kTableBytes<kIQ2_XXS> : 0) + 16 * row_bytes + 8 * 16 * 4 + 8 * 64 * 4 + 128; }
+static int down_lds_bytes(int qt, int row_bytes) { return (qt == kIQ2_XXS ? kTableBytes<kIQ2_XXS> : 0) + 8 * ((16 * row_bytes + 1023) / 1024 * 1024) + 256 * 4 + 8 * 128; }
+
+template <int QT>
+static int launch_gate_up(const FewRoutesParams& p, hipStream_t s) {
+    const int lds = gate_up_lds(QT, p.row_bytes_in);
+    static LdsLimit lim2, lim4;
+    const dim3 grid(p.inter / 8, p.tokens * p.top_k);
+    if (p.hidden <= 2048) {
+        if (int rc = raise_lds_limit(lim2, (const void*)few_routes_gate_up_kernel<QT, 2>, 160 * 1024, "few_routes_gate_up")) return rc;
+        hipLaunchKernelGGL((few_routes_gate_up_kernel<QT, 2>), grid, dim3(512), lds, s, p);
+    } else {
+        if (int rc = raise_lds_limit(lim4, (const void*)few_routes_gate_up_kernel<QT, 4>, 160 * 1024, "few_routes_gate_up")) return rc;
+        hipLaunchKernelGGL((few_routes_gate_up_kernel<QT, 4>), grid, dim3(512), lds, s, p);
+    }
+    return check_launch("few_routes_gate_up");
+}
+template <int QT>
+static int launch_down(const FewRoutesParams& p, hipStream_t s) {
+    static LdsLimit lim;
+    if (int rc = raise_lds_limit(lim, (const void*)few_routes_down_kernel<QT>, 160 * 1024, "few_routes_down")) return rc;
+    hipLaunchKernelGGL(few_routes_down_kernel<QT>, dim3((p.hidden + 15) / 16, p.tokens), dim3(512), down_lds_bytes(QT, p.row_bytes_down), s, p);
+    return check_launch("few_routes_down");
+}
+
+// Up to this many routes every route reads its own expert's weights.
+constexpr int64_t kFewRoutes = 64;
+
+bool few_routes_takes(int qt_in, int qt_down, int64_t tokens, int top_k, int64_t hidden, int64_t inter) {
+    return tokens > 0 && top_k > 0 && top_k <= 16 && tokens * top_k <= kFewRoutes && hidden <= 4096 && inter % 8 == 0 && hidden % 8 == 0 &&
+           gate_up_lds(qt_in, (int)packed_row_bytes(qt_in, hidden)) <= 80 * 1024 && down_lds_bytes(qt_down, (int)packed_row_bytes(qt_down, inter)) <= 160 * 1024;
+}
+
+int few_routes_forward(const void* x, const void* ids, int ids64, const void* weights, int weights_bf16, int64_t tokens, int top_k, int64_t experts, int64_t hidden,
+                       int64_t inter, int qt_in, int qt_down, const void* gate, const void* up, const void* down, const void* a1, const void* b1, int r1,
+                       const void* a2, const void* b2, int r2, float scale, float limit, void* act, void* out, hipStream_t s) {
+    FewRoutesParams p{};
+    p.x = (const bf16_t*)x, p.ids = ids, p.ids64 = ids64, p.weights = weights, p.weights_bf16 = weights_bf16;
+    p.tokens = (int)tokens, p.top_k = top_k, p.experts = (int)experts, p.hidden = (int)hidden, p.inter = (int)inter;
+    p.gate = (const uint8_t*)gate, p.up = (const uint8_t*)up, p.down = (const uint8_t*)down;
+    p.row_bytes_in = (int)packed_row_bytes(qt_in, hidden), p.row_bytes_down = (int)packed_row_bytes(qt_down, inter);
+    p.a1 = (const bf16_t*)a1, p.b1 = (const bf16_t*)b1, p.a2 = (const bf16_t*)a2, p.b2 = (const bf16_t*)b2, p.r1 = r1, p.r2 = r2;
+    p.scale = scale, p.limit = limit, p.act = (bf16_t*)act, p.out = (bf16_t*)out;
+#define GGQ_FEW(F, QT) \
+    case QT: rc = F<QT>(p, s); break
+    int rc = GGQ_ERR_QTYPE;
+    switch (qt_in) {
+        GGQ_FEW(launch_gate_up, kQ8_0); GGQ_FEW(launch_gate_up, kQ2_K); GGQ_FEW(launch_gate_up, kQ3_K); GGQ_FEW(launch_gate_up, kQ4_K);
+        GGQ_FEW(launch_gate_up, kQ5_K); GGQ_FEW(launch_gate_up, kQ6_K); GGQ_FEW(launch_gate_up, kIQ2_XXS);
+    }
+    if (rc) return rc;
+    rc = GGQ_ERR_QTYPE;
+    switch (qt_down) {
+        GGQ_FEW(launch_down, kQ8_0); GGQ_FEW(launch_down, kQ2_K); GGQ_FEW(launch_down, kQ3_K); GGQ_FEW(launch_down, kQ4_K);
+        GGQ_FEW(launch_down, kQ5_K); GGQ_FEW(launch_down, kQ6_K); GGQ_FEW(launch_down, kIQ2_XXS);
+    }
+#undef GGQ_FEW
+    return rc;
+}
+
+}  // namespace ggq

@@ -200,6 +200,20 @@ Tensor experts_forward(const Tensor& x, const Tensor& ids, const Tensor& weights
     return out;
 }
 
+// The forward of a few routes (sampling): two launches, nothing kept.
+bool experts_few_routes(const Tensor& x, const Tensor& ids, const Tensor& weights, const Tensor& gate_w, const Tensor& up_w, const Tensor& down_w, const Tensor& a1,
+                        const Tensor& b1, const Tensor& a2, const Tensor& b2, const ExpertsOptions& o, Tensor& out) {
+    const int64_t tokens = ids.size(0), top_k = ids.size(1), inter = gate_w.size(1), hidden = down_w.size(1);
+    if (!ggq_experts_few_routes_takes((int)o.qt_gate_up, (int)o.qt_down, tokens, (int)top_k, hidden, inter)) return false;
+    Tensor act = empty({tokens * top_k, inter}, at::kBFloat16, x);
+    out = empty(x.sizes(), at::kBFloat16, x);
+    check(ggq_experts_few_routes_forward(x.data_ptr(), ids.data_ptr(), ids.scalar_type() == at::kLong, weights.data_ptr(), weights.scalar_type() == at::kBFloat16,
+                                         tokens, (int)top_k, gate_w.size(0), hidden, inter, (int)o.qt_gate_up, (int)o.qt_down, gate_w.data_ptr(), up_w.data_ptr(),
+                                         down_w.data_ptr(), ptr(a1), ptr(b1), a1.defined() ? (int)a1.size(1) : 0, ptr(a2), ptr(b2), a2.defined() ? (int)a2.size(1) : 0,
+                                         (float)o.scaling, (float)o.limit, act.data_ptr(), out.data_ptr(), stream_of(x)));
+    return true;
+}
+
 struct Experts : torch::autograd::Function<Experts> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& ids, const Tensor& weights, const Tensor& gate_w, const Tensor& up_w,
                           const Tensor& down_w, const Maybe& a1_in, const Maybe& b1_in, const Maybe& a2_in, const Maybe& b2_in, const Tensor& all_experts,
@@ -352,8 +366,7 @@ PyObject* host_experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         ReleaseGil nogil;
         if (any_requires_grad({&x, &weights, &a1, &b1, &a2, &b2})) {
             y = Experts::apply(x, ids, weights, gate, up, down, maybe(a1), maybe(b1), maybe(a2), maybe(b2), all_experts, qt1, qt2, scaling, limit);
-        } else {
-            ExpertsBuffers s;
+        } else if (ExpertsBuffers s; !experts_few_routes(x, ids, weights, gate, up, down, a1, b1, a2, b2, {qt1, qt2, scaling, limit}, y)) {
             y = experts_forward(x, ids, weights, gate, up, down, a1, b1, a2, b2, all_experts, {qt1, qt2, scaling, limit}, s);
         }
     }

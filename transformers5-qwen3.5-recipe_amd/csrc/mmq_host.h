@@ -160,6 +160,15 @@ int64_t dense_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s);
 void dense_force_shape(int shape, int splits);  // test aid: -1 = the automatic choice
 
+// Products of a few rows (gemv.hip).
+constexpr int kShapeFewRows = 7;  // (profile records only)
+bool gemv_takes(int qt, int64_t m, int64_t n, int64_t k, const void* x);
+int gemv(int qt, const void* x, const void* w, int64_t m, int64_t n, int64_t k, const void* lora_a, const void* lora_b, int r, float scale, void* xa_out, void* y, hipStream_t s);
+bool few_routes_takes(int qt_in, int qt_down, int64_t tokens, int top_k, int64_t hidden, int64_t inter);
+int few_routes_forward(const void* x, const void* ids, int ids64, const void* weights, int weights_bf16, int64_t tokens, int top_k, int64_t experts, int64_t hidden,
+                       int64_t inter, int qt_in, int qt_down, const void* gate, const void* up, const void* down, const void* a1, const void* b1, int r1,
+                       const void* a2, const void* b2, int r2, float scale, float limit, void* act, void* out, hipStream_t s);
+
 int pad_factor(const bf16_t* src, bf16_t* dst, int64_t experts, int c, int r, int r_pad, bool transpose, hipStream_t s);
 int transpose_factor(const bf16_t* src, bf16_t* dst, int64_t experts, int c, int r, hipStream_t s);
 int skinny_nt(const SkinnyNtParams& p, int r_pad, int grid_tiles, hipStream_t s);
