@@ -43,6 +43,58 @@ __device__ __forceinline__ int request_bytes(const uint8_t* src, uint8_t* dst, i
     return made;
 }
 
+// A run out of packed rows in LDS.  The blocks of most formats are only 2- or 4-byte aligned, and a wide LDS read that is not
+// aligned to its width is taken apart by the hardware (reading Q6_K runs with 16-byte reads kept the LDS busy for three
+// quarters of the kernel): those formats are read as aligned words, one more than the piece has, and shifted together.
+template <int N>
+__device__ __forceinline__ void lds_words(const uint8_t* lds, int off, uint32_t* out) {
+    const uint32_t* p = (const uint32_t*)(lds + (off & ~3));
+    uint32_t w[N + 1];
+#pragma unroll
+    for (int i = 0; i <= N; i++) w[i] = p[i];
+#pragma unroll
+    for (int i = 0; i < N; i++) out[i] = __builtin_amdgcn_alignbyte(w[i + 1], w[i], off & 3);
+}
+__device__ __forceinline__ uint32_t lds_half(const uint8_t* lds, int off) { return *(const uint16_t*)(lds + off); }
+__device__ __forceinline__ void lds_32_bytes(const uint8_t* lds, int off, uint4& a, uint4& b) {
+    uint32_t w[8];
+    lds_words<8>(lds, off, w);
+    a = make_uint4(w[0], w[1], w[2], w[3]), b = make_uint4(w[4], w[5], w[6], w[7]);
+}
+// row: byte offset of the row in `lds` (even)
+template <int QT>
+__device__ __forceinline__ void load_run(typename Fmt<QT>::Raw& r, const uint8_t* lds, int row, int ksub) {
+    if constexpr (QT == kQ4_K || QT == kQ5_K) {
+        Fmt<QT>::load(r, lds + row, ksub);  // whole 16-byte pieces
+    } else if constexpr (QT == kQ8_0) {
+        const int blk = row + ksub * 34;
+        r.d16 = lds_half(lds, blk);
+        lds_32_bytes(lds, blk + 2, r.q0, r.q1);
+    } else if constexpr (QT == kQ2_K) {
+        const int blk = row + (ksub >> 3) * 84, u = ksub & 7, n = u >> 2, sp = u & 3;
+        const uint32_t* p = (const uint32_t*)(lds + blk + 16 + 32 * n);  // (rows and blocks are multiples of four bytes)
+        r.q0 = make_uint4(p[0], p[1], p[2], p[3]), r.q1 = make_uint4(p[4], p[5], p[6], p[7]);
+        r.sc2 = lds_half(lds, blk + 8 * n + 2 * sp);
+        r.dd = *(const uint32_t*)(lds + blk + 80);
+    } else if constexpr (QT == kQ3_K) {
+        const int blk = row + (ksub >> 3) * 110, u = ksub & 7, n = u >> 2, g = u >> 1, b = 2 * (u & 1);
+        lds_32_bytes(lds, blk, r.h0, r.h1);
+        lds_32_bytes(lds, blk + 32 + 32 * n, r.q0, r.q1);
+        r.sl = lds_half(lds, blk + 96 + 4 * (g & 1) + b), r.sh = lds_half(lds, blk + 104 + b), r.d16 = lds_half(lds, blk + 108);
+    } else if constexpr (QT == kQ6_K) {
+        const int blk = row + (ksub >> 3) * 210, u = ksub & 7, h = u >> 2, p = u & 3;
+        lds_32_bytes(lds, blk + 64 * h + 32 * (p & 1), r.ql[0], r.ql[1]);
+        lds_32_bytes(lds, blk + 128 + 32 * h, r.qh[0], r.qh[1]);
+        r.sc2 = lds_half(lds, blk + 192 + 8 * h + 2 * p), r.d16 = lds_half(lds, blk + 208);
+    } else {
+        const int blk = row + (ksub >> 3) * 66;
+        uint32_t w[2];
+        r.d16 = lds_half(lds, blk);
+        lds_words<2>(lds, blk + 2 + 8 * (ksub & 7), w);
+        r.idx4 = w[0], r.aux = w[1];
+    }
+}
+
 // Eight consecutive factor elements p[0..valid) (zeros past it); vec: 16-byte aligned and whole.
 __device__ __forceinline__ uint4 load_factor8(const bf16_t* p, int valid, bool vec) {
     if (vec && valid >= 8) return *(const uint4*)p;
@@ -138,7 +190,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
         f32x4_t acc[TB];
 #pragma unroll
         for (int tb = 0; tb < TB; tb++) acc[tb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-        const uint8_t* row = stage + buf * p.stage_bytes + min(l16, p.n - block * 16 - 1) * p.row_bytes;
+        const int row = buf * p.stage_bytes + min(l16, p.n - block * 16 - 1) * p.row_bytes;
 #pragma unroll
         for (int sp = 0; sp < SP; sp++) {
             const int span = wave + WAVES * sp;
@@ -146,7 +198,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
             const int run = min(span * 4 + q, (p.k >> 5) - 1);
             typename Fmt<QT>::Raw raw;
             uint32_t v[16];
-            Fmt<QT>::load(raw, row, run);
+            load_run<QT>(raw, stage, row, run);
             Fmt<QT>::decode(raw, run, v, (const uint2*)gemv_lds);
 #pragma unroll
             for (int i = 0; i < 4; i++)
@@ -323,7 +375,7 @@ __global__ __launch_bounds__(512) void few_routes_gate_up_kernel(FewRoutesParams
     wait_loads_at_most(0);
     __syncthreads();
     f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-    const uint8_t* row = stage + l16 * p.row_bytes_in;  // rows 0..7 gate, 8..15 up
+    const int row = l16 * p.row_bytes_in;  // rows 0..7 gate, 8..15 up
     const int spans = (k + kSpan - 1) / kSpan;
 #pragma unroll
     for (int sp = 0; sp < SP; sp++) {
@@ -332,7 +384,7 @@ __global__ __launch_bounds__(512) void few_routes_gate_up_kernel(FewRoutesParams
         const int run = min(span * 4 + q, (k >> 5) - 1);
         typename Fmt<QT>::Raw raw;
         uint32_t v[16];
-        Fmt<QT>::load(raw, row, run);
+        load_run<QT>(raw, stage, row, run);
         Fmt<QT>::decode(raw, run, v, (const uint2*)gu_lds);
 #pragma unroll
         for (int i = 0; i < 4; i++) acc = mfma16(as_operand(make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3])), as_operand(xf[sp][i]), acc);
@@ -383,7 +435,7 @@ __global__ __launch_bounds__(512) void few_routes_down_kernel(FewRoutesParams p)
         f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f}, acc_a[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) acc_a[j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-        const uint8_t* row = mine + min(l16, rows - 1) * p.row_bytes_down;
+        const int row = min(l16, rows - 1) * p.row_bytes_down;
         for (int s0 = 0; s0 < spans; s0 += 4) {  // four spans of x in registers at a time, requested together
             uint4 xf[4][4];
 #pragma unroll
@@ -412,7 +464,7 @@ __global__ __launch_bounds__(512) void few_routes_down_kernel(FewRoutesParams p)
                 const int run = min((s0 + u) * 4 + q, (k >> 5) - 1);  // (past the end x is zero)
                 typename Fmt<QT>::Raw raw;
                 uint32_t v[16];
-                Fmt<QT>::load(raw, row, run);
+                load_run<QT>(raw, mine, row, run);
                 Fmt<QT>::decode(raw, run, v, (const uint2*)down_lds);
 #pragma unroll
                 for (int i = 0; i < 4; i++) acc = mfma16(as_operand(make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3])), as_operand(xf[u][i]), acc);
