@@ -64,34 +64,114 @@ __device__ __forceinline__ void lds_32_bytes(const uint8_t* lds, int off, uint4&
 // row: byte offset of the row in `lds` (even)
 template <int QT>
 __device__ __forceinline__ void load_run(typename Fmt<QT>::Raw& r, const uint8_t* lds, int row, int ksub) {
-    if constexpr (QT == kQ4_K || QT == kQ5_K) {
+    if constexpr (QT == kQ5_K) {
         Fmt<QT>::load(r, lds + row, ksub);  // whole 16-byte pieces
     } else if constexpr (QT == kQ8_0) {
         const int blk = row + ksub * 34;
         r.d16 = lds_half(lds, blk);
         lds_32_bytes(lds, blk + 2, r.q0, r.q1);
-    } else if constexpr (QT == kQ2_K) {
-        const int blk = row + (ksub >> 3) * 84, u = ksub & 7, n = u >> 2, sp = u & 3;
-        const uint32_t* p = (const uint32_t*)(lds + blk + 16 + 32 * n);  // (rows and blocks are multiples of four bytes)
-        r.q0 = make_uint4(p[0], p[1], p[2], p[3]), r.q1 = make_uint4(p[4], p[5], p[6], p[7]);
-        r.sc2 = lds_half(lds, blk + 8 * n + 2 * sp);
-        r.dd = *(const uint32_t*)(lds + blk + 80);
     } else if constexpr (QT == kQ3_K) {
         const int blk = row + (ksub >> 3) * 110, u = ksub & 7, n = u >> 2, g = u >> 1, b = 2 * (u & 1);
         lds_32_bytes(lds, blk, r.h0, r.h1);
         lds_32_bytes(lds, blk + 32 + 32 * n, r.q0, r.q1);
         r.sl = lds_half(lds, blk + 96 + 4 * (g & 1) + b), r.sh = lds_half(lds, blk + 104 + b), r.d16 = lds_half(lds, blk + 108);
-    } else if constexpr (QT == kQ6_K) {
-        const int blk = row + (ksub >> 3) * 210, u = ksub & 7, h = u >> 2, p = u & 3;
-        lds_32_bytes(lds, blk + 64 * h + 32 * (p & 1), r.ql[0], r.ql[1]);
-        lds_32_bytes(lds, blk + 128 + 32 * h, r.qh[0], r.qh[1]);
-        r.sc2 = lds_half(lds, blk + 192 + 8 * h + 2 * p), r.d16 = lds_half(lds, blk + 208);
     } else {
         const int blk = row + (ksub >> 3) * 66;
         uint32_t w[2];
         r.d16 = lds_half(lds, blk);
         lds_words<2>(lds, blk + 2 + 8 * (ksub & 7), w);
         r.idx4 = w[0], r.aux = w[1];
+    }
+}
+
+// The sixteen operand words of a lane for one span of a row: words 4 i .. 4 i + 3 go to MFMA i.
+//
+// Two ways to deal the span's 128 elements to the four lanes of a row.  A contraction may be summed in any order, so each
+// format takes the cheaper one and the other operand follows (span_element):
+//  * by run (Q8_0, Q3_K, Q5_K, IQ2_XXS): lane q owns run q, MFMA i its elements 8 i .. 8 i + 7;
+//  * by position (Q2_K, Q4_K, Q6_K, whose runs share bytes): lane q owns elements 8 q .. 8 q + 7 of all four runs, MFMA i those
+//    of run i: every byte is read and taken apart once (Q6_K by run: 64 bytes and 148 vector instructions per lane and span).
+template <int QT>
+constexpr bool kByPosition = QT == kQ2_K || QT == kQ4_K || QT == kQ6_K;
+template <int QT>
+__device__ __forceinline__ int span_element(int q, int i) { return kByPosition<QT> ? 32 * i + 8 * q : 32 * q + 8 * i; }
+
+// Four small integers in the bytes of w (below 256) -> four bf16 of value scale * integer + offset.
+__device__ __forceinline__ void four_values(uint32_t w, float scale24, float offset, uint32_t* out) {
+    const uint32_t e02 = w & 0x00FF00FFu, e13 = (w >> 8) & 0x00FF00FFu;
+    out[0] = pack_bf16(mix_lo(e02, scale24, offset), mix_lo(e13, scale24, offset));
+    out[1] = pack_bf16(mix_hi(e02, scale24, offset), mix_hi(e13, scale24, offset));
+}
+
+template <int QT>
+__device__ __forceinline__ void decode_span(const uint8_t* lds, int row, int span, int runs, int q, uint32_t* v, const uint2* tables) {
+    if constexpr (QT == kQ4_K) {
+        const uint8_t* blk = lds + row + (span >> 1) * 144;
+        const int h = span & 1;
+        const uint4 hdr = *(const uint4*)blk;
+        const uint2 g0 = *(const uint2*)(blk + 16 + 64 * h + 8 * q), g1 = *(const uint2*)(blk + 48 + 64 * h + 8 * q);
+        const float d = half_bits_to_f32(hdr.x & 0xFFFFu) * kMixScale, dmin = half_bits_to_f32(hdr.x >> 16);
+        // (scale, min) of the four runs, one per byte
+        const uint32_t sc = h ? (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u) : hdr.y & 0x3F3F3F3Fu;
+        const uint32_t mn = h ? ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u) : hdr.z & 0x3F3F3F3Fu;
+        const uint32_t so = opaque(sc), mo = opaque(mn);
+        const float dl[4] = {d * ubyte0(so), d * ubyte1(so), d * ubyte2(so), d * ubyte3(so)};
+        const float nm[4] = {-(dmin * ubyte0(mo)), -(dmin * ubyte1(mo)), -(dmin * ubyte2(mo)), -(dmin * ubyte3(mo))};
+        const uint32_t w[4] = {g0.x, g0.y, g1.x, g1.y};
+#pragma unroll
+        for (int g = 0; g < 2; g++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const uint32_t b = w[2 * g + u];
+                const uint32_t lo02 = b & 0x000F000Fu, hi02 = (b >> 4) & 0x000F000Fu, lo13 = (b >> 8) & 0x000F000Fu, hi13 = (b >> 12) & 0x000F000Fu;
+                uint32_t* even = v + 8 * g + 2 * u;
+                even[0] = pack_bf16(mix_lo(lo02, dl[2 * g], nm[2 * g]), mix_lo(lo13, dl[2 * g], nm[2 * g]));
+                even[1] = pack_bf16(mix_hi(lo02, dl[2 * g], nm[2 * g]), mix_hi(lo13, dl[2 * g], nm[2 * g]));
+                even[4] = pack_bf16(mix_lo(hi02, dl[2 * g + 1], nm[2 * g + 1]), mix_lo(hi13, dl[2 * g + 1], nm[2 * g + 1]));
+                even[5] = pack_bf16(mix_hi(hi02, dl[2 * g + 1], nm[2 * g + 1]), mix_hi(hi13, dl[2 * g + 1], nm[2 * g + 1]));
+            }
+    } else if constexpr (QT == kQ6_K) {
+        const int blk = row + (span >> 1) * 210, h = span & 1;
+        uint32_t a[2], b[2], c[2];
+        lds_words<2>(lds, blk + 64 * h + 8 * q, a);
+        lds_words<2>(lds, blk + 64 * h + 32 + 8 * q, b);
+        lds_words<2>(lds, blk + 128 + 32 * h + 8 * q, c);
+        const float d = half_bits_to_f32(lds_half(lds, blk + 208));
+        uint32_t sw[2];
+        lds_words<2>(lds, blk + 192 + 8 * h, sw);  // the half's eight scales; run i takes scale 2 i + q / 2
+        const int sh = (q >> 1) * 8;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float s = d * (float)(int)(int8_t)((sw[i >> 1] >> (16 * (i & 1) + sh)) & 0xFFu);
+            const float s24 = s * kMixScale, off = -32.0f * s;
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const uint32_t nib = i == 0 ? a[u] & 0x0F0F0F0Fu : i == 1 ? b[u] & 0x0F0F0F0Fu : i == 2 ? (a[u] >> 4) & 0x0F0F0F0Fu : (b[u] >> 4) & 0x0F0F0F0Fu;
+                const uint32_t two = i == 0 ? c[u] << 4 : i == 1 ? c[u] << 2 : i == 2 ? c[u] : c[u] >> 2;
+                four_values(nib | (two & 0x30303030u), s24, off, v + 4 * i + 2 * u);
+            }
+        }
+    } else if constexpr (QT == kQ2_K) {
+        const uint8_t* blk = lds + row + (span >> 1) * 84;  // (rows and blocks are multiples of four bytes)
+        const int n = span & 1;
+        const uint32_t* w = (const uint32_t*)(blk + 16 + 32 * n + 8 * q);
+        const uint32_t w0 = w[0], w1 = w[1], dd = *(const uint32_t*)(blk + 80);
+        const uint32_t* s8 = (const uint32_t*)(blk + 8 * n);  // the half's eight scale bytes; run i takes byte 2 i + q / 2
+        const uint32_t sw[2] = {s8[0], s8[1]};
+        const int sh = (q >> 1) * 8;
+        const float d = half_bits_to_f32(dd & 0xFFFFu) * kMixScale, dmin = half_bits_to_f32(dd >> 16);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t sb = (sw[i >> 1] >> (16 * (i & 1) + sh)) & 0xFFu;
+            const float dl = d * (float)(sb & 0xFu), nm = -(dmin * (float)(sb >> 4));
+            four_values((w0 >> (2 * i)) & 0x03030303u, dl, nm, v + 4 * i);
+            four_values((w1 >> (2 * i)) & 0x03030303u, dl, nm, v + 4 * i + 2);
+        }
+    } else {
+        const int run = min(span * 4 + q, runs - 1);
+        typename Fmt<QT>::Raw raw;
+        load_run<QT>(raw, lds, row, run);
+        Fmt<QT>::decode(raw, run, v, tables);
     }
 }
 
@@ -121,7 +201,7 @@ struct GemvParams {
 };
 
 // WAVES waves deal the spans of the contraction out (span s to wave s % WAVES, at most SP each); TB blocks of sixteen rows of x.
-template <int QT, int WAVES, int SP, int TB>
+template <int QT, int WAVES, int SP, int TB>  // TB <= WAVES
 __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t gemv_lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -143,11 +223,12 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
     for (int sp = 0; sp < SP; sp++)
 #pragma unroll
         for (int tb = 0; tb < TB; tb++) {
-            const int row = min(tb * 16 + l16, p.m - 1), e0 = (wave + WAVES * sp) * kSpan + 32 * q;
-            const bool live = e0 < p.k;  // (k is a multiple of 32: a run is whole or absent)
-            const uint4* src = (const uint4*)(p.x + (int64_t)row * p.k + (live ? e0 : 0));
+            const bf16_t* src = p.x + (int64_t)min(tb * 16 + l16, p.m - 1) * p.k;
 #pragma unroll
-            for (int i = 0; i < 4; i++) xf[sp][tb][i] = live ? src[i] : make_uint4(0, 0, 0, 0);
+            for (int i = 0; i < 4; i++) {
+                const int e = (wave + WAVES * sp) * kSpan + span_element<QT>(q, i);
+                xf[sp][tb][i] = e < p.k ? *(const uint4*)(src + e) : make_uint4(0, 0, 0, 0);  // (k is a multiple of 32: eight elements are whole or absent)
+            }
         }
     if (p.lora_a) {  // x A^T over this wave's spans, added over the waves, kept as bf16 rows in LDS
         for (int r0 = 0; r0 < p.r_pad; r0 += 16) {
@@ -157,11 +238,12 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
             const bf16_t* arow = p.lora_a + (int64_t)min(r0 + l16, p.r - 1) * p.k;
 #pragma unroll
             for (int sp = 0; sp < SP; sp++) {
-                const int e0 = (wave + WAVES * sp) * kSpan + 32 * q;
-                const bool live = e0 < p.k && r0 + l16 < p.r;
                 uint4 a[4];
 #pragma unroll
-                for (int i = 0; i < 4; i++) a[i] = live ? ((const uint4*)(arow + e0))[i] : make_uint4(0, 0, 0, 0);
+                for (int i = 0; i < 4; i++) {
+                    const int e = (wave + WAVES * sp) * kSpan + span_element<QT>(q, i);
+                    a[i] = e < p.k && r0 + l16 < p.r ? *(const uint4*)(arow + e) : make_uint4(0, 0, 0, 0);
+                }
 #pragma unroll
                 for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -187,6 +269,11 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
         if (p.buffers == 2 && next < blocks) wait_loads_at_most(request_block(next, buf ^ 1));
         else wait_loads_at_most(0);
         lds_barrier();
+        // the factor rows of the block's LoRA term, for the waves that will add it, ahead of the work they would wait behind
+        const bool adds = (wave + block) % WAVES < TB;
+        const bf16_t* brow = p.lora_b + (int64_t)min(block * 16 + l16, p.n - 1) * p.r;
+        uint4 b0 = make_uint4(0, 0, 0, 0);
+        if (p.lora_a && adds) b0 = load_factor8(brow + 8 * q, p.r - 8 * q, b_vec);
         f32x4_t acc[TB];
 #pragma unroll
         for (int tb = 0; tb < TB; tb++) acc[tb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
@@ -195,11 +282,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
         for (int sp = 0; sp < SP; sp++) {
             const int span = wave + WAVES * sp;
             if (span >= spans) break;  // uniform over the wave
-            const int run = min(span * 4 + q, (p.k >> 5) - 1);
-            typename Fmt<QT>::Raw raw;
             uint32_t v[16];
-            load_run<QT>(raw, stage, row, run);
-            Fmt<QT>::decode(raw, run, v, (const uint2*)gemv_lds);
+            decode_span<QT>(stage, row, span, p.k >> 5, q, v, (const uint2*)gemv_lds);
 #pragma unroll
             for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -211,16 +295,15 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
         lds_barrier();
         if (p.buffers == 1 && next < blocks) request_block(next, 0);
         // (a buffer is refilled, and the partial sums rewritten, only behind the next barrier)
-        for (int tb = (wave + block) % WAVES; tb < TB; tb += WAVES) {
+        if (const int tb = (wave + block) % WAVES; adds) {
             f32x4_t sum = red[tb * 64 + lane];
             for (int w = 1; w < WAVES; w++) sum += red[(w * TB + tb) * 64 + lane];
             const int col = block * 16 + 4 * q, xrow = tb * 16 + l16;
             if (p.lora_a) {
                 f32x4_t lo = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-                const bf16_t* brow = p.lora_b + (int64_t)min(block * 16 + l16, p.n - 1) * p.r;
                 for (int r0 = 0; r0 < p.r_pad; r0 += 32) {
                     const int j = r0 + 8 * q;
-                    const uint4 b = load_factor8(brow + j, p.r - j, b_vec);
+                    const uint4 b = r0 == 0 ? b0 : load_factor8(brow + j, p.r - j, b_vec);
                     const uint4 xv = j < p.r_pad ? *(const uint4*)(xa + xrow * 64 + j) : make_uint4(0, 0, 0, 0);
                     lo = mfma16(as_operand(b), as_operand(xv), lo);
                 }
@@ -318,11 +401,11 @@ __device__ __forceinline__ int route_expert(const FewRoutesParams& p, int route)
 }
 
 // sum over j of b[j] * xa[j] for the sixteen rows of a block: lane (row lane % 16, quarter) takes every fourth group of eight
-// ranks; every lane of a row returns the row's sum.
-__device__ __forceinline__ float lora_row_dot(const bf16_t* brow, const bf16_t* xa, int r, bool vec, int q) {
+// ranks, the first of them loaded by the caller ahead of the work it would wait behind; every lane of a row returns the sum.
+__device__ __forceinline__ float lora_row_dot(const uint4& first, const bf16_t* brow, const bf16_t* xa, int r, bool vec, int q) {
     float s = 0.f;
     for (int j = 8 * q; j < r; j += 32) {
-        const uint4 b = load_factor8(brow + j, r - j, vec), x = *(const uint4*)(xa + j);
+        const uint4 b = j < 32 ? first : load_factor8(brow + j, r - j, vec), x = *(const uint4*)(xa + j);
         const uint32_t bw[4] = {b.x, b.y, b.z, b.w}, xw[4] = {x.x, x.y, x.z, x.w};
 #pragma unroll
         for (int i = 0; i < 4; i++) s = fmaf(bf16_lo(bw[i]), bf16_lo(xw[i]), s), s = fmaf(bf16_hi(bw[i]), bf16_hi(xw[i]), s);
@@ -352,11 +435,17 @@ __global__ __launch_bounds__(512) void few_routes_gate_up_kernel(FewRoutesParams
     uint4 xf[SP][4];
 #pragma unroll
     for (int sp = 0; sp < SP; sp++) {
-        const int e0 = (wave + WAVES * sp) * kSpan + 32 * q;
 #pragma unroll
-        for (int i = 0; i < 4; i++) xf[sp][i] = e0 < k ? ((const uint4*)(x + e0))[i] : make_uint4(0, 0, 0, 0);
+        for (int i = 0; i < 4; i++) {
+            const int e = (wave + WAVES * sp) * kSpan + span_element<QT>(q, i);
+            xf[sp][i] = e < k ? *(const uint4*)(x + e) : make_uint4(0, 0, 0, 0);
+        }
     }
     const int r_pad = (p.r1 + 15) & ~15;
+    const bool b_vec = (p.r1 & 7) == 0;
+    const bf16_t* brow = p.b1 + ((int64_t)expert * 2 * p.inter + (l16 < 8 ? i0 + l16 : p.inter + i0 + l16 - 8)) * p.r1;
+    uint4 b0 = make_uint4(0, 0, 0, 0);
+    if (p.a1 && wave == 0) b0 = load_factor8(brow + 8 * q, p.r1 - 8 * q, b_vec);
     if (p.a1) {
         const bf16_t* a = p.a1 + (int64_t)expert * p.r1 * k;
         for (int r0 = 0; r0 < r_pad; r0 += 16) {
@@ -364,10 +453,11 @@ __global__ __launch_bounds__(512) void few_routes_gate_up_kernel(FewRoutesParams
             const bf16_t* arow = a + (int64_t)min(r0 + l16, p.r1 - 1) * k;
 #pragma unroll
             for (int sp = 0; sp < SP; sp++) {
-                const int e0 = (wave + WAVES * sp) * kSpan + 32 * q;
-                const bool live = e0 < k && r0 + l16 < p.r1;
 #pragma unroll
-                for (int i = 0; i < 4; i++) acc = mfma16(as_operand(live ? ((const uint4*)(arow + e0))[i] : make_uint4(0, 0, 0, 0)), as_operand(xf[sp][i]), acc);
+                for (int i = 0; i < 4; i++) {
+                    const int e = (wave + WAVES * sp) * kSpan + span_element<QT>(q, i);
+                    acc = mfma16(as_operand(e < k && r0 + l16 < p.r1 ? *(const uint4*)(arow + e) : make_uint4(0, 0, 0, 0)), as_operand(xf[sp][i]), acc);
+                }
             }
             if (l16 == 0) *(f32x4_t*)(red_xa + wave * 64 + r0 + 4 * q) = acc;
         }
@@ -381,11 +471,8 @@ __global__ __launch_bounds__(512) void few_routes_gate_up_kernel(FewRoutesParams
     for (int sp = 0; sp < SP; sp++) {
         const int span = wave + WAVES * sp;
         if (span >= spans) break;
-        const int run = min(span * 4 + q, (k >> 5) - 1);
-        typename Fmt<QT>::Raw raw;
         uint32_t v[16];
-        load_run<QT>(raw, stage, row, run);
-        Fmt<QT>::decode(raw, run, v, (const uint2*)gu_lds);
+        decode_span<QT>(stage, row, span, k >> 5, q, v, (const uint2*)gu_lds);
 #pragma unroll
         for (int i = 0; i < 4; i++) acc = mfma16(as_operand(make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3])), as_operand(xf[sp][i]), acc);
     }
@@ -400,10 +487,7 @@ __global__ __launch_bounds__(512) void few_routes_gate_up_kernel(FewRoutesParams
     if (wave > 0) return;
     float y = 0.f;  // of row l16, in all four quarters
     for (int w = 0; w < WAVES; w++) y += red[w * 16 + l16];
-    if (p.a1) {
-        const int64_t brow = (int64_t)expert * 2 * p.inter + (l16 < 8 ? i0 + l16 : p.inter + i0 + l16 - 8);
-        y = fmaf(p.scale, lora_row_dot(p.b1 + brow * p.r1, xa, p.r1, (p.r1 & 7) == 0, q), y);
-    }
+    if (p.a1) y = fmaf(p.scale, lora_row_dot(b0, brow, xa, p.r1, b_vec, q), y);
     y = bf16_to_f32(to_bf16(y));
     const float up = __shfl(y, (lane & 7) + 8, 64), gate = __shfl(y, lane & 7, 64);
     if (lane < 8) {
@@ -432,6 +516,10 @@ __global__ __launch_bounds__(512) void few_routes_down_kernel(FewRoutesParams p)
         request_bytes(p.down + ((int64_t)expert * p.hidden + h0) * p.row_bytes_down, mine, rows * p.row_bytes_down, 0, 1, lane);
         const bf16_t* x = p.act + (int64_t)route * k;
         const bf16_t* a = p.a2 ? p.a2 + (int64_t)expert * p.r2 * k : nullptr;
+        const bool b_vec = (p.r2 & 7) == 0;
+        const bf16_t* brow = p.b2 + ((int64_t)expert * p.hidden + min(h0 + l16, p.hidden - 1)) * p.r2;
+        uint4 b0 = make_uint4(0, 0, 0, 0);
+        if (a) b0 = load_factor8(brow + 8 * q, p.r2 - 8 * q, b_vec);
         f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f}, acc_a[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) acc_a[j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
@@ -440,9 +528,11 @@ __global__ __launch_bounds__(512) void few_routes_down_kernel(FewRoutesParams p)
             uint4 xf[4][4];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                const int e0 = (s0 + u) * kSpan + 32 * q;
 #pragma unroll
-                for (int i = 0; i < 4; i++) xf[u][i] = e0 < k ? ((const uint4*)(x + e0))[i] : make_uint4(0, 0, 0, 0);
+                for (int i = 0; i < 4; i++) {
+                    const int e = (s0 + u) * kSpan + span_element<QT>(q, i);
+                    xf[u][i] = e < k ? *(const uint4*)(x + e) : make_uint4(0, 0, 0, 0);
+                }
             }
             if (a) {
 #pragma unroll
@@ -451,21 +541,20 @@ __global__ __launch_bounds__(512) void few_routes_down_kernel(FewRoutesParams p)
                     const bf16_t* arow = a + (int64_t)min(16 * j + l16, p.r2 - 1) * k;
 #pragma unroll
                     for (int u = 0; u < 4; u++) {
-                        const int e0 = (s0 + u) * kSpan + 32 * q;
-                        const bool live = e0 < k && 16 * j + l16 < p.r2;
 #pragma unroll
-                        for (int i = 0; i < 4; i++) acc_a[j] = mfma16(as_operand(live ? ((const uint4*)(arow + e0))[i] : make_uint4(0, 0, 0, 0)), as_operand(xf[u][i]), acc_a[j]);
+                        for (int i = 0; i < 4; i++) {
+                            const int e = (s0 + u) * kSpan + span_element<QT>(q, i);
+                            acc_a[j] = mfma16(as_operand(e < k && 16 * j + l16 < p.r2 ? *(const uint4*)(arow + e) : make_uint4(0, 0, 0, 0)), as_operand(xf[u][i]), acc_a[j]);
+                        }
                     }
                 }
             }
             if (s0 == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                const int run = min((s0 + u) * 4 + q, (k >> 5) - 1);  // (past the end x is zero)
-                typename Fmt<QT>::Raw raw;
+                if (s0 + u >= spans) break;  // uniform
                 uint32_t v[16];
-                load_run<QT>(raw, mine, row, run);
-                Fmt<QT>::decode(raw, run, v, (const uint2*)down_lds);
+                decode_span<QT>(mine, row, s0 + u, k >> 5, q, v, (const uint2*)down_lds);
 #pragma unroll
                 for (int i = 0; i < 4; i++) acc = mfma16(as_operand(make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3])), as_operand(xf[u][i]), acc);
             }
@@ -478,7 +567,7 @@ __global__ __launch_bounds__(512) void few_routes_down_kernel(FewRoutesParams p)
         if (l16 == 0) *(f32x4_t*)(red + rank * 16 + 4 * q) = acc;
         if (p.a2) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            const float dot = lora_row_dot(p.b2 + ((int64_t)expert * p.hidden + min(h0 + l16, p.hidden - 1)) * p.r2, xa, p.r2, (p.r2 & 7) == 0, q);
+            const float dot = lora_row_dot(b0, brow, xa, p.r2, b_vec, q);
             if (q == 0) red[rank * 16 + l16] = fmaf(p.scale, dot, red[rank * 16 + l16]);
         }
     }

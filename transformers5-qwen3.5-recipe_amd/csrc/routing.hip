@@ -682,9 +682,8 @@ int swiglu_bwd(const void* gate, const void* up, const void* dh, void* dgate, vo
 
 // ------------------------------------------------------------------------------------------------
 // Router top-k: per token the top_k best of up to 256 expert scores, best first, equal scores in ascending
-// expert index.  One wave per token; lane l holds experts 4l .. 4l+3.  The order is that of the packed key
-// (monotone map of the fp32 score bits) << 16 | (256 - expert): the maximum of the keys is the best score and,
-// among equal scores, the smallest index.  Score functions: 0 = the logit itself (bf16 logits compare as the
+// expert index.  One wave per token; lane l holds experts 4l .. 4l+3.  The order is that of the monotone map of the fp32
+// score bits, and among equal scores that of the expert index.  Score functions: 0 = the logit itself (bf16 logits compare as the
 // fp32 values they are), 1 = sqrt(softplus(logit)) in fp32 plus an optional per-expert bias.
 // Optional routing weights of the selected experts: 1 = softmax over the selected logits in fp32, stored in the
 // logits' type; 2 = sqrt(softplus(logit)) (no bias) / (sum + 1e-20) * scale, stored as fp32.
@@ -693,6 +692,22 @@ __device__ __forceinline__ uint32_t float_order_key(float v) {
     return b ^ ((b & 0x80000000u) ? 0xFFFFFFFFu : 0x80000000u);
 }
 __device__ __forceinline__ float sqrt_softplus(float x) { return sqrtf(fmaxf(x, 0.0f) + logf(1.0f + expf(-fabsf(x)))); }
+
+// Maximum over the 64 lanes, the same in every lane: five data-parallel moves inside rows of sixteen and across them leave it
+// in lane 63.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_max_u32(uint32_t x) {
+    return max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xF, false));
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
+    x = dpp_max_u32<0x111, 0xF>(x);  // row_shr:1
+    x = dpp_max_u32<0x112, 0xF>(x);  // row_shr:2
+    x = dpp_max_u32<0x114, 0xF>(x);  // row_shr:4
+    x = dpp_max_u32<0x118, 0xF>(x);  // row_shr:8
+    x = dpp_max_u32<0x142, 0xA>(x);  // row_bcast:15 into rows 1 and 3
+    x = dpp_max_u32<0x143, 0xC>(x);  // row_bcast:31 into rows 2 and 3
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
 
 template <bool BF16>
 __global__ __launch_bounds__(256) void router_topk_kernel(const void* logits, int64_t tokens, int experts, int top_k, const float* bias,
@@ -713,7 +728,8 @@ __global__ __launch_bounds__(256) void router_topk_kernel(const void* logits, in
             v[0] = r.x, v[1] = r.y, v[2] = r.z, v[3] = r.w;
         }
     }
-    uint64_t key[4];
+    // keys are at least 1: 0 stands for an expert that is absent or already taken
+    uint32_t key[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         float sc = v[j];
@@ -721,30 +737,29 @@ __global__ __launch_bounds__(256) void router_topk_kernel(const void* logits, in
             sc = sqrt_softplus(sc);
             if (bias && e0 < experts) sc += bias[e0 + j];
         }
-        key[j] = e0 < experts ? ((uint64_t)float_order_key(sc) << 16) | (uint64_t)(256 - (e0 + j)) : 0ull;
+        key[j] = e0 < experts ? max(float_order_key(sc), 1u) : 0u;
     }
     float my_logit = 0.0f;  // lane t ends up with the logit of the rank-t expert
+    int my_expert = 0;
     for (int t = 0; t < top_k; t++) {
-        uint64_t best = key[0];
+        // The best key through data-parallel moves (the crossbar behind __shfl takes several times as long), then the first
+        // expert that has it: lanes hold experts in ascending order.
+        const uint32_t best = wave_max_u32(max(max(key[0], key[1]), max(key[2], key[3])));
+        int expert = 1 << 30;
 #pragma unroll
-        for (int j = 1; j < 4; j++) best = key[j] > best ? key[j] : best;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const uint32_t lo = __shfl_xor((uint32_t)best, off), hi = __shfl_xor((uint32_t)(best >> 32), off);
-            const uint64_t other = ((uint64_t)hi << 32) | lo;
-            best = other > best ? other : best;
+        for (int j = 0; j < 4; j++) {
+            const unsigned long long has = __ballot(key[j] == best);
+            if (has) expert = min(expert, 4 * (int)__builtin_ctzll(has) + j);
         }
-        const int expert = 256 - (int)(best & 0xFFFFu);
-        float lg = 0.0f;  // the winner's logit, from the lane that holds it
+        const int owner = expert >> 2, slot = expert & 3;
+        const float mine = slot == 0 ? v[0] : slot == 1 ? v[1] : slot == 2 ? v[2] : v[3];
+        const float lg = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine), owner));
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            if (key[j] == best && best != 0ull) lg = v[j], key[j] = 0ull;
-        // (one lane at most had the key: packed keys are distinct)
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) lg += __shfl_xor(lg, off);
-        if (lane == t) my_logit = lg;
-        if (lane == 0) indices[row * top_k + t] = expert;
+            if (lane == owner && slot == j) key[j] = 0u;
+        if (lane == t) my_logit = lg, my_expert = expert;
     }
+    if (lane < top_k) indices[row * top_k + lane] = my_expert;
     if (weights_mode == 0 || !weights) return;
     const bool in = lane < top_k;
     if (weights_mode == 1) {
