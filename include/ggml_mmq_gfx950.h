@@ -271,6 +271,10 @@ int ggq_swiglu_backward(const void* gate, const void* up, const void* dh, void* 
 int ggq_swiglu_clamped_forward(const void* gate, const void* up, void* h, int64_t elems, float limit, void* stream);
 int ggq_swiglu_clamped_backward(const void* gate, const void* up, const void* dh, void* dgate, void* dup, int64_t elems, float limit, void* stream);
 
+/* Router logits of 1 to 8 tokens, as while sampling: logits [tokens, experts] = hidden_states [tokens, hidden] . weight
+ * [experts, hidden]^T, all bf16 with fp32 sums (fast_moe_ranking.py:273-284; more tokens are a plain library product). */
+int ggq_router_logits(const void* hidden_states, const void* weight, int64_t tokens, int64_t experts, int64_t hidden, void* logits, void* stream);
+
 /* router_topk_indices (fast_moe_ranking.py:197-271; Triton kernel :163-194, key order :71-80 and :119-160): per
  * token the top_k experts of up to 256 router scores, best first, equal scores in ascending expert index.
  *   score_function 0: the logit itself (bf16 or fp32); 1: sqrt(softplus(logit)) in fp32 plus the optional

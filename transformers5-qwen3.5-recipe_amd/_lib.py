@@ -56,6 +56,7 @@ SIGNATURES: dict[str, tuple] = {
     "ggq_route_gather_backward": (_I, [_P, _P, _P, _L, _I, _I, _P]),
     "ggq_route_combine_forward": (_I, [_P, _P, _I, _P, _P, _L, _I, _I, _P]),
     "ggq_route_combine_backward": (_I, [_P, _P, _I, _P, _P, _P, _P, _L, _I, _I, _P]),
+    "ggq_router_logits": (_I, [_P, _P, _L, _L, _L, _P, _P]),
     "ggq_router_topk": (_I, [_P, _I, _L, _I, _I, _P, _I, _P, _P, _I, _F, _P]),
     "ggq_swiglu_forward": (_I, [_P, _P, _P, _L, _P]),
     "ggq_swiglu_backward": (_I, [_P, _P, _P, _P, _P, _L, _P]),

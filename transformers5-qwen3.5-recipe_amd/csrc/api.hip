@@ -757,6 +757,11 @@ int ggq_ptgmm(const void* lhs, const void* grad_out, const int32_t* group_sizes,
     return grouped_gemm_transposed(lhs, grad_out, group_sizes, out, m, k, n, experts, is_f16, ws, ws_bytes, as_stream(stream));
 }
 
+int ggq_router_logits(const void* hidden_states, const void* weight, int64_t tokens, int64_t experts, int64_t hidden, void* logits, void* stream) {
+    if (!hidden_states || !weight || !logits) return set_error(GGQ_ERR_NULL, "router_logits: null pointer");
+    return router_logits(hidden_states, weight, tokens, experts, hidden, logits, as_stream(stream));
+}
+
 int ggq_router_topk(const void* logits, int logits_are_bf16, int64_t tokens, int num_experts, int top_k, const float* correction_bias,
                     int score_function, int64_t* indices, void* weights, int weights_mode, float routed_scaling, void* stream) {
     return router_topk(logits, logits_are_bf16, tokens, num_experts, top_k, correction_bias, score_function, indices, weights,

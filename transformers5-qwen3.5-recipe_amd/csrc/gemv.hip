@@ -372,6 +372,47 @@ int gemv(int qt, const void* x, const void* w, int64_t m, int64_t n, int64_t k, 
 }
 
 // ------------------------------------------------------------------------------------------------
+// Router logits of up to sixteen tokens: y [m, n] = x [m, k] . w [n, k]^T, all bf16.  A workgroup takes sixteen weight rows, its
+// eight waves deal the contraction out in spans of 128.  (A library product of this size costs 19 us of host time per call.)
+__global__ __launch_bounds__(512) void few_rows_bf16_kernel(const bf16_t* x, const bf16_t* w, int m, int n, int k, bf16_t* y) {
+    constexpr int WAVES = 8;
+    __shared__ f32x4_t red[WAVES][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, q = lane >> 4, n0 = blockIdx.x * 16;
+    const bf16_t* wr = w + (int64_t)min(n0 + l16, n - 1) * k;
+    const bf16_t* xr = x + (int64_t)min(l16, m - 1) * k;
+    f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    const int steps = (k + kSpan - 1) / kSpan;
+    for (int s = wave; s < steps; s += WAVES) {
+        uint4 a[4], b[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int e = s * kSpan + 32 * i + 8 * q;
+            a[i] = e < k ? *(const uint4*)(wr + e) : make_uint4(0, 0, 0, 0);
+            b[i] = e < k ? *(const uint4*)(xr + e) : make_uint4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc = mfma16(as_operand(a[i]), as_operand(b[i]), acc);
+    }
+    red[wave][lane] = acc;
+    __syncthreads();
+    if (wave > 0) return;
+    for (int i = 1; i < WAVES; i++) acc += red[i][lane];
+    if (l16 < m) {
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            if (n0 + 4 * q + v < n) y[(int64_t)l16 * n + n0 + 4 * q + v] = to_bf16(acc[v]);
+    }
+}
+
+int router_logits(const void* x, const void* w, int64_t m, int64_t n, int64_t k, void* y, hipStream_t s) {
+    if (m < 1 || m > kRouterLogitsMaxTokens || n < 1 || k < 1 || k % 8 || n >= (1 << 20) || k >= (1 << 20)) return set_error(GGQ_ERR_SHAPE, "router_logits: takes 1 to %d tokens of a multiple of 8 elements", kRouterLogitsMaxTokens);
+    if (((uintptr_t)x | (uintptr_t)w) & 15) return set_error(GGQ_ERR_ALIGN, "router_logits: operands must be 16-byte aligned");
+    hipLaunchKernelGGL(few_rows_bf16_kernel, dim3((unsigned)((n + 15) / 16)), dim3(512), 0, s, (const bf16_t*)x, (const bf16_t*)w, (int)m, (int)n, (int)k, (bf16_t*)y);
+    return check_launch("router_logits");
+}
+
+// ------------------------------------------------------------------------------------------------
 // Expert FFN of a few routes, without a routing plan: with a handful of routes hardly two share an expert, so every route
 // reads its own expert's weights and the four launches of plan and tables, the gather by expert and the combine's pass fall
 // away.  Two launches:

@@ -280,8 +280,13 @@ struct Experts : torch::autograd::Function<Experts> {
 // ------------------------------------------------------------------------------------------------
 // Router logits, selection and softmax weights without autograd.
 void router_forward(const Tensor& weight, const Tensor& flat, int64_t top_k, Tensor& logits, Tensor& scores, Tensor& indices) {
-    at::NoGradGuard no_grad;
-    logits = at::linear(flat, weight);
+    if (flat.size(0) <= 8 && usable(flat, at::kBFloat16) && usable(weight, at::kBFloat16) && flat.size(0) > 0 && flat.size(1) % 8 == 0) {
+        logits = empty({flat.size(0), weight.size(0)}, at::kBFloat16, flat);
+        check(ggq_router_logits(flat.data_ptr(), weight.data_ptr(), flat.size(0), weight.size(0), flat.size(1), logits.data_ptr(), stream_of(flat)));
+    } else {
+        at::NoGradGuard no_grad;
+        logits = at::linear(flat, weight);
+    }
     const int64_t tokens = logits.size(0), experts = logits.size(1);
     indices = empty({tokens, top_k}, at::kLong, logits);
     scores = empty({tokens, top_k}, logits.scalar_type(), logits);

@@ -164,6 +164,8 @@ void dense_force_shape(int shape, int splits);  // test aid: -1 = the automatic 
 constexpr int kShapeFewRows = 7;  // (profile records only)
 bool gemv_takes(int qt, int64_t m, int64_t n, int64_t k, const void* x);
 int gemv(int qt, const void* x, const void* w, int64_t m, int64_t n, int64_t k, const void* lora_a, const void* lora_b, int r, float scale, void* xa_out, void* y, hipStream_t s);
+constexpr int kRouterLogitsMaxTokens = 8;
+int router_logits(const void* x, const void* w, int64_t m, int64_t n, int64_t k, void* y, hipStream_t s);
 bool few_routes_takes(int qt_in, int qt_down, int64_t tokens, int top_k, int64_t hidden, int64_t inter);
 int few_routes_forward(const void* x, const void* ids, int ids64, const void* weights, int weights_bf16, int64_t tokens, int top_k, int64_t experts, int64_t hidden,
                        int64_t inter, int qt_in, int qt_down, const void* gate, const void* up, const void* down, const void* a1, const void* b1, int r1,

@@ -286,13 +286,14 @@ class FastGGUFLoraLinear(torch.nn.Module):
     def forward(self, x: torch.Tensor, *args: Any, **kwargs: Any) -> torch.Tensor:
         if args or kwargs:
             raise TypeError("The packed GGUF MMQ linear path accepts only its input tensor.")
-        base = self.base_layer
+        modules = self._modules  # (what the attribute lookups of Module find, without their cost)
+        base = modules["base_layer"]
         if base.compute_dtype != torch.bfloat16:
             raise RuntimeError("The packed GGUF MMQ linear path requires BF16 compute_dtype.")
         if self.disable_adapters:
             return base(x)
-        name = self.active_adapter
-        y = lora_mmq(_layer_input(x), base.weight, base.weight.quant_type, base.out_features, self.lora_A[name].weight, self.lora_B[name].weight, self.scaling[name])
+        name, weight = self.active_adapter, base.weight
+        y = lora_mmq(_layer_input(x), weight, weight.quant_type, base.out_features, modules["lora_A"][name].weight, modules["lora_B"][name].weight, self.scaling[name])
         if base.bias is not None:
             y = y + base.bias.to(device=y.device, dtype=y.dtype)
         return y

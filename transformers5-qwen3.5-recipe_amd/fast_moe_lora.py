@@ -465,12 +465,24 @@ class GGUFExperts(torch.nn.Module):
         return fn(self, hidden_states, top_k_index, top_k_weights, lora_weights)
 
 
-def _runs_as_one_node(experts: GGUFExperts) -> bool:
-    """Whether nothing asks for the layer's pieces: the switches above are at their defaults, ids need not be validated, and
-    the module's plan and activation are this class's own."""
+def _one_node(experts: GGUFExperts, hidden_states, top_k_index, top_k_weights, gate_up_a, gate_up_b, down_a, down_b, scaling: float):
+    """The whole layer as one native call and one autograd node, or None: when something asks for the layer's pieces (the
+    switches above, id validation, a subclass with an activation or a plan of its own), and for operands the call does not take,
+    whose faults the general path names."""
     cls = type(experts)
-    return (FUSE_GATED_DOWN_COMBINE and SHARE_GROUP_TABLES and not fast_moe_routing.VALIDATE_EXPERT_IDS
-            and cls._apply_split_gate is GGUFExperts._apply_split_gate and cls._prepare_expert_execution is GGUFExperts._prepare_expert_execution)
+    gate, up, down = experts.gate_proj, experts.up_proj, experts.down_proj
+    if not (FUSE_GATED_DOWN_COMBINE and SHARE_GROUP_TABLES) or fast_moe_routing.VALIDATE_EXPERT_IDS \
+            or cls._apply_split_gate is not GGUFExperts._apply_split_gate or cls._prepare_expert_execution is not GGUFExperts._prepare_expert_execution \
+            or experts.projection_layout != "split_gate_up" or experts.has_bias or not experts.has_gate or experts.compute_dtype != torch.bfloat16 \
+            or not (isinstance(gate, GGUFQuantizedTensor) and isinstance(up, GGUFQuantizedTensor) and isinstance(down, GGUFQuantizedTensor)) \
+            or gate.quant_type != up.quant_type:
+        return None
+    x = experts._prepare_expert_hidden_states(hidden_states)
+    out = _lib.host().experts(x, top_k_index, top_k_weights, gate, up, down, gate_up_a, gate_up_b, down_a, down_b, experts._all_experts, gate.quant_type,
+                              down.quant_type, scaling, experts.swiglu_limit or 0.0)
+    if out is None or x is hidden_states:
+        return out
+    return out.to(hidden_states.dtype).reshape(hidden_states.shape)
 
 
 def qwen3_5_moe_gguf_mmq_lora_forward(self: GGUFExperts, hidden_states: torch.Tensor, top_k_index: torch.Tensor,
@@ -478,6 +490,11 @@ def qwen3_5_moe_gguf_mmq_lora_forward(self: GGUFExperts, hidden_states: torch.Te
     """Packed expert FFN with LoRA on gate/up and down (orchestration of fast_moe_lora.py:685-770)."""
     if not isinstance(self, GGUFExperts):
         raise TypeError(f"{EXPERTS_IMPLEMENTATION} requires GGUFExperts, got {type(self).__name__}.")
+    lw = lora_weights
+    factors = (lw.gate_up_a, lw.gate_up_b, lw.down_a, lw.down_b, lw.scaling) if lw is not None else (None, None, None, None, 0.0)
+    out = _one_node(self, hidden_states, top_k_index, top_k_weights, *factors)
+    if out is not None:
+        return out
     if self.projection_layout != "split_gate_up" or self.has_bias or not self.has_gate:
         raise RuntimeError("The GGUF LoRA path requires split, bias-free gate/up expert projections.")
     for w in (self.gate_proj, self.up_proj, self.down_proj):
@@ -493,15 +510,6 @@ def qwen3_5_moe_gguf_mmq_lora_forward(self: GGUFExperts, hidden_states: torch.Te
         raise RuntimeError("Paired grouped GGUF MMQ requires one quantization type.")
 
     compute_hidden_states = self._prepare_expert_hidden_states(hidden_states)
-    if _runs_as_one_node(self):
-        # the whole layer as one native call and one autograd node; operands it does not take go through the nodes below,
-        # whose checks name what is wrong
-        factors = (lora_weights.gate_up_a, lora_weights.gate_up_b, lora_weights.down_a, lora_weights.down_b) if lora_weights is not None else (None,) * 4
-        out = _lib.host().experts(compute_hidden_states, top_k_index, top_k_weights, self.gate_proj, self.up_proj, self.down_proj, *factors,
-                                  self._all_experts, self.gate_proj.quant_type, self.down_proj.quant_type,
-                                  lora_weights.scaling if lora_weights is not None else 0.0, self.swiglu_limit or 0.0)
-        if out is not None:
-            return out if out.dtype == hidden_states.dtype and out.shape == hidden_states.shape else out.to(hidden_states.dtype).reshape(hidden_states.shape)
     tokens, top_k = top_k_index.shape[0], top_k_index.shape[1]
     # The gate/up launch reads the token rows in place where it can; the routed copy is made otherwise.
     in_place = (compute_hidden_states.ndim == 2 and compute_hidden_states.is_contiguous()
@@ -512,7 +520,6 @@ def qwen3_5_moe_gguf_mmq_lora_forward(self: GGUFExperts, hidden_states: torch.Te
         raise RuntimeError("GGUF LoRA requires grouped expert offsets.")
     selected = routing_plan.selected_hidden_states
     expert_indices, expert_offsets = execution_plan.expert_indices, execution_plan.offsets
-    lw = lora_weights
     s = lw.scaling if lw is not None else 0.0
     # the four packed-weight calls of the step see one grouping: its row-tile tables are built once (the calls whose kernels
     # take another tile shape ignore them and build their own)
@@ -770,6 +777,15 @@ class FastGGUFMoeLora(torch.nn.Module):
         return _ExpertLoraWeights(self.lora_A[n].weight, self.lora_B[n].weight, self.lora_A_down[n].weight, self.lora_B_down[n].weight, float(self.scaling[n]))
 
     def forward(self, hidden_states: torch.Tensor, top_k_index: torch.Tensor, top_k_weights: torch.Tensor) -> torch.Tensor:
+        modules = self._modules  # (what the attribute lookups of Module find, without their cost)
+        experts = modules["base_layer"]
+        if not self.disable_adapters and ALL_GGUF_EXPERTS_FUNCTIONS.get(experts.experts_implementation) is qwen3_5_moe_gguf_mmq_lora_forward \
+                and isinstance(experts, GGUFExperts):
+            name = self.active_adapter
+            out = _one_node(experts, hidden_states, top_k_index, top_k_weights, modules["lora_A"][name].weight, modules["lora_B"][name].weight,
+                            modules["lora_A_down"][name].weight, modules["lora_B_down"][name].weight, float(self.scaling[name]))
+            if out is not None:
+                return out
         return self.base_layer(hidden_states, top_k_index, top_k_weights, self._active_lora_weights())
 
     def merge(self, *args: Any, **kwargs: Any) -> None:
