@@ -86,15 +86,18 @@ int64_t ggq_row_bytes(int qt, int64_t k);
  * bit-exact with ggml's dequantize_row_* followed by round-to-nearest-even to bf16. */
 int ggq_dequantize(int qt, const void* packed, int64_t rows, int64_t k, void* out, int out_is_f32, void* stream);
 
-/* torch.ops.torch_ggml_ops.mmq (fast_lora.py:155-160, gguf_liger_loss.py:109-114): y[M,N] = x[M,K] . W^T. */
+/* torch.ops.torch_ggml_ops.mmq (fast_lora.py:155-160, gguf_liger_loss.py:109-114): y[M,N] = x[M,K] . W^T.
+ * Without a workspace the products of many rows decode inside the matmul; ggq_lora_mmq_forward / _backward without factors
+ * (A = B = NULL) take one and are faster there. */
 int ggq_mmq(const void* x, const void* packed, int qt, int64_t m, int64_t n, int64_t k, void* y, void* stream);
 
 /* torch.ops.torch_ggml_ops.mmq_grad_input (gguf_liger_loss.py:172-177; autograd of mmq,
  * test_fast_lora.py:104-105): dx[M,K] = dy[M,N] . W with W decoded to bf16, fp32 accumulation. */
 int ggq_mmq_grad_input(const void* dy, const void* packed, int qt, int64_t m, int64_t n, int64_t k, void* dx, void* stream);
 
-/* Workspace bound for the four LoRA entry points below (n_total = N, or 2N for a pair).  groups = 0 (the dense calls)
- * includes the fp32 partial sums of the factor gradients, whose rows are then dealt over the whole chip. */
+/* Workspace bound for the four LoRA entry points below (n_total = N, or 2N for a pair; r = 0: without factors).  groups = 0
+ * (the dense calls) includes the decoded weights (at most 128 MB at a time), the fp32 partial sums of a split contraction and
+ * those of the factor gradients, whose rows are then dealt over the whole chip. */
 int64_t ggq_lora_workspace_bytes(int64_t rows, int64_t groups, int64_t experts, int64_t n_total, int64_t k, int r);
 
 /* FastGGUFLoraLinear._base_layer_forward + _fused_lora_add (fast_lora.py:34-65, 134-163) in one call:
@@ -172,6 +175,12 @@ int ggq_fixed_grouped_mmq(const void* x, const void* packed_groups, int qt, int6
                           void* stream);
 int ggq_fixed_grouped_mmq_grad_input(const void* dy, const void* packed_groups, int qt, int64_t rows, int groups, int64_t n_group, int64_t k,
                                      void* dx, void* stream);
+/* The same with a workspace of ggq_lora_workspace_bytes(rows, 0, 1, n_group, k, 0) bytes, which every group's launch reuses for
+ * its decoded weights: bit-identical to ggq_lora_mmq_forward / _backward without factors on per-group copies. */
+int ggq_fixed_grouped_mmq_ws(const void* x, const void* packed_groups, int qt, int64_t rows, int groups, int64_t n_group, int64_t k, void* y, void* ws,
+                             int64_t ws_bytes, void* stream);
+int ggq_fixed_grouped_mmq_grad_input_ws(const void* dy, const void* packed_groups, int qt, int64_t rows, int groups, int64_t n_group, int64_t k,
+                                        void* dx, void* ws, int64_t ws_bytes, void* stream);
 
 /* prepare_expert_routing (fast_moe_routing.py:379-428: torch.sort of the flat top-k ids + inverse
  * permutation kernel :88-98) and the grouped-execution offsets of the expert module

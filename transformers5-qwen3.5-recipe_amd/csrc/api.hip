@@ -196,17 +196,22 @@ static int small_tiles_per_wg(int64_t groups, int col_tiles) {
     return per_wg;
 }
 
-// A dense layer's factor gradients deal their rows to at most this many workgroups per column block (fp32 partial sums
-// in the workspace).
-constexpr int64_t kDenseFactorSplits = 32;
+// Partial sums of a dense layer's factor gradient over `cols` columns (fp32, see factor_grad_plan): the rows are dealt to
+// as many workgroups as fill the chip, at most 64.
+static int64_t factor_partials_bytes(int64_t cols, int r_pad) {
+    const int64_t blocks = (cols + 127) / 128;
+    return blocks >= 256 ? 0 : std::min<int64_t>(64, (256 + blocks - 1) / blocks) * cols * r_pad * 4;
+}
 
 int64_t ggq_lora_workspace_bytes(int64_t rows, int64_t groups, int64_t experts, int64_t n_total, int64_t k, int r) {
+    const int64_t panels = groups == 0 ? align256(dense_workspace_bytes(rows, n_total, k)) : 0;
+    if (groups == 0 && r <= 0) return panels + 4096;
     const int rp = rank_pad(r > 0 ? r : 1);
     if (experts < 1) experts = 1;
     const int64_t tiles = rows / 64 + groups + 2;
     return 5 * align256(tiles * (int64_t)sizeof(TileDesc)) + align256(16) + align256(experts * 2 * 4) +
-           align256(experts * n_total * rp * 2) * 2 + align256(experts * k * rp * 2) + align256(rows * rp * 2) + 4096 +
-           (groups == 0 ? align256(kDenseFactorSplits * std::max(n_total, k) * rp * 4) + dense_workspace_bytes(rows, n_total, k) + 256 : 0);
+           align256(experts * n_total * rp * 2) * 2 + align256(experts * k * rp * 2) + align256(rows * rp * 2) + 4096 + panels +
+           (groups == 0 ? align256(factor_partials_bytes(n_total, rp)) + align256(factor_partials_bytes(k, rp)) : 0);
 }
 
 int ggq_lora_mmq_forward(const void* x, const void* packed, int qt, int64_t m, int64_t n, int64_t k, const void* lora_a,
@@ -238,7 +243,7 @@ int ggq_mmq_grad_input(const void* dy, const void* packed, int qt, int64_t m, in
 // a dense matmul over the strided rows x[:, g, :]; it runs as that launch (same tiles, same arithmetic as ggq_mmq on a
 // contiguous copy), so the results are bit-identical to the per-group dense calls.
 static int fixed_grouped(const char* what, int mode, const void* in, const void* packed, int qt, int64_t rows, int groups, int64_t n_group,
-                         int64_t k, void* out, hipStream_t s) {
+                         int64_t k, void* out, void* ws, int64_t ws_bytes, hipStream_t s) {
     if (rows < 0 || groups <= 0 || n_group <= 0 || k <= 0 || rows >= (1ll << 31) || n_group >= (1ll << 30) || k >= (1ll << 30) ||
         (int64_t)groups * std::max(n_group, k) >= (1ll << 31))
         return set_error(GGQ_ERR_SHAPE, "%s: bad shape rows=%lld groups=%d n_group=%lld k=%lld", what, (long long)rows, groups, (long long)n_group, (long long)k);
@@ -252,19 +257,40 @@ static int fixed_grouped(const char* what, int mode, const void* in, const void*
         p.a[0] = (const bf16_t*)in + g * in_cols, p.lda = groups * in_cols;
         p.w[0] = (const uint8_t*)packed + g * p.w_expert_bytes;
         p.c[0] = (bf16_t*)out + g * out_cols, p.ldc = groups * out_cols;
+        if (mode == kModeNT && gemv_takes(qt, rows, n_group, k, p.a[0], p.lda)) {
+            if (int rc = gemv(qt, p.a[0], p.lda, p.w[0], rows, n_group, k, nullptr, nullptr, 0, 0.f, nullptr, p.c[0], p.ldc, s)) return rc;
+            continue;
+        }
+        if (ws && dense_takes(mode, rows, n_group, k, p.a[0], p.lda)) {
+            DenseCall q{};
+            q.qt = qt, q.mode = mode, q.m = rows, q.n = n_group, q.k = k, q.a = p.a[0], q.lda = p.lda, q.w = p.w[0], q.c = p.c[0], q.ldc = p.ldc;
+            if (int rc = dense_mmq(q, ws, ws_bytes, s)) return rc;
+            continue;
+        }
         if (int rc = launch_mmq(qt, mode, kEpiStore, p, s)) return rc;
     }
     return GGQ_OK;
 }
 
-int ggq_fixed_grouped_mmq(const void* x, const void* packed_groups, int qt, int64_t rows, int groups, int64_t n_group, int64_t k, void* y,
-                          void* stream) {
-    return fixed_grouped("fixed_grouped_mmq", kModeNT, x, packed_groups, qt, rows, groups, n_group, k, y, as_stream(stream));
+int64_t ggq_fixed_grouped_mmq_workspace_bytes(int64_t rows, int64_t n_group, int64_t k) { return align256(dense_workspace_bytes(rows, n_group, k)) + 256; }
+
+int ggq_fixed_grouped_mmq(const void* x, const void* packed_groups, int qt, int64_t rows, int groups, int64_t n_group, int64_t k, void* y, void* stream) {
+    return fixed_grouped("fixed_grouped_mmq", kModeNT, x, packed_groups, qt, rows, groups, n_group, k, y, nullptr, 0, as_stream(stream));
 }
 
 int ggq_fixed_grouped_mmq_grad_input(const void* dy, const void* packed_groups, int qt, int64_t rows, int groups, int64_t n_group, int64_t k,
                                      void* dx, void* stream) {
-    return fixed_grouped("fixed_grouped_mmq_grad_input", kModeNN, dy, packed_groups, qt, rows, groups, n_group, k, dx, as_stream(stream));
+    return fixed_grouped("fixed_grouped_mmq_grad_input", kModeNN, dy, packed_groups, qt, rows, groups, n_group, k, dx, nullptr, 0, as_stream(stream));
+}
+
+int ggq_fixed_grouped_mmq_ws(const void* x, const void* packed_groups, int qt, int64_t rows, int groups, int64_t n_group, int64_t k, void* y, void* ws,
+                             int64_t ws_bytes, void* stream) {
+    return fixed_grouped("fixed_grouped_mmq", kModeNT, x, packed_groups, qt, rows, groups, n_group, k, y, ws, ws_bytes, as_stream(stream));
+}
+
+int ggq_fixed_grouped_mmq_grad_input_ws(const void* dy, const void* packed_groups, int qt, int64_t rows, int groups, int64_t n_group, int64_t k,
+                                        void* dx, void* ws, int64_t ws_bytes, void* stream) {
+    return fixed_grouped("fixed_grouped_mmq_grad_input", kModeNN, dy, packed_groups, qt, rows, groups, n_group, k, dx, ws, ws_bytes, as_stream(stream));
 }
 
 // Row-tile tables of one grouping, built once (ggq_group_tables_build) and handed to the launches that share it: the
@@ -345,12 +371,30 @@ static int grouped_forward(const char* what, const void* x, RowIndex x_index, co
     if (int rc = init_params(p, qt, kModeNT, (int)rows, (int)n, (int)k, nseg, pick_shape(qt, rows, groups, direct_ok))) return rc;
     if (x_index.on() && (!forward_reads_indexed_rows(qt, rows, groups, x_index.index_rows, k) || x_index.index_div <= 0))
         return set_error(GGQ_ERR_SHAPE, "%s: this source matrix cannot be read through a row index (ask ggq_grouped_forward_reads_indexed_rows first)", what);
-    if (groups == 0 && !packed2 && !x_index.on() && gemv_takes(qt, rows, n, k, x) && (!lora_a || aligned16(xa_out)))
-        return gemv(qt, x, packed1, rows, n, k, lora_a, lora_b, r, scale, xa_out, y1, s);
+    if (groups == 0 && !packed2 && !x_index.on() && gemv_takes(qt, rows, n, k, x, k) && (!lora_a || aligned16(xa_out)))
+        return gemv(qt, x, k, packed1, rows, n, k, lora_a, lora_b, r, scale, xa_out, y1, n, s);
     p.a[0] = (const bf16_t*)x, p.lda = k, p.a_rows = x_index;
     p.w[0] = (const uint8_t*)packed1, p.w[1] = (const uint8_t*)packed2;
     p.c[0] = y1, p.c[1] = y2, p.ldc = n;
     if (p.shape == kShapeDirect) p.col_tiles_per_wg = direct_tiles_per_wg(rows, groups, nseg * p.col_tiles_per_seg, p.steps_per_seg, kModeNT);
+
+    if (groups == 0 && !packed2 && !x_index.on() && ws && dense_takes(kModeNT, rows, n, k, x, k)) {
+        // (callers without a workspace keep the tile kernel)
+        const int64_t need = dense_workspace_bytes(rows, n, k);
+        void* panels = bump.take(need);
+        if (!panels) return set_error(GGQ_ERR_WORKSPACE, "%s: workspace too small", what);
+        DenseCall q{};
+        q.qt = qt, q.mode = kModeNT, q.m = rows, q.n = n, q.k = k, q.a = x, q.lda = k, q.w = packed1, q.c = y1, q.ldc = n;
+        if (!lora_a) return dense_mmq(q, panels, need, s);
+        q.la = xa_out, q.lb = lora_b, q.r_pad = rp, q.rank = r, q.lora_scale = scale;
+        SkinnyNtParams sp{};
+        sp.in[0] = (const bf16_t*)x, sp.ld_in = k, sp.f = (const bf16_t*)lora_a, sp.ldf = k, sp.out = (bf16_t*)xa_out;
+        sp.m = (int)rows, sp.c = (int)k, sp.r = r, sp.nseg = 1;
+        const DenseSide side{&sp, nullptr, rp};
+        if (dense_side_takes(side)) return dense_mmq(q, panels, need, s, &side);
+        if (int rc = skinny_nt(sp, rp, (int)((rows + 63) / 64), s)) return rc;
+        return dense_mmq(q, panels, need, s);
+    }
 
     const TileDesc* tiles64 = nullptr;
     const int* num_tiles64 = nullptr;
@@ -412,13 +456,6 @@ static int grouped_forward(const char* what, const void* x, RowIndex x_index, co
             lb = padded;
         }
         p.la = (const bf16_t*)xa_out, p.lb = lb, p.lb_expert_elems = (int64_t)nseg * n * rp, p.r_pad = rp, p.lora_scale = scale;
-    }
-    if (groups == 0 && dense_takes(kModeNT, rows, n, k, x, k)) {
-        DenseCall q{};
-        q.qt = qt, q.mode = kModeNT, q.m = rows, q.n = n, q.k = k, q.a = x, q.lda = k, q.w = packed1, q.c = y1, q.ldc = n;
-        if (lora_a) q.la = p.la, q.lb = p.lb, q.r_pad = rp, q.rank = r, q.lora_scale = scale;
-        const int64_t need = dense_workspace_bytes(rows, n, k);
-        if (void* panels = ws ? bump.take(need) : nullptr) return dense_mmq(q, panels, need, s);  // (callers without a workspace keep the tile kernel)
     }
     if (t_small) {
         MmqParams ps = p;
@@ -490,6 +527,39 @@ static int grouped_backward(const char* what, const void* dy1, const void* dy2, 
     p.w[0] = (const uint8_t*)packed1, p.w[1] = (const uint8_t*)packed2;
     p.c[0] = dx, p.ldc = k;
     if (p.shape == kShapeDirect) p.col_tiles_per_wg = direct_tiles_per_wg(rows, groups, p.col_tiles_per_seg, nseg * p.steps_per_seg, kModeNN);
+
+    if (groups == 0 && !packed2 && !dy_index.on() && !x_index.on() && !row_weights && rows > 0 && lora_a && ws && dense_takes(kModeNN, rows, n, k, dy1, n)) {
+        // A dense LoRA layer: dy B and the gradient of B ride in the decoding pass's launch, the gradient of A follows the
+        // grad-input launch, and one pass adds the partial sums of both gradients.
+        SkinnyNtParams sp{};
+        sp.in[0] = (const bf16_t*)dy1, sp.ld_in = n, sp.f = (const bf16_t*)lora_b, sp.ldf = r, sp.f_natural = 1;
+        sp.m = (int)rows, sp.c = (int)n, sp.r = r, sp.nseg = 1;
+        FactorGradParams fb{}, fa{};
+        DenseSide side{&sp, d_lora_b ? &fb : nullptr, rp};
+        if (dense_side_takes(side)) {
+            const int64_t need = dense_workspace_bytes(rows, n, k);
+            bf16_t* dyb = (bf16_t*)bump.take(rows * rp * 2);
+            fb.partials_bytes = factor_partials_bytes(n, rp), fa.partials_bytes = factor_partials_bytes(k, rp);
+            fb.partials = (float*)bump.take(fb.partials_bytes), fa.partials = (float*)bump.take(fa.partials_bytes);
+            void* panels = bump.take(need);
+            if (!panels) return set_error(GGQ_ERR_WORKSPACE, "%s: workspace too small", what);
+            sp.out = dyb;
+            fb.in[0] = (const bf16_t*)dy1, fb.ld_in = n, fb.s = (const bf16_t*)xa, fb.out = (bf16_t*)d_lora_b, fb.c = (int)n, fb.out_j_major = 0;
+            fa.in[0] = (const bf16_t*)x, fa.ld_in = k, fa.s = dyb, fa.out = (bf16_t*)d_lora_a, fa.c = (int)k, fa.out_j_major = 1;
+            for (FactorGradParams* f : {&fb, &fa}) f->m = (int)rows, f->r = r, f->nseg = 1, f->scale = scale;
+            DenseCall q{};
+            q.qt = qt, q.mode = kModeNN, q.m = rows, q.n = n, q.k = k, q.a = dy1, q.lda = n, q.w = packed1, q.c = dx, q.ldc = k;
+            q.la = dyb, q.lb = lora_a, q.r_pad = rp, q.rank = r, q.lora_scale = scale;
+            if (int rc = dense_mmq(q, panels, need, s, &side)) return rc;
+            if (d_lora_a)
+                if (int rc = factor_grad_partial(fa, rp, 1, s)) return rc;
+            const FactorGradParams* both[2];
+            int count = 0;
+            if (d_lora_b) both[count++] = &fb;
+            if (d_lora_a) both[count++] = &fa;
+            return factor_reduce(both, count, rp, s);
+        }
+    }
 
     const TileDesc* tiles64 = nullptr;
     const int* num_tiles64 = nullptr;
@@ -565,7 +635,7 @@ static int grouped_backward(const char* what, const void* dy1, const void* dy2, 
     float* partials = nullptr;
     int64_t partials_bytes = 0;
     if (groups == 0) {  // optional: without it the rows are not split
-        partials_bytes = kDenseFactorSplits * std::max<int64_t>(ntot, k) * rp * 4;
+        partials_bytes = std::max(factor_partials_bytes(ntot, rp), factor_partials_bytes(k, rp));
         partials = (float*)bump.take(partials_bytes);
         if (!partials) partials_bytes = 0;
     }

@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "blocks.h"
+#include "factor_grad.h"
 #include "iq2xxs_grid.h"
 #include "launch.h"
 #include "mmq_host.h"
@@ -30,9 +31,6 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 // ------------------------------------------------------------------------------------------------
 // Decoding passes.  HBM-bound: packed bytes in, two bytes per weight out.
-
-typedef short v4i16_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4i16_t* lds_v4i16_ptr;
 
 // What chunk index of row r is XOR-ed with (r mod 16 counts).
 __device__ __forceinline__ int panel_swizzle(int r) { return (((r >> 1) & 3) << 1) | ((r >> 3) & 1); }
@@ -50,14 +48,28 @@ __device__ __forceinline__ const uint2* stage_tables(uint32_t* lds, int tid, int
 // the eight lanes of a row read adjacent bytes.  The wave's 4 KB go through LDS and leave in whole 1 KB pieces.  The panel
 // holds k0 .. k0 + kcols - 1 of every row; rows from n up to the next multiple of 64 are zeros (a contraction over the rows
 // runs to there).
+struct DecodeParams {
+    const uint8_t* w;
+    int64_t row_bytes;
+    int n, k, k0, kcols;
+    uint8_t* panel;
+};
 template <int QT>
-__global__ __launch_bounds__(256) void decode_panel_kernel(const uint8_t* w, int64_t row_bytes, int n, int k, int k0, int kcols, uint8_t* panel) {
-    __shared__ __attribute__((aligned(16))) uint8_t out_lds[4][4096];
-    __shared__ uint32_t tables[QT == kIQ2_XXS ? Fmt<kIQ2_XXS>::kTableWords : 1];
+struct DecodeLds {
+    uint8_t out[4][4096];
+    uint32_t tables[QT == kIQ2_XXS ? Fmt<kIQ2_XXS>::kTableWords : 1];
+};
+template <int QT>
+__device__ __forceinline__ void decode_panel_body(const DecodeParams& p, int wg, DecodeLds<QT>& lds) {
+    auto& out_lds = lds.out;
+    const uint8_t* w = p.w;
+    const int64_t row_bytes = p.row_bytes;
+    const int n = p.n, k = p.k, k0 = p.k0, kcols = p.kcols;
+    uint8_t* panel = p.panel;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint2* tab = stage_tables<QT>(tables, threadIdx.x, 256);
+    const uint2* tab = stage_tables<QT>(lds.tables, threadIdx.x, 256);
     const int kblocks = (kcols + 255) >> 8, steps = kcols >> 6;
-    const int64_t unit = (int64_t)blockIdx.x * 4 + wave;
+    const int64_t unit = (int64_t)wg * 4 + wave;
     const int group = (int)(unit / kblocks), kb = (int)(unit - (int64_t)group * kblocks);
     if (group * 8 >= ((n + 63) & ~63)) return;
     const int row = group * 8 + (lane >> 3), ksub = min((k0 >> 5) + kb * 8 + (lane & 7), (k >> 5) - 1);
@@ -83,6 +95,124 @@ __global__ __launch_bounds__(256) void decode_panel_kernel(const uint8_t* w, int
     }
 }
 
+template <int QT>
+__global__ __launch_bounds__(256) void decode_panel_kernel(DecodeParams p) {
+    __shared__ __attribute__((aligned(16))) DecodeLds<QT> lds;
+    decode_panel_body<QT>(p, blockIdx.x, lds);
+}
+
+// ---- out[m, 0..r_pad) = In[m, :] . F^T for sixteen rows: the four waves deal the contraction out in spans of 128, the next
+// span's loads in flight under the current one's MFMAs, and add their sums in wave order.  F is [r][ldf] (contraction
+// contiguous), or [contraction][r] (f_natural): then a span of it goes through the wave's own LDS as [128][r_pad] and the
+// operand is read back transposed.
+template <int JB>
+struct ThinLds {
+    bf16_t f[4][128][JB * 16];
+    f32x4_t red[4][JB][64];
+};
+template <int JB>
+__device__ __forceinline__ void thin_product_body(const SkinnyNtParams& p, int wg, ThinLds<JB>& lds) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int li = lane & 15, lq = lane >> 4;
+    const int m0 = wg * 16, spans = (p.c + 127) / 128;
+    const bf16_t* in = p.in[0] + (int64_t)min(m0 + li, p.m - 1) * p.ld_in;
+    const bool vec = (p.r & 7) == 0;
+    f32x4_t acc[JB];
+#pragma unroll
+    for (int jb = 0; jb < JB; jb++) acc[jb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    uint4 x[4], f[JB][4];
+    auto load = [&](int span) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int e = span * 128 + 32 * i + 8 * lq;
+            x[i] = e < p.c ? *(const uint4*)(in + e) : make_uint4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int jb = 0; jb < JB; jb++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                if (p.f_natural) {  // piece (contraction row, eight columns) of the span
+                    const int piece = (jb * 4 + i) * 64 + lane, row = span * 128 + piece / (2 * JB), j = piece % (2 * JB) * 8;
+                    f[jb][i] = load8g(p.f + (int64_t)row * p.r + j, row < p.c ? p.r - j : 0, vec);
+                } else {
+                    const int j = jb * 16 + li, e = span * 128 + 32 * i + 8 * lq;
+                    f[jb][i] = j < p.r && e < p.c ? *(const uint4*)(p.f + (int64_t)j * p.ldf + e) : make_uint4(0, 0, 0, 0);
+                }
+            }
+    };
+    if (wave < spans) load(wave);
+    for (int span = wave; span < spans; span += 4) {
+        bf16x8_t a[4], b[JB][4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) a[i] = __builtin_bit_cast(bf16x8_t, x[i]);
+        if (p.f_natural) {
+            uint4* dst = (uint4*)&lds.f[wave][0][0];
+#pragma unroll
+            for (int jb = 0; jb < JB; jb++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) dst[(jb * 4 + i) * 64 + lane] = f[jb][i];
+            // (LDS serves a wave in order, and no other wave uses this piece)
+#pragma unroll
+            for (int jb = 0; jb < JB; jb++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const bf16_t* src = &lds.f[wave][32 * i + 8 * lq + (li >> 2)][jb * 16 + (li & 3) * 4];
+                    const v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)src);
+                    const v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)(src + 4 * JB * 16));
+                    b[jb][i] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                }
+        } else {
+#pragma unroll
+            for (int jb = 0; jb < JB; jb++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) b[jb][i] = __builtin_bit_cast(bf16x8_t, f[jb][i]);
+        }
+        load(min(span + 4, spans - 1));  // (past the end: the last span again)
+#pragma unroll
+        for (int jb = 0; jb < JB; jb++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[jb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[jb][i], acc[jb], 0, 0, 0);
+    }
+#pragma unroll
+    for (int jb = 0; jb < JB; jb++) lds.red[wave][jb][lane] = acc[jb];
+    __syncthreads();
+    for (int jb = wave; jb < JB; jb += 4) {
+        const f32x4_t sum = ((lds.red[0][jb][lane] + lds.red[1][jb][lane]) + lds.red[2][jb][lane]) + lds.red[3][jb][lane];
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            if (m0 + 4 * lq + v < p.m) p.out[(int64_t)(m0 + 4 * lq + v) * (JB * 16) + jb * 16 + li] = to_bf16(sum[v]);
+    }
+}
+
+// The decoding pass together with the call's rank-sized work that does not read the panel: the thin product, and the gradient
+// of B.  Each alone is a few microseconds of latency on part of the chip; at the sizes of one short sequence they and the gaps
+// between their launches were half of a linear layer's step.  Workgroups are dealt in the order thin product (the longest
+// chain), gradient, decoding.
+struct SidePassParams {
+    DecodeParams decode;
+    SkinnyNtParams product;
+    FactorGradParams gradient;
+    int product_wgs, gradient_wgs;
+};
+template <int QT, int JB>
+__global__ __launch_bounds__(256) void decode_side_kernel(SidePassParams p) {
+    __shared__ __attribute__((aligned(16))) union {
+        DecodeLds<QT> decode;
+        ThinLds<JB> thin;
+        FactorGradLds<JB, 1> narrow;
+        FactorGradLds<JB, 2> wide;
+    } lds;
+    int wg = blockIdx.x;
+    if (wg < p.product_wgs) return thin_product_body<JB>(p.product, wg, lds.thin);
+    wg -= p.product_wgs;
+    if (wg < p.gradient_wgs) {
+        if (p.gradient.c % 128 == 0) factor_grad_body<JB, 2>(p.gradient, wg, lds.wide);
+        else factor_grad_body<JB, 1>(p.gradient, wg, lds.narrow);
+        return;
+    }
+    decode_panel_body<QT>(p.decode, wg - p.gradient_wgs, lds.decode);
+}
+
 // ------------------------------------------------------------------------------------------------
 // The tile kernel: C[m, col] = sum_t A[m, t] * W(col, t), plus scale * LA . LB when a LoRA term comes along.
 struct DenseParams {
@@ -97,7 +227,7 @@ struct DenseParams {
     const float* row_scale;  // accumulate epilogue
     int splits;            // contraction dealt to this many workgroups (partial epilogue)
     int64_t split_stride;  // floats between two splits' partial sums
-    // LoRA: la [m, r_pad]; lb [cols][r_pad], or (lb_k_major) [rank][lb_ld] with the columns contiguous
+    // LoRA: la [m, r_pad]; lb [cols][rank], or (lb_k_major) [rank][lb_ld] with the columns contiguous
     const bf16_t *la, *lb;
     int r_pad, rank, lb_k_major;
     int64_t lb_ld;
@@ -206,7 +336,7 @@ __device__ __forceinline__ void dense_body(const DenseParams& p, uint8_t* lds) {
             for (int j = 0; j < CB; j++) {
                 const int col = min(col0 + (wn * CB + j) * 32 + l32, p.cols - 1);
                 if (!p.lb_k_major) {
-                    lbv[j] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(p.lb + (int64_t)col * p.r_pad + r0 + 8 * half));
+                    lbv[j] = __builtin_bit_cast(bf16x8_t, load8g(p.lb + (int64_t)col * p.rank + r0 + 8 * half, p.rank - (r0 + 8 * half), (p.rank & 7) == 0));
                 } else {
                     uint32_t e[8];
 #pragma unroll
@@ -458,22 +588,43 @@ static void shape_size(int shape, int& bm, int& bn) {
 }
 
 template <int QT>
-static int launch_decode_panel(const uint8_t* w, int64_t row_bytes, int n, int k, int k0, int kcols, uint8_t* panel, hipStream_t s) {
-    const int64_t units = (int64_t)((n + 63) / 64 * 8) * ((kcols + 255) / 256);
-    hipLaunchKernelGGL(decode_panel_kernel<QT>, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, w, row_bytes, n, k, k0, kcols, panel);
-    return check_launch("decode_panel");
+static int launch_decode_panel(const DecodeParams& d, const DenseSide* side, hipStream_t s) {
+    const int64_t units = (int64_t)((d.n + 63) / 64 * 8) * ((d.kcols + 255) / 256), wgs = (units + 3) / 4;
+    if (!side) {
+        hipLaunchKernelGGL(decode_panel_kernel<QT>, dim3((unsigned)wgs), dim3(256), 0, s, d);
+        return check_launch("decode_panel");
+    }
+    SidePassParams p{};
+    p.decode = d;
+    if (side->product) p.product = *side->product, p.product_wgs = (p.product.m + 15) / 16;
+    if (side->gradient) {
+        p.gradient_wgs = (int)factor_grad_plan(*side->gradient, side->r_pad, 1);
+        p.gradient = *side->gradient;
+    }
+    const dim3 grid((unsigned)(wgs + p.product_wgs + p.gradient_wgs));
+    if (side->r_pad == 16) hipLaunchKernelGGL((decode_side_kernel<QT, 1>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((decode_side_kernel<QT, 2>), grid, dim3(256), 0, s, p);
+    return check_launch("decode_side");
 }
-static int decode_panel(int qt, const uint8_t* w, int64_t row_bytes, int n, int k, int k0, int kcols, uint8_t* panel, hipStream_t s) {
+static int decode_panel(int qt, const DecodeParams& d, const DenseSide* side, hipStream_t s) {
     switch (qt) {
-        case kQ8_0: return launch_decode_panel<kQ8_0>(w, row_bytes, n, k, k0, kcols, panel, s);
-        case kQ2_K: return launch_decode_panel<kQ2_K>(w, row_bytes, n, k, k0, kcols, panel, s);
-        case kQ3_K: return launch_decode_panel<kQ3_K>(w, row_bytes, n, k, k0, kcols, panel, s);
-        case kQ4_K: return launch_decode_panel<kQ4_K>(w, row_bytes, n, k, k0, kcols, panel, s);
-        case kQ5_K: return launch_decode_panel<kQ5_K>(w, row_bytes, n, k, k0, kcols, panel, s);
-        case kQ6_K: return launch_decode_panel<kQ6_K>(w, row_bytes, n, k, k0, kcols, panel, s);
-        case kIQ2_XXS: return launch_decode_panel<kIQ2_XXS>(w, row_bytes, n, k, k0, kcols, panel, s);
+        case kQ8_0: return launch_decode_panel<kQ8_0>(d, side, s);
+        case kQ2_K: return launch_decode_panel<kQ2_K>(d, side, s);
+        case kQ3_K: return launch_decode_panel<kQ3_K>(d, side, s);
+        case kQ4_K: return launch_decode_panel<kQ4_K>(d, side, s);
+        case kQ5_K: return launch_decode_panel<kQ5_K>(d, side, s);
+        case kQ6_K: return launch_decode_panel<kQ6_K>(d, side, s);
+        case kIQ2_XXS: return launch_decode_panel<kIQ2_XXS>(d, side, s);
     }
     return set_error(GGQ_ERR_QTYPE, "unsupported GGML type id %d", qt);
+}
+
+// Aligned rows in eights, one segment without an index, rank up to kDenseSideMaxRank.
+bool dense_side_takes(const DenseSide& side) {
+    if (side.r_pad > kDenseSideMaxRank) return false;
+    if (const SkinnyNtParams* q = side.product)
+        if (q->nseg != 1 || q->in_rows.on() || q->c % 8 || q->ld_in % 8 || ((uintptr_t)q->in[0] & 15) || (!q->f_natural && (q->ldf % 8 || ((uintptr_t)q->f & 15)))) return false;
+    return true;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -519,7 +670,7 @@ static void pick_tile(int64_t m, int64_t cols, int64_t steps, bool can_split, in
 }
 
 int64_t dense_workspace_bytes(int64_t m, int64_t n, int64_t k) {
-    if (m <= 0 || n <= 0 || k <= 0) return 0;
+    if (m < kDenseMinRows || n <= 0 || k <= 0) return 0;
     const int64_t nt = slab_columns(n, k) * ((k + 63) / 64) * 128, nn = slab_columns(k, n) * ((n + 63) / 64) * 128;
     int64_t partial = 0;
     for (int mode = 0; mode < 2; mode++) {
@@ -537,7 +688,7 @@ bool dense_takes(int mode, int64_t m, int64_t n, int64_t k, const void* a, int64
     return m >= kDenseMinRows && ((uintptr_t)a & 15) == 0 && lda % 8 == 0 && (contraction % 8 == 0 || a_zero_padded) && 256 * lda < (1ll << 30) && cols > 0;
 }
 
-int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s) {
+int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s, const DenseSide* side) {
     const int64_t cols = q.mode == kModeNT ? q.n : q.k, contraction = q.mode == kModeNT ? q.k : q.n, steps = (contraction + 63) / 64;
     const int64_t slab = slab_columns(cols, contraction), panel_bytes = (slab * steps * 128 + 255) / 256 * 256;
     if (!ws || ws_bytes < panel_bytes) return set_error(GGQ_ERR_WORKSPACE, "dense_gemm: workspace too small");
@@ -549,13 +700,14 @@ int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s) {
         const uint8_t* w = (const uint8_t*)q.w + (q.mode == kModeNT ? c0 * row_bytes : 0);
         const int kcols = (int)(q.mode == kModeNT ? q.k : cn);
         if (!q.panel_ready)
-            if (int rc = decode_panel(q.qt, w, row_bytes, (int)(q.mode == kModeNT ? cn : q.n), (int)q.k, (int)(q.mode == kModeNT ? 0 : c0), kcols, panel, s)) return rc;
+            if (int rc = decode_panel(q.qt, DecodeParams{w, row_bytes, (int)(q.mode == kModeNT ? cn : q.n), (int)q.k, (int)(q.mode == kModeNT ? 0 : c0), kcols, panel},
+                                      c0 == 0 ? side : nullptr, s)) return rc;
         DenseParams p{};
         p.a = (const bf16_t*)q.a, p.lda = q.lda, p.contraction = (int)(q.a_zero_padded ? steps * 64 : contraction);
         p.panel = panel, p.panel_steps = kcols / 64, p.m = (int)q.m, p.cols = (int)cn, p.ldc = q.ldc, p.row_scale = q.row_scale;
         if (q.la) {
             p.la = (const bf16_t*)q.la, p.r_pad = q.r_pad, p.rank = q.rank, p.lora_scale = q.lora_scale, p.lb_k_major = q.mode == kModeNN, p.lb_ld = q.k;
-            p.lb = (const bf16_t*)q.lb + (q.mode == kModeNT ? c0 * q.r_pad : c0);
+            p.lb = (const bf16_t*)q.lb + (q.mode == kModeNT ? c0 * q.rank : c0);
         }
         int shape, splits;
         const bool can_split = cn % 4 == 0 && q.ldc % 4 == 0 && ((uintptr_t)q.c & 7) == 0;

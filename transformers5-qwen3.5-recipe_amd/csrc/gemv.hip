@@ -189,10 +189,12 @@ __device__ __forceinline__ uint4 load_factor8(const bf16_t* p, int valid, bool v
 // Dense: y [m, n] = x [m, k] . W [n, k]^T (+ scale (x A^T) B^T).
 struct GemvParams {
     const bf16_t* x;
+    int64_t ldx;
     int m, n, k;
     const uint8_t* w;
     int row_bytes;
     bf16_t* y;
+    int64_t ldy;
     const bf16_t *lora_a, *lora_b;  // [r][k], [n][r]; null: none
     bf16_t* xa_out;                 // [m][r_pad]
     int r, r_pad;
@@ -223,7 +225,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
     for (int sp = 0; sp < SP; sp++)
 #pragma unroll
         for (int tb = 0; tb < TB; tb++) {
-            const bf16_t* src = p.x + (int64_t)min(tb * 16 + l16, p.m - 1) * p.k;
+            const bf16_t* src = p.x + min(tb * 16 + l16, p.m - 1) * p.ldx;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int e = (wave + WAVES * sp) * kSpan + span_element<QT>(q, i);
@@ -310,8 +312,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
                 sum += lo * p.lora_scale;
             }
             if (xrow < p.m) {
-                bf16_t* dst = p.y + (int64_t)xrow * p.n + col;
-                if ((p.n & 3) == 0 && ((uintptr_t)p.y & 7) == 0) {
+                bf16_t* dst = p.y + xrow * p.ldy + col;
+                if (((p.n | p.ldy) & 3) == 0 && ((uintptr_t)p.y & 7) == 0) {
                     if (col < p.n) *(uint2*)dst = make_uint2(pack_bf16(sum[0], sum[1]), pack_bf16(sum[2], sum[3]));
                 } else {
 #pragma unroll
@@ -346,15 +348,17 @@ static int launch_gemv_qt(const GemvParams& p, hipStream_t s) {
 }
 
 // Rows up to which x fits the registers of the waves that share it: 64 of 2048 elements, 32 of 4096, 16 of 8192.
-bool gemv_takes(int qt, int64_t m, int64_t n, int64_t k, const void* x) {
-    if (m < 1 || n < 1 || k > 8192 || ((uintptr_t)x & 15)) return false;
+bool gemv_takes(int qt, int64_t m, int64_t n, int64_t k, const void* x, int64_t ldx) {
+    if (m < 1 || n < 1 || k > 8192 || ((uintptr_t)x & 15) || ldx % 8) return false;
     if (m > (k <= 2048 ? 64 : k <= 4096 ? 32 : 16)) return false;
     return 16 * packed_row_bytes(qt, k) <= (k <= 4096 ? 72 : 136) * 1024;
 }
 
-int gemv(int qt, const void* x, const void* w, int64_t m, int64_t n, int64_t k, const void* lora_a, const void* lora_b, int r, float scale, void* xa_out, void* y, hipStream_t s) {
+int gemv(int qt, const void* x, int64_t ldx, const void* w, int64_t m, int64_t n, int64_t k, const void* lora_a, const void* lora_b, int r, float scale, void* xa_out,
+         void* y, int64_t ldy, hipStream_t s) {
     GemvParams p{};
     p.x = (const bf16_t*)x, p.m = (int)m, p.n = (int)n, p.k = (int)k, p.w = (const uint8_t*)w, p.row_bytes = (int)packed_row_bytes(qt, k), p.y = (bf16_t*)y;
+    p.ldx = ldx, p.ldy = ldy;
     if (lora_a) p.lora_a = (const bf16_t*)lora_a, p.lora_b = (const bf16_t*)lora_b, p.r = r, p.r_pad = (r + 15) / 16 * 16, p.lora_scale = scale, p.xa_out = (bf16_t*)xa_out;
     p.stage_bytes = (16 * p.row_bytes + 1023) / 1024 * 1024;
     p.buffers = (p.n + 15) / 16 > 256 && p.stage_bytes <= 36 * 1024 ? 2 : 1;  // (one block per workgroup needs one buffer)

@@ -72,7 +72,10 @@ Tensor linear_forward(const Tensor& x, const Tensor& payload, const Tensor& a, c
     shape.back() = n;
     Tensor y = empty(shape, at::kBFloat16, x);
     if (!a.defined()) {
-        if (m) check(ggq_mmq(x.data_ptr(), payload.data_ptr(), (int)qt, m, n, k, y.data_ptr(), stream_of(x)));
+        if (m) {
+            Tensor ws = empty_bytes(ggq_lora_workspace_bytes(m, 0, 1, n, k, 0), x);
+            check(ggq_lora_mmq_forward(x.data_ptr(), payload.data_ptr(), (int)qt, m, n, k, nullptr, nullptr, 0, 0.f, nullptr, y.data_ptr(), ws.data_ptr(), ws.numel(), stream_of(x)));
+        }
         return y;
     }
     const int64_t r = a.size(0);
@@ -115,7 +118,11 @@ struct Linear : torch::autograd::Function<Linear> {
         if (!lora) {
             if (!ctx->needs_input_grad(0)) return out;
             out[0] = empty(shape, at::kBFloat16, g);
-            if (m) check(ggq_mmq_grad_input(g.data_ptr(), payload.data_ptr(), qt, m, n, k, out[0].data_ptr(), stream_of(g)));
+            if (m) {
+                Tensor ws = empty_bytes(ggq_lora_workspace_bytes(m, 0, 1, n, k, 0), g);
+                check(ggq_lora_mmq_backward(g.data_ptr(), payload.data_ptr(), qt, m, n, k, nullptr, nullptr, nullptr, nullptr, 0, 0.f, out[0].data_ptr(), nullptr, nullptr,
+                                            ws.data_ptr(), ws.numel(), stream_of(g)));
+            }
             return out;
         }
         const Tensor &x = saved[1], &xa = saved[2], &a = saved[3], &b = saved[4];

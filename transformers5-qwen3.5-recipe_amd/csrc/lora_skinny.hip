@@ -5,22 +5,11 @@
 //   factor_grad    G[e][c, j] = s * sum_{m in group e} In[m, c] * S[m, j]   (dB, dA; fixed order, no atomics)
 //   pad / transpose helpers that lay the factors out [cols][r_pad] for the tile kernel.
 #include <algorithm>
-#include "common.h"
+#include "factor_grad.h"
 #include "launch.h"
 #include "mmq_host.h"
 
 namespace ggq {
-
-__device__ __forceinline__ uint4 load8g(const bf16_t* p, int valid, bool vec) {
-    if (valid >= 8 && vec) return *(const uint4*)p;
-    uint4 v = make_uint4(0, 0, 0, 0);
-    if (valid <= 0) return v;
-    uint32_t e[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) e[i] = i < valid ? (uint32_t)p[i] : 0u;
-    v.x = e[0] | (e[1] << 16), v.y = e[2] | (e[3] << 16), v.z = e[4] | (e[5] << 16), v.w = e[6] | (e[7] << 16);
-    return v;
-}
 
 // ---- out[m, 0..r_pad) = In[m, :] . F[e][0..r, :]^T.  One workgroup per 16 rows; its four waves deal the
 // contraction out in 128-wide trips (trip t to wave t % 4), so a 64-row tile keeps sixteen waves of loads
@@ -130,9 +119,6 @@ __global__ __launch_bounds__(256) void skinny_nt_kernel(SkinnyNtParams p) {
 // 64-wide step of it is one contiguous run, copied as it is; the operand reads transpose it on the way out
 // of LDS (ds_read_b64_tr_b16: within 16 lanes, lane L gets element L % 4 of the 8 bytes addressed by lanes
 // L / 4 + 4 t, t = 0..3, so source lane s points at contraction row s / 4, factor columns 4 (s % 4) .. +3).
-typedef short v4i16_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4i16_t* lds_v4i16_ptr;
-
 template <int JB, bool FNAT>
 __global__ __launch_bounds__(256) void skinny_nt_direct_kernel(SkinnyNtParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t sk_lds[];
@@ -266,183 +252,36 @@ __global__ __launch_bounds__(256) void skinny_nt_direct_kernel(SkinnyNtParams p)
             }
 }
 
-// ---- G[e][c, j] = s * sum_m In[m, c] * S[m, j] over the rows of expert e.  One workgroup per
-// (expert, 64 * CB columns); each wave owns CB blocks of 16 columns; rows are consumed 32 at a time
-// through LDS, where the operands of the contraction over m are read with transposing loads.  The loads
-// of four 32-row slices are issued together and the slices then go through two alternating LDS buffers,
-// one barrier each.  Experts without rows get zeros.
 template <int JB, int CB>
 __global__ __launch_bounds__(256) void factor_grad_kernel(FactorGradParams p) {
-    // rows are contraction rows m; the operands are read with transposing 8-byte LDS reads (lane L of a
-    // 16-lane group gets element L % 4 of the 8 bytes addressed by lanes L / 4 + 4 t), so the tiles stay as
-    // loaded; the row pitches keep four consecutive rows' 32-byte pieces on distinct banks
-    constexpr int kCols = 64 * CB, kPitch = kCols + 32, kSPitch = JB * 16 + 8;
-    __shared__ __attribute__((aligned(16))) bf16_t in_t[2][32][kPitch];
-    __shared__ __attribute__((aligned(16))) bf16_t s_t[2][32][kSPitch];
-    __shared__ __attribute__((aligned(16))) bf16_t g_t[4][16][JB * 16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int blocks_per_seg = (p.c + kCols - 1) / kCols;
-    const int col_blocks = p.nseg * blocks_per_seg;
+    __shared__ __attribute__((aligned(16))) FactorGradLds<JB, CB> lds;
     // contiguous runs of (expert, column block) units per XCD: one L2 sees whole rows of an expert
     const int per_xcd = ((int)gridDim.x + 7) >> 3;
     const int unit = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= per_xcd || unit >= p.units) return;
-    const int splits = p.row_splits > 1 ? p.row_splits : 1;
-    const int split = unit % splits, ucb = unit / splits;
-    const int e = ucb / col_blocks, cblk = ucb - e * col_blocks;
-    const int seg = cblk / blocks_per_seg;
-    const int c0 = (cblk - seg * blocks_per_seg) * kCols;
-    int row_begin = 0, row_end = p.m;
-    if (p.ranges) {
-        row_begin = p.ranges[2 * e];
-        row_end = p.ranges[2 * e + 1];
-    } else if (splits > 1) {  // this workgroup's share of the rows, in whole 32-row slices
-        const int share = (((p.m + splits - 1) / splits) + 31) & ~31;
-        row_begin = min(p.m, split * share);
-        row_end = min(p.m, row_begin + share);
-    }
-    const bf16_t* in = p.in[seg];
-    const bool vec = ((p.ld_in & 7) == 0) && (((uintptr_t)in & 15) == 0);
-    const int li = lane & 15, lq = lane >> 4;
-    f32x4_t acc[CB][JB];
-#pragma unroll
-    for (int cb = 0; cb < CB; cb++)
-#pragma unroll
-        for (int jb = 0; jb < JB; jb++) acc[cb][jb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-    constexpr int rp = JB * 16;
-    const int tr = threadIdx.x >> 3, tch = threadIdx.x & 7;           // In slice: 32 rows x CB x 8 chunks of 8
-    const int sr = threadIdx.x / (rp / 8), sch = threadIdx.x % (rp / 8);  // S slice: 32 rows x rp/8 chunks
-    int buf = 0;
-    for (int m0 = row_begin; m0 < row_end; m0 += 128) {
-        uint4 vin[4][CB], vs[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int r = m0 + 32 * u + tr;
-            const int src = r < row_end ? p.in_rows.source(r) : 0;
-#pragma unroll
-            for (int cb = 0; cb < CB; cb++) {
-                const int tcc = c0 + cb * 64 + tch * 8;
-                vin[u][cb] = load8g(in + (int64_t)src * p.ld_in + tcc, r < row_end ? p.c - tcc : 0, vec);
-            }
-            vs[u] = make_uint4(0, 0, 0, 0);
-            if (sr < 32 && m0 + 32 * u + sr < row_end) {
-                const int64_t row = m0 + 32 * u + sr;
-                vs[u] = *(const uint4*)(p.s + row * rp + sch * 8);
-                if (p.s_weights) {
-                    const int64_t wi = p.s_weight_index[row];
-                    // (routing weights act at bf16 precision everywhere on the path)
-                    const float w = p.s_weights_are_bf16 ? bf16_to_f32(((const bf16_t*)p.s_weights)[wi]) : bf16_to_f32(to_bf16(((const float*)p.s_weights)[wi]));
-                    vs[u] = make_uint4(pack_bf16(bf16_lo(vs[u].x) * w, bf16_hi(vs[u].x) * w), pack_bf16(bf16_lo(vs[u].y) * w, bf16_hi(vs[u].y) * w),
-                                       pack_bf16(bf16_lo(vs[u].z) * w, bf16_hi(vs[u].z) * w), pack_bf16(bf16_lo(vs[u].w) * w, bf16_hi(vs[u].w) * w));
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            if (m0 + 32 * u >= row_end) break;  // uniform over the workgroup
-#pragma unroll
-            for (int cb = 0; cb < CB; cb++) *(uint4*)&in_t[buf][tr][cb * 64 + tch * 8] = vin[u][cb];
-            if (sr < 32) *(uint4*)&s_t[buf][sr][sch * 8] = vs[u];
-            // one barrier per slice: the slice after the next reuses this buffer, and every wave passes the
-            // next barrier only after its reads of this one
-            __syncthreads();
-            // B operand (n = factor column j, contraction m): source lane s = li points at contraction row
-            // 8*lq + s/4 (+4 for the second read), factor columns 4*(s%4) .. +3 of the block's 16
-            bf16x8_t b[JB];
-#pragma unroll
-            for (int jb = 0; jb < JB; jb++) {
-                const bf16_t* b_src = &s_t[buf][8 * lq + (li >> 2)][jb * 16 + (li & 3) * 4];
-                const v4i16_t b_lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)b_src);
-                const v4i16_t b_hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)(b_src + 4 * kSPitch));
-                b[jb] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(b_lo, b_hi, 0, 1, 2, 3, 4, 5, 6, 7));
-            }
-            // A operand (row = column c, contraction m): the same pattern over the wave's 16 columns of block cb
-#pragma unroll
-            for (int cb = 0; cb < CB; cb++) {
-                const bf16_t* a_src = &in_t[buf][8 * lq + (li >> 2)][cb * 64 + wave * 16 + (li & 3) * 4];
-                const v4i16_t a_lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)a_src);
-                const v4i16_t a_hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)(a_src + 4 * kPitch));
-                const bf16x8_t a = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(a_lo, a_hi, 0, 1, 2, 3, 4, 5, 6, 7));
-#pragma unroll
-                for (int jb = 0; jb < JB; jb++) acc[cb][jb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[jb], acc[cb][jb], 0, 0, 0);
-            }
-            buf ^= 1;
-        }
-    }
-    // acc[cb][jb][v]: c = c0 + 64*cb + wave*16 + 4*lq + v, j = 16*jb + li
-    const int64_t ctot = (int64_t)p.nseg * p.c;
-    if (splits > 1) {  // unscaled fp32 partial sums [split][column][r_pad]; factor_reduce_kernel finishes
-        float* part = p.partials + (int64_t)split * ctot * rp;
-#pragma unroll
-        for (int cb = 0; cb < CB; cb++)
-#pragma unroll
-            for (int jb = 0; jb < JB; jb++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int c = c0 + 64 * cb + wave * 16 + 4 * lq + v;
-                    if (c < p.c) part[((int64_t)seg * p.c + c) * rp + jb * 16 + li] = acc[cb][jb][v];
-                }
-        return;
-    }
-    bf16_t* out = p.out + (int64_t)e * p.out_expert_elems;
-    const bool vec4 = (ctot & 3) == 0 && (((uintptr_t)out & 7) == 0);
-    const bool vec8 = (p.r & 7) == 0 && (((uintptr_t)out & 15) == 0);
-#pragma unroll
-    for (int cb = 0; cb < CB; cb++) {
-        const int cw0 = c0 + 64 * cb + wave * 16;  // first column of this wave's block
-        if (p.out_j_major) {
-            // [r][columns]: a lane holds four consecutive columns of factor row j: one 8-byte store
-#pragma unroll
-            for (int jb = 0; jb < JB; jb++) {
-                const int j = jb * 16 + li, c = cw0 + 4 * lq;
-                if (j >= p.r) continue;
-                bf16_t* dst = out + (int64_t)j * ctot + (int64_t)seg * p.c + c;
-                if (vec4 && c + 3 < p.c) {
-                    *(uint2*)dst = make_uint2(pack_bf16(acc[cb][jb][0] * p.scale, acc[cb][jb][1] * p.scale), pack_bf16(acc[cb][jb][2] * p.scale, acc[cb][jb][3] * p.scale));
-                } else {
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        if (c + v < p.c) dst[v] = to_bf16(acc[cb][jb][v] * p.scale);
-                }
-            }
-        } else if (vec8) {
-            // [columns][r]: the wave's 16 columns x r are one contiguous run; transpose through LDS (each wave
-            // reads back only what it wrote; LDS serves a wave in order) and store 16 bytes per lane
-#pragma unroll
-            for (int jb = 0; jb < JB; jb++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) g_t[wave][4 * lq + v][jb * 16 + li] = to_bf16(acc[cb][jb][v] * p.scale);
-            const int chunks_per_row = p.r >> 3;
-            bf16_t* dst = out + ((int64_t)seg * p.c + cw0) * p.r;
-            for (int id = lane; id < 16 * chunks_per_row; id += 64) {
-                const int row = id / chunks_per_row, ch = id - row * chunks_per_row;
-                const uint4 piece = *(const uint4*)&g_t[wave][row][ch * 8];
-                if (cw0 + row < p.c) *(uint4*)(dst + (int64_t)id * 8) = piece;
-            }
-        } else {
-#pragma unroll
-            for (int jb = 0; jb < JB; jb++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int c = cw0 + 4 * lq + v, j = jb * 16 + li;
-                    if (c < p.c && j < p.r) out[((int64_t)seg * p.c + c) * p.r + j] = to_bf16(acc[cb][jb][v] * p.scale);
-                }
-        }
-    }
+    factor_grad_body<JB, CB>(p, unit, lds);
 }
 
-// out = bf16(scale * sum over the row splits, in split order) of the partial sums of a split factor_grad launch.
-// One lane per (column, j < r_pad); lanes of a wave run along j, then columns: contiguous reads.
-__global__ __launch_bounds__(256) void factor_reduce_kernel(const float* partials, bf16_t* out, int64_t ctot, int r, int r_pad, int splits, int out_j_major,
-                                                            float scale) {
-    const int64_t total = ctot * r_pad;
+// out = bf16(scale * sum over the row splits, in split order) of the partial sums of split factor_grad launches, one or two of
+// them (blockIdx.y).  One lane per (column, j < r_pad); lanes of a wave run along j, then columns: contiguous reads.
+struct FactorReduceParams {
+    const float* partials[2];
+    bf16_t* out[2];
+    int64_t ctot[2];
+    int splits[2], out_j_major[2];
+    int r, r_pad;
+    float scale;
+};
+__global__ __launch_bounds__(256) void factor_reduce_kernel(FactorReduceParams p) {
+    const int w = blockIdx.y;
+    const int64_t total = p.ctot[w] * p.r_pad;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-        const int64_t c = i / r_pad;
-        const int j = (int)(i - c * r_pad);
-        if (j >= r) continue;
+        const int64_t c = i / p.r_pad;
+        const int j = (int)(i - c * p.r_pad);
+        if (j >= p.r) continue;
         float sum = 0.f;
-        for (int sp = 0; sp < splits; sp++) sum += partials[(int64_t)sp * total + i];
-        out[out_j_major ? (int64_t)j * ctot + c : c * r + j] = to_bf16(sum * scale);
+        for (int sp = 0; sp < p.splits[w]; sp++) sum += p.partials[w][(int64_t)sp * total + i];
+        p.out[w][p.out_j_major[w] ? (int64_t)j * p.ctot[w] + c : c * p.r + j] = to_bf16(sum * p.scale);
     }
 }
 
@@ -568,22 +407,8 @@ int skinny_nt(const SkinnyNtParams& p, int r_pad, int grid_tiles, hipStream_t s)
 }
 
 template <int CB>
-static int launch_factor_grad(const FactorGradParams& p_in, int r_pad, int64_t experts, hipStream_t s) {
-    const int col_blocks = p_in.nseg * ((p_in.c + 64 * CB - 1) / (64 * CB));
-    FactorGradParams p = p_in;
-    // One row range for everything (a dense layer) leaves only the column blocks to spread over the compute units: deal
-    // the rows out as well, enough to give every unit a workgroup, in shares of at least 128 rows.
-    p.row_splits = 1;
-    if (!p.ranges && experts == 1 && p.partials && col_blocks < 256 && p.m >= 256) {
-        const int64_t want = (256 + col_blocks - 1) / col_blocks;
-        const int64_t fit = p.partials_bytes / ((int64_t)p.nseg * p.c * r_pad * 4);
-        p.row_splits = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, p.m / 128), std::min<int64_t>(fit, 64)));
-    }
-    const int64_t units = experts * col_blocks * p.row_splits;
-    if (units <= 0) return 0;
-    if (units > 0x7FFFFFF0) return set_error(GGQ_ERR_SHAPE, "factor_grad: grid too large");
-    const int64_t grid = (units + 7) / 8 * 8;
-    p.units = (int)units;
+static int launch_factor_grad(const FactorGradParams& p, int r_pad, hipStream_t s) {
+    const int64_t grid = ((int64_t)p.units + 7) / 8 * 8;
     switch (r_pad / 16) {
         case 1: hipLaunchKernelGGL((factor_grad_kernel<1, CB>), dim3((unsigned)grid), dim3(256), 0, s, p); break;
         case 2: hipLaunchKernelGGL((factor_grad_kernel<2, CB>), dim3((unsigned)grid), dim3(256), 0, s, p); break;
@@ -591,19 +416,38 @@ static int launch_factor_grad(const FactorGradParams& p_in, int r_pad, int64_t e
         case 4: hipLaunchKernelGGL((factor_grad_kernel<4, CB>), dim3((unsigned)grid), dim3(256), 0, s, p); break;
         default: return set_error(GGQ_ERR_SHAPE, "LoRA rank must be between 1 and 64");
     }
-    if (int rc = check_launch("factor_grad")) return rc;
-    if (p.row_splits > 1) {
-        const int64_t ctot = (int64_t)p.nseg * p.c;
-        const unsigned blocks = (unsigned)std::min<int64_t>((ctot * r_pad + 255) / 256, 4096);
-        hipLaunchKernelGGL(factor_reduce_kernel, dim3(blocks), dim3(256), 0, s, p.partials, p.out, ctot, p.r, r_pad, p.row_splits, p.out_j_major, p.scale);
-        return check_launch("factor_reduce");
-    }
-    return 0;
+    return check_launch("factor_grad");
 }
 
-int factor_grad(const FactorGradParams& p, int r_pad, int64_t experts, hipStream_t s) {
-    // wide column blocks (256 contiguous bytes per row and workgroup) when they divide the segment
-    return p.c % 128 == 0 ? launch_factor_grad<2>(p, r_pad, experts, s) : launch_factor_grad<1>(p, r_pad, experts, s);
+int factor_grad_partial(FactorGradParams& p, int r_pad, int64_t experts, hipStream_t s) {
+    const int64_t units = factor_grad_plan(p, r_pad, experts);
+    if (units <= 0) return 0;
+    if (units > 0x7FFFFFF0) return set_error(GGQ_ERR_SHAPE, "factor_grad: grid too large");
+    return p.c % 128 == 0 ? launch_factor_grad<2>(p, r_pad, s) : launch_factor_grad<1>(p, r_pad, s);
+}
+
+int factor_reduce(const FactorGradParams* const* ps, int count, int r_pad, hipStream_t s) {
+    FactorReduceParams q{};
+    int n = 0;
+    int64_t most = 0;
+    for (int i = 0; i < count; i++) {
+        const FactorGradParams& p = *ps[i];
+        if (p.row_splits <= 1) continue;  // its launch wrote the result
+        q.partials[n] = p.partials, q.out[n] = p.out, q.ctot[n] = (int64_t)p.nseg * p.c, q.splits[n] = p.row_splits, q.out_j_major[n] = p.out_j_major;
+        q.r = p.r, q.r_pad = r_pad, q.scale = p.scale;
+        most = std::max(most, q.ctot[n] * r_pad);
+        n++;
+    }
+    if (!n) return 0;
+    hipLaunchKernelGGL(factor_reduce_kernel, dim3((unsigned)std::min<int64_t>((most + 255) / 256, 4096), n), dim3(256), 0, s, q);
+    return check_launch("factor_reduce");
+}
+
+int factor_grad(const FactorGradParams& p_in, int r_pad, int64_t experts, hipStream_t s) {
+    FactorGradParams p = p_in;
+    if (int rc = factor_grad_partial(p, r_pad, experts, s)) return rc;
+    const FactorGradParams* one = &p;
+    return factor_reduce(&one, 1, r_pad, s);
 }
 
 }  // namespace ggq

@@ -150,20 +150,29 @@ struct DenseCall {
     bool fp32;            // c is fp32 (a multiple of four columns)
     bool accumulate;      // fp32: c = c * row_scale[m] + result instead of c = result
     const float* row_scale;
-    const void *la, *lb;  // LoRA: la [m, r_pad]; lb NT [n, r_pad], NN the factor A [rank, k]
+    const void *la, *lb;  // LoRA: la [m, r_pad]; lb NT the factor B [n, rank], NN the factor A [rank, k]
     int r_pad, rank;
     float lora_scale;
 };
+// Rank-sized work of a dense LoRA call that depends on nothing its decoding pass writes, and runs in that pass's launch.
+struct DenseSide {
+    const SkinnyNtParams* product;  // x A^T, or dy B; null: none
+    FactorGradParams* gradient;     // dB; null: none (its row_splits are set)
+    int r_pad;
+};
+constexpr int kDenseSideMaxRank = 32;
+bool dense_side_takes(const DenseSide& side);
 bool dense_takes(int mode, int64_t m, int64_t n, int64_t k, const void* a, int64_t lda, bool a_zero_padded = false);
 bool dense_panel_whole(int64_t n, int64_t k);
 int64_t dense_workspace_bytes(int64_t m, int64_t n, int64_t k);
-int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s);
+int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s, const DenseSide* side = nullptr);
 void dense_force_shape(int shape, int splits);  // test aid: -1 = the automatic choice
 
 // Products of a few rows (gemv.hip).
 constexpr int kShapeFewRows = 7;  // (profile records only)
-bool gemv_takes(int qt, int64_t m, int64_t n, int64_t k, const void* x);
-int gemv(int qt, const void* x, const void* w, int64_t m, int64_t n, int64_t k, const void* lora_a, const void* lora_b, int r, float scale, void* xa_out, void* y, hipStream_t s);
+bool gemv_takes(int qt, int64_t m, int64_t n, int64_t k, const void* x, int64_t ldx);
+int gemv(int qt, const void* x, int64_t ldx, const void* w, int64_t m, int64_t n, int64_t k, const void* lora_a, const void* lora_b, int r, float scale, void* xa_out,
+         void* y, int64_t ldy, hipStream_t s);
 constexpr int kRouterLogitsMaxTokens = 8;
 int router_logits(const void* x, const void* w, int64_t m, int64_t n, int64_t k, void* y, hipStream_t s);
 bool few_routes_takes(int qt_in, int qt_down, int64_t tokens, int top_k, int64_t hidden, int64_t inter);
@@ -176,6 +185,9 @@ int transpose_factor(const bf16_t* src, bf16_t* dst, int64_t experts, int c, int
 int skinny_nt(const SkinnyNtParams& p, int r_pad, int grid_tiles, hipStream_t s);
 bool skinny_nt_takes_natural_factor(const SkinnyNtParams& p);
 int factor_grad(const FactorGradParams& p, int r_pad, int64_t experts, hipStream_t s);
+// The same in two parts, so that one pass adds the partial sums of several: the launch (sets p.row_splits), and the sums.
+int factor_grad_partial(FactorGradParams& p, int r_pad, int64_t experts, hipStream_t s);
+int factor_reduce(const FactorGradParams* const* ps, int count, int r_pad, hipStream_t s);
 
 // Builds the row-tile table of an expert-sorted layout on the device (no host sync):
 // tiles[0..*num_tiles) in group order, tile height bm; optionally per-expert row ranges.

@@ -43,13 +43,9 @@ def _flat_bf16(x: torch.Tensor, name: str) -> torch.Tensor:
 
 
 def _mmq_forward(x: torch.Tensor, payload: torch.Tensor, quant_type: int, out_features: int) -> torch.Tensor:
-    x2 = _flat_bf16(x, "mmq input")
-    m, k = x2.shape
-    _check_packed(payload, quant_type, out_features, k, "mmq")
-    y = torch.empty(m, out_features, dtype=torch.bfloat16, device=x.device)
-    if m:
-        _lib.check(_lib.load().ggq_mmq(x2.data_ptr(), payload.data_ptr(), quant_type, m, out_features, k, y.data_ptr(), _lib.stream_handle(x.device)))
-    return y.reshape(*x.shape[:-1], out_features)
+    """``mmq`` outside autograd (what the registered operators call)."""
+    with torch.no_grad():
+        return mmq(x, payload, quant_type, out_features)
 
 
 def mmq_grad_input(grad_output: torch.Tensor, payload: torch.Tensor, quant_type: int, in_features: int) -> torch.Tensor:
@@ -61,7 +57,9 @@ def mmq_grad_input(grad_output: torch.Tensor, payload: torch.Tensor, quant_type:
     _check_packed(payload, quant_type, n, in_features, "mmq_grad_input")
     dx = torch.empty(m, in_features, dtype=torch.bfloat16, device=grad_output.device)
     if m:
-        _lib.check(_lib.load().ggq_mmq_grad_input(g2.data_ptr(), payload.data_ptr(), quant_type, m, n, in_features, dx.data_ptr(), _lib.stream_handle(g2.device)))
+        ws = _panel_workspace(g2.device, m, n, in_features)
+        _lib.check(_lib.load().ggq_lora_mmq_backward(g2.data_ptr(), payload.data_ptr(), quant_type, m, n, in_features, None, None, None, None, 0, 0.0,
+                                                     dx.data_ptr(), None, None, ws.data_ptr(), ws.numel(), _lib.stream_handle(g2.device)))
     return dx.reshape(*grad_output.shape[:-1], in_features)
 
 
@@ -69,6 +67,10 @@ def mmq(x: torch.Tensor, payload: torch.Tensor, quant_type: int, out_features: i
     """Y = X . W^T over packed rows (the reference's ``torch_ggml_ops.mmq``, fast_lora.py:155-160)."""
     y = _lib.host().linear(x, payload, int(quant_type), int(out_features), None, None, 0.0)
     return y if y is not None else _rejected_linear(x, payload, int(quant_type), int(out_features), None, None, "mmq")
+
+
+def _panel_workspace(device, rows: int, n: int, k: int) -> torch.Tensor:
+    return torch.empty(_lib.load().ggq_lora_workspace_bytes(rows, 0, 1, n, k, 0), dtype=torch.uint8, device=device)
 
 
 class _FixedGroupedMmq(torch.autograd.Function):
@@ -82,8 +84,9 @@ class _FixedGroupedMmq(torch.autograd.Function):
         _check_packed(packed_groups[0], quant_type, n_group, k, "fixed grouped MMQ")
         rows = x.numel() // (groups * k)
         y = torch.empty(*x.shape[:-1], n_group, dtype=torch.bfloat16, device=x.device)
-        _lib.check(_lib.load().ggq_fixed_grouped_mmq(x.data_ptr(), packed_groups.data_ptr(), quant_type, rows, groups, n_group, k, y.data_ptr(),
-                                                     _lib.stream_handle(x.device)))
+        ws = _panel_workspace(x.device, rows, n_group, k)
+        _lib.check(_lib.load().ggq_fixed_grouped_mmq_ws(x.data_ptr(), packed_groups.data_ptr(), quant_type, rows, groups, n_group, k, y.data_ptr(),
+                                                        ws.data_ptr(), ws.numel(), _lib.stream_handle(x.device)))
         ctx.save_for_backward(packed_groups)
         ctx.quant_type, ctx.k = quant_type, k
         return y
@@ -96,11 +99,7 @@ class _FixedGroupedMmq(torch.autograd.Function):
             return None, None, None
         (packed_groups,) = ctx.saved_tensors
         g = grad_output.contiguous()
-        groups, n_group = packed_groups.shape[0], packed_groups.shape[1]
-        rows = g.numel() // (groups * n_group)
-        dx = torch.empty(*g.shape[:-1], ctx.k, dtype=torch.bfloat16, device=g.device)
-        _lib.check(_lib.load().ggq_fixed_grouped_mmq_grad_input(g.data_ptr(), packed_groups.data_ptr(), ctx.quant_type, rows, groups, n_group, ctx.k,
-                                                                dx.data_ptr(), _lib.stream_handle(g.device)))
+        dx = fixed_grouped_mmq_grad_input(g, packed_groups, ctx.quant_type, ctx.k)
         return dx, None, None
 
 
@@ -120,8 +119,9 @@ def fixed_grouped_mmq_grad_input(grad_output: torch.Tensor, packed_groups: torch
         raise ValueError(f"fixed grouped cotangent {tuple(grad_output.shape)} does not fit packed groups {tuple(packed_groups.shape)} of type {quant_type}")
     rows = grad_output.numel() // (groups * n_group)
     dx = torch.empty(*grad_output.shape[:-1], in_features, dtype=torch.bfloat16, device=grad_output.device)
-    _lib.check(_lib.load().ggq_fixed_grouped_mmq_grad_input(grad_output.data_ptr(), packed_groups.data_ptr(), quant_type, rows, groups, n_group, in_features,
-                                                            dx.data_ptr(), _lib.stream_handle(grad_output.device)))
+    ws = _panel_workspace(grad_output.device, rows, n_group, in_features)
+    _lib.check(_lib.load().ggq_fixed_grouped_mmq_grad_input_ws(grad_output.data_ptr(), packed_groups.data_ptr(), quant_type, rows, groups, n_group, in_features,
+                                                               dx.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_handle(grad_output.device)))
     return dx
 
 
