@@ -68,11 +68,6 @@ int ggq_set_factor_gradient_overlap(int enabled);
  * the stated tolerances whatever is chosen. */
 int ggq_debug_force_grouped_shape(int shape);
 
-/* Test aid: forces the output tile of the dense launches that run over decoded panels (0: 256 x 256, 1: 256 x 128,
- * 2: 128 x 128, 3: 64 x 64; -1: the library's choice) and, where the contraction may be split, the number of splits
- * (0: the library's choice).  Workspace sizes follow the setting. */
-int ggq_debug_force_dense_shape(int shape, int splits);
-
 /* fast_lora.py:24-31 (_NATIVE_MMQ_QUANT_TYPES / supports_native_mmq): 1 if this library has kernels
  * for the GGML type id. */
 int ggq_supports_quant_type(int qt);

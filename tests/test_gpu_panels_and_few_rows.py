@@ -1,0 +1,133 @@
+"""The dense launches over decoded panels, the products of a few rows, and the layers' native host calls, at the sizes
+where they can go wrong: tile edges, split contractions, ragged rows and columns, the ends of each range."""
+
+import contextlib
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import ALL_TYPES, TYPE_NAMES, assert_close_bf16, bf16_randn, make_payload
+from oracle import gguf_blocks as gb
+from oracle import lora_matmul as ref
+from oracle import routing as rref
+
+pytestmark = pytest.mark.gpu
+
+
+def _lora_case(seed, m, n, k, r, qt):
+    gen = torch.Generator().manual_seed(seed)
+    payload = make_payload(seed, qt, n, k, "random")
+    return payload, bf16_randn(gen, m, k), bf16_randn(gen, r, k, std=k ** -0.5), bf16_randn(gen, n, r, std=0.02), bf16_randn(gen, m, n)
+
+
+def _check_lora(pkg, dev, payload, qt, x, a, b, s, dy):
+    """Against fp32 products on the device of the oracle's decoded weights (bf16 values: their products are exact in fp32)."""
+    w, n = ref.weights_bf16(payload, qt).to(dev).float(), b.shape[0]
+    xd, ad, bd = (t.to(dev).requires_grad_(True) for t in (x, a, b))
+    y = pkg.fast_lora.lora_mmq(xd, torch.from_numpy(payload).to(dev), qt, n, ad, bd, s)
+    y.backward(dy.to(dev))
+    xf, af, bf, df = (t.to(dev).float() for t in (x, a, b, dy))
+    xa, dyb = (xf @ af.T).bfloat16().float(), (df @ bf).bfloat16().float()
+    assert_close_bf16(y, xf @ w.T + s * xa @ bf.T, "Y")
+    assert_close_bf16(xd.grad, df @ w + s * dyb @ af, "dX")
+    assert_close_bf16(ad.grad, s * dyb.T @ xf, "dA")
+    assert_close_bf16(bd.grad, s * df.T @ xa, "dB")
+
+
+@pytest.mark.parametrize("m,n,k,r", [
+    (48, 64, 256, 16),      # the fewest rows
+    (49, 65, 512, 5),       # one row and one column past a tile; a rank that is no multiple of eight; columns that no split takes
+    (63, 511, 4096, 32),    # the widest rank of the shared launch
+    (64, 512, 8192, 16),    # eight contraction splits
+    (257, 520, 2048, 33),   # a rank of the separate launches
+    (1500, 2052, 1024, 8),  # 128 x 128 tiles forward
+    (3001, 5001, 256, 16),  # 256 x 256 tiles, ragged both ways; the shortest contraction
+    (4096, 1028, 2048, 4),
+])
+@pytest.mark.parametrize("qt", [gb.Q8_0, gb.Q4_K, gb.IQ2_XXS], ids=lambda q: TYPE_NAMES[q])
+def test_dense_lora_over_panels(pkg, dev, qt, m, n, k, r):
+    payload, x, a, b, dy = _lora_case(7000 + m + n, m, n, k, r, qt)
+    _check_lora(pkg, dev, payload, qt, x, a, b, 32.0 / r, dy)
+
+
+def test_dense_matrix_in_slabs(pkg, dev):
+    # more than 128 MB of decoded weights: forward in slabs of output columns (70000 x 1024 x 2 bytes)
+    qt, m, n, k = gb.Q8_0, 50, 70001, 1024
+    payload, x, *_ = _lora_case(88, m, n, k, 4, qt)
+    y = pkg.fast_lora.mmq(x.to(dev), torch.from_numpy(payload).to(dev), qt, n)
+    assert_close_bf16(y, x.to(dev).float() @ ref.weights_bf16(payload, qt).to(dev).float().T, "Y")
+
+
+@pytest.mark.parametrize("m,n,k,r", [
+    (1, 1, 256, 1), (1, 4099, 2048, 16), (16, 17, 512, 64), (17, 48, 2048, 24), (64, 5000, 2048, 8),  # two LDS buffers from 4097 columns
+    (32, 100, 4096, 40), (16, 33, 8192, 16), (47, 31, 1024, 5),
+])
+@pytest.mark.parametrize("qt", ALL_TYPES, ids=[TYPE_NAMES[q] for q in ALL_TYPES])
+def test_few_rows(pkg, dev, qt, m, n, k, r):
+    payload, x, a, b, _ = _lora_case(9000 + m + n, m, n, k, r, qt)
+    w = ref.weights_bf16(payload, qt).to(dev).float()
+    p, xf, s = torch.from_numpy(payload).to(dev), x.to(dev).float(), 2.0
+    y = pkg.fast_lora.lora_mmq(x.to(dev), p, qt, n, a.to(dev), b.to(dev), s)
+    xa = (xf @ a.to(dev).float().T).bfloat16().float()
+    assert_close_bf16(y, xf @ w.T + s * xa @ b.to(dev).float().T, "Y with LoRA")
+    assert_close_bf16(pkg.fast_lora.mmq(x.to(dev), p, qt, n), xf @ w.T, "Y")
+
+
+@pytest.mark.parametrize("k", [64, 192, 320])
+def test_few_rows_of_a_contraction_that_ends_inside_a_span(pkg, dev, k):
+    # 128-element spans; only the 32-element block format has such lengths
+    payload, x, *_ = _lora_case(k, 5, 70, k, 4, gb.Q8_0)
+    y = pkg.fast_lora.mmq(x.to(dev), torch.from_numpy(payload).to(dev), gb.Q8_0, 70)
+    assert_close_bf16(y, x.to(dev).float() @ ref.weights_bf16(payload, gb.Q8_0).to(dev).float().T, "Y")
+
+
+def _expert_layer(pkg, dev, qt, qt_down, experts, hidden, inter, r, limit=None, seed=0):
+    gen = torch.Generator().manual_seed(4000 + seed)
+    planes = [np.stack([make_payload(seed + 31 * i + e, q, n, k, "random") for e in range(experts)])
+              for i, (q, n, k) in enumerate([(qt, inter, hidden), (qt, inter, hidden), (qt_down, hidden, inter)])]
+    packed = [pkg.gguf.GGUFQuantizedTensor(torch.from_numpy(p).to(dev), q, (experts, n, k))
+              for p, (q, n, k) in zip(planes, [(qt, inter, hidden), (qt, inter, hidden), (qt_down, hidden, inter)])]
+    base = pkg.fast_moe_lora.GGUFExperts(*packed)
+    if limit:
+        base.swiglu_limit = limit
+    layer = pkg.fast_moe_lora.FastGGUFMoeLora(base, r=r, lora_alpha=2 * r)
+    factors = {"lora_A": (experts, r, hidden), "lora_B": (experts, 2 * inter, r), "lora_A_down": (experts, r, inter), "lora_B_down": (experts, hidden, r)}
+    with torch.no_grad():
+        for name, shape in factors.items():
+            getattr(layer, name)["default"].weight.copy_(bf16_randn(gen, *shape, std=0.02).to(dev))
+    return layer, [ref.weights_bf16(p, q) for p, q in zip(planes, (qt, qt, qt_down))], gen
+
+
+@pytest.mark.parametrize("tokens,top_k,hidden,inter,r,limit,ids", [
+    (1, 8, 2048, 512, 16, None, torch.int64), (8, 8, 256, 256, 5, 0.25, torch.int32),   # 64 routes: the most
+    (4, 16, 512, 768, 64, None, torch.int64), (3, 1, 4096, 256, 24, None, torch.int32),
+])
+@pytest.mark.parametrize("qt", ALL_TYPES, ids=[TYPE_NAMES[q] for q in ALL_TYPES])
+def test_experts_of_a_few_routes(pkg, dev, qt, tokens, top_k, hidden, inter, r, limit, ids):
+    experts = max(top_k, 4)
+    layer, (wg, wu, wd), gen = _expert_layer(pkg, dev, qt, qt, experts, hidden, inter, r, limit)
+    x = bf16_randn(gen, tokens, hidden)
+    top = torch.stack([torch.randperm(experts, generator=gen)[:top_k] for _ in range(tokens)])
+    weights = torch.softmax(torch.randn(tokens, top_k, generator=gen), -1)
+    with torch.no_grad():
+        got = layer(x.to(dev), top.to(dev, ids), weights.to(dev))
+    _, perm, inv = rref.plan(top)
+    active, offsets = rref.active_offsets(rref.expert_counts(top, experts))
+    factors = [getattr(layer, name)["default"].weight.detach().cpu() for name in ("lora_A", "lora_B", "lora_A_down", "lora_B_down")]
+    rows = ref.expert_layer(rref.gather_forward(x, perm, top_k), active, offsets, wg, wu, wd, *factors, 2.0, limit=limit)["out"]
+    want = rref.combine_forward(ref.bf16_round(rows).to(torch.bfloat16), weights, inv)
+    # bf16 roundings that a sum in another order may land on the other side of: x A^T, gate and up, the activation, a route's row
+    assert_close_bf16(got, want, "experts", ulps=4)
+
+
+@pytest.mark.parametrize("tokens,experts,hidden", [(1, 4, 8), (1, 256, 2048), (8, 100, 1000), (5, 8, 136)])
+def test_router_logits_of_a_few_tokens(pkg, dev, tokens, experts, hidden):
+    gen = torch.Generator().manual_seed(tokens + experts)
+    x, w = bf16_randn(gen, tokens, hidden), bf16_randn(gen, experts, hidden, std=hidden ** -0.5)
+    with torch.no_grad():
+        logits, scores, ids = pkg.fast_moe_ranking.qwen_router_forward(w.to(dev), x.to(dev), 4)
+    assert_close_bf16(logits, x.double() @ w.double().T, "logits")
+    want, order = torch.sort(logits.float().cpu(), dim=-1, descending=True, stable=True)
+    assert torch.equal(ids.cpu(), order[:, :4])
+    assert_close_bf16(scores, torch.softmax(want[:, :4].double(), -1), "scores")

@@ -133,12 +133,6 @@ int ggq_debug_force_grouped_shape(int shape) {
     return GGQ_OK;
 }
 
-int ggq_debug_force_dense_shape(int shape, int splits) {
-    if (shape < -1 || shape > 3 || splits < 0 || splits > 8) return set_error(GGQ_ERR_SHAPE, "debug_force_dense_shape: unknown shape %d or %d splits", shape, splits);
-    dense_force_shape(shape, splits);
-    return GGQ_OK;
-}
-
 int ggq_set_factor_gradient_overlap(int enabled) {
     g_overlap_enabled.store(enabled ? 1 : 0, std::memory_order_relaxed);
     return GGQ_OK;

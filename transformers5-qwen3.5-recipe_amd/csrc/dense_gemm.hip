@@ -13,7 +13,6 @@
 // (ds_read_b64_tr_b16).  The swizzle keeps both free of bank conflicts: sixteen consecutive rows at one chunk cover all
 // bank groups, and four consecutive rows at an aligned pair of chunks cover four distinct 32-byte bank runs of each half.
 #include <algorithm>
-#include <atomic>
 #include <type_traits>
 
 #include "blocks.h"
@@ -250,7 +249,6 @@ __device__ __forceinline__ void wait_loads(int n) {  // at most n of this wave's
     switch (n) {
         case 0: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
         case 4: asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); break;
-        case 6: asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); break;
         case 8: asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); break;
         case 12: asm volatile("s_waitcnt vmcnt(12)" ::: "memory"); break;
         default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
@@ -572,19 +570,14 @@ template <int MODE, int EPI>
 static int launch_shape_mode(int shape, const DenseParams& p, hipStream_t s) {
     switch (shape) {
         case 0: return launch_tile<MODE, 2, 4, 4, 2, 2, EPI>(p, s);   // 256 x 256
-        case 1: return launch_tile<MODE, 4, 2, 2, 2, 3, EPI>(p, s);   // 256 x 128
-        case 2: return launch_tile<MODE, 2, 2, 2, 2, 2, EPI>(p, s);   // 128 x 128, two workgroups per compute unit
-        case 3: return launch_tile<MODE, 2, 2, 1, 1, 4, EPI>(p, s);   // 64 x 64, two workgroups per compute unit
+        case 1: return launch_tile<MODE, 2, 2, 2, 2, 2, EPI>(p, s);   // 128 x 128, two workgroups per compute unit
+        case 2: return launch_tile<MODE, 2, 2, 1, 1, 4, EPI>(p, s);   // 64 x 64, two workgroups per compute unit
     }
     return set_error(GGQ_ERR_SHAPE, "dense_gemm: unknown tile shape");
 }
 template <int EPI>
 static int launch_shape(int mode, int shape, const DenseParams& p, hipStream_t s) {
     return mode == kModeNT ? launch_shape_mode<kModeNT, EPI>(shape, p, s) : launch_shape_mode<kModeNN, EPI>(shape, p, s);
-}
-static void shape_size(int shape, int& bm, int& bn) {
-    bm = shape <= 1 ? 256 : shape == 2 ? 128 : 64;
-    bn = shape == 0 ? 256 : shape <= 2 ? 128 : 64;
 }
 
 template <int QT>
@@ -644,23 +637,16 @@ bool dense_panel_whole(int64_t n, int64_t k) { return slab_columns(n, k) >= n &&
 
 // Tile shape and number of contraction splits for an [m, cols] output: the smallest estimate of
 // rounds of workgroups x (steps x time per step + fixed cost), plus the pass that adds split partial sums.
-static std::atomic<int> g_force_shape{-1}, g_force_splits{0};
-void dense_force_shape(int shape, int splits) { g_force_shape.store(shape), g_force_splits.store(splits); }
-
 static void pick_tile(int64_t m, int64_t cols, int64_t steps, bool can_split, int& shape, int& splits) {
     // microseconds per 64-wide step with every slot of the chip busy, workgroups per chip, and cost of a tile's start and end
-    static const struct { double step, fixed; int slots; } kShape[4] = {{1.15, 6.0, 256}, {0.65, 4.5, 256}, {0.60, 4.0, 512}, {0.25, 3.0, 512}};
+    static const struct { double step, fixed; int slots; } kShape[3] = {{1.15, 6.0, 256}, {0.60, 4.0, 512}, {0.25, 3.0, 512}};
     double best = 1e30;
     shape = 0, splits = 1;
-    const int forced = g_force_shape.load();
-    for (int sh = 0; sh < 4; sh++) {
-        if (forced >= 0 && sh != forced) continue;
-        int bm, bn;
-        shape_size(sh, bm, bn);
-        const int64_t tiles = ((m + bm - 1) / bm) * ((cols + bn - 1) / bn);
+    for (int sh = 0; sh < 3; sh++) {
+        const int side = 256 >> sh;
+        const int64_t tiles = ((m + side - 1) / side) * ((cols + side - 1) / side);
         for (int sp = 1; sp <= kMaxSplits; sp *= 2) {
             if (sp > 1 && (!can_split || steps < 4 * sp)) break;
-            if (g_force_splits.load() > 0 && sp != g_force_splits.load() && can_split) continue;
             const double rounds = (double)((tiles * sp + kShape[sh].slots - 1) / kShape[sh].slots);
             double t = rounds * (((steps + sp - 1) / sp) * kShape[sh].step + kShape[sh].fixed);
             if (sp > 1) t += 3.0 + (double)m * cols * 4.0 * (2 * sp) / 4.5e6;

@@ -166,7 +166,6 @@ bool dense_takes(int mode, int64_t m, int64_t n, int64_t k, const void* a, int64
 bool dense_panel_whole(int64_t n, int64_t k);
 int64_t dense_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s, const DenseSide* side = nullptr);
-void dense_force_shape(int shape, int splits);  // test aid: -1 = the automatic choice
 
 // Products of a few rows (gemv.hip).
 constexpr int kShapeFewRows = 7;  // (profile records only)
