@@ -131,3 +131,46 @@ def test_router_logits_of_a_few_tokens(pkg, dev, tokens, experts, hidden):
     want, order = torch.sort(logits.float().cpu(), dim=-1, descending=True, stable=True)
     assert torch.equal(ids.cpu(), order[:, :4])
     assert_close_bf16(scores, torch.softmax(want[:, :4].double(), -1), "scores")
+
+
+# ------------------------------------------------------------------------------------------------
+# What stands around a call: saved-tensor hooks, module hooks, tracing, forward mode.
+def _small_linear(pkg, dev):
+    payload, x, a, b, dy = _lora_case(5, 64, 96, 256, 8, gb.Q4_K)
+    return torch.from_numpy(payload).to(dev), *(t.to(dev) for t in (x, a, b, dy))
+
+
+def test_saved_tensor_hooks_reach_the_native_nodes(pkg, dev):
+    p, x, a, b, dy = _small_linear(pkg, dev)
+
+    def grads(hooks):
+        xs = [t.clone().requires_grad_(True) for t in (x, a, b)]
+        with hooks:
+            y = pkg.fast_lora.lora_mmq(xs[0], p, gb.Q4_K, 96, xs[1], xs[2], 2.0)
+        y.backward(dy)
+        return [t.grad for t in xs]
+
+    for got, want in zip(grads(torch.autograd.graph.save_on_cpu()), grads(contextlib.nullcontext())):
+        assert torch.equal(got, want)
+
+
+def test_a_traced_linear_computes_on_its_inputs(pkg, dev):
+    p, x, a, b, _ = _small_linear(pkg, dev)
+
+    def call(inp):
+        return pkg.fast_lora.lora_mmq(inp, p, gb.Q4_K, 96, a, b, 2.0)
+
+    with torch.no_grad():
+        traced = torch.jit.trace(call, (x,), check_trace=False)
+        other = x.flip(0).contiguous()
+        assert torch.equal(traced(other), call(other)), "the trace holds the first call's result"
+
+
+def test_forward_mode_is_refused(pkg, dev):
+    import torch.autograd.forward_ad as fwad
+
+    p, x, a, b, _ = _small_linear(pkg, dev)
+    with fwad.dual_level(), torch.no_grad():
+        dual = fwad.make_dual(x, torch.ones_like(x))
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            pkg.fast_lora.lora_mmq(dual, p, gb.Q4_K, 96, a, b, 2.0)

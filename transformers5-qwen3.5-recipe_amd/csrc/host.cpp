@@ -4,8 +4,9 @@
 // takes the interpreter lock on the engine's thread), and a dozen tensor methods per check.  At the sizes of one short
 // sequence that was most of a step's time.
 //
-// Every entry returns None when an operand is not what the kernels take; the Python caller then runs its own checks,
-// which name what is wrong (one place for the error texts), or takes its general path.
+// Every entry returns None when an operand is not what the kernels take, and while a call is being traced or carries
+// forward-mode tangents (neither sees launches made here); the Python caller then runs its own checks, which name what is
+// wrong (one place for the error texts), or takes its general path.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -56,6 +57,14 @@ Tensor usable_cotangent(const Tensor& g, const char* what) {
 }
 
 void refuse_higher_order(const char* what) { TORCH_CHECK(!at::GradMode::is_enabled(), what, " does not support higher-order gradients"); }
+
+// Tracing records Python autograd functions, and forward mode has them refuse: those calls are left to the general path.
+bool traced_or_forward_mode(std::initializer_list<const Tensor*> ts) {
+    if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer)) return true;
+    for (const Tensor* t : ts)
+        if (t->defined() && t->_fw_grad(0).defined()) return true;
+    return false;
+}
 
 bool any_requires_grad(std::initializer_list<const Tensor*> ts) {
     if (!at::GradMode::is_enabled()) return false;
@@ -327,6 +336,7 @@ PyObject* host_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const Tensor x = arg_tensor(args[0]), payload = arg_tensor(args[1]), a = arg_tensor(args[4]), b = arg_tensor(args[5]);
     const int64_t qt = arg_int(args[2]), n = arg_int(args[3]);
     const double scaling = arg_double(args[6]);
+    if (traced_or_forward_mode({&x, &a, &b})) Py_RETURN_NONE;
     if (!usable(x, at::kBFloat16) || x.dim() < 1 || !usable_weight(payload, 2, qt, x.size(-1)) || payload.size(0) != n || x.device() != payload.device()) Py_RETURN_NONE;
     if (a.defined() != b.defined()) Py_RETURN_NONE;
     if (a.defined() && (!usable(a, at::kBFloat16) || !usable(b, at::kBFloat16) || a.dim() != 2 || b.dim() != 2 || a.size(1) != x.size(-1) || b.size(0) != n ||
@@ -351,6 +361,7 @@ PyObject* host_experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                  all_experts = arg_tensor(args[10]);
     const int64_t qt1 = arg_int(args[11]), qt2 = arg_int(args[12]);
     const double scaling = arg_double(args[13]), limit = arg_double(args[14]);
+    if (traced_or_forward_mode({&x, &weights, &a1, &b1, &a2, &b2})) Py_RETURN_NONE;
     if (!usable(x, at::kBFloat16) || x.dim() < 2 || x.size(-1) % 8 || x.size(-1) == 0) Py_RETURN_NONE;
     const int64_t hidden = x.size(-1), tokens = x.numel() / hidden;
     if (!ids.defined() || !ids.is_cuda() || (ids.scalar_type() != at::kLong && ids.scalar_type() != at::kInt) || !ids.is_contiguous() || ids.dim() != 2 ||
@@ -394,7 +405,7 @@ PyObject* host_router(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const int64_t top_k = arg_int(args[2]);
     if (!weight.defined() || !hidden.defined() || !weight.is_cuda() || hidden.device() != weight.device() || weight.dim() != 2 || hidden.dim() != 2 ||
         weight.scalar_type() != hidden.scalar_type() || (weight.scalar_type() != at::kBFloat16 && weight.scalar_type() != at::kFloat) ||
-        hidden.size(1) != weight.size(1) || any_requires_grad({&weight, &hidden}))
+        hidden.size(1) != weight.size(1) || any_requires_grad({&weight, &hidden}) || traced_or_forward_mode({&weight, &hidden}))
         Py_RETURN_NONE;
     const int64_t experts = weight.size(0);
     if (experts > 256 || experts % 4 || top_k < 1 || top_k > std::min<int64_t>(8, experts)) Py_RETURN_NONE;

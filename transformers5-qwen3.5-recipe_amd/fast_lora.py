@@ -66,7 +66,7 @@ def mmq_grad_input(grad_output: torch.Tensor, payload: torch.Tensor, quant_type:
 def mmq(x: torch.Tensor, payload: torch.Tensor, quant_type: int, out_features: int) -> torch.Tensor:
     """Y = X . W^T over packed rows (the reference's ``torch_ggml_ops.mmq``, fast_lora.py:155-160)."""
     y = _lib.host().linear(x, payload, int(quant_type), int(out_features), None, None, 0.0)
-    return y if y is not None else _rejected_linear(x, payload, int(quant_type), int(out_features), None, None, "mmq")
+    return y if y is not None else _general_linear(x, payload, int(quant_type), int(out_features), None, None, 0.0, "mmq")
 
 
 def _panel_workspace(device, rows: int, n: int, k: int) -> torch.Tensor:
@@ -125,22 +125,66 @@ def fixed_grouped_mmq_grad_input(grad_output: torch.Tensor, packed_groups: torch
     return dx
 
 
-def _rejected_linear(x, payload, quant_type, out_features, lora_a, lora_b, what):
-    """Raises the error that says why the native call did not take its operands."""
-    x2 = _flat_bf16(x, f"{what} input")
-    k = x2.shape[1]
-    _check_packed(payload.as_subclass(torch.Tensor), quant_type, out_features, k, what)
+class _Linear(torch.autograd.Function):
+    """The packed linear as a Python autograd function, with or without the LoRA term: what tracing records and forward mode
+    refuses (the native call returns None for both)."""
+
+    @staticmethod
+    def forward(ctx, x, payload, quant_type, out_features, lora_a, lora_b, scaling):
+        x2 = x.reshape(-1, x.shape[-1])
+        m, k = x2.shape
+        r = 0 if lora_a is None else lora_a.shape[0]
+        y = torch.empty(m, out_features, dtype=torch.bfloat16, device=x.device)
+        xa = torch.empty(m, (r + 15) // 16 * 16, dtype=torch.bfloat16, device=x.device)
+        if m:
+            ws = torch.empty(_lib.load().ggq_lora_workspace_bytes(m, 0, 1, out_features, k, r), dtype=torch.uint8, device=x.device)
+            _lib.check(_lib.load().ggq_lora_mmq_forward(
+                x2.data_ptr(), payload.data_ptr(), quant_type, m, out_features, k, _lib.ptr(lora_a), _lib.ptr(lora_b), r, scaling,
+                xa.data_ptr() if r else None, y.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_handle(x.device)))
+        ctx.save_for_backward(x2, xa, payload, lora_a, lora_b)
+        ctx.meta = (quant_type, out_features, scaling, x.shape)
+        return y.reshape(*x.shape[:-1], out_features)
+
+    @staticmethod
+    def backward(ctx, grad_output):
+        if torch.is_grad_enabled():
+            raise RuntimeError("packed MMQ linear does not support higher-order gradients")
+        x2, xa, payload, lora_a, lora_b = ctx.saved_tensors
+        quant_type, n, scaling, x_shape = ctx.meta
+        g2 = _flat_bf16(grad_output.contiguous(), "LoRA linear cotangent")
+        if lora_a is None:
+            return (mmq_grad_input(g2, payload, quant_type, x2.shape[1]).reshape(x_shape) if ctx.needs_input_grad[0] else None), *([None] * 6)
+        m, k = x2.shape
+        r = lora_a.shape[0]
+        dx = torch.empty_like(x2)
+        da = torch.empty_like(lora_a) if ctx.needs_input_grad[4] else None
+        db = torch.empty_like(lora_b) if ctx.needs_input_grad[5] else None
+        ws = torch.empty(_lib.load().ggq_lora_workspace_bytes(m, 0, 1, n, k, r), dtype=torch.uint8, device=x2.device)
+        _lib.check(_lib.load().ggq_lora_mmq_backward(
+            g2.data_ptr(), payload.data_ptr(), quant_type, m, n, k, x2.data_ptr(), xa.data_ptr(), lora_a.data_ptr(), lora_b.data_ptr(), r, scaling,
+            dx.data_ptr(), _lib.ptr(da), _lib.ptr(db), ws.data_ptr(), ws.numel(), _lib.stream_handle(x2.device)))
+        return (dx.reshape(x_shape) if ctx.needs_input_grad[0] else None), None, None, None, da, db, None
+
+
+def _general_linear(x, payload, quant_type, out_features, lora_a, lora_b, scaling, what):
+    """For operands the native call did not take: raises the error that says why, or runs the Python autograd function."""
+    payload = payload.as_subclass(torch.Tensor)
+    k = _flat_bf16(x, f"{what} input").shape[1]
+    _check_packed(payload, quant_type, out_features, k, what)
     if lora_a is not None:
         _lib.require_device_tensor(lora_a, "lora_A", torch.bfloat16)
         _lib.require_device_tensor(lora_b, "lora_B", torch.bfloat16)
-        raise ValueError(f"LoRA factors must be A [r,{k}] and B [{out_features},r], got {tuple(lora_a.shape)} and {tuple(lora_b.shape)}")
-    raise ValueError(f"{what}: operands do not describe a packed linear on one device")
+        if tuple(lora_a.shape) != (lora_a.shape[0], k) or tuple(lora_b.shape) != (out_features, lora_a.shape[0]):
+            raise ValueError(f"LoRA factors must be A [r,{k}] and B [{out_features},r], got {tuple(lora_a.shape)} and {tuple(lora_b.shape)}")
+    if any(t is not None and t.device != x.device for t in (payload, lora_a, lora_b)):
+        raise ValueError(f"{what}: operands do not describe a packed linear on one device")
+    return _Linear.apply(x, payload, quant_type, out_features, lora_a, lora_b, scaling)
 
 
 def lora_mmq(x, payload, quant_type, out_features, lora_a, lora_b, scaling) -> torch.Tensor:
     """Base matmul + LoRA residual in one forward call; dX, dA, dB in one backward call."""
     y = _lib.host().linear(x, payload, int(quant_type), int(out_features), lora_a, lora_b, float(scaling))
-    return y if y is not None else _rejected_linear(x, payload, int(quant_type), int(out_features), lora_a, lora_b, "LoRA linear")
+    return y if y is not None else _general_linear(x, payload, int(quant_type), int(out_features), lora_a, lora_b, float(scaling), "LoRA linear")
 
 
 def _fused_lora_add(result, x, lora_A: torch.nn.Linear, lora_B: torch.nn.Linear, dropout: torch.nn.Module, scaling: float):
