@@ -154,6 +154,15 @@ def test_saved_tensor_hooks_reach_the_native_nodes(pkg, dev):
         assert torch.equal(got, want)
 
 
+def test_module_hooks_of_the_expert_base_layer_run(pkg, dev):
+    layer, _, gen = _expert_layer(pkg, dev, gb.Q4_K, gb.Q4_K, 4, 256, 256, 8)
+    seen = []
+    layer.base_layer.register_forward_hook(lambda module, args, out: seen.append(tuple(out.shape)))
+    with torch.no_grad():
+        layer(bf16_randn(gen, 3, 256).to(dev), torch.tensor([[0, 1], [2, 3], [1, 0]], device=dev), torch.full((3, 2), 0.5, device=dev))
+    assert seen == [(3, 256)]
+
+
 def test_a_traced_linear_computes_on_its_inputs(pkg, dev):
     p, x, a, b, _ = _small_linear(pkg, dev)
 

@@ -777,15 +777,6 @@ class FastGGUFMoeLora(torch.nn.Module):
         return _ExpertLoraWeights(self.lora_A[n].weight, self.lora_B[n].weight, self.lora_A_down[n].weight, self.lora_B_down[n].weight, float(self.scaling[n]))
 
     def forward(self, hidden_states: torch.Tensor, top_k_index: torch.Tensor, top_k_weights: torch.Tensor) -> torch.Tensor:
-        modules = self._modules  # (what the attribute lookups of Module find, without their cost)
-        experts = modules["base_layer"]
-        if not self.disable_adapters and ALL_GGUF_EXPERTS_FUNCTIONS.get(experts.experts_implementation) is qwen3_5_moe_gguf_mmq_lora_forward \
-                and isinstance(experts, GGUFExperts):
-            name = self.active_adapter
-            out = _one_node(experts, hidden_states, top_k_index, top_k_weights, modules["lora_A"][name].weight, modules["lora_B"][name].weight,
-                            modules["lora_A_down"][name].weight, modules["lora_B_down"][name].weight, float(self.scaling[name]))
-            if out is not None:
-                return out
         return self.base_layer(hidden_states, top_k_index, top_k_weights, self._active_lora_weights())
 
     def merge(self, *args: Any, **kwargs: Any) -> None:
