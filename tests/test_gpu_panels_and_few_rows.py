@@ -100,8 +100,8 @@ def _expert_layer(pkg, dev, qt, qt_down, experts, hidden, inter, r, limit=None, 
 
 
 @pytest.mark.parametrize("tokens,top_k,hidden,inter,r,limit,ids", [
-    (1, 8, 2048, 512, 16, None, torch.int64), (8, 8, 256, 256, 5, 0.25, torch.int32),   # 64 routes: the most
-    (4, 16, 512, 768, 64, None, torch.int64), (3, 1, 4096, 256, 24, None, torch.int32),
+    (1, 8, 2048, 512, 16, None, torch.int64), (8, 8, 256, 256, 5, 0.25, torch.int32),   # 64 routes: past every limit of the path without a plan
+    (4, 16, 512, 768, 64, None, torch.int64), (2, 16, 256, 512, 40, None, torch.int64), (3, 1, 4096, 256, 24, None, torch.int32),
 ])
 @pytest.mark.parametrize("qt", ALL_TYPES, ids=[TYPE_NAMES[q] for q in ALL_TYPES])
 def test_experts_of_a_few_routes(pkg, dev, qt, tokens, top_k, hidden, inter, r, limit, ids):
@@ -183,3 +183,26 @@ def test_forward_mode_is_refused(pkg, dev):
         dual = fwad.make_dual(x, torch.ones_like(x))
         with pytest.raises((RuntimeError, NotImplementedError)):
             pkg.fast_lora.lora_mmq(dual, p, gb.Q4_K, 96, a, b, 2.0)
+
+
+# ------------------------------------------------------------------------------------------------
+# Expert-sorted rows while an expert has a few: row tiles of sixteen, one to eight waves per contraction.
+@pytest.mark.parametrize("n,k,r", [(40, 256, 5), (64, 512, 16), (264, 768, 40), (48, 2048, 16), (24, 4096, 64)])
+@pytest.mark.parametrize("qt", ALL_TYPES, ids=[TYPE_NAMES[q] for q in ALL_TYPES])
+def test_grouped_forward_of_a_few_rows_per_expert(pkg, dev, qt, n, k, r):
+    sizes = [1, 0, 16, 17, 0, 40, 3, 0, 15, 2, 33, 0] if qt != gb.Q4_K else [1, 0, 0, 17, 0, 0, 3, 0] + [0] * 40
+    experts, offsets = torch.arange(len(sizes)), torch.tensor(np.cumsum(sizes), dtype=torch.int32)
+    rows, s = sum(sizes), 2.0
+    gen = torch.Generator().manual_seed(n + k)
+    planes = [np.stack([make_payload(seed + e % 12, qt, n, k, "random") for e in range(len(sizes))]) for seed in (300, 400)]
+    x, a = bf16_randn(gen, rows, k), bf16_randn(gen, len(sizes), r, k, std=k ** -0.5)
+    b = bf16_randn(gen, len(sizes), 2 * n, r, std=0.02)
+    args = experts.to(dev), offsets.to(dev), qt, n
+    with torch.no_grad():
+        gate, up = pkg.fast_moe_lora.grouped_lora_mmq_pair(x.to(dev), *(torch.from_numpy(p).to(dev) for p in planes), *args, a.to(dev), b.to(dev), s)
+        single = pkg.fast_moe_lora.grouped_mmq(x.to(dev), torch.from_numpy(planes[1]).to(dev), *args)
+    w = [ref.weights_bf16(p, qt) for p in planes]
+    want = ref.grouped_lora_linear(x, torch.cat(w, dim=1), experts, offsets, a, b, s)["y"]
+    assert_close_bf16(gate, want[:, :n], "gate")
+    assert_close_bf16(up, want[:, n:], "up")
+    assert_close_bf16(single, ref.grouped_lora_linear(x, w[1], experts, offsets)["y"], "single")

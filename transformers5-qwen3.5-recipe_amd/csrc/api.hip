@@ -203,7 +203,8 @@ int64_t ggq_lora_workspace_bytes(int64_t rows, int64_t groups, int64_t experts, 
     const int rp = rank_pad(r > 0 ? r : 1);
     if (experts < 1) experts = 1;
     const int64_t tiles = rows / 64 + groups + 2;
-    return 5 * align256(tiles * (int64_t)sizeof(TileDesc)) + align256(16) + align256(experts * 2 * 4) +
+    // (rows / 16: tiles of the few-row forward)
+    return align256(groups > 0 ? (rows / 16 + groups) * (int64_t)sizeof(TileDesc) : 0) + 5 * align256(tiles * (int64_t)sizeof(TileDesc)) + align256(16) + align256(experts * 2 * 4) +
            align256(experts * n_total * rp * 2) * 2 + align256(experts * k * rp * 2) + align256(rows * rp * 2) + 4096 + panels +
            (groups == 0 ? align256(factor_partials_bytes(n_total, rp)) + align256(factor_partials_bytes(k, rp)) : 0);
 }
@@ -291,10 +292,10 @@ int ggq_fixed_grouped_mmq_grad_input_ws(const void* dy, const void* packed_group
 // main table in group order and sorted by size, the 64-row table of the LoRA side kernels, the two tile counts, the
 // per-expert row ranges.  Only the decoding-wave kernels' tile height is covered; a launch of another shape builds its own.
 struct GroupTablesView {
-    TileDesc *t_main, *t_sorted, *t64;
+    TileDesc *t_main, *t_sorted, *t64, *t_few;  // (t_few: while groups are small)
     int* counts;
     int* ranges;
-    int max_main, max64;
+    int max_main, max64, max_few;
 };
 static int64_t group_tables_layout(void* base, int64_t rows, int64_t groups, int64_t experts, GroupTablesView& v) {
     Bump b{(char*)base, INT64_MAX, 0};
@@ -302,6 +303,8 @@ static int64_t group_tables_layout(void* base, int64_t rows, int64_t groups, int
     v.t_main = (TileDesc*)b.take((int64_t)v.max_main * sizeof(TileDesc));
     v.t_sorted = (TileDesc*)b.take((int64_t)v.max_main * sizeof(TileDesc));
     v.t64 = (TileDesc*)b.take((int64_t)v.max64 * sizeof(TileDesc));
+    v.max_few = rows <= kFewRowsPerGroup * groups ? (int)(rows / kFewRowsTile + groups) : 0;
+    v.t_few = (TileDesc*)b.take((int64_t)v.max_few * sizeof(TileDesc));
     v.counts = (int*)b.take(16);
     v.ranges = (int*)b.take(experts * 2 * 4);
     return b.used;
@@ -325,6 +328,7 @@ int ggq_group_tables_build(const int64_t* expert_ids, const int32_t* end_offsets
     RowTileTables tb{};
     tb.add(kDirectBM, 0, 0x7FFFFFFF, v.t_main, v.counts, v.t_sorted);
     tb.add(64, 0, 0x7FFFFFFF, v.t64, v.counts + 1);
+    if (v.max_few) tb.add(kFewRowsTile, 0, 0x7FFFFFFF, v.t_few, v.counts + 2);
     return build_row_tile_tables(expert_ids, end_offsets, (int)groups, tb, v.ranges, (int)experts, as_stream(stream));
 }
 
@@ -388,6 +392,29 @@ static int grouped_forward(const char* what, const void* x, RowIndex x_index, co
         if (dense_side_takes(side)) return dense_mmq(q, panels, need, s, &side);
         if (int rc = skinny_nt(sp, rp, (int)((rows + 63) / 64), s)) return rc;
         return dense_mmq(q, panels, need, s);
+    }
+
+    if (groups > 0 && g_shape_override.load() < 0 && (!lora_a || aligned16(xa_out)) && grouped_few_rows_takes(qt, rows, groups, n, k, x)) {
+        GroupedFewRowsCall c{};
+        c.x = x, c.x_rows = x_index, c.rows = rows, c.groups = groups, c.n = n, c.k = k, c.w1 = packed1, c.w2 = packed2, c.y1 = y1, c.y2 = y2;
+        c.lora_a = lora_a, c.lora_b = lora_b, c.xa_out = xa_out, c.r = r, c.lora_scale = scale;
+        c.max_tiles = (int)(rows / kFewRowsTile + groups);
+        if (group_tables) {
+            GroupTablesView v;
+            group_tables_layout(const_cast<void*>(group_tables), rows, groups, experts, v);
+            c.tiles = v.t_few, c.num_tiles = v.counts + 2;
+            return grouped_few_rows(qt, c, s);
+        }
+        TileDesc* tiles = (TileDesc*)bump.take((int64_t)c.max_tiles * sizeof(TileDesc));
+        int* count = (int*)bump.take(16);
+        if (tiles && count) {
+            RowTileTables tb{};
+            tb.add(kFewRowsTile, 0, 0x7FFFFFFF, tiles, count);
+            if (int rc = build_row_tile_tables(expert_ids, end_offsets, (int)groups, tb, nullptr, 0, s)) return rc;
+            c.tiles = tiles, c.num_tiles = count;
+            return grouped_few_rows(qt, c, s);
+        }
+        bump = Bump{(char*)ws, ws_bytes, 0};  // (a workspace for 64-row tiles only)
     }
 
     const TileDesc* tiles64 = nullptr;

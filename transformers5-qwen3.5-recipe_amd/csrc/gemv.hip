@@ -31,15 +31,28 @@ __device__ __forceinline__ void stage_tables(uint8_t* lds, int tid, int threads)
 __device__ __forceinline__ bf16x8_t as_operand(const uint4& v) { return __builtin_bit_cast(bf16x8_t, v); }
 __device__ __forceinline__ f32x4_t mfma16(const bf16x8_t& a, const bf16x8_t& b, const f32x4_t& c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
-// A run of packed bytes global -> LDS, dealt to the workgroup's waves in 1 KB requests; both ends 16-byte aligned except for
-// the length, whose odd end (less than 16 bytes) a few lanes carry.  Returns the requests this wave made.
+// Where byte `off` of packed rows lies in LDS.  Q4_K rows of 2048 and 4096 elements are an odd and an even number of 128-byte
+// pieces, and the same byte of sixteen rows falls on an eighth of the banks and less: bank conflicts took half of the cycles
+// of a launch.  32 bytes left free behind every 1024 put eight rows on eight different eighths.  (Every piece of a Q4_K block that is
+// read at once is 16-byte aligned, so none straddles a gap; the other formats' rows spread over the banks as they are, or are read as words.)
+template <int QT>
+constexpr int kPieceGap = QT == kQ4_K ? 32 : 0;
+template <int QT>
+__host__ __device__ __forceinline__ int lds_at(int off) { return kPieceGap<QT> ? off + (off >> 10) * kPieceGap<QT> : off; }
+__host__ __device__ __forceinline__ int row_block_bytes(int qt, int bytes) {  // LDS bytes of `bytes` of packed rows
+    return (bytes + 1023) / 1024 * (1024 + (qt == kQ4_K ? kPieceGap<kQ4_K> : 0));
+}
+
+// A run of packed bytes global -> LDS, dealt to the workgroup's waves in 1 KB requests (kGap free bytes behind each); both ends
+// 16-byte aligned except for the length, whose odd end (less than 16 bytes) a few lanes carry.  Returns the requests this wave made.
+template <int kGap = 0>
 __device__ __forceinline__ int request_bytes(const uint8_t* src, uint8_t* dst, int bytes, int wave, int waves, int lane) {
     const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)dst;
     const int whole = bytes & ~15;
     int made = 0;
     for (int c = wave; c * 1024 < whole; c += waves, made++)
-        if (c * 1024 + lane * 16 < whole) load16_to_lds(lds + c * 1024, (uint32_t)lane * 16u, src + c * 1024);
-    if (wave == 0 && lane * 2 < bytes - whole) *(uint16_t*)(dst + whole + lane * 2) = *(const uint16_t*)(src + whole + lane * 2);
+        if (c * 1024 + lane * 16 < whole) load16_to_lds(__builtin_amdgcn_readfirstlane(lds + c * (1024 + kGap)), (uint32_t)lane * 16u, src + c * 1024);
+    if (wave == 0 && lane * 2 < bytes - whole) *(uint16_t*)(dst + whole + (whole >> 10) * kGap + lane * 2) = *(const uint16_t*)(src + whole + lane * 2);
     return made;
 }
 
@@ -106,16 +119,18 @@ __device__ __forceinline__ void four_values(uint32_t w, float scale24, float off
 template <int QT>
 __device__ __forceinline__ void decode_span(const uint8_t* lds, int row, int span, int runs, int q, uint32_t* v, const uint2* tables) {
     if constexpr (QT == kQ4_K) {
-        const uint8_t* blk = lds + row + (span >> 1) * 144;
-        const int h = span & 1;
-        const uint4 hdr = *(const uint4*)blk;
-        const uint2 g0 = *(const uint2*)(blk + 16 + 64 * h + 8 * q), g1 = *(const uint2*)(blk + 48 + 64 * h + 8 * q);
+        const int blk = row + (span >> 1) * 144, h = span & 1;
+        const uint4 hdr = *(const uint4*)(lds + lds_at<QT>(blk));
+        const int low = blk + 16 + 64 * h + 8 * q;
+        const uint2 g0 = *(const uint2*)(lds + lds_at<QT>(low)), g1 = *(const uint2*)(lds + lds_at<QT>(low + 32));
         const float d = half_bits_to_f32(hdr.x & 0xFFFFu) * kMixScale, dmin = half_bits_to_f32(hdr.x >> 16);
         // (scale, min) of the four runs, one per byte
         const uint32_t sc = h ? (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u) : hdr.y & 0x3F3F3F3Fu;
         const uint32_t mn = h ? ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u) : hdr.z & 0x3F3F3F3Fu;
         const uint32_t so = opaque(sc), mo = opaque(mn);
-        const float dl[4] = {d * ubyte0(so), d * ubyte1(so), d * ubyte2(so), d * ubyte3(so)};
+        // (the high nibbles of runs 1 and 3 stay in place and are read as sixteen times their value)
+        const float d16 = d * 0.0625f;
+        const float dl[4] = {d * ubyte0(so), d16 * ubyte1(so), d * ubyte2(so), d16 * ubyte3(so)};
         const float nm[4] = {-(dmin * ubyte0(mo)), -(dmin * ubyte1(mo)), -(dmin * ubyte2(mo)), -(dmin * ubyte3(mo))};
         const uint32_t w[4] = {g0.x, g0.y, g1.x, g1.y};
 #pragma unroll
@@ -123,7 +138,7 @@ __device__ __forceinline__ void decode_span(const uint8_t* lds, int row, int spa
 #pragma unroll
             for (int u = 0; u < 2; u++) {
                 const uint32_t b = w[2 * g + u];
-                const uint32_t lo02 = b & 0x000F000Fu, hi02 = (b >> 4) & 0x000F000Fu, lo13 = (b >> 8) & 0x000F000Fu, hi13 = (b >> 12) & 0x000F000Fu;
+                const uint32_t b8 = b >> 8, lo02 = b & 0x000F000Fu, hi02 = b & 0x00F000F0u, lo13 = b8 & 0x000F000Fu, hi13 = b8 & 0x00F000F0u;
                 uint32_t* even = v + 8 * g + 2 * u;
                 even[0] = pack_bf16(mix_lo(lo02, dl[2 * g], nm[2 * g]), mix_lo(lo13, dl[2 * g], nm[2 * g]));
                 even[1] = pack_bf16(mix_hi(lo02, dl[2 * g], nm[2 * g]), mix_hi(lo13, dl[2 * g], nm[2 * g]));
@@ -214,7 +229,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
     const int blocks = (p.n + 15) / 16, spans = (p.k + kSpan - 1) / kSpan;
     int block = blockIdx.x;
     auto request_block = [&](int b, int buf) __attribute__((always_inline)) {
-        return request_bytes(p.w + (int64_t)b * 16 * p.row_bytes, stage + buf * p.stage_bytes, min(16, p.n - b * 16) * p.row_bytes, wave, WAVES, lane);
+        return request_bytes<kPieceGap<QT>>(p.w + (int64_t)b * 16 * p.row_bytes, stage + buf * p.stage_bytes, min(16, p.n - b * 16) * p.row_bytes, wave, WAVES, lane);
     };
     // (the barriers here order LDS traffic only: __syncthreads would also wait for the block requested ahead)
     if (block < blocks) request_block(block, 0);
@@ -279,13 +294,13 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
         f32x4_t acc[TB];
 #pragma unroll
         for (int tb = 0; tb < TB; tb++) acc[tb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-        const int row = buf * p.stage_bytes + min(l16, p.n - block * 16 - 1) * p.row_bytes;
+        const int row = min(l16, p.n - block * 16 - 1) * p.row_bytes;
 #pragma unroll
         for (int sp = 0; sp < SP; sp++) {
             const int span = wave + WAVES * sp;
             if (span >= spans) break;  // uniform over the wave
             uint32_t v[16];
-            decode_span<QT>(stage, row, span, p.k >> 5, q, v, (const uint2*)gemv_lds);
+            decode_span<QT>(stage + buf * p.stage_bytes, row, span, p.k >> 5, q, v, (const uint2*)gemv_lds);
 #pragma unroll
             for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -360,7 +375,7 @@ int gemv(int qt, const void* x, int64_t ldx, const void* w, int64_t m, int64_t n
     p.x = (const bf16_t*)x, p.m = (int)m, p.n = (int)n, p.k = (int)k, p.w = (const uint8_t*)w, p.row_bytes = (int)packed_row_bytes(qt, k), p.y = (bf16_t*)y;
     p.ldx = ldx, p.ldy = ldy;
     if (lora_a) p.lora_a = (const bf16_t*)lora_a, p.lora_b = (const bf16_t*)lora_b, p.r = r, p.r_pad = (r + 15) / 16 * 16, p.lora_scale = scale, p.xa_out = (bf16_t*)xa_out;
-    p.stage_bytes = (16 * p.row_bytes + 1023) / 1024 * 1024;
+    p.stage_bytes = row_block_bytes(qt, 16 * p.row_bytes);
     p.buffers = (p.n + 15) / 16 > 256 && p.stage_bytes <= 36 * 1024 ? 2 : 1;  // (one block per workgroup needs one buffer)
     TimedScope timed(qt, kModeNT, kEpiStore, kShapeFewRows, s);
     switch (qt) {
@@ -376,7 +391,255 @@ int gemv(int qt, const void* x, int64_t ldx, const void* w, int64_t m, int64_t n
 }
 
 // ------------------------------------------------------------------------------------------------
-// Router logits of up to sixteen tokens: y [m, n] = x [m, k] . w [n, k]^T, all bf16.  A workgroup takes sixteen weight rows, its
+// Grouped: the forward of expert-sorted rows (a projection, or a gate / up pair) while an expert has a few rows.  Such a launch
+// ought to cost the packed bytes of the active experts; what bounds it is the decoding (about four vector instructions per
+// weight and lane).  The tile kernels and the decoding-wave kernels pad an expert's rows to 32 at least and stage activations
+// for 64 to 192.  Here a workgroup takes one row tile (up to sixteen rows of one expert, as operands in registers) and a part
+// of the expert's weight rows, sixteen at a time, requested up to three blocks ahead.  Its waves form TEAMS teams of KW: a team
+// deals the contraction of a sixteen-row block out to its waves (of a short contraction every wave takes a block of its own).
+// x A^T is formed in the same launch.
+// Router-less expert FFN with LoRA rank 16, 256 experts, top-8, before -> after:
+//   Q6_K / Q8_0, 2048 / 512:       64 tokens 409 -> 260 us, 256 tokens 441 -> 278 us (tile kernel)
+//   IQ2_XXS / Q2_K, 2048 / 2048:   64 tokens 565 -> 410 us, 192 tokens 651 -> 421 us (decoding-wave and tile kernel)
+//   IQ2_XXS, 4096 / 1024:         128 tokens 534 -> 411 us
+struct GroupedFewRowsParams {
+    const bf16_t* x;
+    int64_t ldx;
+    RowIndex x_rows;
+    const TileDesc* tiles;
+    const int* num_tiles;
+    int max_tiles, parts;
+    const uint8_t* w[2];            // planes [experts][n][row_bytes]
+    int64_t w_expert_bytes;
+    int row_bytes, n, k, nseg;
+    bf16_t* y[2];
+    int64_t ldy;
+    const bf16_t *lora_a, *lora_b;  // [experts][r][k], [experts][nseg * n][r]; null: none
+    bf16_t* xa_out;                 // [rows][r_pad]
+    int r, r_pad;
+    float lora_scale;
+    int lb_offset, stage_bytes, buffers;  // LDS bytes of sixteen packed rows, of those with their rows of B behind them; two to four buffers per team
+};
+
+template <int QT, int KW>
+__global__ __launch_bounds__(64 * (KW < 4 ? 4 : KW)) __attribute__((amdgpu_waves_per_eu(4))) void grouped_few_rows_kernel(GroupedFewRowsParams p) {
+    constexpr int WAVES = KW < 4 ? 4 : KW, TEAMS = WAVES / KW, SP = 4;
+    extern __shared__ __attribute__((aligned(16))) uint8_t gfr_lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, q = lane >> 4, kw = wave % KW, team = wave / KW;
+    // the parts of a row tile follow one another on one XCD: they share its activation and factor rows in that L2
+    const int slot = (int)(blockIdx.x >> 3), tile_id = (slot / p.parts) * 8 + (int)(blockIdx.x & 7), part = slot % p.parts;
+    if (tile_id >= min(*p.num_tiles, p.max_tiles)) return;
+    TileDesc tile = p.tiles[tile_id];
+    tile.row_begin = __builtin_amdgcn_readfirstlane(tile.row_begin), tile.row_end = __builtin_amdgcn_readfirstlane(tile.row_end);
+    tile.expert = __builtin_amdgcn_readfirstlane(tile.expert);
+    const int rows = min(tile.row_end - tile.row_begin, kFewRowsTile);
+    if (rows <= 0) return;
+    const int seg_blocks = (p.n + 15) / 16, blocks = p.nseg * seg_blocks;
+    const int b_begin = (int)((int64_t)blocks * part / p.parts), count = (int)((int64_t)blocks * (part + 1) / p.parts) - b_begin;
+    const int spans = (p.k + kSpan - 1) / kSpan;
+    uint8_t* stage = gfr_lds + kTableBytes<QT> + team * p.buffers * p.stage_bytes;
+    f32x4_t* red_all = (f32x4_t*)(gfr_lds + kTableBytes<QT> + TEAMS * p.buffers * p.stage_bytes);  // [WAVES][64]
+    f32x4_t* red = red_all + team * KW * 64;
+    bf16_t* xa = (bf16_t*)(red_all + WAVES * 64);                                                  // [16][64]
+    // A block's packed rows and its rows of the factor B, into one buffer.  (B comes with the untracked requests too: a load the
+    // compiler tracks is waited for with vmcnt(0) where it is used, and that wait would cover every block requested ahead.)
+    auto request_block = [&](int i, int buf) __attribute__((always_inline)) {
+        const int b = b_begin + i, seg = b >= seg_blocks, row0 = (b - seg * seg_blocks) * 16, block_rows = min(16, p.n - row0);
+        uint8_t* dst = stage + buf * p.stage_bytes;
+        int made = request_bytes<kPieceGap<QT>>((seg ? p.w[1] : p.w[0]) + (int64_t)tile.expert * p.w_expert_bytes + (int64_t)row0 * p.row_bytes, dst,
+                                                block_rows * p.row_bytes, kw, KW, lane);
+        if (p.lora_a)
+            made += request_bytes((const uint8_t*)(p.lora_b + ((int64_t)tile.expert * p.nseg * p.n + (int64_t)seg * p.n + row0) * p.r), dst + p.lb_offset,
+                                  block_rows * p.r * 2, (kw + 1) % KW, KW, lane);
+        return made;
+    };
+    // (the barriers here order LDS traffic only: __syncthreads would also wait for the blocks requested ahead)
+    int ahead[2] = {0, 0};  // this wave's requests for the two blocks after the current one
+    if (team < count) request_block(team, 0);
+#pragma unroll
+    for (int i = 1; i < 3; i++)
+        if (i < p.buffers - 1 && team + i * TEAMS < count) ahead[i - 1] = request_block(team + i * TEAMS, i);
+    stage_tables<QT>(gfr_lds, threadIdx.x, 64 * WAVES);
+
+    uint4 xf[SP][4];
+    {
+        const bf16_t* src = p.x + (int64_t)p.x_rows.source(tile.row_begin + min(l16, rows - 1)) * p.ldx;
+#pragma unroll
+        for (int sp = 0; sp < SP; sp++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int e = (kw + KW * sp) * kSpan + span_element<QT>(q, i);
+                xf[sp][i] = e < p.k ? *(const uint4*)(src + e) : make_uint4(0, 0, 0, 0);
+            }
+    }
+    if (p.lora_a) {  // x A^T: a team takes sixteen factor rows at a time; kept as bf16 rows in LDS
+        const bf16_t* a0 = p.lora_a + (int64_t)tile.expert * p.r * p.k;
+        for (int base = 0; base < p.r_pad; base += 16 * TEAMS) {
+            const int r0 = base + 16 * team;  // (past r_pad: zeros that nobody stores)
+            f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+            const bf16_t* arow = a0 + (int64_t)min(r0 + l16, p.r - 1) * p.k;
+#pragma unroll
+            for (int sp = 0; sp < SP; sp++) {
+                uint4 a[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int e = (kw + KW * sp) * kSpan + span_element<QT>(q, i);
+                    a[i] = e < p.k && r0 + l16 < p.r ? *(const uint4*)(arow + e) : make_uint4(0, 0, 0, 0);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc = mfma16(as_operand(a[i]), as_operand(xf[sp][i]), acc);
+            }
+            red[kw * 64 + lane] = acc;
+            lds_barrier();
+            if (kw == 0 && r0 < p.r_pad) {
+                f32x4_t sum = red[lane];
+#pragma unroll
+                for (int w = 1; w < KW; w++) sum += red[w * 64 + lane];
+                const uint2 v = make_uint2(pack_bf16(sum[0], sum[1]), pack_bf16(sum[2], sum[3]));  // factor rows r0 + 4 q .. + 3 of tile row l16
+                *(uint2*)(xa + l16 * 64 + r0 + 4 * q) = v;
+                if (part == 0 && l16 < rows) *(uint2*)(p.xa_out + (int64_t)(tile.row_begin + l16) * p.r_pad + r0 + 4 * q) = v;
+            }
+            lds_barrier();
+        }
+    }
+    const bool b_vec = (p.r & 7) == 0;
+    const bool whole = ((p.n | p.ldy) & 3) == 0 && (((uintptr_t)p.y[0] | (uintptr_t)p.y[1]) & 7) == 0;
+    int turn = 0, buf = 0;
+    for (int i0 = 0; i0 < count; i0 += TEAMS) {  // uniform over the workgroup; a team's last block may not exist
+        const int i = i0 + team, last = i + (p.buffers - 1) * TEAMS;
+        const bool live = i < count;
+        const int b = b_begin + i, seg = b >= seg_blocks, col0 = (b - seg * seg_blocks) * 16;
+        wait_loads_at_most(ahead[0] + ahead[1]);
+        lds_barrier();
+        {  // every wave is done with the block before: its buffer takes the last block that fits ahead
+            const int made = last < count ? request_block(last, buf == 0 ? p.buffers - 1 : buf - 1) : 0;
+            if (p.buffers == 4) ahead[0] = ahead[1], ahead[1] = made;
+            else if (p.buffers == 3) ahead[0] = made;
+        }
+        const uint8_t* block = stage + buf * p.stage_bytes;
+        f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        if (live) {
+            const int row = min(l16, p.n - col0 - 1) * p.row_bytes;
+#pragma unroll
+            for (int sp = 0; sp < SP; sp++) {
+                const int span = kw + KW * sp;
+                if (span >= spans) break;  // uniform over the wave
+                uint32_t v[16];
+                decode_span<QT>(block, row, span, p.k >> 5, q, v, (const uint2*)gfr_lds);
+#pragma unroll
+                for (int m = 0; m < 4; m++) acc = mfma16(as_operand(make_uint4(v[4 * m], v[4 * m + 1], v[4 * m + 2], v[4 * m + 3])), as_operand(xf[sp][m]), acc);
+            }
+        }
+        red[kw * 64 + lane] = acc;
+        lds_barrier();
+        // (a buffer is refilled, and the partial sums rewritten, only behind the next barrier)
+        if (live && kw == turn) {
+            f32x4_t sum = red[lane];
+#pragma unroll
+            for (int w = 1; w < KW; w++) sum += red[w * 64 + lane];
+            const int col = col0 + 4 * q;
+            if (p.lora_a) {
+                const bf16_t* brow = (const bf16_t*)(block + p.lb_offset) + min(l16, p.n - col0 - 1) * p.r;
+                f32x4_t lo = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+                for (int r0 = 0; r0 < p.r_pad; r0 += 32) {
+                    const int j = r0 + 8 * q;
+                    const uint4 xv = j < p.r_pad ? *(const uint4*)(xa + l16 * 64 + j) : make_uint4(0, 0, 0, 0);
+                    lo = mfma16(as_operand(load_factor8(brow + j, p.r - j, b_vec)), as_operand(xv), lo);
+                }
+                sum += lo * p.lora_scale;
+            }
+            if (l16 < rows) {
+                bf16_t* dst = (seg ? p.y[1] : p.y[0]) + (int64_t)(tile.row_begin + l16) * p.ldy + col;
+                if (whole) {
+                    if (col < p.n) *(uint2*)dst = make_uint2(pack_bf16(sum[0], sum[1]), pack_bf16(sum[2], sum[3]));
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                        if (col + v < p.n) dst[v] = to_bf16(sum[v]);
+                }
+            }
+        }
+        turn = turn + 1 == KW ? 0 : turn + 1;  // the wave that adds the partial sums changes from block to block
+        buf = buf + 1 == p.buffers ? 0 : buf + 1;
+    }
+}
+
+template <int QT, int KW>
+static int grouped_few_rows_lds(int stage_bytes, int buffers) {
+    constexpr int kWaves = KW < 4 ? 4 : KW;
+    return kTableBytes<QT> + kWaves / KW * buffers * stage_bytes + kWaves * 64 * 16 + 16 * 64 * 2;
+}
+static int few_rows_waves(int64_t k) { return k <= 512 ? 1 : k <= 1024 ? 2 : k <= 2048 ? 4 : 8; }  // waves that share a contraction
+static int64_t few_rows_stage(int qt, int64_t k) { return row_block_bytes(qt, (int)(16 * packed_row_bytes(qt, k))); }
+
+// Rows per expert, in the mean of a call, up to which these kernels are the faster ones.  Against the tile kernel (most
+// formats) and the IQ2_XXS decoding waves the line is where experts with more than one row tile become common, each tile
+// decoding the weights again: IQ2_XXS 4096 / 1024 at 8 rows 650 against 563 us, IQ2_XXS / Q2_K at 8 rows 554 against 654 us.
+// The Q4_K decoding waves, whose waves share no decoded weight either, are as fast from half a row on (120 us both at 16 tokens
+// of 2048 / 512, 212 against 203 us at 128).
+static bool few_rows_per_expert(int qt, int64_t rows, int64_t groups) {
+    if (qt == kQ4_K) return 2 * rows <= groups;
+    return rows <= (qt == kIQ2_XXS ? 6 : kFewRowsPerGroup) * groups;
+}
+bool grouped_few_rows_takes(int qt, int64_t rows, int64_t groups, int64_t n, int64_t k, const void* x) {
+    if (!few_rows_per_expert(qt, rows, groups) || k > 4096 || ((uintptr_t)x & 15) || n % 8) return false;  // (planes of B and of packed rows start at 16-byte addresses)
+    const int waves = few_rows_waves(k), teams = waves < 4 ? 4 / waves : 1;
+    return teams * 2 * (few_rows_stage(qt, k) + 2048) <= 140 * 1024;  // (two buffers, the partial sums, x A^T and tables: within 160 KB)
+}
+
+template <int QT, int KW>
+static int launch_grouped_few_rows(GroupedFewRowsParams p, hipStream_t s) {
+    constexpr int kThreadsWG = 64 * (KW < 4 ? 4 : KW);
+    static LdsLimit lim;
+    if (int rc = raise_lds_limit(lim, (const void*)grouped_few_rows_kernel<QT, KW>, 160 * 1024, "grouped_few_rows")) return rc;
+    // as many buffers as leave room for sixteen waves on a compute unit, or else for two workgroups
+    p.buffers = 4;
+    while (p.buffers > 2 && grouped_few_rows_lds<QT, KW>(p.stage_bytes, p.buffers) > 160 * 1024 / (1024 / kThreadsWG)) p.buffers--;
+    const int64_t grid = (int64_t)(p.max_tiles + 7) / 8 * 8 * p.parts;
+    if (grid > 0x7FFFFFF0) return set_error(GGQ_ERR_SHAPE, "grouped_few_rows: too many tiles for one launch");
+    const int lds = grouped_few_rows_lds<QT, KW>(p.stage_bytes, p.buffers);
+    hipLaunchKernelGGL((grouped_few_rows_kernel<QT, KW>), dim3((unsigned)grid), dim3(kThreadsWG), lds, s, p);
+    return check_launch("grouped_few_rows");
+}
+template <int QT>
+static int launch_grouped_few_rows_qt(const GroupedFewRowsParams& p, hipStream_t s) {
+    switch (few_rows_waves(p.k)) {
+        case 1: return launch_grouped_few_rows<QT, 1>(p, s);
+        case 2: return launch_grouped_few_rows<QT, 2>(p, s);
+        case 4: return launch_grouped_few_rows<QT, 4>(p, s);
+    }
+    return launch_grouped_few_rows<QT, 8>(p, s);
+}
+
+int grouped_few_rows(int qt, const GroupedFewRowsCall& c, hipStream_t s) {
+    GroupedFewRowsParams p{};
+    p.x = (const bf16_t*)c.x, p.ldx = c.k, p.x_rows = c.x_rows, p.tiles = c.tiles, p.num_tiles = c.num_tiles, p.max_tiles = c.max_tiles;
+    p.row_bytes = (int)packed_row_bytes(qt, c.k), p.n = (int)c.n, p.k = (int)c.k, p.nseg = c.w2 ? 2 : 1, p.w_expert_bytes = c.n * p.row_bytes;
+    p.w[0] = (const uint8_t*)c.w1, p.w[1] = (const uint8_t*)c.w2, p.y[0] = (bf16_t*)c.y1, p.y[1] = (bf16_t*)c.y2, p.ldy = c.n;
+    if (c.lora_a)
+        p.lora_a = (const bf16_t*)c.lora_a, p.lora_b = (const bf16_t*)c.lora_b, p.xa_out = (bf16_t*)c.xa_out, p.r = c.r, p.r_pad = (c.r + 15) / 16 * 16,
+        p.lora_scale = c.lora_scale;
+    p.lb_offset = (int)few_rows_stage(qt, c.k), p.stage_bytes = p.lb_offset + (p.lora_a ? 16 * p.r_pad * 2 : 0);
+    const int64_t kSlots = few_rows_waves(c.k) <= 4 ? 1024 : 512;
+    // a workgroup for every slot of the chip (sixteen waves per compute unit), while a part keeps four blocks per team
+    const int64_t tiles = std::min<int64_t>(c.max_tiles, std::min(c.groups, c.rows)), blocks = p.nseg * ((c.n + 15) / 16), waves = few_rows_waves(c.k), teams = waves < 4 ? 4 / waves : 1;
+    p.parts = (int)std::max<int64_t>(1, std::min((kSlots + tiles / 2) / std::max<int64_t>(1, tiles), blocks / (4 * teams)));
+    TimedScope timed(qt, kModeNT, kEpiStore, kShapeFewRows, s);
+    switch (qt) {
+        case kQ8_0: return launch_grouped_few_rows_qt<kQ8_0>(p, s);
+        case kQ2_K: return launch_grouped_few_rows_qt<kQ2_K>(p, s);
+        case kQ3_K: return launch_grouped_few_rows_qt<kQ3_K>(p, s);
+        case kQ4_K: return launch_grouped_few_rows_qt<kQ4_K>(p, s);
+        case kQ5_K: return launch_grouped_few_rows_qt<kQ5_K>(p, s);
+        case kQ6_K: return launch_grouped_few_rows_qt<kQ6_K>(p, s);
+        case kIQ2_XXS: return launch_grouped_few_rows_qt<kIQ2_XXS>(p, s);
+    }
+    return set_error(GGQ_ERR_QTYPE, "unsupported GGML type id %d", qt);
+}
+
+// ------------------------------------------------------------------------------------------------
+// Router logits of up to eight tokens: y [m, n] = x [m, k] . w [n, k]^T, all bf16.  A workgroup takes sixteen weight rows, its
 // eight waves deal the contraction out in spans of 128.  (A library product of this size costs 19 us of host time per call.)
 __global__ __launch_bounds__(512) void few_rows_bf16_kernel(const bf16_t* x, const bf16_t* w, int m, int n, int k, bf16_t* y) {
     constexpr int WAVES = 8;
@@ -459,22 +722,26 @@ __device__ __forceinline__ float lora_row_dot(const uint4& first, const bf16_t* 
     return s + __shfl_xor(s, 32, 64);
 }
 
+__host__ __device__ __forceinline__ int gate_up_half_lds(int qt, int row_bytes) {
+    const int bytes = 8 * row_bytes;
+    return qt == kQ4_K ? (bytes + (bytes >> 10) * kPieceGap<kQ4_K> + 127) & ~127 : bytes;
+}
 template <int QT, int SP>
 __global__ __launch_bounds__(512) void few_routes_gate_up_kernel(FewRoutesParams p) {
     constexpr int WAVES = 8;
     extern __shared__ __attribute__((aligned(16))) uint8_t gu_lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, q = lane >> 4;
-    const int half_bytes = 8 * p.row_bytes_in;
+    const int half_bytes = 8 * p.row_bytes_in, half_lds = gate_up_half_lds(QT, p.row_bytes_in);
     uint8_t* stage = gu_lds + kTableBytes<QT>;
-    float* red = (float*)(stage + 2 * half_bytes);   // [WAVES][16]
+    float* red = (float*)(stage + 2 * half_lds);   // [WAVES][16]
     float* red_xa = red + WAVES * 16;                // [WAVES][64]
     bf16_t* xa = (bf16_t*)(red_xa + WAVES * 64);     // [64]
     const int route = blockIdx.y, i0 = blockIdx.x * 8, k = p.hidden;
     const int expert = route_expert(p, route);
     const int64_t row0 = (int64_t)expert * p.inter + i0;
-    request_bytes(p.gate + row0 * p.row_bytes_in, stage, half_bytes, wave, WAVES, lane);
-    request_bytes(p.up + row0 * p.row_bytes_in, stage + half_bytes, half_bytes, (wave + 4) & 7, WAVES, lane);
+    request_bytes<kPieceGap<QT>>(p.gate + row0 * p.row_bytes_in, stage, half_bytes, wave, WAVES, lane);
+    request_bytes<kPieceGap<QT>>(p.up + row0 * p.row_bytes_in, stage + half_lds, half_bytes, (wave + 4) & 7, WAVES, lane);
     stage_tables<QT>(gu_lds, threadIdx.x, 512);
     const bf16_t* x = p.x + (int64_t)(route / p.top_k) * k;
     uint4 xf[SP][4];
@@ -510,14 +777,15 @@ __global__ __launch_bounds__(512) void few_routes_gate_up_kernel(FewRoutesParams
     wait_loads_at_most(0);
     __syncthreads();
     f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-    const int row = l16 * p.row_bytes_in;  // rows 0..7 gate, 8..15 up
+    const uint8_t* half = stage + (l16 < 8 ? 0 : half_lds);  // rows 0..7 gate, 8..15 up
+    const int row = (l16 & 7) * p.row_bytes_in;
     const int spans = (k + kSpan - 1) / kSpan;
 #pragma unroll
     for (int sp = 0; sp < SP; sp++) {
         const int span = wave + WAVES * sp;
         if (span >= spans) break;
         uint32_t v[16];
-        decode_span<QT>(stage, row, span, k >> 5, q, v, (const uint2*)gu_lds);
+        decode_span<QT>(half, row, span, k >> 5, q, v, (const uint2*)gu_lds);
 #pragma unroll
         for (int i = 0; i < 4; i++) acc = mfma16(as_operand(make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3])), as_operand(xf[sp][i]), acc);
     }
@@ -547,7 +815,7 @@ __global__ __launch_bounds__(512) void few_routes_down_kernel(FewRoutesParams p)
     extern __shared__ __attribute__((aligned(16))) uint8_t down_lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, q = lane >> 4;
-    const int stage_bytes = (16 * p.row_bytes_down + 1023) / 1024 * 1024;
+    const int stage_bytes = row_block_bytes(QT, 16 * p.row_bytes_down);
     uint8_t* mine = down_lds + kTableBytes<QT> + wave * stage_bytes;
     float* red = (float*)(down_lds + kTableBytes<QT> + 8 * stage_bytes);  // [16 routes][16]
     bf16_t* xa = (bf16_t*)(red + 256) + wave * 64;
@@ -558,7 +826,7 @@ __global__ __launch_bounds__(512) void few_routes_down_kernel(FewRoutesParams p)
     for (int rank = wave; rank < p.top_k; rank += 8) {
         const int route = token * p.top_k + rank, expert = route_expert(p, route);
         // this wave's own sixteen rows: no other wave touches them, so no barrier stands between their requests and their use
-        request_bytes(p.down + ((int64_t)expert * p.hidden + h0) * p.row_bytes_down, mine, rows * p.row_bytes_down, 0, 1, lane);
+        request_bytes<kPieceGap<QT>>(p.down + ((int64_t)expert * p.hidden + h0) * p.row_bytes_down, mine, rows * p.row_bytes_down, 0, 1, lane);
         const bf16_t* x = p.act + (int64_t)route * k;
         const bf16_t* a = p.a2 ? p.a2 + (int64_t)expert * p.r2 * k : nullptr;
         const bool b_vec = (p.r2 & 7) == 0;
@@ -628,8 +896,8 @@ __global__ __launch_bounds__(512) void few_routes_down_kernel(FewRoutesParams p)
     }
 }
 
-static int gate_up_lds(int qt, int row_bytes) { return (qt == kIQ2_XXS ? kTableBytes<kIQ2_XXS> : 0) + 16 * row_bytes + 8 * 16 * 4 + 8 * 64 * 4 + 128; }
-static int down_lds_bytes(int qt, int row_bytes) { return (qt == kIQ2_XXS ? kTableBytes<kIQ2_XXS> : 0) + 8 * ((16 * row_bytes + 1023) / 1024 * 1024) + 256 * 4 + 8 * 128; }
+static int gate_up_lds(int qt, int row_bytes) { return (qt == kIQ2_XXS ? kTableBytes<kIQ2_XXS> : 0) + 2 * gate_up_half_lds(qt, row_bytes) + 8 * 16 * 4 + 8 * 64 * 4 + 128; }
+static int down_lds_bytes(int qt, int row_bytes) { return (qt == kIQ2_XXS ? kTableBytes<kIQ2_XXS> : 0) + 8 * row_block_bytes(qt, 16 * row_bytes) + 256 * 4 + 8 * 128; }
 
 template <int QT>
 static int launch_gate_up(const FewRoutesParams& p, hipStream_t s) {
@@ -653,11 +921,14 @@ static int launch_down(const FewRoutesParams& p, hipStream_t s) {
     return check_launch("few_routes_down");
 }
 
-// Up to this many routes every route reads its own expert's weights.
-constexpr int64_t kFewRoutes = 64;
+// Up to this many routes every route reads its own expert's weights.  Beyond, the routing plan and the grouped kernels are
+// faster: 2048 / 512, 256 experts, 32 / 64 routes: Q4_K 54 / 97 against 54 / 70 us, Q6_K with Q8_0 58 / 111 against 62 / 92 us; the
+// decoder's tables, staged by every workgroup, set the line lower: IQ2_XXS 8 / 16 / 64 routes of 4096 / 1024: 52 / 95 / 351
+// against 54 / 69 / 135 us.
+static int64_t few_routes_limit(int qt_in, int qt_down) { return qt_in == kIQ2_XXS || qt_down == kIQ2_XXS ? 4 : 32; }
 
 bool few_routes_takes(int qt_in, int qt_down, int64_t tokens, int top_k, int64_t hidden, int64_t inter) {
-    return tokens > 0 && top_k > 0 && top_k <= 16 && tokens * top_k <= kFewRoutes && hidden <= 4096 && inter % 8 == 0 && hidden % 8 == 0 &&
+    return tokens > 0 && top_k > 0 && top_k <= 16 && tokens * top_k <= few_routes_limit(qt_in, qt_down) && hidden <= 4096 && inter % 8 == 0 && hidden % 8 == 0 &&
            gate_up_lds(qt_in, (int)packed_row_bytes(qt_in, hidden)) <= 80 * 1024 && down_lds_bytes(qt_down, (int)packed_row_bytes(qt_down, inter)) <= 160 * 1024;
 }
 

@@ -172,6 +172,25 @@ constexpr int kShapeFewRows = 7;  // (profile records only)
 bool gemv_takes(int qt, int64_t m, int64_t n, int64_t k, const void* x, int64_t ldx);
 int gemv(int qt, const void* x, int64_t ldx, const void* w, int64_t m, int64_t n, int64_t k, const void* lora_a, const void* lora_b, int r, float scale, void* xa_out,
          void* y, int64_t ldy, hipStream_t s);
+// Expert-sorted rows while an expert has few of them: row tiles of kFewRowsTile, never more than kFewRowsPerGroup rows per
+// expert in the mean.
+constexpr int kFewRowsTile = 16, kFewRowsPerGroup = 10;
+struct GroupedFewRowsCall {
+    const void* x;
+    RowIndex x_rows;
+    const TileDesc* tiles;  // of kFewRowsTile rows
+    const int* num_tiles;
+    int max_tiles;
+    int64_t rows, groups, n, k;
+    const void *w1, *w2;    // w2: gate / up pair
+    void *y1, *y2;
+    const void *lora_a, *lora_b;
+    void* xa_out;
+    int r;
+    float lora_scale;
+};
+bool grouped_few_rows_takes(int qt, int64_t rows, int64_t groups, int64_t n, int64_t k, const void* x);
+int grouped_few_rows(int qt, const GroupedFewRowsCall& c, hipStream_t s);
 constexpr int kRouterLogitsMaxTokens = 8;
 int router_logits(const void* x, const void* w, int64_t m, int64_t n, int64_t k, void* y, hipStream_t s);
 bool few_routes_takes(int qt_in, int qt_down, int64_t tokens, int top_k, int64_t hidden, int64_t inter);
