@@ -32,14 +32,17 @@ std::atomic<int> g_shape_override{-1};  // ggq_debug_force_grouped_shape (a test
 
 // ---------------------------------------------------------------------------------------------------
 // The factor gradients dA / dB of a backward call depend on nothing the grad-input launch writes, are HBM-bound and
-// small, while the grad-input launch is MFMA-bound and leaves compute units idle at its tail: they run on a second
-// stream of the library's own, forked from the caller's stream behind the rank-sized product they read and joined back
+// small, while the grad-input launch is MFMA-bound and leaves compute units idle at its tail: in a captured call they run on a
+// second stream of the library's own.  A call that is not captured keeps them in line unless asked: there the two events leave
+// gaps of 18 us a call, more than the overlap gives (training step of 256 Q4_K experts, 2048 / 512, top-8, forked against in line:
+// 997 tokens 515 against 493 us, 4096 tokens 910 against 893 us; IQ2_XXS 4096 / 2048, 2048 tokens: 3347 against 3319 us).  They are forked from the caller's stream behind the rank-sized product they read and joined back
 // into it before the call returns, so that to the caller the call is still one ordered piece of work on its stream.
 // Under stream capture the fork and the join become graph edges.  One side stream and event pair per device (default
 // priority); the lock is held while a call enqueues its forked section, so calls from several threads do not mix their
 // event records.  A stream that is being captured when the side stream does not exist yet runs the call unforked
 // (nothing is created during a capture).
-std::atomic<int> g_overlap_enabled{1};
+enum : int { kOverlapNever = 0, kOverlapAlways = 1, kOverlapCaptured = 2 };
+std::atomic<int> g_overlap_mode{kOverlapCaptured};
 constexpr int kMaxDevices = 64;
 struct SideStream {
     hipStream_t stream = nullptr;
@@ -52,7 +55,8 @@ std::mutex g_side_lock;
 class Forked {  // fork on construction (when allowed), join in done() or on destruction
 public:
     explicit Forked(hipStream_t main_stream) : main_(main_stream), lock_(g_side_lock, std::defer_lock) {
-        if (!g_overlap_enabled.load(std::memory_order_relaxed)) return;
+        const int mode = g_overlap_mode.load(std::memory_order_relaxed);
+        if (mode == kOverlapNever) return;
         int device = -1;
         if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices) return;
         lock_.lock();
@@ -72,6 +76,12 @@ public:
                 lock_.unlock();
                 return;
             }
+        }
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (mode == kOverlapCaptured && (hipStreamIsCapturing(main_, &capture) != hipSuccess || capture != hipStreamCaptureStatusActive)) {
+            (void)hipGetLastError();  // (the stream and events above are there for a capture to come)
+            lock_.unlock();
+            return;
         }
         if (hipEventRecord(st.fork, main_) != hipSuccess || hipStreamWaitEvent(st.stream, st.fork, 0) != hipSuccess) {
             (void)hipGetLastError();
@@ -133,8 +143,8 @@ int ggq_debug_force_grouped_shape(int shape) {
     return GGQ_OK;
 }
 
-int ggq_set_factor_gradient_overlap(int enabled) {
-    g_overlap_enabled.store(enabled ? 1 : 0, std::memory_order_relaxed);
+int ggq_set_factor_gradient_overlap(int mode) {
+    g_overlap_mode.store(mode == kOverlapCaptured ? kOverlapCaptured : mode ? kOverlapAlways : kOverlapNever, std::memory_order_relaxed);
     return GGQ_OK;
 }
 
