@@ -188,6 +188,10 @@ int64_t ggq_route_plan_workspace_bytes(int64_t tokens, int top_k, int num_expert
 int ggq_route_plan(const void* topk_ids, int ids_are_int64, int64_t tokens, int top_k, int num_experts, int64_t* sorted_ids,
                    int64_t* permutation, int64_t* inverse, int32_t* counts, int32_t* end_offsets, int64_t* active_ids,
                    int32_t* active_end_offsets, int32_t* status, void* ws, int64_t ws_bytes, void* stream);
+/* The plan together with the row-tile tables of its layout (ggq_group_tables_build with groups = experts, in the plan's order). */
+int ggq_route_plan_with_tables(const void* topk_ids, int ids_are_int64, int64_t tokens, int top_k, int num_experts, int64_t* sorted_ids,
+                               int64_t* permutation, int64_t* inverse, int32_t* counts, int32_t* end_offsets, int64_t* active_ids,
+                               int32_t* active_end_offsets, int32_t* status, void* tables, int64_t tables_bytes, void* ws, int64_t ws_bytes, void* stream);
 
 /* ggq_route_plan without a workspace and without any allocation.  No counterpart in the reference: it is for callers
  * that cannot allocate device memory around the call (code under HIP graph capture, tight serving loops, harnesses

@@ -206,3 +206,31 @@ def test_grouped_forward_of_a_few_rows_per_expert(pkg, dev, qt, n, k, r):
     assert_close_bf16(gate, want[:, :n], "gate")
     assert_close_bf16(up, want[:, n:], "up")
     assert_close_bf16(single, ref.grouped_lora_linear(x, w[1], experts, offsets)["y"], "single")
+
+
+@pytest.mark.parametrize("ids_type", [torch.int64, torch.int32])
+@pytest.mark.parametrize("tokens,top_k,experts", [(1, 1, 1), (1, 8, 256), (128, 8, 256), (515, 8, 250), (997, 3, 1024), (1536, 8, 256), (1537, 8, 60)])
+def test_plan_and_tables_in_one_launch(pkg, dev, tokens, top_k, experts, ids_type):
+    # one chunk, several, the most that one launch takes (12 of 1024 routes), and one more (separate launches)
+    lib, stream = pkg._lib.load(), torch.cuda.current_stream().cuda_stream
+    gen = torch.Generator().manual_seed(tokens)
+    ids = (torch.rand(tokens, top_k, generator=gen) ** 2 * experts).long().clamp_(max=experts - 1)  # (uneven groups)
+    d_ids, routes = ids.to(dev, ids_type), tokens * top_k
+    i64 = [torch.empty(n, dtype=torch.int64, device=dev) for n in (routes, routes, routes, experts)]
+    i32 = [torch.empty(n, dtype=torch.int32, device=dev) for n in (experts, experts, experts, 2)]
+    tables = [torch.zeros(lib.ggq_group_tables_bytes(routes, experts, experts), dtype=torch.uint8, device=dev) for _ in range(2)]
+    ws = torch.empty(lib.ggq_route_plan_workspace_bytes(tokens, top_k, experts), dtype=torch.uint8, device=dev)
+    sorted_ids, perm, inv, active = i64
+    counts, ends, active_ends, status = i32
+    pkg._lib.check(lib.ggq_route_plan_with_tables(d_ids.data_ptr(), ids_type == torch.int64, tokens, top_k, experts, sorted_ids.data_ptr(), perm.data_ptr(), inv.data_ptr(),
+                                                  counts.data_ptr(), ends.data_ptr(), active.data_ptr(), active_ends.data_ptr(), status.data_ptr(), tables[0].data_ptr(),
+                                                  tables[0].numel(), ws.data_ptr(), ws.numel(), stream))
+    pkg._lib.check(lib.ggq_group_tables_build(torch.arange(experts, device=dev).data_ptr(), ends.data_ptr(), experts, experts, routes, tables[1].data_ptr(), tables[1].numel(), stream))
+    for got, want in zip((sorted_ids, perm, inv), rref.plan(ids)):
+        assert torch.equal(got.cpu(), want)
+    want_counts = rref.expert_counts(ids, experts)
+    assert torch.equal(counts.cpu(), want_counts) and torch.equal(ends.cpu(), torch.cumsum(want_counts.long(), 0).int())
+    want_active, want_ends = rref.active_offsets(want_counts)
+    assert status.tolist() == [want_active.numel(), 0]
+    assert torch.equal(active[:want_active.numel()].cpu(), want_active) and torch.equal(active_ends[:want_active.numel()].cpu(), want_ends)
+    assert torch.equal(*tables)

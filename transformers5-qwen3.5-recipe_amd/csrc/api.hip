@@ -320,6 +320,15 @@ static int64_t group_tables_layout(void* base, int64_t rows, int64_t groups, int
     return b.used;
 }
 
+static RowTileTables group_tables(void* base, int64_t rows, int64_t groups, int64_t experts, GroupTablesView& v) {
+    group_tables_layout(base, rows, groups, experts, v);
+    RowTileTables tb{};
+    tb.add(kDirectBM, 0, 0x7FFFFFFF, v.t_main, v.counts, v.t_sorted);
+    tb.add(64, 0, 0x7FFFFFFF, v.t64, v.counts + 1);
+    if (v.max_few) tb.add(kFewRowsTile, 0, 0x7FFFFFFF, v.t_few, v.counts + 2);
+    return tb;
+}
+
 int64_t ggq_group_tables_bytes(int64_t rows, int64_t groups, int64_t experts) {
     if (rows < 0 || groups < 1 || experts < 1 || rows >= (1ll << 31)) return -1;
     GroupTablesView v;
@@ -334,11 +343,7 @@ int ggq_group_tables_build(const int64_t* expert_ids, const int32_t* end_offsets
     if (need < 0) return set_error(GGQ_ERR_SHAPE, "group_tables_build: bad sizes rows=%lld groups=%lld experts=%lld", (long long)rows, (long long)groups, (long long)experts);
     if (tables_bytes < need) return set_error(GGQ_ERR_WORKSPACE, "group_tables_build: buffer of %lld bytes, %lld needed", (long long)tables_bytes, (long long)need);
     GroupTablesView v;
-    group_tables_layout(tables, rows, groups, experts, v);
-    RowTileTables tb{};
-    tb.add(kDirectBM, 0, 0x7FFFFFFF, v.t_main, v.counts, v.t_sorted);
-    tb.add(64, 0, 0x7FFFFFFF, v.t64, v.counts + 1);
-    if (v.max_few) tb.add(kFewRowsTile, 0, 0x7FFFFFFF, v.t_few, v.counts + 2);
+    const RowTileTables tb = group_tables(tables, rows, groups, experts, v);
     return build_row_tile_tables(expert_ids, end_offsets, (int)groups, tb, v.ranges, (int)experts, as_stream(stream));
 }
 
@@ -765,6 +770,22 @@ int ggq_route_plan(const void* topk_ids, int ids_are_int64, int64_t tokens, int 
         return set_error(GGQ_ERR_NULL, "route_plan: null pointer");
     return route_plan(topk_ids, ids_are_int64, tokens, top_k, num_experts, sorted_ids, permutation, inverse, counts, end_offsets,
                       active_ids, active_end_offsets, status, ws, ws_bytes, as_stream(stream));
+}
+
+int ggq_route_plan_with_tables(const void* topk_ids, int ids_are_int64, int64_t tokens, int top_k, int num_experts, int64_t* sorted_ids,
+                               int64_t* permutation, int64_t* inverse, int32_t* counts, int32_t* end_offsets, int64_t* active_ids,
+                               int32_t* active_end_offsets, int32_t* status, void* tables, int64_t tables_bytes, void* ws, int64_t ws_bytes, void* stream) {
+    if (!topk_ids || !sorted_ids || !permutation || !inverse || !counts || !end_offsets || !active_ids || !active_end_offsets || !status || !tables || !ws)
+        return set_error(GGQ_ERR_NULL, "route_plan_with_tables: null pointer");
+    if (!aligned16(tables)) return set_error(GGQ_ERR_ALIGN, "route_plan_with_tables: the table buffer must be 16-byte aligned");
+    if (tokens < 0 || top_k <= 0 || num_experts <= 0) return set_error(GGQ_ERR_SHAPE, "route_plan_with_tables: bad shape");
+    const int64_t need = ggq_group_tables_bytes(tokens * top_k, num_experts, num_experts);
+    if (need < 0) return set_error(GGQ_ERR_SHAPE, "route_plan_with_tables: more than 2^31 routes");
+    if (tables_bytes < need) return set_error(GGQ_ERR_WORKSPACE, "route_plan_with_tables: table buffer of %lld bytes, %lld needed", (long long)tables_bytes, (long long)need);
+    GroupTablesView v;
+    const RowTileTables tb = group_tables(tables, tokens * top_k, num_experts, num_experts, v);
+    return route_plan(topk_ids, ids_are_int64, tokens, top_k, num_experts, sorted_ids, permutation, inverse, counts, end_offsets, active_ids, active_end_offsets,
+                      status, ws, ws_bytes, as_stream(stream), &tb, v.ranges);
 }
 
 int ggq_route_plan_static(const void* topk_ids, int ids_are_int64, int64_t tokens, int top_k, int num_experts, int64_t* sorted_ids,

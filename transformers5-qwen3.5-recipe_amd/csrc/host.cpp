@@ -192,10 +192,13 @@ Tensor experts_forward(const Tensor& x, const Tensor& ids, const Tensor& weights
     void* stream = stream_of(x);
     s.plan = empty_bytes(plan_view(nullptr, tokens, top_k, experts, tables).bytes, x);
     const PlanView v = plan_view(s.plan.data_ptr(), tokens, top_k, experts, tables);
-    check(ggq_route_plan(ids.data_ptr(), ids.scalar_type() == at::kLong, tokens, (int)top_k, (int)experts, v.sorted_ids, v.permutation, v.inverse, v.counts,
-                         v.ends, v.active_ids, v.active_ends, v.status, v.scratch, v.scratch_bytes, stream));
     const int64_t* groups = all_experts.const_data_ptr<int64_t>();
-    if (tables) check(ggq_group_tables_build(groups, v.ends, experts, experts, routes, v.tables, v.tables_bytes, stream));
+    if (tables)
+        check(ggq_route_plan_with_tables(ids.data_ptr(), ids.scalar_type() == at::kLong, tokens, (int)top_k, (int)experts, v.sorted_ids, v.permutation, v.inverse,
+                                         v.counts, v.ends, v.active_ids, v.active_ends, v.status, v.tables, v.tables_bytes, v.scratch, v.scratch_bytes, stream));
+    else
+        check(ggq_route_plan(ids.data_ptr(), ids.scalar_type() == at::kLong, tokens, (int)top_k, (int)experts, v.sorted_ids, v.permutation, v.inverse, v.counts,
+                             v.ends, v.active_ids, v.active_ends, v.status, v.scratch, v.scratch_bytes, stream));
     s.gate = empty({routes, inter}, at::kBFloat16, x), s.up = empty({routes, inter}, at::kBFloat16, x), s.act = empty({routes, inter}, at::kBFloat16, x);
     if (lora) s.xa_gate_up = empty({routes, rank_pad(r1)}, at::kBFloat16, x), s.xa_down = empty({routes, rank_pad(r2)}, at::kBFloat16, x);
     Tensor y = empty({routes, hidden}, at::kBFloat16, x);

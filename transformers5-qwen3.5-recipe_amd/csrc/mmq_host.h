@@ -232,7 +232,8 @@ int build_row_tiles(const int64_t* expert_ids, const int32_t* end_offsets, int g
 int64_t route_plan_workspace_bytes(int64_t routes, int num_experts);
 int route_plan(const void* topk_ids, int ids_are_int64, int64_t tokens, int top_k, int num_experts,
                int64_t* sorted_ids, int64_t* permutation, int64_t* inverse, int* counts, int* end_offsets,
-               int64_t* active_ids, int* active_end, int* num_active, void* ws, int64_t ws_bytes, hipStream_t s);
+               int64_t* active_ids, int* active_end, int* num_active, void* ws, int64_t ws_bytes, hipStream_t s,
+               const RowTileTables* tables = nullptr, int* expert_ranges = nullptr);  // (tables: of the layout, group = expert)
 int route_plan_static(const void* topk_ids, int ids_are_int64, int64_t tokens, int top_k, int num_experts,
                       int64_t* sorted_ids, int64_t* permutation, int64_t* inverse, int* counts, int* end_offsets,
                       int64_t* active_ids, int* active_end, int* num_active, hipStream_t s);  // no workspace: a built-in scratch array
