@@ -159,6 +159,10 @@ struct ExpertsBuffers {  // what the backward needs beside the inputs
     Tensor plan, gate, up, act, xa_gate_up, xa_down;
 };
 
+// Whether some launch of the layer reads row-tile tables built once: Q4_K launches, and the forwards of a few rows per expert (in
+// every format; without the plan's tables each of them builds its own, 5 us in front of a launch).
+bool shares_tables(int64_t qt_gate_up, int64_t qt_down, int64_t routes, int64_t experts) { return qt_gate_up == 12 || qt_down == 12 || routes <= 10 * experts; }
+
 // Pieces of the one buffer that holds the routing plan, the row-tile tables and the plan's scratch.
 struct PlanView {
     int64_t *sorted_ids, *permutation, *inverse, *active_ids;
@@ -188,7 +192,7 @@ Tensor experts_forward(const Tensor& x, const Tensor& ids, const Tensor& weights
     const int64_t experts = gate_w.size(0), inter = gate_w.size(1), hidden = down_w.size(1);
     const bool lora = a1.defined();
     const int64_t r1 = lora ? a1.size(1) : 0, r2 = lora ? a2.size(1) : 0;
-    const bool tables = o.qt_gate_up == 12 || o.qt_down == 12;  // the block format whose launches share row-tile tables
+    const bool tables = shares_tables(o.qt_gate_up, o.qt_down, routes, experts);
     void* stream = stream_of(x);
     s.plan = empty_bytes(plan_view(nullptr, tokens, top_k, experts, tables).bytes, x);
     const PlanView v = plan_view(s.plan.data_ptr(), tokens, top_k, experts, tables);
@@ -261,7 +265,7 @@ struct Experts : torch::autograd::Function<Experts> {
         const int r1 = lora ? (int)a1.size(1) : 0, r2 = lora ? (int)a2.size(1) : 0, w_bf16 = weights.scalar_type() == at::kBFloat16;
         const Tensor g = usable_cotangent(grads[0], "combined output cotangent");
         void* stream = stream_of(g);
-        const PlanView v = plan_view(plan.data_ptr(), tokens, top_k, experts, qt1 == 12 || qt2 == 12);
+        const PlanView v = plan_view(plan.data_ptr(), tokens, top_k, experts, shares_tables(qt1, qt2, routes, experts));
         const int64_t* groups = all_experts.const_data_ptr<int64_t>();
         variable_list out(15);
         if (ctx->needs_input_grad(2)) out[2] = empty(weights.sizes(), weights.scalar_type(), g);
