@@ -440,7 +440,7 @@ def main() -> None:
     ap.add_argument("--warmup", type=int, default=3)
     ap.add_argument("--settle-ms", type=float, default=300.0, help="moe_q4k: milliseconds of untimed step replays ahead of the warm-up steps (0: none)")
     ap.add_argument("--no-cpu-baseline", action="store_true")
-    ap.add_argument("--chunk", type=int, default=1024, help="lmhead_q6k: rows per chunk (1024 in the BASELINE configuration; from 4096 rows on the logits of a chunk are kept)")
+    ap.add_argument("--chunk", type=int, default=1024, help="lmhead_q6k: rows per chunk (1024 in the BASELINE configuration; the sweep takes up to 4096 rows whatever the chunk)")
     ap.add_argument("--graph", type=int, default=1, help="replay the step from a captured HIP graph (1) or run it eagerly (0)")
     ap.add_argument("--iq2-pool", type=int, default=256, help="moe_iq2xxs: number of distinct experts drawn and quantized (the others repeat them)")
     ap.add_argument("--overlap", type=int, default=1, help="factor gradients of the grouped backward calls on the library's side stream (1, what the library does in a captured step) or on the launch stream (0)")
