@@ -8,11 +8,10 @@
 // tile and issues no MFMA on empty blocks.  Per contraction step of 64
 //   * the A tile goes global -> LDS directly (no registers), three steps ahead, through a ring of four stages; rows are
 //     unpadded with XOR-swizzled 16-byte slots (a_slot), every wave reads all of them;
-//   * the packed quant bytes go global -> LDS directly as well, half a 256-wide block (two steps) of the wave's 32
-//     columns at a time, four lanes per row so that a row's bytes are requested by adjacent lanes, into a ring of three
-//     wave-private buffers; a block's 16-byte headers follow the same way, one lane per column, a block ahead;
-//   * a lane reads its 16 quant bytes of the step from its wave's buffer and decodes them in registers into the operands
-//     of the step's four MFMA sub-steps (mmq_direct.h).  No decoded weight ever touches LDS.
+//   * the packed blocks go global -> LDS directly as well, the whole 144-byte blocks (header and quant bytes, four steps)
+//     of the wave's 32 columns at a time, nine adjacent lanes per row, into two wave-private buffers;
+//   * a lane reads its 16 quant bytes of the step, and once per block its header, from its wave's buffer and decodes them
+//     in registers into the operands of the step's four MFMA sub-steps (mmq_direct.h).  No decoded weight ever touches LDS.
 // A single wave issues at most one instruction per four to five cycles, whatever its kind, so a step's decode
 // arithmetic, LDS reads, requests and waits (about eight instructions per MFMA) cannot hide behind that wave's own
 // MFMAs; with two waves per SIMD one wave's MFMAs run while the other decodes, reads and waits.
@@ -21,6 +20,11 @@
 // there.  A workgroup takes a run of column tiles of its row tile and treats their steps as one stream, so the requests
 // of a tile's first steps are in flight while the tile before it finishes.  The requests are inline-asm loads the
 // compiler does not track; the step waits for them with exact counts (vector memory operations complete in issue order).
+//
+// What bounds it: the clock the matrix cores leave (1.9 GHz at 128 rows and more), plus what does not overlap them: 256
+// experts, 2 x 512 columns, k 2048 take 88 us at 32 rows each and 22 us for every 32 rows more (302 MB of packed weights: 58
+// us at 5.2 TB/s).  Whole-block requests, staging of its own, and cursors that only add: 102 / 88 / 107 / 153 / 182 / 204 us
+// at 16 / 32 / 64 / 128 / 160 / 192 rows, before 109 / 95 / 114 / 160 / 187 / 209.
 #pragma once
 #include "mmq_direct.h"
 
@@ -28,27 +32,32 @@ namespace ggq {
 
 struct Direct8 {
     static constexpr int kTM = kDirectBM, kTN = kDirectBN;
-    static constexpr int kStages = 4;
     static constexpr int kWaves = 8;
     static constexpr int kThreadsWG = 64 * kWaves;
-    static constexpr int kMaxLoadsPerStage = (kTM / 32 + 1) / 2;            // one direct-to-LDS instruction of the workgroup moves 64 rows
-    static constexpr int kRingBytes = kStages * kMaxLoadsPerStage * 8192;  // 96 KB
-    // Packed weights: per wave a ring of three buffers of 32 rows x 64 bytes, the quant bytes of two steps (half a
-    // 256-wide block) of the wave's 32 columns.  A finished tile's output rows are staged in the buffer just read.
-    static constexpr int kWBufBytes = 32 * 64, kWBufs = 3;
-    static constexpr int kWBase = kRingBytes;
-    static constexpr int kLaBase = kWBase + kWaves * kWBufs * kWBufBytes;  // + 48 KB: then the row tile's LA rows (rank <= 16), 32 bytes each
-    static constexpr int kHdrBase = kLaBase + kTM * 32;                    // + 6 KB: then per wave the 16-byte headers of a block of its 32 columns
-    static constexpr int kLdsBytes = kHdrBase + kWaves * 512;              // + 4 KB = 154 KB
-
+    // Packed weights: per wave two buffers of 32 rows x 144 bytes, a block of each of the wave's 32 columns (a row pitch of
+    // 144 bytes spreads the lane-per-row reads over all banks); then per wave 2 KB in which a finished row block's output is
+    // staged; then the row tile's LA rows (rank <= 16), 32 bytes each; then the A ring.  Six row blocks leave no room for
+    // staging: they stage in the packed buffer just read, and request its next contents only behind the store path.
+    static constexpr int kWBufBytes = 32 * 144;
+    static constexpr int kOutBase = kWaves * 2 * kWBufBytes;               // 72 KB
+    static constexpr int kLdsBytes = 160 * 1024 - 4096;  // 156 KB
+    template <int LIVE>
+    struct Layout {
+        static constexpr int kStages = LIVE <= 4 ? 4 : 3;
+        static constexpr bool kOwnStaging = LIVE <= 5;
+        static constexpr int kLaBase = kOutBase + (kOwnStaging ? kWaves * 2048 : 0), kABase = kLaBase + LIVE * 1024;
+    };
+    static_assert(kOutBase + kWaves * 2048 + 4 * (1024 + 4 * 4096) <= kLdsBytes && kOutBase + kWaves * 2048 + 5 * (1024 + 3 * 4096) <= kLdsBytes && kOutBase + 6 * (1024 + 3 * 4096) <= kLdsBytes, "LDS");
     using Scales = Direct::Scales;
     using RowCtx = Direct::RowCtx;
 
     template <int LIVE>
     static __device__ __forceinline__ void work(const MmqParams& p, const RowCtx& c, int ct0, int ct1) {
         extern __shared__ __attribute__((aligned(16))) uint8_t smem_raw[];
-        constexpr int NI = (LIVE + 1) / 2;       // direct-to-LDS instructions per A stage and wave
-        constexpr int kStageBytes = NI * 8192;   // (an odd block count leaves the last 32 rows of a stage as copies of the last row)
+        using L = Layout<LIVE>;
+        constexpr int kStages = L::kStages, kLaBase = L::kLaBase, kABase = L::kABase;
+        constexpr int NI = (LIVE + 1) / 2;       // direct-to-LDS instructions per A stage and wave (the last of an odd block count: half its lanes)
+        constexpr int kStageBytes = LIVE * 4096;
         constexpr int kStores = 2 * LIVE - 1;    // 16-byte store instructions a tile certainly issues per wave (two per full row block, one for the last)
         const int tid = threadIdx.x, lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -56,16 +65,17 @@ struct Direct8 {
         const int steps = p.steps_per_seg, blocks = steps >> 2;
         const int out_cols = p.n;
         const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem_raw;
-        // A tile loads: instruction i fills slots 512 i + tid: tile row 64 i + tid / 8, slot tid % 8.  Rows past the
-        // group's end repeat its last row (their results are never stored).  With a row index the lane offsets carry
-        // the whole stored row (the host keeps the matrix under 4 GiB).
-        const bf16_t* a_base = p.a[0] + (p.a_rows.on() ? 0 : (int64_t)c.row_begin * p.lda);
+        // A tile loads: instruction i fills slots 512 i + tid: tile row 64 i + tid / 8, slot tid % 8; the last instruction of
+        // an odd block count has half the rows, 32 lanes of every wave.  Rows past the group's end repeat its first rows
+        // (their results are never stored; one row repeated by all of them cost 2 % of a launch of 16-row groups).  With a
+        // row index the lane offsets carry the whole stored row (the host keeps the matrix under 4 GiB).
+        const bf16_t* a_src = p.a[0] + (p.a_rows.on() ? 0 : (int64_t)c.row_begin * p.lda);
         uint32_t a_voff[NI];
 #pragma unroll
         for (int i = 0; i < NI; i++) {
-            const int r = 64 * i + (tid >> 3), s = tid & 7;
+            const int r = 64 * i + (2 * i + 1 < LIVE ? tid >> 3 : 4 * wave + (lane_c >> 3)), s = tid & 7;
             const int kc = s ^ ((r >> 1) & 7);
-            const int rr = min(r, c.rows_valid - 1);
+            const int rr = r < c.rows_valid ? r : min(r - c.rows_valid, c.rows_valid - 1);
             const int src = p.a_rows.on() ? p.a_rows.source(c.row_begin + rr) : rr;
             a_voff[i] = (uint32_t)(((int64_t)src * p.lda + kc * 8) * 2);
         }
@@ -73,83 +83,82 @@ struct Direct8 {
             seg = ct / p.col_tiles_per_seg;
             col0 = (ct - seg * p.col_tiles_per_seg) * kTN;
         };
-        // The A cursor: (column tile, step) of the next step to request; it only moves the contraction offset.
-        int i_step = 0;
+        // The A cursor: the next step to request; it only moves the contraction offset, the same way for every column tile.
+        const bf16_t* a_next = a_src;
+        int a_left = steps;
         int a_wr = 0;  // byte offset of the stage the next request fills
-        auto issue_a = [&]() __attribute__((always_inline)) {
-            const uint32_t dst = lds_base + a_wr + wave * 1024;
-            const bf16_t* a_step = a_base + i_step * 64;
-#pragma unroll
-            for (int i = 0; i < NI; i++) load16_to_lds(dst + i * 8192, a_voff[i], a_step);
+        uint32_t ph_dst;  // the open phase's A stage and source
+        const bf16_t* ph_src;
+        auto phase_open = [&]() __attribute__((always_inline)) {
+            ph_dst = lds_base + kABase + a_wr;
+            ph_src = a_next;
             a_wr = a_wr == (kStages - 1) * kStageBytes ? 0 : a_wr + kStageBytes;
-            if (++i_step == steps) i_step = 0;
+            a_next += 64;
+            if (--a_left == 0) a_left = steps, a_next = a_src;
         };
-        // The W cursor: (column tile, 256-wide block) of the next block to request.  Packed quant bytes go global ->
-        // LDS directly, half a block (two steps) of the wave's 32 columns per buffer: instruction j moves 64 bytes of
-        // each of the rows 16 j .. 16 j + 15, four lanes per row, so that a row's bytes are requested by adjacent lanes
-        // (a lane-per-row load of 16 bytes costs the vector cache one access per lane).  The 16-byte chunks of a row
-        // are XOR-swizzled with (row / 2) % 4: the reads below (lane = row, 16 bytes) meet no bank conflict.
+        auto request_a = [&](auto i_c) __attribute__((always_inline)) {
+            constexpr int I = decltype(i_c)::value;
+            if constexpr (2 * I + 1 < LIVE) load16_to_lds(ph_dst + I * 8192 + wave * 1024, a_voff[I], ph_src);
+            else if constexpr (2 * I < LIVE) {
+                if (lane_h == 0) load16_to_lds(ph_dst + I * 8192 + wave * 512, a_voff[I], ph_src);
+            }
+        };
+        // The W cursor: (column tile, 256-wide block) of the next block to request.  Whole blocks go global -> LDS directly:
+        // the 288 16-byte chunks of the wave's 32 blocks in row order, chunk 64 j + lane by instruction j (the fifth moves
+        // 32).  What a request costs is the cache lines it touches: a step's blocks as separate headers and quant halves,
+        // 16 rows x 64 bytes each, kept the vector cache busy for 204 ns (L2 hits), as whole blocks for 88.
         int w_tile_i = ct0, w_blk = 0;
-        const uint8_t* w_next;  // packed row of the cursor tile's first column, at the cursor's block (scalar)
-        uint32_t wq_voff[2];    // this lane's byte offset from there in instruction j
-        uint32_t wh_voff;       // and for the block header of its column (both lane halves read the same 16 bytes)
+        const uint8_t* w_next;  // packed row of the cursor tile's first column (scalar)
+        uint32_t w_voff[5];     // this lane's byte offset from the cursor's block there in instruction j
         auto w_cursor_rows = [&]() __attribute__((always_inline)) {
             int seg, col0;
             tile_origin(w_tile_i, seg, col0);
             w_next = (seg ? p.w[1] : p.w[0]) + c.expert * p.w_expert_bytes + (int64_t)col0 * p.w_row_bytes;
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const int row = 16 * j + (lane >> 2), kc = (lane & 3) ^ ((row >> 1) & 3);
-                wq_voff[j] = (uint32_t)min(32 * wave + row, out_cols - 1 - col0) * (uint32_t)p.w_row_bytes + 16u * kc;
+            for (int j = 0; j < 5; j++) {
+                const int chunk = j < 4 ? 64 * j + lane : 256 + lane_c, row = chunk / 9;
+                w_voff[j] = (uint32_t)min(32 * wave + row, out_cols - 1 - col0) * (uint32_t)p.w_row_bytes + 16u * (chunk - 9 * row);
             }
-            wh_voff = (uint32_t)min(32 * wave + lane_c, out_cols - 1 - col0) * (uint32_t)p.w_row_bytes;
         };
         w_cursor_rows();
-        int w_wr = 0;  // byte offset (inside the wave's ring) of the buffer the next request fills
-        const uint32_t w_lds = lds_base + kWBase + wave * (kWBufs * kWBufBytes);
-        auto issue_w_half = [&](auto half_c) __attribute__((always_inline)) {  // quant bytes 64 half .. +63 of the cursor's block
-            constexpr int HALF = decltype(half_c)::value;
-            // (no immediate offset: a direct-to-LDS load adds it to the LDS address as well)
-            const uint8_t* src = w_next + w_blk * 144 + 16 + 64 * HALF;
-#pragma unroll
-            for (int j = 0; j < 2; j++) load16_to_lds(w_lds + w_wr + j * 1024, wq_voff[j], src);
-            w_wr = w_wr == (kWBufs - 1) * kWBufBytes ? 0 : w_wr + kWBufBytes;
-        };
-        // The headers of the cursor's block go global -> LDS as well, one lane per column (a load of 64 lanes that names
-        // each of 32 addresses twice costs the vector cache twice the accesses), into the wave's one header buffer: a
-        // block's headers are read out of it (below) a whole step before the request of the next block's goes out.
-        const uint32_t hdr_lds = lds_base + kHdrBase + wave * 512;
-        const uint8_t* const hdr_row = smem_raw + kHdrBase + wave * 512 + lane_c * 16;
-        auto issue_w_header = [&]() __attribute__((always_inline)) {
-            if (lane_h == 0) load16_to_lds(hdr_lds, wh_voff, w_next + w_blk * 144);
+        int w_wr = 0;  // byte offset (inside the wave's pair) of the buffer the open block's requests fill
+        const uint32_t w_lds = lds_base + wave * (2 * kWBufBytes);
+        auto request_w = [&](auto j_c) __attribute__((always_inline)) {
+            constexpr int J = decltype(j_c)::value;
+            if constexpr (J < 4) load16_to_lds(w_lds + w_wr + J * 1024, w_voff[J], w_next + w_blk * 144);
+            else if (lane_h == 0) load16_to_lds(w_lds + w_wr + J * 1024, w_voff[J], w_next + w_blk * 144);
         };
         auto w_cursor_advance = [&]() __attribute__((always_inline)) {  // past the last block of the last tile the cursor stays
+            w_wr ^= kWBufBytes;
             if (w_blk + 1 < blocks) w_blk++;
             else if (w_tile_i + 1 < ct1) w_tile_i++, w_blk = 0, w_cursor_rows();
         };
 
         f32x16_t acc[LIVE];
         // LDS read addresses: block rb is tile rows 32 rb + lane_c; sub-step I reads chunk 4 (I / 2) + 2 h + (I % 2)
-        const uint8_t* a_row = smem_raw + lane_c * kARowBytes;
+        const uint8_t* a_row = smem_raw + kABase + lane_c * kARowBytes;
         int a_koff[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) a_koff[i] = a_slot(lane_c, 4 * (i >> 1) + 2 * lane_h + (i & 1)) * 16;
         bf16x8_t ao[LIVE];
-        // this lane's 16 quant bytes of the first / second step of a buffer
-        const uint8_t* const w_rows = smem_raw + kWBase + wave * (kWBufs * kWBufBytes) + lane_c * 64;
-        const int w_roff[2] = {((lane_h) ^ ((lane_c >> 1) & 3)) * 16, ((2 + lane_h) ^ ((lane_c >> 1) & 3)) * 16};
-        int w_rd = 0;  // byte offset of the buffer of the current pair of steps
+        const uint8_t* const w_row = smem_raw + wave * (2 * kWBufBytes) + lane_c * 144;  // this lane's block (+ 16 + 32 S + 16 h: its quant bytes of step S)
+        const int w_q = 16 + 16 * lane_h;
+        int w_rd = 0;  // byte offset of the buffer of the current block
         int a_rd = 0;  // byte offset of the A stage of the current step
 
         u32x4_t qc, qn;  // quant bytes of the current / next step
         u32x4_t hc, hn;  // headers of the current / next block
-        issue_w_header();
-        issue_w_half(std::integral_constant<int, 0>{});
-        issue_w_half(std::integral_constant<int, 1>{});
-        w_cursor_advance();
-        issue_a();
-        issue_a();
-        issue_a();
+        auto request_w_block = [&]() __attribute__((always_inline)) {
+            request_w(std::integral_constant<int, 0>{}), request_w(std::integral_constant<int, 1>{}), request_w(std::integral_constant<int, 2>{});
+            request_w(std::integral_constant<int, 3>{}), request_w(std::integral_constant<int, 4>{});
+            w_cursor_advance();
+        };
+        request_w_block();
+#pragma unroll
+        for (int i = 0; i < kStages - 1; i++) {
+            phase_open();
+            request_a(std::integral_constant<int, 0>{}), request_a(std::integral_constant<int, 1>{}), request_a(std::integral_constant<int, 2>{});
+        }
         // the first 16 rank columns of the row tile's LA rows stay in LDS for all the column tiles of this workgroup: the
         // epilogue then reads them with LDS reads, which no pending store or request stands in front of
         if (p.r_pad > 0) {
@@ -158,30 +167,16 @@ struct Direct8 {
                 *(uint4*)(smem_raw + kLaBase + row * 32 + half * 16) = *(const uint4*)(p.la + (int64_t)(c.row_begin + min(row, c.rows_valid - 1)) * p.r_pad + half * 8);
             }
         }
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NI) : "memory");  // the first block's bytes and the first step's A stage have landed
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kStages - 2) * NI) : "memory");  // the first blocks and the first step's A stage have landed
         lds_barrier();
-        hc = *(const u32x4_t*)hdr_row;
-        asm volatile("" : "+v"(hc));  // (read out before the request below refills the buffer)
+        hc = *(const u32x4_t*)w_row;
         // Phase p = the last sub-step of step p - 1 and the first three of step p: it reads A stage p only, and its
         // requests (behind the barrier that opens it) fill the stage of step p - 1.  A phase's first A instruction goes
-        // out in its first sub-step, the others in the next step's first two; ph_dst / ph_src carry them across.
-        uint32_t ph_dst;
-        const bf16_t* ph_src;
-        auto phase_open = [&]() __attribute__((always_inline)) {
-            ph_dst = lds_base + a_wr + wave * 1024;
-            ph_src = a_base + i_step * 64;
-            a_wr = a_wr == (kStages - 1) * kStageBytes ? 0 : a_wr + kStageBytes;
-            if (++i_step == steps) i_step = 0;
-        };
-        auto request_a = [&](auto i_c) __attribute__((always_inline)) {
-            constexpr int I = decltype(i_c)::value;
-            if constexpr (I < NI) load16_to_lds(ph_dst + I * 8192, a_voff[I], ph_src);
-        };
-        issue_w_half(std::integral_constant<int, 0>{});  // phase 0: the first half of block 1 and its headers, A of step 3
-        issue_w_header();
+        // out in its first sub-step, the others in the next step's first two.
+        request_w_block();  // phase 0: block 1, A of step kStages - 1
         phase_open();
         request_a(std::integral_constant<int, 0>{});
-        qc = *(const u32x4_t*)(w_rows + w_roff[0]);
+        qc = *(const u32x4_t*)(w_row + w_q);
         Scales sc;
         uint32_t bx[4], by[4];  // B operands of the current / next sub-step
         sc = Direct::chunk_scales<0>(hc);
@@ -222,18 +217,18 @@ struct Direct8 {
                                               : (const void*)(p.w[0] + c.expert * p.w_expert_bytes);
                 asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(lb0_raw) : "v"(src) : "memory");
             }
-            // the first half of the next block's quant bytes goes out with a block's last sub-step, except behind a
-            // tile's last block, where the store path below still uses the buffer it would fill
-            if (ct > ct0) issue_w_half(std::integral_constant<int, 0>{});
-            for (int kb = 0; kb < blocks; kb++) {
-                // Requests per phase P (= step index % 4): the A stage three steps on [NI]; P = 0: the first half of the
-                // next block's quant bytes [2] and its headers [1]; P = 2: the second half [2].
+            if (!L::kOwnStaging && ct > ct0) request_w_block();
+            auto block = [&](auto first_c, bool last) __attribute__((always_inline)) {
+                constexpr bool FIRST = decltype(first_c)::value;
+                // Requests per phase P (= step index % 4): an A stage [NI]; P = 3 and 0: the next block but one, into the buffer
+                // whose last quant bytes step 2 has read [3 + 2] (staging in that buffer: behind a tile's last block all of it
+                // in phase 0, behind the store path).
                 auto step = [&](auto s_c) __attribute__((always_inline)) {
                     constexpr int S = decltype(s_c)::value;
-                    // the quant bytes of the next step: second step of this buffer, or the first of the next one
-                    const int w_rd_next = w_rd == (kWBufs - 1) * kWBufBytes ? 0 : w_rd + kWBufBytes;
-                    qn = *(const u32x4_t*)(w_rows + ((S & 1) ? w_rd_next + w_roff[0] : w_rd + w_roff[1]));
-                    if (S == 3) hn = *(const u32x4_t*)hdr_row;  // the next block's headers: requested a block ago, landed by the last step's wait
+                    // the quant bytes of the next step: of this block, or the first of the next one, with its header
+                    if (S == 3) w_rd ^= kWBufBytes;
+                    qn = *(const u32x4_t*)(w_row + w_rd + w_q + 32 * ((S + 1) & 3));
+                    if (S == 3) hn = *(const u32x4_t*)(w_row + w_rd);
                     const int a_rd_next = a_rd == (kStages - 1) * kStageBytes ? 0 : a_rd + kStageBytes;
                     __builtin_amdgcn_sched_barrier(0);
                     sub_step(bx, a_rd, 1, [&](auto k_c) __attribute__((always_inline)) { Direct::decode_half<1, decltype(k_c)::value>(qc, sc, by); },
@@ -247,12 +242,16 @@ struct Direct8 {
                     // the barrier every wave's part has, and every wave is done reading stage S, which the next phase's
                     // requests overwrite.  Requests complete in order, so the distance matters: packed bytes come from
                     // HBM, and a wait that covered requests only one step old stalled on them.
-                    // (Behind a tile's stores and the request of the LoRA factor row, which went out inside phase 0's requests,
-                    // the first two steps allow for them.)
-                    constexpr int kGroup[4] = {NI + 3, NI, NI + 2, NI};
-                    constexpr int kBehind = kGroup[S] + kGroup[(S + 3) & 3];
-                    if (S < 2 && kb == 0 && stores_behind) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBehind + kStores + 1) : "memory");
-                    else if (S < 2 && kb == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBehind + 1) : "memory");
+                    // (Three stages: A stages are requested one phase later, and only this phase's requests may be outstanding.)
+                    // A tile's phase 0 also holds the tile before's stores and the request of the LoRA factor row.
+                    constexpr int kTwo = kStages - 3;  // 1: the phase before this one counts, 0: it does not
+                    constexpr int kLate = L::kOwnStaging ? 0 : 3;  // packed requests of phase 3 that come in phase 0 at a tile's end
+                    constexpr int kGroup[4] = {NI + 2 + (FIRST ? 1 + kLate : 0), NI, NI, NI + 3}, kLastOfTile = NI + 3 - kLate;
+                    constexpr int kBehind = kGroup[S] + kTwo * (S == 0 && FIRST ? kLastOfTile : kGroup[(S + 3) & 3]);
+                    if (FIRST && (S == 0 || (S == 1 && kTwo))) {
+                        if (stores_behind) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBehind + kStores) : "memory");
+                        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBehind) : "memory");
+                    } else if (S == 3 && kLate && last) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBehind - kLate) : "memory");
                     else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBehind) : "memory");
                     lds_barrier();
                     phase_open();
@@ -263,22 +262,22 @@ struct Direct8 {
                         if (K == 0) sc = Direct::chunk_scales<(S + 1) & 3>(S == 3 ? hn : hc);
                         Direct::decode_half<0, K>(qn, sc, bx);
                     }, [&]() __attribute__((always_inline)) {
-                        if (S == 3 && kb + 1 < blocks) issue_w_half(std::integral_constant<int, 0>{});
-                        if (S == 3) issue_w_header();  // (behind the barrier: every read of the buffer's last contents has returned)
-                        if (S == 1) issue_w_half(std::integral_constant<int, 1>{});
+                        const bool here = L::kOwnStaging || !last;
+                        if (S == 2 && here) request_w(std::integral_constant<int, 0>{}), request_w(std::integral_constant<int, 1>{}), request_w(std::integral_constant<int, 2>{});
+                        if (S == 3 && here) request_w(std::integral_constant<int, 3>{}), request_w(std::integral_constant<int, 4>{}), w_cursor_advance();
                         request_a(std::integral_constant<int, 0>{});
                     });
                     qc = qn;
                     a_rd = a_rd_next;
-                    if (S & 1) w_rd = w_rd_next;
-                    if (S == 2) w_cursor_advance();
                 };
                 step(std::integral_constant<int, 0>{});
                 step(std::integral_constant<int, 1>{});
                 step(std::integral_constant<int, 2>{});
                 step(std::integral_constant<int, 3>{});
                 hc = hn;
-            }
+            };
+            block(std::true_type{}, blocks == 1);
+            for (int kb = 1; kb < blocks; kb++) block(std::false_type{}, kb + 1 == blocks);
             // ---- LoRA term and store.  A lane holds four consecutive columns of one row: acc[rb][i] is tile row
             // 32 rb + lane_c, column 32 wave + 8 (i / 4) + 4 h + (i % 4): a row block goes out as 64-byte row pieces.
             // (own, opaque copies of the lane coordinates: none of this part's address arithmetic may be hoisted in
@@ -306,9 +305,7 @@ struct Direct8 {
                 for (int rb = 0; rb < LIVE; rb++)
                     la0[rb] = *(const bf16x8_t*)(smem_raw + kLaBase + (32 * rb + lane_ce) * 32 + lane_he * 16);
             }
-            // the staging block: the buffer of the pair of steps just finished (the next request into it comes with the
-            // next tile's first step, after the reads below have returned their data to the stores)
-            uint8_t* const stage = smem_raw + kWBase + wave * (kWBufs * kWBufBytes) + (w_rd == 0 ? (kWBufs - 1) * kWBufBytes : w_rd - kWBufBytes);
+            uint8_t* const stage = smem_raw + (L::kOwnStaging ? kOutBase + wave * 2048 : wave * (2 * kWBufBytes) + (w_rd ^ kWBufBytes));
 #pragma unroll
             for (int rb = 0; rb < LIVE; rb++) {
                 const int row = 32 * rb + lane_ce;

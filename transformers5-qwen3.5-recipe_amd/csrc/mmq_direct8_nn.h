@@ -7,15 +7,19 @@
 // wave w owns sub-block w of it (32 columns: the low or the high nibbles of quant group w / 2), for up to six 32-row
 // blocks of 32x32x16 accumulators.  Per contraction step of 64 weight rows
 //   * the A tile (cotangent rows) goes global -> LDS directly, as in the forward kernel;
-//   * the step's packed bytes - 64 rows x (16-byte header + 128 quant bytes), contiguous per row - go global -> LDS
-//     directly too, requested by the whole workgroup with adjacent lanes on adjacent bytes (one row's bytes asked
-//     for lane by lane, 16 bytes each, cost the vector cache one access per lane), and are shared by the eight waves;
+//   * the step's packed bytes - 64 blocks of 144 bytes, header and quants together - go global -> LDS directly too,
+//     requested by the whole workgroup with nine adjacent lanes on a block (one row's bytes asked for lane by lane,
+//     16 bytes each, cost the vector cache one access per lane), and are shared by the eight waves;
 //   * lane l of every wave decodes weight row l for the wave's 32 columns (one scale and one min per row) and
 //     writes the 32 values as one row of the wave's own [64][32] LDS block; the MFMA operands (eight consecutive
 //     contraction rows of one column per lane) come back out of that block through transposing reads.  LDS accesses
 //     of one wave execute in order, so the block needs neither a barrier nor a second buffer.
 // The weights are the MFMA's first operand (accumulator registers hold four consecutive columns of one row), the
 // store path and the LoRA term are those of the forward kernel; the factor tile is transposed through the same block.
+//
+// What bounds it: instructions a wave issues per step, and LDS (the decoded block's way out and back).  256 experts, 2 x 512
+// rows of W, k 2048: 116 / 117 / 138 / 191 / 220 / 245 us at 16 / 32 / 64 / 128 / 160 / 192 rows; with separate headers,
+// addresses computed per request and waits chosen by branches 117 / 118 / 142 / 197 / 225 / 250.
 #pragma once
 #include "mmq_direct8.h"
 
@@ -26,7 +30,7 @@ struct Direct8NN {
     static constexpr int kWaves = 8;
     static constexpr int kThreadsWG = 64 * kWaves;
     static constexpr int kARingBytes = 9 * 8192;                       // 4 stages x 16 KB (up to 128 rows) or 3 x 24 KB (up to 192)
-    static constexpr int kRawStageBytes = 64 * 128 + 64 * 16;          // a step's quant bytes [64 rows][128], then its headers [64][16]
+    static constexpr int kRawStageBytes = 64 * 144;                    // a step's blocks; the pitch spreads the row-per-lane reads over all banks
     static constexpr int kRawBase = kARingBytes;
     static constexpr int kDecPitch = 80;                               // bytes per row of a wave's decoded block (32 bf16 + pad)
     static constexpr int kDecBlock = 64 * kDecPitch;
@@ -71,8 +75,9 @@ struct Direct8NN {
         extern __shared__ __attribute__((aligned(16))) uint8_t smem_raw[];
         constexpr int NI = (LIVE + 1) / 2;        // direct-to-LDS instructions per A stage and wave
         constexpr int kStages = LIVE <= 4 ? 4 : 3;
-        constexpr int kStageBytes = NI * 8192;
-        constexpr int kGroup = NI + 1;            // requests per phase and wave: A [NI], quant bytes [1]; wave 0 one more: the headers
+        constexpr int kStageBytes = LIVE * 4096;
+        constexpr int kGroup = NI + 1;            // requests per phase and wave: A [NI] (of an odd block count, the last with half its lanes), packed bytes [1]; wave 0 one more
+        constexpr int kBehind = (kStages - 2) * kGroup;  // requests that may be outstanding at a phase's end (wave 0 waits for one or two more than it needs)
         constexpr int kStores = 2 * LIVE - 1;     // 16-byte store instructions a tile certainly issues per wave
         const int tid = threadIdx.x, lane = tid & 63;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -84,59 +89,59 @@ struct Direct8NN {
         uint32_t a_voff[NI];
 #pragma unroll
         for (int i = 0; i < NI; i++) {
-            const int r = 64 * i + (tid >> 3), s = tid & 7;
+            const int r = 64 * i + (2 * i + 1 < LIVE ? tid >> 3 : 4 * wave + (lane_c >> 3)), s = tid & 7;
             const int kc = s ^ ((r >> 1) & 7);
-            const int rr = min(r, c.rows_valid - 1);
+            const int rr = r < c.rows_valid ? r : min(r - c.rows_valid, c.rows_valid - 1);
             // with a row index (one cotangent matrix read through it) the lane offsets carry the whole stored row
             const int src = p.a_rows.on() ? p.a_rows.source(c.row_begin + rr) : rr;
             a_voff[i] = (uint32_t)(((int64_t)src * p.lda + kc * 8) * 2);
         }
-        // packed bytes of a step: lane t of the workgroup moves quant chunk (t % 8) ^ swizzle of weight row t / 8
-        // (the 16-byte chunks of a row are XOR-swizzled like an A row's: the per-row reads below meet no bank conflict);
-        // wave 0 moves the 64 headers of the step with one request (one request of eight lanes
-        // per wave took the same time to 0.1 % of a training step, at eight times the requests)
-        const uint32_t wq_voff = (uint32_t)((tid >> 3) * (int)p.w_row_bytes + 16 + 16 * ((tid & 7) ^ (((tid >> 3) >> 1) & 7)));
-        const uint32_t wh_voff = (uint32_t)(lane * (int)p.w_row_bytes);
-        const bool hdr_wave = wave == 0;
-        // waits: at most `behind` phases of requests (and `extra` other operations) of this wave outstanding
-        auto wait_behind = [&](auto extra_c) __attribute__((always_inline)) {
-            constexpr int X = decltype(extra_c)::value;
-            if (hdr_wave) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kStages - 2) * (kGroup + 1) + X) : "memory");
-            else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kStages - 2) * kGroup + X) : "memory");
-        };
-        // Cursors: (column tile, step) of the next A stage / packed-byte stage to request; past the last tile they
-        // stay on it (what they request again is never used).
-        int a_step_i = 0, a_wr = 0;
-        int w_tile_i = ct0, w_step_i = 0, w_wr = 0;
-        auto step_src_a = [&](int st) __attribute__((always_inline)) {
-            const int seg = st >= sps ? 1 : 0, local = st - seg * sps;
-            return (seg ? p.a[1] : p.a[0]) + (p.a_rows.on() ? 0 : (int64_t)c.row_begin * p.lda) + local * 64;
-        };
-        auto step_src_w = [&](int ct, int st) __attribute__((always_inline)) {
-            const int seg = st >= sps ? 1 : 0, local = st - seg * sps;
-            return (seg ? p.w[1] : p.w[0]) + c.expert * p.w_expert_bytes + (int64_t)local * 64 * p.w_row_bytes + ct * 144;
-        };
+        // packed bytes of a step: the 576 16-byte chunks of its 64 blocks in row order, chunk `tid` by lane `tid` of the
+        // workgroup, the last 64 by wave 0.  What a request costs is the cache lines it touches: with the headers in a
+        // request of their own (64 rows x 16 bytes) the vector cache was busy twice as long.
+        const uint32_t w_voff = (uint32_t)((tid / 9) * (int)p.w_row_bytes + 16 * (tid % 9));
+        const uint32_t w_voff_last = (uint32_t)(((512 + lane) / 9) * (int)p.w_row_bytes + 16 * ((512 + lane) % 9));
+        const bool last_wave = wave == 0;
+        // Cursors: the next A stage / packed-byte stage to request.  They advance by additions and change segment and column
+        // tile (a branch that is rarely taken) when their steps run out: computed from (tile, segment, step) for every
+        // request, the addresses were a third of the loop's instructions, and with two waves per SIMD a wave's time is the
+        // instructions it issues.  Past the last tile they stay on it (what they request again is never used).
+        const int64_t a_row0 = p.a_rows.on() ? 0 : (int64_t)c.row_begin * p.lda;
+        const bf16_t* a_src = p.a[0] + a_row0;
+        const uint8_t* const w_plane[2] = {p.w[0] + c.expert * p.w_expert_bytes, p.nseg > 1 ? p.w[1] + c.expert * p.w_expert_bytes : nullptr};
+        const uint8_t* w_src = w_plane[0] + ct0 * 144;
+        const int64_t w_step = 64 * p.w_row_bytes;
+        int a_left = sps, a_seg = 0, a_wr = 0;
+        int w_left = sps, w_seg = 0, w_tile = ct0, w_wr = 0;
         uint32_t ph_dst;       // the open phase's A requests (its first goes out at once, the others in the next sub-steps)
         const bf16_t* ph_src;
         auto open_a = [&]() __attribute__((always_inline)) {
-            ph_dst = lds_base + a_wr + wave * 1024;
-            ph_src = step_src_a(a_step_i);
+            ph_dst = lds_base + a_wr;
+            ph_src = a_src;
             a_wr = a_wr == (kStages - 1) * kStageBytes ? 0 : a_wr + kStageBytes;
-            if (++a_step_i == steps) a_step_i = 0;
+            a_src += 64;
+            if (--a_left == 0) {
+                a_left = sps, a_seg = a_seg + 1 < p.nseg ? a_seg + 1 : 0;
+                a_src = (a_seg ? p.a[1] : p.a[0]) + a_row0;
+            }
         };
         auto request_a = [&](auto i_c) __attribute__((always_inline)) {
             constexpr int I = decltype(i_c)::value;
-            if constexpr (I < NI) load16_to_lds(ph_dst + I * 8192, a_voff[I], ph_src);
+            if constexpr (2 * I + 1 < LIVE) load16_to_lds(ph_dst + I * 8192 + wave * 1024, a_voff[I], ph_src);
+            else if constexpr (2 * I < LIVE) {
+                if (lane_h == 0) load16_to_lds(ph_dst + I * 8192 + wave * 512, a_voff[I], ph_src);
+            }
         };
         auto request_w = [&]() __attribute__((always_inline)) {
-            const uint8_t* src = step_src_w(w_tile_i, w_step_i);
             const uint32_t dst = lds_base + kRawBase + w_wr;
-            load16_to_lds(dst + wave * 1024, wq_voff, src);
-            if (hdr_wave) load16_to_lds(dst + 64 * 128, wh_voff, src);
+            load16_to_lds(dst + wave * 1024, w_voff, w_src);
+            if (last_wave) load16_to_lds(dst + 8 * 1024, w_voff_last, w_src);
             w_wr = w_wr == (kStages - 1) * kRawStageBytes ? 0 : w_wr + kRawStageBytes;
-            if (++w_step_i == steps) {
-                w_step_i = 0;
-                if (w_tile_i + 1 < ct1) w_tile_i++;
+            w_src += w_step;
+            if (--w_left == 0) {
+                w_left = sps;
+                if (++w_seg == p.nseg) w_seg = 0, w_tile = min(w_tile + 1, ct1 - 1);
+                w_src = (w_seg ? w_plane[1] : w_plane[0]) + w_tile * 144;
             }
         };
 
@@ -146,11 +151,9 @@ struct Direct8NN {
 #pragma unroll
         for (int i = 0; i < 4; i++) a_koff[i] = a_slot(lane_c, 2 * i + lane_h) * 16;
         bf16x8_t ao[LIVE];
-        // this lane's weight row in a packed-byte stage: the two chunks of its wave's quant group, and its header
-        const int grp = wave >> 1;
-        const uint8_t* const raw_row = smem_raw + kRawBase + lane * 128;
-        const int raw_qoff[2] = {((2 * grp) ^ ((lane >> 1) & 7)) * 16, ((2 * grp + 1) ^ ((lane >> 1) & 7)) * 16};
-        const uint8_t* const raw_hdr = smem_raw + kRawBase + 64 * 128 + lane * 16;
+        // this lane's weight row in a packed-byte stage: the block's header, and the 32 bytes of its wave's quant group
+        const uint8_t* const raw_row = smem_raw + kRawBase + lane * 144;
+        const int raw_q = 16 + 32 * (wave >> 1);
         const uint32_t nib_mask = (wave & 1) ? 0x00F000F0u : 0x000F000Fu;
         // this wave's decoded block, the row this lane writes, and where its transposing reads start
         uint8_t* const dblk = smem_raw + kDecBase + wave * kDecBlock;
@@ -164,9 +167,9 @@ struct Direct8NN {
         u32x4_t rq0, rq1, rh;  // raw bytes of the step being decoded
         float dl, nm;
         auto raw_fetch = [&](int off) __attribute__((always_inline)) {
-            rq0 = *(const u32x4_t*)(raw_row + off + raw_qoff[0]);
-            rq1 = *(const u32x4_t*)(raw_row + off + raw_qoff[1]);
-            rh = *(const u32x4_t*)(raw_hdr + off);
+            rq0 = *(const u32x4_t*)(raw_row + off + raw_q);
+            rq1 = *(const u32x4_t*)(raw_row + off + raw_q + 16);
+            rh = *(const u32x4_t*)(raw_row + off);
         };
         // quarter Q (0..3) of the row: words 2 Q, 2 Q + 1 of the 32 quant bytes -> columns 8 Q .. 8 Q + 7
         auto decode_quarter = [&](auto q_c) __attribute__((always_inline)) {
@@ -201,7 +204,7 @@ struct Direct8NN {
                 *(uint4*)(smem_raw + kLaBase + row * 32 + half * 16) = *(const uint4*)(p.la + (int64_t)(c.row_begin + min(row, c.rows_valid - 1)) * p.r_pad + half * 8);
             }
         }
-        wait_behind(std::integral_constant<int, 0>{});
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBehind) : "memory");
         lds_barrier();
         int a_rd = 0;   // byte offset of the A stage of the current step
         int w_rd = 0;   // byte offset of the packed-byte stage of the step being decoded (one ahead of the A stage)
@@ -239,7 +242,6 @@ struct Direct8NN {
             one(std::integral_constant<int, 3>{}), one(std::integral_constant<int, 4>{}), one(std::integral_constant<int, 5>{});
         };
         bool stores_behind = false;  // the tile before this one went out through the staged store path
-        int relax = 0;               // steps of this tile whose wait still allows for the stores of the tile before
         for (int ct = ct0; ct < ct1; ct++) {
 #pragma unroll
             for (int i = 0; i < LIVE; i++)
@@ -256,72 +258,74 @@ struct Direct8NN {
                                               : (const void*)(p.w[0] + c.expert * p.w_expert_bytes);
                 asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(lbraw) : "v"(src) : "memory");
             }
-            relax = kStages - 2;
-            for (int st = 0; st < steps; st += 2) {
-                // One step.  Its B operands were read at the end of the step before; the next step's weight rows are
-                // decoded behind its MFMAs (a half of a quarter row per slot) and read back at its end.
-                auto step = [&](auto par_c) __attribute__((always_inline)) {
-                    constexpr int P = decltype(par_c)::value;
-                    const bf16x8_t* b = bops[P];
-                    raw_fetch(w_rd);
-                    const int a_rd_next = a_rd == (kStages - 1) * kStageBytes ? 0 : a_rd + kStageBytes;
-                    __builtin_amdgcn_sched_barrier(0);
-                    // The next step's weight row of this lane is decoded in eight pieces (one quant word = four columns
-                    // each) spread evenly over the 3 LIVE MFMA slots of the first three sub-steps, so that the block is
-                    // complete before the phase ends; its transposing reads are spread over the last sub-step's slots and
-                    // have landed when the next step starts.
-                    uint32_t o[4];
-                    auto decode_piece = [&](auto hp_c) __attribute__((always_inline)) {
-                        constexpr int HP = decltype(hp_c)::value, Q = HP >> 1, K = HP & 1;
-                        const u32x4_t& src = Q < 2 ? rq0 : rq1;
-                        if (HP == 0) sub_block_scale(rh, wave, dl, nm);
-                        decode_word(src[2 * (Q & 1) + K], nib_mask, dl, nm, o + 2 * K);
-                        if (K == 1) *(uint4*)(d_my_row + Q * 16) = make_uint4(o[0], o[1], o[2], o[3]);
-                    };
-                    auto decode_slots = [&](auto i_c) __attribute__((always_inline)) {  // sub-step I's share
-                        return [&](auto rb_c) __attribute__((always_inline)) {
-                            constexpr int T = decltype(i_c)::value * LIVE + decltype(rb_c)::value;
-                            auto maybe = [&](auto hp_c) __attribute__((always_inline)) {
-                                if constexpr (decltype(hp_c)::value * 3 * LIVE / 8 == T) decode_piece(hp_c);
-                            };
-                            maybe(std::integral_constant<int, 0>{}), maybe(std::integral_constant<int, 1>{}), maybe(std::integral_constant<int, 2>{}), maybe(std::integral_constant<int, 3>{});
-                            maybe(std::integral_constant<int, 4>{}), maybe(std::integral_constant<int, 5>{}), maybe(std::integral_constant<int, 6>{}), maybe(std::integral_constant<int, 7>{});
-                            if constexpr (decltype(rb_c)::value == 0 && decltype(i_c)::value == 0) request_a(std::integral_constant<int, 1>{});
-                            if constexpr (decltype(rb_c)::value == 0 && decltype(i_c)::value == 1) request_a(std::integral_constant<int, 2>{});
-                        };
-                    };
-                    sub_step(b[0], a_rd, 1, decode_slots(std::integral_constant<int, 0>{}));
-                    sub_step(b[1], a_rd, 2, decode_slots(std::integral_constant<int, 1>{}));
-                    sub_step(b[2], a_rd, 3, decode_slots(std::integral_constant<int, 2>{}));
-                    // End of the phase: all but the requests of this phase (and, with four stages, the one before it)
-                    // have landed - this wave's parts of the next step's A stage and of the packed bytes of the step
-                    // after it.  Behind the barrier every wave's parts have, and every wave is done with the stages the
-                    // next phase's requests overwrite.  (Behind a tile's stores and the request of the LoRA factor piece, which went out
-                    // inside a phase's requests, the steps whose awaited requests are older than that phase allow for them.)
-                    if (relax > 0 && stores_behind) wait_behind(std::integral_constant<int, kStores + 1>{});
-                    else if (relax > 0) wait_behind(std::integral_constant<int, 1>{});
-                    else wait_behind(std::integral_constant<int, 0>{});
-                    lds_barrier();
-                    open_a();
-                    bf16x8_t* bn = bops[P ^ 1];
-                    sub_step(b[3], a_rd_next, 0, [&](auto rb_c) __attribute__((always_inline)) {
-                        constexpr int RB = decltype(rb_c)::value;
-                        if constexpr (RB == 0) {
-                            request_w();
-                            request_a(std::integral_constant<int, 0>{});
-                        }
-                        // the next step's operands: its rows are in the block (LDS accesses of a wave execute in order), and
-                        // the writes of the step after it come behind these reads
-#pragma unroll
-                        for (int ks = 0; ks < 4; ks++)
-                            if (ks * LIVE / 4 == RB) bn[ks] = read_tr(tr_src + ks * 16 * kDecPitch, kDecPitch);
-                    });
-                    a_rd = a_rd_next;
-                    w_rd = w_rd == (kStages - 1) * kRawStageBytes ? 0 : w_rd + kRawStageBytes;
-                    relax--;
+            // One step.  Its B operands were read at the end of the step before; the next step's weight rows are
+            // decoded behind its MFMAs (a half of a quarter row per slot) and read back at its end.  P: parity; FIRST: of the
+            // tile's first kStages - 2 steps, whose waits allow for the stores and the factor request of the tile's start.
+            auto step = [&](auto par_c, auto first_c) __attribute__((always_inline)) {
+                constexpr int P = decltype(par_c)::value;
+                const bf16x8_t* b = bops[P];
+                raw_fetch(w_rd);
+                const int a_rd_next = a_rd == (kStages - 1) * kStageBytes ? 0 : a_rd + kStageBytes;
+                __builtin_amdgcn_sched_barrier(0);
+                // The next step's weight row of this lane is decoded in eight pieces (one quant word = four columns
+                // each) spread evenly over the 3 LIVE MFMA slots of the first three sub-steps, so that the block is
+                // complete before the phase ends; its transposing reads are spread over the last sub-step's slots and
+                // have landed when the next step starts.
+                uint32_t o[4];
+                auto decode_piece = [&](auto hp_c) __attribute__((always_inline)) {
+                    constexpr int HP = decltype(hp_c)::value, Q = HP >> 1, K = HP & 1;
+                    const u32x4_t& src = Q < 2 ? rq0 : rq1;
+                    if (HP == 0) sub_block_scale(rh, wave, dl, nm);
+                    decode_word(src[2 * (Q & 1) + K], nib_mask, dl, nm, o + 2 * K);
+                    if (K == 1) *(uint4*)(d_my_row + Q * 16) = make_uint4(o[0], o[1], o[2], o[3]);
                 };
-                step(std::integral_constant<int, 0>{});
-                step(std::integral_constant<int, 1>{});
+                auto decode_slots = [&](auto i_c) __attribute__((always_inline)) {  // sub-step I's share
+                    return [&](auto rb_c) __attribute__((always_inline)) {
+                        constexpr int T = decltype(i_c)::value * LIVE + decltype(rb_c)::value;
+                        auto maybe = [&](auto hp_c) __attribute__((always_inline)) {
+                            if constexpr (decltype(hp_c)::value * 3 * LIVE / 8 == T) decode_piece(hp_c);
+                        };
+                        maybe(std::integral_constant<int, 0>{}), maybe(std::integral_constant<int, 1>{}), maybe(std::integral_constant<int, 2>{}), maybe(std::integral_constant<int, 3>{});
+                        maybe(std::integral_constant<int, 4>{}), maybe(std::integral_constant<int, 5>{}), maybe(std::integral_constant<int, 6>{}), maybe(std::integral_constant<int, 7>{});
+                        if constexpr (decltype(rb_c)::value == 0 && decltype(i_c)::value == 0) request_a(std::integral_constant<int, 1>{});
+                        if constexpr (decltype(rb_c)::value == 0 && decltype(i_c)::value == 1) request_a(std::integral_constant<int, 2>{});
+                    };
+                };
+                sub_step(b[0], a_rd, 1, decode_slots(std::integral_constant<int, 0>{}));
+                sub_step(b[1], a_rd, 2, decode_slots(std::integral_constant<int, 1>{}));
+                sub_step(b[2], a_rd, 3, decode_slots(std::integral_constant<int, 2>{}));
+                // End of the phase: all but the requests of this phase (and, with four stages, the one before it)
+                // have landed - this wave's parts of the next step's A stage and of the packed bytes of the step
+                // after it.  Behind the barrier every wave's parts have, and every wave is done with the stages the
+                // next phase's requests overwrite.  (Behind a tile's stores and the request of the LoRA factor piece, which went out
+                // inside a phase's requests, the steps whose awaited requests are older than that phase allow for them.)
+                if constexpr (decltype(first_c)::value) {
+                    if (stores_behind) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBehind + kStores + 1) : "memory");
+                    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBehind + 1) : "memory");
+                } else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBehind) : "memory");
+                lds_barrier();
+                open_a();
+                bf16x8_t* bn = bops[P ^ 1];
+                sub_step(b[3], a_rd_next, 0, [&](auto rb_c) __attribute__((always_inline)) {
+                    constexpr int RB = decltype(rb_c)::value;
+                    if constexpr (RB == 0) {
+                        request_w();
+                        request_a(std::integral_constant<int, 0>{});
+                    }
+                    // the next step's operands: its rows are in the block (LDS accesses of a wave execute in order), and
+                    // the writes of the step after it come behind these reads
+#pragma unroll
+                    for (int ks = 0; ks < 4; ks++)
+                        if (ks * LIVE / 4 == RB) bn[ks] = read_tr(tr_src + ks * 16 * kDecPitch, kDecPitch);
+                });
+                a_rd = a_rd_next;
+                w_rd = w_rd == (kStages - 1) * kRawStageBytes ? 0 : w_rd + kRawStageBytes;
+            };
+            step(std::integral_constant<int, 0>{}, std::true_type{});
+            step(std::integral_constant<int, 1>{}, std::integral_constant<bool, kStages == 4>{});
+            for (int st = 2; st < steps; st += 2) {
+                step(std::integral_constant<int, 0>{}, std::false_type{});
+                step(std::integral_constant<int, 1>{}, std::false_type{});
             }
             // ---- LoRA term and store (accumulator layout and staging as in the forward kernel; the staging block is this
             // wave's decoded block, whose rows have been read)
