@@ -39,11 +39,13 @@ def _check_lora(pkg, dev, payload, qt, x, a, b, s, dy):
     (48, 64, 256, 16),      # the fewest rows
     (49, 65, 512, 5),       # one row and one column past a tile; a rank that is no multiple of eight; columns that no split takes
     (63, 511, 4096, 32),    # the widest rank of the shared launch
-    (64, 512, 8192, 16),    # eight contraction splits
+    (64, 512, 8192, 16),    # sixteen contraction splits
     (257, 520, 2048, 33),   # a rank of the separate launches
     (1500, 2052, 1024, 8),  # 128 x 128 tiles forward
     (3001, 5001, 256, 16),  # 256 x 256 tiles, ragged both ways; the shortest contraction
     (4096, 1028, 2048, 4),
+    (1999, 4097, 2048, 16),  # 128 x 256 tiles forward, ragged both ways
+    (4003, 4100, 2048, 24),  # and in the grad-input; a contraction that ends inside a step
 ])
 @pytest.mark.parametrize("qt", [gb.Q8_0, gb.Q4_K, gb.IQ2_XXS], ids=lambda q: TYPE_NAMES[q])
 def test_dense_lora_over_panels(pkg, dev, qt, m, n, k, r):

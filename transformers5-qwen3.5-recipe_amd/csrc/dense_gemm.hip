@@ -31,8 +31,8 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 // ------------------------------------------------------------------------------------------------
 // Decoding passes.  HBM-bound: packed bytes in, two bytes per weight out.
 
-// What chunk index of row r is XOR-ed with (r mod 16 counts).
-__device__ __forceinline__ int panel_swizzle(int r) { return (((r >> 1) & 3) << 1) | ((r >> 3) & 1); }
+// What chunk index of row r is XOR-ed with (r mod 32 counts).
+__device__ __forceinline__ int panel_swizzle(int r) { return ((((r >> 1) & 3) << 1) | ((r >> 3) & 1)) ^ (((r >> 4) & 1) << 2); }
 
 template <int QT>
 __device__ __forceinline__ const uint2* stage_tables(uint32_t* lds, int tid, int threads) {
@@ -234,21 +234,25 @@ struct DenseParams {
 };
 enum : int { kDenseStore = 0, kDenseAccum = 1, kDensePartial = 2 };
 
-// Waves form a WM x WN grid, each owning RB x CB blocks of 32 x 32; NS stages of 64 contraction elements in LDS.
+// Waves form a WM x WN grid, each owning RB x CB blocks of 16 x 16; NS stages of 64 contraction elements in LDS.
+//
+// What bounds it at a few thousand rows is power: on every compute unit at once the chip holds 1.7 to 2.0 GHz, and 16x16x32
+// MFMAs get 2.05 PFLOP/s out of that (random operands in registers), 32x32x16 ones 1.83.
 template <int WM, int WN, int RB, int CB, int NS>
 struct DenseTile {
-    static constexpr int kBM = WM * RB * 32, kBN = WN * CB * 32, kWaves = WM * WN, kThreadsWG = 64 * kWaves;
+    static constexpr int kBM = WM * RB * 16, kBN = WN * CB * 16, kWaves = WM * WN, kThreadsWG = 64 * kWaves;
     static constexpr int kLoadsA = kBM / 8 / kWaves, kLoadsB = kBN / 8 / kWaves, kLoads = kLoadsA + kLoadsB;
     static constexpr int kStageA = kBM * 128, kStage = (kBM + kBN) * 128;
     static constexpr int kLdsBytes = NS * kStage;
-    static constexpr int kOutPitch = CB * 64 + 16;  // bytes of a staged output row
-    static_assert(kWaves * 32 * kOutPitch <= kLdsBytes, "output staging");
+    static constexpr int kOutPitch = CB * 32 + 16;  // bytes of a staged output row
+    static_assert(kWaves * 16 * kOutPitch <= kLdsBytes, "output staging");
 };
 
 __device__ __forceinline__ void wait_loads(int n) {  // at most n of this wave's requests outstanding (n known at compile time after inlining)
     switch (n) {
         case 0: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
         case 4: asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); break;
+        case 6: asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); break;
         case 8: asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); break;
         case 12: asm volatile("s_waitcnt vmcnt(12)" ::: "memory"); break;
         default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
@@ -318,89 +322,91 @@ __device__ __forceinline__ void dense_body(const DenseParams& p, uint8_t* lds) {
         }
     };
 
-    f32x16_t acc[RB][CB];
+    f32x4_t acc[RB][CB];
 #pragma unroll
     for (int i = 0; i < RB; i++)
 #pragma unroll
-        for (int j = 0; j < CB; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+        for (int j = 0; j < CB; j++) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 
-    const int l32 = lane & 31, half = lane >> 5;
-    if (p.la && split == 0) {  // scale * LA . LB first (operands straight from memory: one to four MFMAs per block and tile)
-        for (int r0 = 0; r0 < p.r_pad; r0 += 16) {
+    const int l16 = lane & 15, quarter = lane >> 4;
+    if (p.la && split == 0) {  // scale * LA . LB first (operands straight from memory: one or two MFMAs per block and tile)
+        for (int r0 = 0; r0 < p.r_pad; r0 += 32) {
+            const int r = r0 + 8 * quarter;  // this lane's eight ranks (zeros past the rank in both operands)
             bf16x8_t lbv[CB];
 #pragma unroll
             for (int j = 0; j < CB; j++) {
-                const int col = min(col0 + (wn * CB + j) * 32 + l32, p.cols - 1);
+                const int col = min(col0 + (wn * CB + j) * 16 + l16, p.cols - 1);
                 if (!p.lb_k_major) {
-                    lbv[j] = __builtin_bit_cast(bf16x8_t, load8g(p.lb + (int64_t)col * p.rank + r0 + 8 * half, p.rank - (r0 + 8 * half), (p.rank & 7) == 0));
+                    lbv[j] = __builtin_bit_cast(bf16x8_t, load8g(p.lb + (int64_t)col * p.rank + r, p.rank - r, (p.rank & 7) == 0));
                 } else {
                     uint32_t e[8];
 #pragma unroll
                     for (int i = 0; i < 8; i++) {
-                        const int r = r0 + 8 * half + i;
-                        const uint32_t x = p.lb[(int64_t)min(r, p.rank - 1) * p.lb_ld + col];
-                        e[i] = r < p.rank ? x : 0u;
+                        const uint32_t x = p.lb[(int64_t)min(r + i, p.rank - 1) * p.lb_ld + col];
+                        e[i] = r + i < p.rank ? x : 0u;
                     }
                     lbv[j] = __builtin_bit_cast(bf16x8_t, make_uint4(e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)));
                 }
             }
 #pragma unroll
             for (int i = 0; i < RB; i++) {
-                const int row = row0 + min((wm * RB + i) * 32 + l32, rows_valid - 1);
-                const bf16x8_t lav = __builtin_bit_cast(bf16x8_t, *(const uint4*)(p.la + (int64_t)row * p.r_pad + r0 + 8 * half));
+                const int row = row0 + min((wm * RB + i) * 16 + l16, rows_valid - 1);
+                const bf16x8_t lav = __builtin_bit_cast(bf16x8_t, r < p.r_pad ? *(const uint4*)(p.la + (int64_t)row * p.r_pad + r) : make_uint4(0, 0, 0, 0));
 #pragma unroll
-                for (int j = 0; j < CB; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lbv[j], lav, acc[i][j], 0, 0, 0);
+                for (int j = 0; j < CB; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lbv[j], lav, acc[i][j], 0, 0, 0);
             }
         }
 #pragma unroll
         for (int i = 0; i < RB; i++)
 #pragma unroll
-            for (int j = 0; j < CB; j++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) acc[i][j][v] *= p.lora_scale;
+            for (int j = 0; j < CB; j++) acc[i][j] *= p.lora_scale;
     }
 
-    // Main loop.  A step is four sub-steps of 16 contraction elements; a sub-step's operands are read from LDS during the one
-    // before it.  In front of the last sub-step every wave has the whole stage in registers: there the step's one barrier
-    // stands, behind it the stage is refilled with step s + NS and the next stage's first operands are read, both under
-    // the MFMAs of the last sub-step, so no wave meets the barrier with an idle matrix pipe behind it.
+    // Main loop.  A step is two sub-steps of 32 contraction elements (chunks kk, 2 + kk, 4 + kk, 6 + kk of a row, one per lane
+    // quarter: any order serves a sum, and these meet no bank conflict), each RB rows of CB MFMAs.  A row block's operand of
+    // the next sub-step is read into the registers its row has just released, the last row's at the start of that sub-step; column
+    // operands have two sets.  The step's one barrier stands kBarrierRow rows into the second sub-step, where every read of the
+    // stage has returned: behind it the stage is refilled with step s + NS and the next stage's first operands are read, all
+    // under MFMAs, so no wave meets the barrier with an idle matrix pipe behind it.
 #pragma unroll
     for (int s = 0; s < NS; s++)
         if (s < steps)
 #pragma unroll
             for (int q = 0; q < T::kLoads; q++) request(s, s * T::kStage, q, false);
-    // LDS offsets of this lane's operand chunks: rows by sub-step; columns by sub-step (forward), or by half of the eight
-    // contraction rows and column block (grad-input: lane s of sixteen points at row s / 4, columns 4 (s % 4) .. + 3)
-    uint32_t ra[4], rb[MODE == kModeNT ? 4 : 2 * CB];
+    // LDS offsets of this lane's operand chunks, by sub-step: rows (and forward's columns) of even and odd blocks of sixteen;
+    // grad-input: lane s of sixteen points at row s / 4 of four contraction rows, columns 4 (s % 4) .. + 3
+    uint32_t ra[2][2], rb[2][MODE == kModeNT ? 2 : 2 * CB];
 #pragma unroll
-    for (int kk = 0; kk < 4; kk++) {
-        const uint32_t slot = (uint32_t)((2 * kk + half) ^ panel_swizzle(l32)) * 16u;
-        ra[kk] = (uint32_t)(wm * RB * 32 + l32) * 128u + slot;
-        if (MODE == kModeNT) rb[kk] = (uint32_t)T::kStageA + (uint32_t)(wn * CB * 32 + l32) * 128u + slot;
-    }
+    for (int kk = 0; kk < 2; kk++)
+#pragma unroll
+        for (int odd = 0; odd < 2; odd++) {
+            const uint32_t slot = (uint32_t)((2 * quarter + kk) ^ panel_swizzle(16 * odd + l16)) * 16u;
+            ra[kk][odd] = (uint32_t)(wm * RB * 16 + l16) * 128u + slot;
+            if (MODE == kModeNT) rb[kk][odd] = (uint32_t)T::kStageA + (uint32_t)(wn * CB * 16 + l16) * 128u + slot;
+        }
     if (MODE == kModeNN) {
-        const int src = lane & 15, sub = (lane >> 4) & 1;
 #pragma unroll
-        for (int j = 0; j < CB; j++)
+        for (int kk = 0; kk < 2; kk++)
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
-                const int col = (wn * CB + j) * 32 + 16 * sub + 4 * (src & 3), row = 8 * half + 4 * t + (src >> 2);
-                rb[2 * j + t] = (uint32_t)T::kStageA + (uint32_t)(col >> 6) * 8192u + (uint32_t)row * 128u +
-                                (uint32_t)(((col & 63) >> 3) ^ panel_swizzle(row)) * 16u + (uint32_t)(src & 1) * 8u;
-            }
+            for (int j = 0; j < CB; j++)
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    const int col = (wn * CB + j) * 16 + 4 * (l16 & 3), row = 8 * (2 * quarter + kk) + 4 * t + (l16 >> 2);
+                    rb[kk][2 * j + t] = (uint32_t)T::kStageA + (uint32_t)(col >> 6) * 8192u + (uint32_t)row * 128u +
+                                        (uint32_t)(((col & 63) >> 3) ^ panel_swizzle(row)) * 16u + (uint32_t)(l16 & 1) * 8u;
+                }
     }
-    bf16x8_t fa[2][RB], fb[2][CB];
-    auto read_a = [&](int set, int i, uint32_t stage_off, int kk) __attribute__((always_inline)) {
-        fa[set][i] = *(const bf16x8_t*)(lds + stage_off + ra[kk] + i * 4096);
+    constexpr int kSets = RB <= 4 ? 2 : 1;  // row operand sets
+    bf16x8_t fa[kSets][RB], fb[2][CB];
+    auto read_a = [&](int i, uint32_t stage_off, int kk) __attribute__((always_inline)) {
+        fa[kk & (kSets - 1)][i] = *(const bf16x8_t*)(lds + stage_off + ra[kk][(wm * RB + i) & 1] + i * 2048);
     };
     auto read_b = [&](int set, int j, uint32_t stage_off, int kk) __attribute__((always_inline)) {
         if constexpr (MODE == kModeNT) {
-            fb[set][j] = *(const bf16x8_t*)(lds + stage_off + rb[kk] + j * 4096);
+            fb[set][j] = *(const bf16x8_t*)(lds + stage_off + rb[kk][(wn * CB + j) & 1] + j * 2048);
         } else {
-            const v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)(lds + stage_off + rb[2 * j] + kk * 2048));
-            const v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)(lds + stage_off + rb[2 * j + 1] + kk * 2048));
+            const v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)(lds + stage_off + rb[kk][2 * j]));
+            const v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)(lds + stage_off + rb[kk][2 * j + 1]));
             fb[set][j] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
         }
     };
@@ -411,39 +417,53 @@ __device__ __forceinline__ void dense_body(const DenseParams& p, uint8_t* lds) {
 #pragma unroll
         for (int j = 0; j < CB; j++) read_b(0, j, 0, 0);
 #pragma unroll
-        for (int i = 0; i < RB; i++) read_a(0, i, 0, 0);
+        for (int i = 0; i < (kSets == 2 ? RB : RB - 1); i++) read_a(i, 0, 0);
         uint32_t cur = 0;
-        constexpr int kM = RB * CB, kReads = RB + CB;
+        static_assert(RB % 2 == 0 && CB % 2 == 0, "blocks of sixteen alternate between two read offsets");
+        constexpr int kBarrierRow = kSets == 2 ? 0 : RB / 4;
         // one step; WHOLE: step s + NS exists and is not the contraction's last
         auto step = [&](int s, auto whole_tag) __attribute__((always_inline)) {
             constexpr bool WHOLE = decltype(whole_tag)::value;
             const uint32_t nxt = cur == (NS - 1) * T::kStage ? 0u : cur + T::kStage;
 #pragma unroll
-            for (int kk = 0; kk < 4; kk++) {
-                const int set = kk & 1;
-                if (kk == 3) {
-                    // step s + 1 has landed when only the requests of the steps after it are outstanding
-                    if (WHOLE || s + NS - 1 < steps) wait_loads((NS - 2) * T::kLoads);
-                    else wait_loads(0);
-                    lds_barrier();
-                }
-                const uint32_t from = kk == 3 ? nxt : cur;
+            for (int kk = 0; kk < 2; kk++) {
+                const uint32_t from = kk == 1 ? nxt : cur;  // where the next sub-step's operands are
+                constexpr int kFirst[2] = {kSets == 2 ? 0 : 1, kBarrierRow};  // the row from which on they are read
+                const int first = kFirst[kk];
 #pragma unroll
-                for (int x = 0; x < kM; x++) {
-                    // reads of the next sub-step, ahead of the MFMAs as far as they go: column operands first, in the order
-                    // the MFMAs take them
-                    constexpr int kPer = (kReads + kM - 1) / kM;
-#pragma unroll
-                    for (int q = x * kPer; q < (x + 1) * kPer && q < kReads; q++) {
-                        if (q < CB) read_b(set ^ 1, q, from, (kk + 1) & 3);
-                        else read_a(set ^ 1, q - CB, from, (kk + 1) & 3);
+                for (int i = 0; i < RB; i++) {
+                    if (kk == 1 && i == kBarrierRow) {
+                        // step s + 1 has landed when only the requests of the steps after it are outstanding
+                        if (WHOLE || s + NS - 1 < steps) wait_loads((NS - 2) * T::kLoads);
+                        else wait_loads(0);
+                        lds_barrier();
                     }
-                    if (kk == 3 && (WHOLE || s + NS < steps)) {
+                    if (kSets == 1 && i == 0) read_a(RB - 1, cur, kk);
+                    if constexpr (kSets == 2) {  // all of the next sub-step's operands, in the first half of the rows
+                        constexpr int kPer = (RB + CB + RB / 2 - 1) / (RB / 2);
 #pragma unroll
-                        for (int q = x * T::kLoads / kM; q < (x + 1) * T::kLoads / kM; q++) request(s + NS, cur, q, WHOLE);
+                        for (int q = i * kPer; q < (i + 1) * kPer && q < RB + CB; q++) {
+                            if (q < CB) read_b(kk ^ 1, q, from, kk ^ 1);
+                            else read_a(q - CB, from, kk ^ 1);
+                        }
+                    } else if (i >= first) {  // column operands first, then the operands of the rows done so far
+                        const int u = i - first;
+#pragma unroll
+                        for (int j = u * 2; j < (u + 1) * 2 && j < CB; j++) read_b(kk ^ 1, j, from, kk ^ 1);
+                        const int lo = u == 0 ? 0 : kk == 0 ? i - 1 : min(i - 1, 2 * u - 1), hi = kk == 0 ? i : min(i, 2 * u + 1);
+#pragma unroll
+                        for (int r = lo; r < hi; r++) read_a(r, from, kk ^ 1);
                     }
-                    acc[x / CB][x % CB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[set][x % CB], fa[set][x / CB], acc[x / CB][x % CB], 0, 0, 0);
-                    __builtin_amdgcn_sched_barrier(0);
+                    if (kk == 1 && i >= kBarrierRow && (WHOLE || s + NS < steps)) {
+                        constexpr int kRows = RB - kBarrierRow;
+#pragma unroll
+                        for (int q = (i - kBarrierRow) * T::kLoads / kRows; q < (i - kBarrierRow + 1) * T::kLoads / kRows; q++) request(s + NS, cur, q, WHOLE);
+                    }
+#pragma unroll
+                    for (int j = 0; j < CB; j++) {
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[kk][j], fa[kk & (kSets - 1)][i], acc[i][j], 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                 }
             }
             cur = nxt;
@@ -453,27 +473,24 @@ __device__ __forceinline__ void dense_body(const DenseParams& p, uint8_t* lds) {
         for (; s < steps; s++) step(s, std::false_type{});
     }
 
-    // acc[i][j][v]: row 32 (wm RB + i) + lane % 32, column 32 (wn CB + j) + 8 (v / 4) + 4 (lane / 32) + v % 4
+    // acc[i][j][v]: row 16 (wm RB + i) + lane % 16, column 16 (wn CB + j) + 4 (lane / 16) + v
     if constexpr (EPI == kDenseStore) {
         __syncthreads();  // every wave is done with the stages; the (surplus) operand reads have returned
-        uint8_t* stage = lds + wave * 32 * T::kOutPitch;
-        constexpr int kLanesPerRow = CB * 4, kRowsPerStore = 64 / kLanesPerRow;
-        const int cw = col0 + wn * CB * 32;
+        uint8_t* stage = lds + wave * 16 * T::kOutPitch;
+        constexpr int kLanesPerRow = CB * 2, kRowsPerStore = 64 / kLanesPerRow;
+        const int cw = col0 + wn * CB * 16;
         const bool whole = (p.ldc & 7) == 0 && (((uintptr_t)p.c) & 15) == 0;
 #pragma unroll
         for (int i = 0; i < RB; i++) {
 #pragma unroll
             for (int j = 0; j < CB; j++)
-#pragma unroll
-                for (int g = 0; g < 4; g++)
-                    *(uint2*)(stage + l32 * T::kOutPitch + j * 64 + g * 16 + half * 8) =
-                        make_uint2(pack_bf16(acc[i][j][4 * g], acc[i][j][4 * g + 1]), pack_bf16(acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]));
+                *(uint2*)(stage + l16 * T::kOutPitch + j * 32 + quarter * 8) = make_uint2(pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
             const int ch = lane % kLanesPerRow;
 #pragma unroll
-            for (int u = 0; u < 32 / kRowsPerStore; u++) {
+            for (int u = 0; u < 16 / kRowsPerStore; u++) {
                 const int rl = u * kRowsPerStore + lane / kLanesPerRow;
                 const uint4 piece = *(const uint4*)(stage + rl * T::kOutPitch + ch * 16);
-                const int row = (wm * RB + i) * 32 + rl, col = cw + ch * 8;
+                const int row = (wm * RB + i) * 16 + rl, col = cw + ch * 8;
                 if (row < rows_valid) {
                     bf16_t* dst = (bf16_t*)p.c + (int64_t)(row0 + row) * p.ldc + col;
                     if (whole && col + 8 <= p.cols) {
@@ -491,24 +508,22 @@ __device__ __forceinline__ void dense_body(const DenseParams& p, uint8_t* lds) {
         float* c = (float*)p.c + (EPI == kDensePartial ? (int64_t)split * p.split_stride : 0);
 #pragma unroll
         for (int i = 0; i < RB; i++) {
-            const int row = (wm * RB + i) * 32 + l32;
+            const int row = (wm * RB + i) * 16 + l16;
             if (row >= rows_valid) continue;
             const float rs = EPI == kDenseAccum && p.row_scale ? p.row_scale[row0 + row] : 1.0f;
             float* dst_row = c + (int64_t)(row0 + row) * p.ldc;
 #pragma unroll
-            for (int j = 0; j < CB; j++)
-#pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const int col = col0 + (wn * CB + j) * 32 + g * 8 + half * 4;
-                    if (col >= p.cols) continue;  // (fp32 outputs have a multiple of four columns)
-                    float4* dst = (float4*)(dst_row + col);
-                    float4 o = make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
-                    if (EPI == kDenseAccum) {
-                        const float4 old = *dst;
-                        o.x = fmaf(old.x, rs, o.x), o.y = fmaf(old.y, rs, o.y), o.z = fmaf(old.z, rs, o.z), o.w = fmaf(old.w, rs, o.w);
-                    }
-                    *dst = o;
+            for (int j = 0; j < CB; j++) {
+                const int col = col0 + (wn * CB + j) * 16 + quarter * 4;
+                if (col >= p.cols) continue;  // (fp32 outputs have a multiple of four columns)
+                float4* dst = (float4*)(dst_row + col);
+                float4 o = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+                if (EPI == kDenseAccum) {
+                    const float4 old = *dst;
+                    o.x = fmaf(old.x, rs, o.x), o.y = fmaf(old.y, rs, o.y), o.z = fmaf(old.z, rs, o.z), o.w = fmaf(old.w, rs, o.w);
                 }
+                *dst = o;
+            }
         }
     }
 }
@@ -569,9 +584,10 @@ static int launch_tile(const DenseParams& p, hipStream_t s) {
 template <int MODE, int EPI>
 static int launch_shape_mode(int shape, const DenseParams& p, hipStream_t s) {
     switch (shape) {
-        case 0: return launch_tile<MODE, 2, 4, 4, 2, 2, EPI>(p, s);   // 256 x 256
-        case 1: return launch_tile<MODE, 2, 2, 2, 2, 2, EPI>(p, s);   // 128 x 128, two workgroups per compute unit
-        case 2: return launch_tile<MODE, 2, 2, 1, 1, 4, EPI>(p, s);   // 64 x 64, two workgroups per compute unit
+        case 0: return launch_tile<MODE, 2, 4, 8, 4, 2, EPI>(p, s);   // 256 x 256
+        case 1: return launch_tile<MODE, 2, 2, 4, 4, 2, EPI>(p, s);   // 128 x 128, two workgroups per compute unit
+        case 2: return launch_tile<MODE, 2, 2, 2, 2, 4, EPI>(p, s);   // 64 x 64, two workgroups per compute unit
+        case 3: return launch_tile<MODE, 2, 4, 4, 4, 3, EPI>(p, s);   // 128 x 256
     }
     return set_error(GGQ_ERR_SHAPE, "dense_gemm: unknown tile shape");
 }
@@ -624,7 +640,7 @@ bool dense_side_takes(const DenseSide& side) {
 // Panels of at most this many bytes are decoded at a time: small enough to be read back out of the 256 MB memory-side cache,
 // large enough that a slab's launch fills the chip.  Larger matrices go in slabs of output columns.
 constexpr int64_t kPanelBytes = 128ll << 20;
-constexpr int kMaxSplits = 8;
+constexpr int kMaxSplits = 16;
 
 static int64_t slab_columns(int64_t cols, int64_t contraction) {
     const int64_t steps = (contraction + 63) / 64, fit = kPanelBytes / (steps * 128) / 256 * 256;
@@ -635,22 +651,30 @@ static int64_t slab_columns(int64_t cols, int64_t contraction) {
 // Whether both directions of an [n, k] matrix run over one panel of all of it.
 bool dense_panel_whole(int64_t n, int64_t k) { return slab_columns(n, k) >= n && slab_columns(k, n) >= k; }
 
-// Tile shape and number of contraction splits for an [m, cols] output: the smallest estimate of
-// rounds of workgroups x (steps x time per step + fixed cost), plus the pass that adds split partial sums.
+// Tile shape and number of contraction splits for an [m, cols] output: the smallest estimate of the launch, plus the pass that
+// adds split partial sums.  A tile's 64-wide step slows down with the share of the chip that is busy (clock and L2), by shape
+// from `idle` to `full` microseconds; measured at one tile, a quarter, a half and all of the slots, within 10 % of the estimate:
+//   256 x 256, one per compute unit:  1.07 / 1.08 / 1.13 / 1.40     128 x 256, one: 0.52 / 0.56 / 0.65 / 0.80
+//   128 x 128, two:                   0.33 / 0.45 / 0.60 / 0.90      64 x 64, two: 0.12 / 0.14 / 0.16 / 0.30
+// A larger tile reads less per output: 256 x 256 wins where it fills the chip in whole rounds or by splits (4096 x 8192 over
+// 2048: 119 us against 128 with 128 x 128), 128 x 256 where it would leave a half of it idle (4096 x 2048 over 8192: 113 us
+// against 154, and 122 with 128 x 128), the smaller ones for short sequences.
 static void pick_tile(int64_t m, int64_t cols, int64_t steps, bool can_split, int& shape, int& splits) {
-    // microseconds per 64-wide step with every slot of the chip busy, workgroups per chip, and cost of a tile's start and end
-    static const struct { double step, fixed; int slots; } kShape[3] = {{1.15, 6.0, 256}, {0.60, 4.0, 512}, {0.25, 3.0, 512}};
+    static const struct { int rows, cols, slots; double idle, full, fixed; } kShape[4] = {
+        {256, 256, 256, 1.05, 1.40, 6.0}, {128, 128, 512, 0.30, 0.90, 4.0}, {64, 64, 512, 0.08, 0.30, 2.5}, {128, 256, 256, 0.50, 0.80, 5.0}};  // (fixed: a tile's start and end)
     double best = 1e30;
     shape = 0, splits = 1;
-    for (int sh = 0; sh < 3; sh++) {
-        const int side = 256 >> sh;
-        const int64_t tiles = ((m + side - 1) / side) * ((cols + side - 1) / side);
-        for (int sp = 1; sp <= kMaxSplits; sp *= 2) {
-            if (sp > 1 && (!can_split || steps < 4 * sp)) break;
-            const double rounds = (double)((tiles * sp + kShape[sh].slots - 1) / kShape[sh].slots);
-            double t = rounds * (((steps + sp - 1) / sp) * kShape[sh].step + kShape[sh].fixed);
-            if (sp > 1) t += 3.0 + (double)m * cols * 4.0 * (2 * sp) / 4.5e6;
-            if (t < best) best = t, shape = sh, splits = sp;
+    for (int sh = 0; sh < 4; sh++) {
+        const auto& t = kShape[sh];
+        const int64_t tiles = ((m + t.rows - 1) / t.rows) * ((cols + t.cols - 1) / t.cols);
+        for (int sp = 1; sp <= (can_split ? kMaxSplits : 1); sp++) {
+            const int64_t per = (steps + sp - 1) / sp;
+            if (sp > 1 && (per < 4 || (sp - 1) * per >= steps)) continue;
+            const int64_t units = tiles * sp, rounds = units / t.slots, rest = units % t.slots;
+            const double load = (double)rest / t.slots, slow = sh == 0 ? load * load : load;
+            double est = 3.0 + rounds * (per * t.full + t.fixed) + (rest ? per * (t.idle + (t.full - t.idle) * slow) + t.fixed : 0.0);
+            if (sp > 1) est += 3.0 + (double)m * cols * 4.0 * (1.5 * sp) / 5e6;
+            if (est < best * 0.999) best = est, shape = sh, splits = sp;
         }
     }
 }
