@@ -232,9 +232,9 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
         return request_bytes<kPieceGap<QT>>(p.w + (int64_t)b * 16 * p.row_bytes, stage + buf * p.stage_bytes, p.head + min(16, p.n - b * 16) * p.row_bytes, wave, WAVES, lane);
     };
     // (the barriers here order LDS traffic only: __syncthreads would also wait for the block requested ahead)
-    if (block < blocks) request_block(block, 0);
-    stage_tables<QT>(gemv_lds, threadIdx.x, 64 * WAVES);
-
+    // With a LoRA term x and the first sixteen factor rows go out ahead of the packed bytes: requests complete in order, and
+    // x A^T is formed while the packed bytes are on their way.
+    if (!p.lora_a && block < blocks) request_block(block, 0);
     uint4 xf[SP][TB][4];
 #pragma unroll
     for (int sp = 0; sp < SP; sp++)
@@ -247,24 +247,34 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
                 xf[sp][tb][i] = e < p.k ? *(const uint4*)(src + e) : make_uint4(0, 0, 0, 0);  // (k is a multiple of 32: eight elements are whole or absent)
             }
         }
+    uint4 a[SP][4];
+    auto load_a = [&](int r0) __attribute__((always_inline)) {
+        const bf16_t* arow = p.lora_a + (int64_t)min(r0 + l16, p.r - 1) * p.k;
+#pragma unroll
+        for (int sp = 0; sp < SP; sp++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int e = (wave + WAVES * sp) * kSpan + span_element<QT>(q, i);
+                a[sp][i] = e < p.k && r0 + l16 < p.r ? *(const uint4*)(arow + e) : make_uint4(0, 0, 0, 0);
+            }
+    };
+    if (p.lora_a) {
+        load_a(0);
+        if (block < blocks) request_block(block, 0);
+    }
+    stage_tables<QT>(gemv_lds, threadIdx.x, 64 * WAVES);
     if (p.lora_a) {  // x A^T over this wave's spans, added over the waves, kept as bf16 rows in LDS
         for (int r0 = 0; r0 < p.r_pad; r0 += 16) {
             f32x4_t acc[TB];
 #pragma unroll
             for (int tb = 0; tb < TB; tb++) acc[tb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-            const bf16_t* arow = p.lora_a + (int64_t)min(r0 + l16, p.r - 1) * p.k;
+            if (r0 > 0) load_a(r0);
 #pragma unroll
             for (int sp = 0; sp < SP; sp++) {
-                uint4 a[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int e = (wave + WAVES * sp) * kSpan + span_element<QT>(q, i);
-                    a[i] = e < p.k && r0 + l16 < p.r ? *(const uint4*)(arow + e) : make_uint4(0, 0, 0, 0);
-                }
 #pragma unroll
                 for (int i = 0; i < 4; i++)
 #pragma unroll
-                    for (int tb = 0; tb < TB; tb++) acc[tb] = mfma16(as_operand(a[i]), as_operand(xf[sp][tb][i]), acc[tb]);
+                    for (int tb = 0; tb < TB; tb++) acc[tb] = mfma16(as_operand(a[sp][i]), as_operand(xf[sp][tb][i]), acc[tb]);
             }
 #pragma unroll
             for (int tb = 0; tb < TB; tb++) red[(wave * TB + tb) * 64 + lane] = acc[tb];
@@ -688,10 +698,11 @@ int router_logits(const void* x, const void* w, int64_t m, int64_t n, int64_t k,
 // Expert FFN of a few routes, without a routing plan: with a handful of routes hardly two share an expert, so every route
 // reads its own expert's weights and the four launches of plan and tables, the gather by expert and the combine's pass fall
 // away.  Two launches:
-//   act[route] = silu(gate) * up         one workgroup per (route, eight gate rows and the eight up rows of the same columns)
+//   act[route] = silu(gate) * up         one workgroup per (route, eight or sixteen gate rows and the up rows of the same columns)
 //   out[token] = sum w[route] * down     one workgroup per (token, sixteen output columns), one wave per route
 // The LoRA products x A^T are formed by every workgroup for itself (64 KB of factor out of the L2 at rank 16 and 2048
-// columns): cheaper than a launch.
+// columns): cheaper than a launch.  One token, 8 of 256 Q4_K experts, 2048 / 512: 7.6 and 9.6 us; with the factor rows read
+// as MFMA operands and eight gate rows per workgroup 10.4 and 11.3.
 struct FewRoutesParams {
     const bf16_t* x;       // [tokens, hidden]
     const void* ids;
@@ -704,6 +715,7 @@ struct FewRoutesParams {
     const bf16_t *a1, *b1, *a2, *b2;
     int r1, r2;
     float scale, limit;
+    int x_in_lds;          // down: room for 512 elements of x per wave
     bf16_t* act;           // [routes, inter]
     bf16_t* out;           // [tokens, hidden]
 };
@@ -727,91 +739,115 @@ __device__ __forceinline__ float lora_row_dot(const uint4& first, const bf16_t* 
     return s + __shfl_xor(s, 32, 64);
 }
 
-__host__ __device__ __forceinline__ int gate_up_half_lds(int qt, int row_bytes) {
-    const int bytes = 8 * row_bytes;
-    return qt == kQ4_K ? (bytes + (bytes >> 10) * kPieceGap<kQ4_K> + 127) & ~127 : bytes;
+// x . row for a row of k bf16 values, eight of every 512 per lane (x as loaded by load_row_pieces); the sum over the lanes is the caller's.
+template <int PIECES>
+__device__ __forceinline__ void load_row_pieces(const bf16_t* row, int k, int lane, uint4 (&v)[PIECES]) {
+#pragma unroll
+    for (int t = 0; t < PIECES; t++) {
+        const int e = 512 * t + 8 * lane;
+        v[t] = e < k ? *(const uint4*)(row + e) : make_uint4(0, 0, 0, 0);
+    }
 }
-template <int QT, int SP>
+__device__ __forceinline__ float dot8(const uint4& a, const uint4& b, float s) {
+    const uint32_t aw[4] = {a.x, a.y, a.z, a.w}, bw[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) s = fmaf(bf16_lo(aw[i]), bf16_lo(bw[i]), s), s = fmaf(bf16_hi(aw[i]), bf16_hi(bw[i]), s);
+    return s;
+}
+__device__ __forceinline__ float wave_sum(float s) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) s += __shfl_xor(s, off, 64);
+    return s;
+}
+
+// Eight gate rows and eight up rows per set; a workgroup takes SETS sets of one route.  What bounds it is latency and the
+// vector cache's requests: every workgroup forms x A^T for itself, and as MFMA operands (16 rows x 64 bytes a request) the 64 KB
+// of A cost two workgroups of a compute unit 2.3 us.  So each wave takes whole rows of A (1 KB a request, half the time, under
+// the weights' latency), x comes to LDS once, and two sets share one x A^T where that leaves enough workgroups.
+__host__ __device__ __forceinline__ int gate_up_half_lds(int qt, int row_bytes, int sets) {
+    const int bytes = 8 * sets * row_bytes;
+    return qt == kQ4_K ? (bytes + (bytes >> 10) * kPieceGap<kQ4_K> + 127) & ~127 : (bytes + 15) & ~15;
+}
+template <int QT, int SP, int SETS>
 __global__ __launch_bounds__(512) void few_routes_gate_up_kernel(FewRoutesParams p) {
-    constexpr int WAVES = 8;
+    constexpr int WAVES = 8, PIECES = SP * 2;  // 512-element pieces of x: k <= 1024 SP
     extern __shared__ __attribute__((aligned(16))) uint8_t gu_lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, q = lane >> 4;
-    const int half_bytes = 8 * p.row_bytes_in, half_lds = gate_up_half_lds(QT, p.row_bytes_in);
+    const int half_bytes = 8 * SETS * p.row_bytes_in, half_lds = gate_up_half_lds(QT, p.row_bytes_in, SETS);
     uint8_t* stage = gu_lds + kTableBytes<QT>;
-    float* red = (float*)(stage + 2 * half_lds);   // [WAVES][16]
-    float* red_xa = red + WAVES * 16;                // [WAVES][64]
-    bf16_t* xa = (bf16_t*)(red_xa + WAVES * 64);     // [64]
-    const int route = blockIdx.y, i0 = blockIdx.x * 8, k = p.hidden;
+    bf16_t* xs = (bf16_t*)(stage + 2 * half_lds);     // [512 PIECES]
+    float* red = (float*)(xs + 512 * PIECES);         // [SETS][WAVES][16]
+    bf16_t* xa = (bf16_t*)(red + SETS * WAVES * 16);  // [64]
+    const int route = blockIdx.y, i0 = blockIdx.x * 8 * SETS, k = p.hidden;
+    const bf16_t* x = p.x + (int64_t)(route / p.top_k) * k;
+    uint4 xr[PIECES];
+    load_row_pieces(x, k, lane, xr);
     const int expert = route_expert(p, route);
     const int64_t row0 = (int64_t)expert * p.inter + i0;
     request_bytes<kPieceGap<QT>>(p.gate + row0 * p.row_bytes_in, stage, half_bytes, wave, WAVES, lane);
     request_bytes<kPieceGap<QT>>(p.up + row0 * p.row_bytes_in, stage + half_lds, half_bytes, (wave + 4) & 7, WAVES, lane);
     stage_tables<QT>(gu_lds, threadIdx.x, 512);
-    const bf16_t* x = p.x + (int64_t)(route / p.top_k) * k;
-    uint4 xf[SP][4];
-#pragma unroll
-    for (int sp = 0; sp < SP; sp++) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int e = (wave + WAVES * sp) * kSpan + span_element<QT>(q, i);
-            xf[sp][i] = e < k ? *(const uint4*)(x + e) : make_uint4(0, 0, 0, 0);
-        }
-    }
     const int r_pad = (p.r1 + 15) & ~15;
     const bool b_vec = (p.r1 & 7) == 0;
-    const bf16_t* brow = p.b1 + ((int64_t)expert * 2 * p.inter + (l16 < 8 ? i0 + l16 : p.inter + i0 + l16 - 8)) * p.r1;
+    // the wave that finishes set `wave`: its row of B ahead of the work it would wait behind
+    const int own_row = (l16 < 8 ? i0 + l16 : p.inter + i0 + l16 - 8) + 8 * wave;
+    const bf16_t* brow = p.b1 + ((int64_t)expert * 2 * p.inter + own_row) * p.r1;
     uint4 b0 = make_uint4(0, 0, 0, 0);
-    if (p.a1 && wave == 0) b0 = load_factor8(brow + 8 * q, p.r1 - 8 * q, b_vec);
+    if (p.a1 && wave < SETS) b0 = load_factor8(brow + 8 * q, p.r1 - 8 * q, b_vec);
     if (p.a1) {
         const bf16_t* a = p.a1 + (int64_t)expert * p.r1 * k;
-        for (int r0 = 0; r0 < r_pad; r0 += 16) {
-            f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-            const bf16_t* arow = a + (int64_t)min(r0 + l16, p.r1 - 1) * k;
+        for (int j0 = wave; j0 < r_pad; j0 += 2 * WAVES) {  // ranks j0 and j0 + 8 together
+            uint4 a0[PIECES], a8[PIECES];
+            load_row_pieces(a + (int64_t)min(j0, p.r1 - 1) * k, k, lane, a0);
+            load_row_pieces(a + (int64_t)min(j0 + WAVES, p.r1 - 1) * k, k, lane, a8);
+            float s0 = 0.f, s8 = 0.f;
 #pragma unroll
-            for (int sp = 0; sp < SP; sp++) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int e = (wave + WAVES * sp) * kSpan + span_element<QT>(q, i);
-                    acc = mfma16(as_operand(e < k && r0 + l16 < p.r1 ? *(const uint4*)(arow + e) : make_uint4(0, 0, 0, 0)), as_operand(xf[sp][i]), acc);
-                }
-            }
-            if (l16 == 0) *(f32x4_t*)(red_xa + wave * 64 + r0 + 4 * q) = acc;
+            for (int t = 0; t < PIECES; t++) s0 = dot8(a0[t], xr[t], s0), s8 = dot8(a8[t], xr[t], s8);
+            s0 = wave_sum(s0), s8 = wave_sum(s8);
+            if (lane == 0) xa[j0] = j0 < p.r1 ? to_bf16(s0) : (bf16_t)0, xa[j0 + WAVES] = j0 + WAVES < p.r1 ? to_bf16(s8) : (bf16_t)0;
         }
     }
+#pragma unroll
+    for (int t = 0; t < PIECES; t++)
+        if (wave == t % WAVES) *(uint4*)(xs + 512 * t + 8 * lane) = xr[t];
     wait_loads_at_most(0);
     __syncthreads();
-    f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     const uint8_t* half = stage + (l16 < 8 ? 0 : half_lds);  // rows 0..7 gate, 8..15 up
-    const int row = (l16 & 7) * p.row_bytes_in;
     const int spans = (k + kSpan - 1) / kSpan;
+    f32x4_t acc[SETS];
+#pragma unroll
+    for (int b = 0; b < SETS; b++) acc[b] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int sp = 0; sp < SP; sp++) {
         const int span = wave + WAVES * sp;
         if (span >= spans) break;
-        uint32_t v[16];
-        decode_span<QT>(half, row, span, k >> 5, q, v, (const uint2*)gu_lds);
+        uint4 xf[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) acc = mfma16(as_operand(make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3])), as_operand(xf[sp][i]), acc);
+        for (int i = 0; i < 4; i++) xf[i] = *(const uint4*)(xs + span * kSpan + span_element<QT>(q, i));  // (zeros past k)
+#pragma unroll
+        for (int b = 0; b < SETS; b++) {
+            uint32_t v[16];
+            decode_span<QT>(half, (8 * b + (l16 & 7)) * p.row_bytes_in, span, k >> 5, q, v, (const uint2*)gu_lds);
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[b] = mfma16(as_operand(make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3])), as_operand(xf[i]), acc[b]);
+        }
     }
-    if (l16 == 0) *(f32x4_t*)(red + wave * 16 + 4 * q) = acc;
-    if (p.a1 && wave == 0) {  // (red_xa is complete since the barrier above)
-        float s = 0.f;
-        if (lane < r_pad)
-            for (int w = 0; w < WAVES; w++) s += red_xa[w * 64 + lane];
-        xa[lane] = lane < r_pad ? to_bf16(s) : (bf16_t)0;
-    }
+#pragma unroll
+    for (int b = 0; b < SETS; b++)
+        if (l16 == 0) *(f32x4_t*)(red + (b * WAVES + wave) * 16 + 4 * q) = acc[b];
     __syncthreads();
-    if (wave > 0) return;
-    float y = 0.f;  // of row l16, in all four quarters
-    for (int w = 0; w < WAVES; w++) y += red[w * 16 + l16];
+    if (wave >= SETS) return;
+    float y = 0.f;  // of row l16 of set `wave`, in all four quarters
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) y += red[(wave * WAVES + w) * 16 + l16];
     if (p.a1) y = fmaf(p.scale, lora_row_dot(b0, brow, xa, p.r1, b_vec, q), y);
     y = bf16_to_f32(to_bf16(y));
     const float up = __shfl(y, (lane & 7) + 8, 64), gate = __shfl(y, lane & 7, 64);
     if (lane < 8) {
         const float hi = p.limit > 0.0f ? p.limit : INFINITY;
         const float g = fminf(gate, hi), u = fminf(fmaxf(up, -hi), hi);
-        p.act[(int64_t)route * p.inter + i0 + lane] = to_bf16(g / (1.0f + __expf(-g)) * u);
+        p.act[(int64_t)route * p.inter + i0 + 8 * wave + lane] = to_bf16(g / (1.0f + __expf(-g)) * u);
     }
 }
 
@@ -824,12 +860,15 @@ __global__ __launch_bounds__(512) void few_routes_down_kernel(FewRoutesParams p)
     uint8_t* mine = down_lds + kTableBytes<QT> + wave * stage_bytes;
     float* red = (float*)(down_lds + kTableBytes<QT> + 8 * stage_bytes);  // [16 routes][16]
     bf16_t* xa = (bf16_t*)(red + 256) + wave * 64;
+    bf16_t* xs = (bf16_t*)(red + 256) + 8 * 64 + wave * 512;  // this wave's 512 elements of x (where the LDS has room for them)
     const int token = blockIdx.y, h0 = blockIdx.x * 16, k = p.inter, spans = (k + kSpan - 1) / kSpan;
     const int rows = min(16, p.hidden - h0);
     stage_tables<QT>(down_lds, threadIdx.x, 512);
     if (kTableBytes<QT>) __syncthreads();
     for (int rank = wave; rank < p.top_k; rank += 8) {
         const int route = token * p.top_k + rank, expert = route_expert(p, route);
+        // (ahead of the work: behind the last barrier its latency would be the workgroup's)
+        const float weight = p.weights_bf16 ? bf16_to_f32(((const bf16_t*)p.weights)[route]) : ((const float*)p.weights)[route];
         // this wave's own sixteen rows: no other wave touches them, so no barrier stands between their requests and their use
         request_bytes<kPieceGap<QT>>(p.down + ((int64_t)expert * p.hidden + h0) * p.row_bytes_down, mine, rows * p.row_bytes_down, 0, 1, lane);
         const bf16_t* x = p.act + (int64_t)route * k;
@@ -838,33 +877,44 @@ __global__ __launch_bounds__(512) void few_routes_down_kernel(FewRoutesParams p)
         const bf16_t* brow = p.b2 + ((int64_t)expert * p.hidden + min(h0 + l16, p.hidden - 1)) * p.r2;
         uint4 b0 = make_uint4(0, 0, 0, 0);
         if (a) b0 = load_factor8(brow + 8 * q, p.r2 - 8 * q, b_vec);
-        f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f}, acc_a[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc_a[j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        float part[4] = {0.f, 0.f, 0.f, 0.f};  // x A^T of rank 16 j + lane / 4, of a sixteenth of the elements
         const int row = min(l16, rows - 1) * p.row_bytes_down;
-        for (int s0 = 0; s0 < spans; s0 += 4) {  // four spans of x in registers at a time, requested together
+        for (int s0 = 0; s0 < spans; s0 += 4) {  // 512 elements of x at a time
+            uint4 xr[1];
+            load_row_pieces(x + s0 * kSpan, k - s0 * kSpan, lane, xr);
+            if (a) {
+                // Sixteen ranks at a time, whole rows of A (1 KB a request: as MFMA operands, 16 rows x 64 bytes, a request cost
+                // the vector cache twice that): each lane has eight terms of every rank, and four exchanges leave each with one rank.
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if (16 * j >= p.r2) break;
+                    float d[16];
+#pragma unroll
+                    for (int h = 0; h < 16; h++) {
+                        uint4 av[1];
+                        load_row_pieces(a + (int64_t)min(16 * j + h, p.r2 - 1) * k + s0 * kSpan, k - s0 * kSpan, lane, av);
+                        d[h] = dot8(av[0], xr[0], 0.f);
+                    }
+#pragma unroll
+                    for (int n = 8, bit = 32; n >= 1; n >>= 1, bit >>= 1)
+#pragma unroll
+                        for (int h = 0; h < n; h++) {
+                            const float give = (lane & bit) ? d[h] : d[h + n], keep = (lane & bit) ? d[h + n] : d[h];
+                            d[h] = keep + __shfl_xor(give, bit, 64);
+                        }
+                    part[j] += d[0];  // of rank 16 j + lane / 4, summed over all lanes but the low two bits
+                }
+            }
+            if (p.x_in_lds) *(uint4*)(xs + 8 * lane) = xr[0];
             uint4 xf[4][4];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const int e = (s0 + u) * kSpan + span_element<QT>(q, i);
-                    xf[u][i] = e < k ? *(const uint4*)(x + e) : make_uint4(0, 0, 0, 0);
-                }
-            }
-            if (a) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    if (16 * j >= p.r2) break;
-                    const bf16_t* arow = a + (int64_t)min(16 * j + l16, p.r2 - 1) * k;
-#pragma unroll
-                    for (int u = 0; u < 4; u++) {
-#pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            const int e = (s0 + u) * kSpan + span_element<QT>(q, i);
-                            acc_a[j] = mfma16(as_operand(e < k && 16 * j + l16 < p.r2 ? *(const uint4*)(arow + e) : make_uint4(0, 0, 0, 0)), as_operand(xf[u][i]), acc_a[j]);
-                        }
-                    }
+                    const int e = u * kSpan + span_element<QT>(q, i);
+                    if (p.x_in_lds) xf[u][i] = *(const uint4*)(xs + e);  // (LDS serves a wave in order)
+                    else xf[u][i] = s0 * kSpan + e < k ? *(const uint4*)(x + s0 * kSpan + e) : make_uint4(0, 0, 0, 0);
                 }
             }
             if (s0 == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -877,52 +927,58 @@ __global__ __launch_bounds__(512) void few_routes_down_kernel(FewRoutesParams p)
                 for (int i = 0; i < 4; i++) acc = mfma16(as_operand(make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3])), as_operand(xf[u][i]), acc);
             }
         }
-        if (a && l16 == 0) {
+        if (a) {
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                if (16 * j < p.r2) *(uint2*)(xa + 16 * j + 4 * q) = make_uint2(pack_bf16(acc_a[j][0], acc_a[j][1]), pack_bf16(acc_a[j][2], acc_a[j][3]));
+            for (int j = 0; j < 4; j++) {
+                if (16 * j >= p.r2) break;
+                float t = part[j] + __shfl_xor(part[j], 1, 64);
+                t += __shfl_xor(t, 2, 64);
+                const int rank_a = 16 * j + (lane >> 2);
+                if ((lane & 3) == 0) xa[rank_a] = rank_a < p.r2 ? to_bf16(t) : (bf16_t)0;
+            }
         }
         if (l16 == 0) *(f32x4_t*)(red + rank * 16 + 4 * q) = acc;
-        if (p.a2) {
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            const float dot = lora_row_dot(b0, brow, xa, p.r2, b_vec, q);
-            if (q == 0) red[rank * 16 + l16] = fmaf(p.scale, dot, red[rank * 16 + l16]);
-        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        float y = red[rank * 16 + l16];
+        if (p.a2) y = fmaf(p.scale, lora_row_dot(b0, brow, xa, p.r2, b_vec, q), y);
+        // (weights and rows act at bf16 precision: their product is exact)
+        if (q == 0) red[rank * 16 + l16] = bf16_to_f32(to_bf16(y)) * bf16_to_f32(to_bf16(weight));
     }
     __syncthreads();
-    if ((int)threadIdx.x < rows) {  // the combine: routes in rank order, weights and rows at bf16 precision
+    if ((int)threadIdx.x < rows) {  // the combine: routes in rank order
         float sum = 0.f;
-        for (int rank = 0; rank < p.top_k; rank++) {
-            const int64_t route = (int64_t)token * p.top_k + rank;
-            const float w = p.weights_bf16 ? bf16_to_f32(((const bf16_t*)p.weights)[route]) : bf16_to_f32(to_bf16(((const float*)p.weights)[route]));
-            sum = fmaf(bf16_to_f32(to_bf16(red[rank * 16 + threadIdx.x])), w, sum);
-        }
+        for (int rank = 0; rank < p.top_k; rank++) sum += red[rank * 16 + threadIdx.x];
         p.out[(int64_t)token * p.hidden + h0 + threadIdx.x] = to_bf16(sum);
     }
 }
 
-static int gate_up_lds(int qt, int row_bytes) { return (qt == kIQ2_XXS ? kTableBytes<kIQ2_XXS> : 0) + 2 * gate_up_half_lds(qt, row_bytes) + 8 * 16 * 4 + 8 * 64 * 4 + 128; }
+static int gate_up_lds(int qt, int row_bytes, int64_t hidden, int sets) {
+    return (qt == kIQ2_XXS ? kTableBytes<kIQ2_XXS> : 0) + 2 * gate_up_half_lds(qt, row_bytes, sets) + (hidden <= 2048 ? 4096 : 8192) + sets * 8 * 16 * 4 + 128;
+}
 static int down_lds_bytes(int qt, int row_bytes) { return (qt == kIQ2_XXS ? kTableBytes<kIQ2_XXS> : 0) + 8 * row_block_bytes(qt, 16 * row_bytes) + 256 * 4 + 8 * 128; }
 
+template <int QT, int SP, int SETS>
+static int launch_gate_up_sets(const FewRoutesParams& p, hipStream_t s) {
+    static LdsLimit lim;
+    if (int rc = raise_lds_limit(lim, (const void*)few_routes_gate_up_kernel<QT, SP, SETS>, 160 * 1024, "few_routes_gate_up")) return rc;
+    hipLaunchKernelGGL((few_routes_gate_up_kernel<QT, SP, SETS>), dim3(p.inter / (8 * SETS), p.tokens * p.top_k), dim3(512), gate_up_lds(QT, p.row_bytes_in, p.hidden, SETS), s, p);
+    return check_launch("few_routes_gate_up");
+}
 template <int QT>
 static int launch_gate_up(const FewRoutesParams& p, hipStream_t s) {
-    const int lds = gate_up_lds(QT, p.row_bytes_in);
-    static LdsLimit lim2, lim4;
-    const dim3 grid(p.inter / 8, p.tokens * p.top_k);
-    if (p.hidden <= 2048) {
-        if (int rc = raise_lds_limit(lim2, (const void*)few_routes_gate_up_kernel<QT, 2>, 160 * 1024, "few_routes_gate_up")) return rc;
-        hipLaunchKernelGGL((few_routes_gate_up_kernel<QT, 2>), grid, dim3(512), lds, s, p);
-    } else {
-        if (int rc = raise_lds_limit(lim4, (const void*)few_routes_gate_up_kernel<QT, 4>, 160 * 1024, "few_routes_gate_up")) return rc;
-        hipLaunchKernelGGL((few_routes_gate_up_kernel<QT, 4>), grid, dim3(512), lds, s, p);
-    }
-    return check_launch("few_routes_gate_up");
+    // two sets where every compute unit still has a workgroup, and two workgroups of a unit fit its LDS
+    const bool two = p.inter % 16 == 0 && (int64_t)p.tokens * p.top_k * p.inter / 16 >= 256 && gate_up_lds(QT, p.row_bytes_in, p.hidden, 2) <= 80 * 1024;
+    if (p.hidden <= 2048) return two ? launch_gate_up_sets<QT, 2, 2>(p, s) : launch_gate_up_sets<QT, 2, 1>(p, s);
+    return two ? launch_gate_up_sets<QT, 4, 2>(p, s) : launch_gate_up_sets<QT, 4, 1>(p, s);
 }
 template <int QT>
 static int launch_down(const FewRoutesParams& p, hipStream_t s) {
     static LdsLimit lim;
     if (int rc = raise_lds_limit(lim, (const void*)few_routes_down_kernel<QT>, 160 * 1024, "few_routes_down")) return rc;
-    hipLaunchKernelGGL(few_routes_down_kernel<QT>, dim3((p.hidden + 15) / 16, p.tokens), dim3(512), down_lds_bytes(QT, p.row_bytes_down), s, p);
+    FewRoutesParams q = p;
+    const int lds = down_lds_bytes(QT, p.row_bytes_down);
+    q.x_in_lds = lds + 8 * 1024 <= 160 * 1024;
+    hipLaunchKernelGGL(few_routes_down_kernel<QT>, dim3((p.hidden + 15) / 16, p.tokens), dim3(512), lds + (q.x_in_lds ? 8 * 1024 : 0), s, q);
     return check_launch("few_routes_down");
 }
 
@@ -934,7 +990,7 @@ static int64_t few_routes_limit(int qt_in, int qt_down) { return qt_in == kIQ2_X
 
 bool few_routes_takes(int qt_in, int qt_down, int64_t tokens, int top_k, int64_t hidden, int64_t inter) {
     return tokens > 0 && top_k > 0 && top_k <= 16 && tokens * top_k <= few_routes_limit(qt_in, qt_down) && hidden <= 4096 && inter % 8 == 0 && hidden % 8 == 0 &&
-           gate_up_lds(qt_in, (int)packed_row_bytes(qt_in, hidden)) <= 80 * 1024 && down_lds_bytes(qt_down, (int)packed_row_bytes(qt_down, inter)) <= 160 * 1024;
+           gate_up_lds(qt_in, (int)packed_row_bytes(qt_in, hidden), hidden, 1) <= 88 * 1024 && down_lds_bytes(qt_down, (int)packed_row_bytes(qt_down, inter)) <= 160 * 1024;
 }
 
 int few_routes_forward(const void* x, const void* ids, int ids64, const void* weights, int weights_bf16, int64_t tokens, int top_k, int64_t experts, int64_t hidden,
