@@ -59,6 +59,7 @@ struct FactorGradParams {
     float* partials;      // null: no splitting
     int64_t partials_bytes;
     int row_splits;
+    int blocks_outer;     // order of the units: column blocks outer, experts inner (set by factor_grad)
 };
 
 constexpr int kBM = 256, kBN = 128, kBK = 64;  // the tall tile shape (dense launches, large expert groups)
