@@ -109,9 +109,11 @@ constexpr bool kByPosition = QT == kQ2_K || QT == kQ4_K || QT == kQ6_K;
 template <int QT>
 __device__ __forceinline__ int span_element(int q, int i) { return kByPosition<QT> ? 32 * i + 8 * q : 32 * q + 8 * i; }
 
-// Four small integers in the bytes of w (below 256) -> four bf16 of value scale * integer + offset.
+// Four small integers in the bytes of w (the bits of MASK) -> four bf16 of value scale * integer + offset.
+template <uint32_t MASK = 0x00FF00FFu>
 __device__ __forceinline__ void four_values(uint32_t w, float scale24, float offset, uint32_t* out) {
-    const uint32_t e02 = w & 0x00FF00FFu, e13 = (w >> 8) & 0x00FF00FFu;
+    // (opaque: taken apart by bytes instead, the two words would be three)
+    const uint32_t e02 = opaque(w & MASK), e13 = opaque((w >> 8) & MASK);
     out[0] = pack_bf16(mix_lo(e02, scale24, offset), mix_lo(e13, scale24, offset));
     out[1] = pack_bf16(mix_hi(e02, scale24, offset), mix_hi(e13, scale24, offset));
 }
@@ -161,9 +163,11 @@ __device__ __forceinline__ void decode_span(const uint8_t* lds, int row, int spa
             const float s24 = s * kMixScale, off = -32.0f * s;
 #pragma unroll
             for (int u = 0; u < 2; u++) {
-                const uint32_t nib = i == 0 ? a[u] & 0x0F0F0F0Fu : i == 1 ? b[u] & 0x0F0F0F0Fu : i == 2 ? (a[u] >> 4) & 0x0F0F0F0Fu : (b[u] >> 4) & 0x0F0F0F0Fu;
+                // low four bits of a byte from one word, the next two from the other (one v_bfi_b32); what is left above them
+                // falls to the masks below
+                const uint32_t nib = i == 0 ? a[u] : i == 1 ? b[u] : i == 2 ? a[u] >> 4 : b[u] >> 4;
                 const uint32_t two = i == 0 ? c[u] << 4 : i == 1 ? c[u] << 2 : i == 2 ? c[u] : c[u] >> 2;
-                four_values(nib | (two & 0x30303030u), s24, off, v + 4 * i + 2 * u);
+                four_values<0x003F003Fu>((nib & 0x0F0F0F0Fu) | (two & 0xF0F0F0F0u), s24, off, v + 4 * i + 2 * u);
             }
         }
     } else if constexpr (QT == kQ2_K) {
@@ -218,7 +222,9 @@ struct GemvParams {
 };
 
 // WAVES waves deal the spans of the contraction out (span s to wave s % WAVES, at most SP each); TB blocks of sixteen rows of x.
-template <int QT, int WAVES, int SP, int TB>  // TB <= WAVES
+// LORA is a template parameter because a load the compiler tracks may stand nowhere in the block loop of a plain product: on
+// whatever path, it makes every iteration wait for all requests, the block requested ahead among them.
+template <int QT, int WAVES, int SP, int TB, bool LORA>  // TB <= WAVES
 __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t gemv_lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -234,7 +240,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
     // (the barriers here order LDS traffic only: __syncthreads would also wait for the block requested ahead)
     // With a LoRA term x and the first sixteen factor rows go out ahead of the packed bytes: requests complete in order, and
     // x A^T is formed while the packed bytes are on their way.
-    if (!p.lora_a && block < blocks) request_block(block, 0);
+    if (!LORA && block < blocks) request_block(block, 0);
     uint4 xf[SP][TB][4];
 #pragma unroll
     for (int sp = 0; sp < SP; sp++)
@@ -258,12 +264,12 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
                 a[sp][i] = e < p.k && r0 + l16 < p.r ? *(const uint4*)(arow + e) : make_uint4(0, 0, 0, 0);
             }
     };
-    if (p.lora_a) {
+    if constexpr (LORA) {
         load_a(0);
         if (block < blocks) request_block(block, 0);
     }
     stage_tables<QT>(gemv_lds, threadIdx.x, 64 * WAVES);
-    if (p.lora_a) {  // x A^T over this wave's spans, added over the waves, kept as bf16 rows in LDS
+    if constexpr (LORA) {  // x A^T over this wave's spans, added over the waves, kept as bf16 rows in LDS
         for (int r0 = 0; r0 < p.r_pad; r0 += 16) {
             f32x4_t acc[TB];
 #pragma unroll
@@ -301,7 +307,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
         const bool adds = (wave + block) % WAVES < TB;
         const bf16_t* brow = p.lora_b + (int64_t)min(block * 16 + l16, p.n - 1) * p.r;
         uint4 b0 = make_uint4(0, 0, 0, 0);
-        if (p.lora_a && adds) b0 = load_factor8(brow + 8 * q, p.r - 8 * q, b_vec);
+        if (LORA && adds) b0 = load_factor8(brow + 8 * q, p.r - 8 * q, b_vec);
         f32x4_t acc[TB];
 #pragma unroll
         for (int tb = 0; tb < TB; tb++) acc[tb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
@@ -327,7 +333,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
             f32x4_t sum = red[tb * 64 + lane];
             for (int w = 1; w < WAVES; w++) sum += red[(w * TB + tb) * 64 + lane];
             const int col = block * 16 + 4 * q, xrow = tb * 16 + l16;
-            if (p.lora_a) {
+            if constexpr (LORA) {
                 f32x4_t lo = (f32x4_t){0.f, 0.f, 0.f, 0.f};
                 for (int r0 = 0; r0 < p.r_pad; r0 += 32) {
                     const int j = r0 + 8 * q;
@@ -352,25 +358,34 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
     }
 }
 
-template <int QT, int WAVES, int SP, int TB>
+// One row block of up to 2048 elements without a LoRA term: three workgroups per compute unit with one LDS buffer each, instead of
+// two with two.  A block's way through its workgroup (requests, decoding, two barriers) is longer than the memory's, and three
+// independent ones hide more of it than a request ahead does: 151936 x 2048 Q6_K, one row, 66.5 -> 58.0 us; Q8_0 109 -> 103.  (A
+// fourth needs 64 registers and spills: 67 us.  Sixteen waves on one block: 88 us with two to five buffers.)
+static bool many_small_workgroups(bool lora, int64_t m, int64_t k) { return !lora && m <= 16 && k <= 2048; }
+template <int QT, int WAVES, int SP, int TB, bool LORA>
 static int launch_gemv(const GemvParams& p, hipStream_t s) {
     const int lds = kTableBytes<QT> + p.buffers * p.stage_bytes + WAVES * TB * 64 * 16 + TB * 16 * 64 * 2;
     static LdsLimit lim;
-    if (int rc = raise_lds_limit(lim, (const void*)gemv_kernel<QT, WAVES, SP, TB>, 160 * 1024, "gemv")) return rc;
-    const int per_cu = std::max(1, std::min(160 * 1024 / lds, 16 / WAVES));
-    hipLaunchKernelGGL((gemv_kernel<QT, WAVES, SP, TB>), dim3(std::min((p.n + 15) / 16, 256 * per_cu)), dim3(64 * WAVES), lds, s, p);
+    if (int rc = raise_lds_limit(lim, (const void*)gemv_kernel<QT, WAVES, SP, TB, LORA>, 160 * 1024, "gemv")) return rc;
+    const int per_cu = std::max(1, std::min(160 * 1024 / lds, (many_small_workgroups(LORA, p.m, p.k) ? 24 : 16) / WAVES));
+    hipLaunchKernelGGL((gemv_kernel<QT, WAVES, SP, TB, LORA>), dim3(std::min((p.n + 15) / 16, 256 * per_cu)), dim3(64 * WAVES), lds, s, p);
     return check_launch("gemv");
 }
-template <int QT>
+template <int QT, bool LORA>
 static int launch_gemv_qt(const GemvParams& p, hipStream_t s) {
     const int tb = (p.m + 15) / 16;
     if (p.k <= 2048) {
-        if (tb == 1) return launch_gemv<QT, 8, 2, 1>(p, s);
-        if (tb == 2) return launch_gemv<QT, 8, 2, 2>(p, s);
-        return launch_gemv<QT, 8, 2, 4>(p, s);
+        if (tb == 1) return launch_gemv<QT, 8, 2, 1, LORA>(p, s);
+        if (tb == 2) return launch_gemv<QT, 8, 2, 2, LORA>(p, s);
+        return launch_gemv<QT, 8, 2, 4, LORA>(p, s);
     }
-    if (p.k <= 4096) return tb == 1 ? launch_gemv<QT, 8, 4, 1>(p, s) : launch_gemv<QT, 8, 4, 2>(p, s);
-    return launch_gemv<QT, 16, 4, 1>(p, s);
+    if (p.k <= 4096) return tb == 1 ? launch_gemv<QT, 8, 4, 1, LORA>(p, s) : launch_gemv<QT, 8, 4, 2, LORA>(p, s);
+    return launch_gemv<QT, 16, 4, 1, LORA>(p, s);
+}
+template <int QT>
+static int launch_gemv_qt(const GemvParams& p, hipStream_t s) {
+    return p.lora_a ? launch_gemv_qt<QT, true>(p, s) : launch_gemv_qt<QT, false>(p, s);
 }
 
 // Rows up to which x fits the registers of the waves that share it: 64 of 2048 elements, 32 of 4096, 16 of 8192.
@@ -391,7 +406,7 @@ int gemv(int qt, const void* x, int64_t ldx, const void* w, int64_t m, int64_t n
     p.ldx = ldx, p.ldy = ldy;
     if (lora_a) p.lora_a = (const bf16_t*)lora_a, p.lora_b = (const bf16_t*)lora_b, p.r = r, p.r_pad = (r + 15) / 16 * 16, p.lora_scale = scale, p.xa_out = (bf16_t*)xa_out;
     p.stage_bytes = row_block_bytes(qt, p.head + 16 * p.row_bytes);
-    p.buffers = (p.n + 15) / 16 > 256 && p.stage_bytes <= 36 * 1024 ? 2 : 1;  // (one block per workgroup needs one buffer)
+    p.buffers = (p.n + 15) / 16 > 256 && p.stage_bytes <= 36 * 1024 && !many_small_workgroups(lora_a != nullptr, m, k) ? 2 : 1;  // (one block per workgroup needs one buffer)
     TimedScope timed(qt, kModeNT, kEpiStore, kShapeFewRows, s);
     switch (qt) {
         case kQ8_0: return launch_gemv_qt<kQ8_0>(p, s);
