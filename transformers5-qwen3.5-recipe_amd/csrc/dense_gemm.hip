@@ -245,7 +245,7 @@ struct DenseTile {
     static constexpr int kStageA = kBM * 128, kStage = (kBM + kBN) * 128;
     static constexpr int kLdsBytes = NS * kStage;
     static constexpr int kOutPitch = CB * 32 + 16;  // bytes of a staged output row
-    static_assert(kWaves * 16 * kOutPitch <= kLdsBytes, "output staging");
+    static_assert(kWaves * 32 * kOutPitch <= kLdsBytes, "output staging");
 };
 
 __device__ __forceinline__ void wait_loads(int n) {  // at most n of this wave's requests outstanding (n known at compile time after inlining)
@@ -388,13 +388,17 @@ __device__ __forceinline__ void dense_body(const DenseParams& p, uint8_t* lds) {
 #pragma unroll
         for (int kk = 0; kk < 2; kk++)
 #pragma unroll
-            for (int j = 0; j < CB; j++)
+            for (int t = 0; t < 2; t++) {
+                // chunk (2 j + x) ^ swizzle of the row: j only meets the swizzle's upper two bits, so a block's offset is the
+                // first one's with two address bits flipped
+                const int row = 8 * (2 * quarter + kk) + 4 * t + (l16 >> 2), sw = panel_swizzle(row) ^ ((l16 & 3) >> 1);
+                const uint32_t first = (uint32_t)T::kStageA + (uint32_t)row * 128u + (uint32_t)sw * 16u + (uint32_t)(l16 & 1) * 8u;
 #pragma unroll
-                for (int t = 0; t < 2; t++) {
-                    const int col = (wn * CB + j) * 16 + 4 * (l16 & 3), row = 8 * (2 * quarter + kk) + 4 * t + (l16 >> 2);
-                    rb[kk][2 * j + t] = (uint32_t)T::kStageA + (uint32_t)(col >> 6) * 8192u + (uint32_t)row * 128u +
-                                        (uint32_t)(((col & 63) >> 3) ^ panel_swizzle(row)) * 16u + (uint32_t)(l16 & 1) * 8u;
+                for (int j = 0; j < CB; j++) {
+                    const int col = (wn * CB + j) * 16;
+                    rb[kk][2 * j + t] = (first ^ (uint32_t)((col & 63) * 2)) + (uint32_t)(col >> 6) * 8192u;
                 }
+            }
     }
     constexpr int kSets = RB <= 4 ? 2 : 1;  // row operand sets
     bf16x8_t fa[kSets][RB], fb[2][CB];
@@ -476,18 +480,21 @@ __device__ __forceinline__ void dense_body(const DenseParams& p, uint8_t* lds) {
     // acc[i][j][v]: row 16 (wm RB + i) + lane % 16, column 16 (wn CB + j) + 4 (lane / 16) + v
     if constexpr (EPI == kDenseStore) {
         __syncthreads();  // every wave is done with the stages; the (surplus) operand reads have returned
-        uint8_t* stage = lds + wave * 16 * T::kOutPitch;
+        uint8_t* stage = lds + wave * 32 * T::kOutPitch;
         constexpr int kLanesPerRow = CB * 2, kRowsPerStore = 64 / kLanesPerRow;
         const int cw = col0 + wn * CB * 16;
         const bool whole = (p.ldc & 7) == 0 && (((uintptr_t)p.c) & 15) == 0;
 #pragma unroll
-        for (int i = 0; i < RB; i++) {
+        for (int i = 0; i < RB; i += 2) {  // 32 rows at a time
 #pragma unroll
-            for (int j = 0; j < CB; j++)
-                *(uint2*)(stage + l16 * T::kOutPitch + j * 32 + quarter * 8) = make_uint2(pack_bf16(acc[i][j][0], acc[i][j][1]), pack_bf16(acc[i][j][2], acc[i][j][3]));
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int j = 0; j < CB; j++)
+                    *(uint2*)(stage + (16 * h + l16) * T::kOutPitch + j * 32 + quarter * 8) =
+                        make_uint2(pack_bf16(acc[i + h][j][0], acc[i + h][j][1]), pack_bf16(acc[i + h][j][2], acc[i + h][j][3]));
             const int ch = lane % kLanesPerRow;
 #pragma unroll
-            for (int u = 0; u < 16 / kRowsPerStore; u++) {
+            for (int u = 0; u < 32 / kRowsPerStore; u++) {
                 const int rl = u * kRowsPerStore + lane / kLanesPerRow;
                 const uint4 piece = *(const uint4*)(stage + rl * T::kOutPitch + ch * 16);
                 const int row = (wm * RB + i) * 16 + rl, col = cw + ch * 8;
@@ -655,13 +662,13 @@ bool dense_panel_whole(int64_t n, int64_t k) { return slab_columns(n, k) >= n &&
 // adds split partial sums.  A tile's 64-wide step slows down with the share of the chip that is busy (clock and L2), by shape
 // from `idle` to `full` microseconds; measured at one tile, a quarter, a half and all of the slots, within 10 % of the estimate:
 //   256 x 256, one per compute unit:  1.07 / 1.08 / 1.13 / 1.40     128 x 256, one: 0.52 / 0.56 / 0.65 / 0.80
-//   128 x 128, two:                   0.33 / 0.45 / 0.60 / 0.90      64 x 64, two: 0.12 / 0.14 / 0.16 / 0.30
+//   128 x 128, two:                   0.37 / 0.55 / 0.62 / 0.90      64 x 64, two: 0.12 / 0.14 / 0.16 / 0.30
 // A larger tile reads less per output: 256 x 256 wins where it fills the chip in whole rounds or by splits (4096 x 8192 over
 // 2048: 119 us against 128 with 128 x 128), 128 x 256 where it would leave a half of it idle (4096 x 2048 over 8192: 113 us
 // against 154, and 122 with 128 x 128), the smaller ones for short sequences.
 static void pick_tile(int64_t m, int64_t cols, int64_t steps, bool can_split, int& shape, int& splits) {
     static const struct { int rows, cols, slots; double idle, full, fixed; } kShape[4] = {
-        {256, 256, 256, 1.05, 1.40, 6.0}, {128, 128, 512, 0.30, 0.90, 4.0}, {64, 64, 512, 0.08, 0.30, 2.5}, {128, 256, 256, 0.50, 0.80, 5.0}};  // (fixed: a tile's start and end)
+        {256, 256, 256, 1.05, 1.40, 6.0}, {128, 128, 512, 0.36, 0.90, 2.5}, {64, 64, 512, 0.11, 0.30, 2.5}, {128, 256, 256, 0.50, 0.80, 5.0}};  // (fixed: a tile's start and end)
     double best = 1e30;
     shape = 0, splits = 1;
     for (int sh = 0; sh < 4; sh++) {
