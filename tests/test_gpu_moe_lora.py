@@ -90,6 +90,50 @@ def test_q4k_grouped_grad_input_decoding_waves(pkg, dev):
     assert_close_bf16(dx_single, want_g["dx"], "single dX")
 
 
+@pytest.mark.parametrize("sizes,n,r,pair", [
+    ([1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 0, 97, 5, 2], 256, 16, True),  # every count of 16-row blocks, groups walked in two and three parts
+    ([1, 40, 16, 0, 3], 256, 0, False),
+    ([20, 7, 48, 33], 128, 4, True),      # four 64-row steps, the fewest; a rank padded to 16
+    ([9, 33, 50], 320 + 64, 40, False),   # a rank padded to 48: a half-filled second factor step
+])
+def test_q4k_grad_input_of_few_rows_per_group(pkg, dev, sizes, n, r, pair):
+    # the grad-input kernel that keeps decoded weights out of LDS: k = 512 * 8, so that 64 groups give it the workgroups it asks for
+    ml = pkg.fast_moe_lora
+    qt, k, groups, planes, s = gb.Q4_K, 4096, 64, 4, 2.0
+    sizes = (sizes * groups)[:groups]
+    assert sum(sizes) <= 40 * groups
+    ids, ends, rows = torch.arange(groups, dtype=torch.int64), torch.tensor(np.cumsum(sizes), dtype=torch.int32), sum(sizes)
+    gen = torch.Generator().manual_seed(97 + n + r)
+    p1, p2 = _expert_payload(700, qt, planes, n, k), _expert_payload(750, qt, planes, n, k)
+    w = torch.cat([ref.weights_bf16(p1, qt), ref.weights_bf16(p2, qt)], dim=1) if pair else ref.weights_bf16(p1, qt)
+    which = torch.arange(groups) % planes
+    p1, p2 = (torch.from_numpy(p)[which].contiguous().to(dev) for p in (p1, p2))
+    nt = w.shape[1]
+    dy, x = bf16_randn(gen, rows, nt), bf16_randn(gen, rows, k)
+    e_d, o_d = _to(dev, ids, ends)
+    parts = [dy[:, i * n : (i + 1) * n].contiguous().to(dev) for i in range(nt // n)]
+    if r:
+        a, b = bf16_randn(gen, groups, r, k, std=k ** -0.5), bf16_randn(gen, groups, nt, r, std=0.02)
+        xd, ad, bd = (t.to(dev).requires_grad_(True) for t in (x, a, b))
+        if pair:
+            out = ml.grouped_lora_mmq_pair(xd, p1, p2, e_d, o_d, qt, n, ad, bd, s)
+        else:
+            out = (ml.grouped_lora_mmq(xd, p1, e_d, o_d, qt, n, ad, bd, s),)
+        torch.autograd.backward(out, parts)
+        got = xd.grad
+    else:
+        got = ml.grouped_mmq_grad_input(parts[0], p1, e_d, o_d, qt, k)
+    begin = 0
+    for g, size in enumerate(sizes):
+        d = dy[begin : begin + size].float()
+        want = d @ w[g % planes].float()
+        if r:
+            want += s * (d @ b[g].float()).bfloat16().float() @ a[g].float()
+        if size:
+            assert_close_bf16(got[begin : begin + size], want, f"dX of group {g} of {size} rows")
+        begin += size
+
+
 def test_constant_byte_iq2_xxs_experts(pkg, dev):
     # test_deepseek_v4_moe_lora.py:55-118: payload of all bytes 32, experts [0,1], offsets [3,7]
     ml = pkg.fast_moe_lora

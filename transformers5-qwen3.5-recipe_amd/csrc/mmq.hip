@@ -2,6 +2,7 @@
 #include "mmq_tile.h"
 #include "mmq_direct8.h"
 #include "mmq_direct8_nn.h"
+#include "mmq_small_nn.h"
 #include "mmq_small_iq2.h"
 #include "launch.h"
 
@@ -127,8 +128,11 @@ template <int MODE>
 static int launch_direct(const MmqParams& p, hipStream_t s) {
     const int col_tiles = (MODE == kModeNT ? p.nseg : 1) * p.col_tiles_per_seg;
     if (p.col_tiles_per_wg < 1) return set_error(GGQ_ERR_SHAPE, "mmq: column tiles per workgroup must be at least 1");
+    const bool few_rows = MODE == kModeNN && p.few_rows;  // 512 columns per workgroup
+    if (few_rows && (p.k & 511)) return set_error(GGQ_ERR_SHAPE, "mmq: the grad-input kernel for few rows needs whole pairs of blocks");
     // row tiles are dealt round-robin over the eight XCDs; each XCD walks its row tiles' column-tile runs
-    const int64_t total = (int64_t)((p.max_row_tiles + 7) / 8) * ((col_tiles + p.col_tiles_per_wg - 1) / p.col_tiles_per_wg);
+    const int per_wg = few_rows ? 2 : p.col_tiles_per_wg;
+    const int64_t total = (int64_t)((p.max_row_tiles + 7) / 8) * ((col_tiles + per_wg - 1) / per_wg);
     if (total <= 0) return GGQ_OK;
     const int64_t grid = total * 8;
     if (grid > 0x7FFFFFF0) return set_error(GGQ_ERR_SHAPE, "mmq: too many tiles for one launch");
@@ -141,6 +145,11 @@ static int launch_direct(const MmqParams& p, hipStream_t s) {
         t->qt = kQ4_K, t->mode = MODE, t->epi = kEpiStore, t->shape = kShapeDirect;
         g_timed_count++;
         (void)hipEventRecord(t->start, s);
+    }
+    if (few_rows) {  // (its 40 KB need no raised limit)
+        hipLaunchKernelGGL(mmq_small_nn_q4k_kernel, dim3((unsigned)grid), dim3(SmallNN::kThreadsWG), SmallNN::kLdsBytes, s, p);
+        if (t) (void)hipEventRecord(t->stop, s);
+        return check_launch("mmq_small_nn_q4k_kernel");
     }
     constexpr int kSmemBytes = MODE == kModeNT ? Direct8::kLdsBytes : Direct8NN::kLdsBytes;
     const void* fn = MODE == kModeNT ? (const void*)mmq_direct8_q4k_kernel : (const void*)mmq_direct8_nn_q4k_kernel;

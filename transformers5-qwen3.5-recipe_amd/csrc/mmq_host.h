@@ -103,6 +103,7 @@ struct MmqParams {
     int max_row_tiles2;
     int col_tiles_per_seg2;
     int col_tiles_per_wg;   // direct shape: column tiles one workgroup walks through (>= 1)
+    int few_rows;           // direct shape, NN: the groups average few rows (mmq_small_nn.h)
     int shape;  // kShapeTall / kShapeWide / kShapeDirect: which kernel the sizes above are for
     // LoRA
     const bf16_t* la;     // [rows, r_pad]  (x A^T in NT, dY B in NN)
