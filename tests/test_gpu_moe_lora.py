@@ -90,18 +90,21 @@ def test_q4k_grouped_grad_input_decoding_waves(pkg, dev):
     assert_close_bf16(dx_single, want_g["dx"], "single dX")
 
 
-@pytest.mark.parametrize("sizes,n,r,pair", [
-    ([1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 0, 97, 5, 2], 256, 16, True),  # every count of 16-row blocks, groups walked in two and three parts
-    ([1, 40, 16, 0, 3], 256, 0, False),
-    ([20, 7, 48, 33], 128, 4, True),      # four 64-row steps, the fewest; a rank padded to 16
-    ([9, 33, 50], 320 + 64, 40, False),   # a rank padded to 48: a half-filled second factor step
+@pytest.mark.parametrize("qt,sizes,n,r,pair", [
+    (gb.Q4_K, [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 0, 97, 5, 2], 256, 16, True),  # every count of 16-row blocks, groups walked in two and three parts
+    (gb.Q4_K, [1, 40, 16, 0, 3], 256, 0, False),
+    (gb.Q4_K, [20, 7, 48, 33], 128, 4, True),      # four 64-row steps, the fewest; a rank padded to 16
+    (gb.Q4_K, [9, 33, 50], 320 + 64, 40, False),   # a rank padded to 48: a half-filled second factor step
+    (gb.IQ2_XXS, [1, 15, 16, 17, 33, 48, 49, 64, 65, 80, 81, 128, 129, 0, 2], 128, 16, True),  # ... groups walked in two parts, a tall tile
+    (gb.IQ2_XXS, [3, 0, 79, 64], 128, 0, False),   # one group of four steps
+    (gb.IQ2_XXS, [70, 9, 96], 384, 40, False),
 ])
-def test_q4k_grad_input_of_few_rows_per_group(pkg, dev, sizes, n, r, pair):
-    # the grad-input kernel that keeps decoded weights out of LDS: k = 512 * 8, so that 64 groups give it the workgroups it asks for
+def test_grad_input_of_few_rows_per_group(pkg, dev, qt, sizes, n, r, pair):
+    # the grad-input kernels that keep decoded weights out of LDS: k = 512 * 8, so that 64 groups give them the workgroups they ask for
     ml = pkg.fast_moe_lora
-    qt, k, groups, planes, s = gb.Q4_K, 4096, 64, 4, 2.0
+    k, groups, planes, s = 4096, 64, 4, 2.0
     sizes = (sizes * groups)[:groups]
-    assert sum(sizes) <= 40 * groups
+    assert sum(sizes) <= (40 if qt == gb.Q4_K else 72) * groups
     ids, ends, rows = torch.arange(groups, dtype=torch.int64), torch.tensor(np.cumsum(sizes), dtype=torch.int32), sum(sizes)
     gen = torch.Generator().manual_seed(97 + n + r)
     p1, p2 = _expert_payload(700, qt, planes, n, k), _expert_payload(750, qt, planes, n, k)

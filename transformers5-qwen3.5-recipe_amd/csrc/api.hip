@@ -202,6 +202,14 @@ static bool grad_input_of_few_rows(int64_t rows, int64_t groups, int64_t k) {
     return k % 512 == 0 && rows <= 40 * groups && groups * (k / 512) >= 512;
 }
 
+// IQ2_XXS, grad-input: groups that average at most 72 rows take the kernel that keeps decoded weights out of LDS (its tiles have 80
+// rows; a group with more decodes the weights again, 1490 us against the tile kernel's 1140 if all have), where its 512-column
+// tiles give every compute unit two workgroups.  256 experts, 4096 / 2048, 2048 tokens, top-8 (64 rows): gate / up and down
+// together 1680 -> 1420 us, the training step of that layer 3390 -> 3080.
+static bool iq2_grad_input_of_few_rows(int64_t rows, int64_t groups, int64_t n, int64_t k) {
+    return k % 512 == 0 && n % 128 == 0 && n < (1 << 22) && k < (1 << 22) && rows <= 72 * groups && groups * (k / 512) >= 512;
+}
+
 // Small shape: a workgroup stages the decoder's tables and its row tile's LoRA rows once, so it walks up to four column
 // tiles while that still leaves every compute unit eight workgroups.
 static int small_tiles_per_wg(int64_t groups, int col_tiles) {
@@ -611,6 +619,8 @@ static int grouped_backward(const char* what, const void* dy1, const void* dy2, 
     TileDesc* t_tall = nullptr;
     const int* n_tall = nullptr;
     int max_tall = 0;
+    TileDesc* t_small = nullptr;
+    const int* n_small = nullptr;
     if (groups > 0 && group_tables && p.shape == kShapeDirect) {  // tables the caller built once for this grouping
         GroupTablesView v;
         group_tables_layout(const_cast<void*>(group_tables), rows, groups, experts, v);
@@ -628,16 +638,22 @@ static int grouped_backward(const char* what, const void* dy1, const void* dy2, 
         TileDesc* t_sorted = direct ? (TileDesc*)bump.take((int64_t)max128 * sizeof(TileDesc)) : nullptr;
         t_tall = wide ? (TileDesc*)bump.take((int64_t)max_tall * sizeof(TileDesc)) : nullptr;
         TileDesc* t64 = lora_a ? (TileDesc*)bump.take((int64_t)max_tiles64 * sizeof(TileDesc)) : nullptr;
+        // IQ2_XXS, small groups: the groups of at most 128 rows leave the wide table for a launch of their own
+        const bool small = wide && qt == 16 /* GGML IQ2_XXS */ && iq2_grad_input_of_few_rows(rows, groups, n, k) && aligned16(dy1) && (!dy2 || aligned16(dy2)) &&
+                           (!lora_a || (aligned16(lora_a) && aligned16(ws))) && g_shape_override.load() != kShapeWide;
+        t_small = small ? (TileDesc*)bump.take((int64_t)groups * sizeof(TileDesc)) : nullptr;
+        TileDesc* t_small_sorted = small ? (TileDesc*)bump.take((int64_t)groups * sizeof(TileDesc)) : nullptr;  // most row blocks first
         int* counts = (int*)bump.take(16);
         int* rg = lora_a ? (int*)bump.take(experts * 2 * 4) : nullptr;
-        if (!t128 || !counts || (lora_a && (!t64 || !rg)) || (wide && !t_tall) || (direct && !t_sorted)) return set_error(GGQ_ERR_WORKSPACE, "%s: workspace too small", what);
+        if (!t128 || !counts || (lora_a && (!t64 || !rg)) || (wide && !t_tall) || (direct && !t_sorted) || (small && (!t_small || !t_small_sorted))) return set_error(GGQ_ERR_WORKSPACE, "%s: workspace too small", what);
         RowTileTables tb{};
-        tb.add(bm_main, 0, wide ? kWideBM : 0x7FFFFFFF, t128, counts, t_sorted);
+        tb.add(bm_main, small ? kSmallBM : 0, wide ? kWideBM : 0x7FFFFFFF, t128, counts, t_sorted);
         if (direct) t128 = t_sorted;
         if (wide) tb.add(kBM, kWideBM, 0x7FFFFFFF, t_tall, counts + 2), n_tall = counts + 2;
         if (lora_a) tb.add(64, 0, 0x7FFFFFFF, t64, counts + 1);
+        if (small) tb.add(kSmallBM, 0, kSmallBM, t_small, counts + 3, t_small_sorted), n_small = counts + 3, t_small = t_small_sorted;
         if (int rc = build_row_tile_tables(expert_ids, end_offsets, (int)groups, tb, rg, (int)experts, s)) return rc;
-        p.expert_ids = expert_ids, p.tiles = t128, p.num_tiles = counts, p.max_row_tiles = max128;
+        p.expert_ids = expert_ids, p.tiles = t128, p.num_tiles = counts, p.max_row_tiles = small ? 0 : max128;  // (small: the wide table stays empty)
         tiles64 = t64, num_tiles64 = counts + 1, ranges = rg;
     }
     if (lora_a) {
@@ -670,6 +686,11 @@ static int grouped_backward(const char* what, const void* dy1, const void* dy2, 
             if (lora_a) q.la = p.la, q.lb = p.lb, q.r_pad = rp, q.rank = r, q.lora_scale = scale;
             const int64_t need = dense_workspace_bytes(rows, n, k);
             if (void* panels = ws && aligned16(ws) ? bump.take(need) : nullptr) return dense_mmq(q, panels, need, s);
+        }
+        if (t_small) {
+            MmqParams ps = p;
+            ps.tiles = t_small, ps.num_tiles = n_small, ps.max_row_tiles = (int)groups;
+            if (int rc = launch_mmq_small_nn(ps, s)) return rc;
         }
         if (t_tall) return launch_wide_and_tall(qt, kModeNN, p, (int)rows, (int)n, (int)k, nseg, t_tall, n_tall, max_tall, s);
         return launch_mmq(qt, kModeNN, kEpiStore, p, s);

@@ -4,6 +4,7 @@
 #include "mmq_direct8_nn.h"
 #include "mmq_small_nn.h"
 #include "mmq_small_iq2.h"
+#include "mmq_small_nn_iq2.h"
 #include "launch.h"
 
 #include <stdarg.h>
@@ -210,6 +211,20 @@ int launch_mmq_small(const MmqParams& p, hipStream_t s) {
     hipLaunchKernelGGL(mmq_small_iq2xxs_kernel, dim3((unsigned)grid), dim3(SmallIq2::kThreadsWG), SmallIq2::kLdsBytes, s, p);
     if (t) (void)hipEventRecord(t->stop, s);
     return check_launch("mmq_small_iq2xxs_kernel");
+}
+
+// IQ2_XXS, grad-input, store epilogue: entries of up to kSmallBM rows (p.tiles).
+int launch_mmq_small_nn(const MmqParams& p, hipStream_t s) {
+    if ((p.k & 511) || (p.n & 127)) return set_error(GGQ_ERR_SHAPE, "mmq: the small-group grad-input kernel needs whole pairs of blocks and a contraction of whole groups of 128 rows");
+    // row tiles are dealt round-robin over the eight XCDs; the column tiles of a row tile follow one another
+    const int64_t grid = (int64_t)((p.max_row_tiles + 7) / 8) * (p.k / SmallNNIq2::kCols) * 8;
+    if (grid <= 0) return GGQ_OK;
+    if (grid > 0x7FFFFFF0) return set_error(GGQ_ERR_SHAPE, "mmq: too many tiles for one launch");
+    TimedScope timed(kIQ2_XXS, kModeNN, kEpiStore, kShapeSmall, s);
+    static LdsLimit lds_limit;
+    if (int rc = raise_lds_limit(lds_limit, (const void*)mmq_small_nn_iq2xxs_kernel, SmallNNIq2::kLdsBytes, "mmq")) return rc;
+    hipLaunchKernelGGL(mmq_small_nn_iq2xxs_kernel, dim3((unsigned)grid), dim3(SmallNNIq2::kThreadsWG), SmallNNIq2::kLdsBytes, s, p);
+    return check_launch("mmq_small_nn_iq2xxs_kernel");
 }
 
 int launch_mmq_mixed(int qt, int mode, const MmqParams& p, hipStream_t s) {

@@ -123,6 +123,7 @@ const char* last_error();
 int launch_mmq(int qt, int mode, int epi, const MmqParams& p, hipStream_t s);
 int launch_mmq_mixed(int qt, int mode, const MmqParams& p, hipStream_t s);  // Q4_K, store epilogue, tiles + tiles2
 int launch_mmq_small(const MmqParams& p, hipStream_t s);  // IQ2_XXS forward, store epilogue, tiles of kSmallBM rows
+int launch_mmq_small_nn(const MmqParams& p, hipStream_t s);  // its grad-input
 int init_params(MmqParams& p, int qt, int mode, int m, int n, int k, int nseg, int shape = kShapeTall);
 
 // Event pair around the launches of its lifetime, when launches are being timed (profile_begin).
