@@ -21,7 +21,7 @@
 // k 4096: 595 / 714 / 804 / 910 us at 16 / 48 / 64 / 80 rows per expert, against 853 / 986 / 1000 / 1132 of the tile kernel; 4096
 // rows of W, k 2048: 323 / 391 / 445 / 490 against 426 / 513 / 539 / 582.  Groups of more than 80 rows decode the weights again.
 #pragma once
-#include "mmq_direct.h"
+#include "mmq_small_iq2.h"
 
 namespace ggq {
 
@@ -44,24 +44,6 @@ struct SmallNNIq2 {
     template <class T>
     static __device__ __forceinline__ __attribute__((address_space(3))) T* lds(uint32_t address) {
         return (__attribute__((address_space(3))) T*)(uintptr_t)address;
-    }
-    // Bitwise functions and doublings as instructions of full rate (a left shift and v_and_or take twice as long)
-    static __device__ __forceinline__ uint32_t flip_signs(uint32_t x, uint32_t flips) {  // x ^ (flips & 0x80008000)
-        uint32_t o;
-        asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0x78" : "=v"(o) : "v"(x), "v"(flips), "s"(0x80008000u));
-        return o;
-    }
-    static __device__ __forceinline__ uint32_t twice(uint32_t x) {
-        uint32_t o;
-        asm("v_add_u32 %0, %1, %1" : "=v"(o) : "v"(x));
-        return o;
-    }
-    // Signs of the eight weights of a group: pair j's at bits 15 and 31 after j doublings (the eighth is the parity of the other seven)
-    static __device__ __forceinline__ uint32_t sign_word(uint32_t s7) {
-        const uint32_t s = s7 | ((uint32_t)(__builtin_popcount(s7) & 1) << 7);
-        uint32_t w = 0;
-        for (int j = 0; j < 4; j++) w |= ((s >> (2 * j)) & 1u) << (15 - j) | ((s >> (2 * j + 1)) & 1u) << (31 - j);
-        return w;
     }
     // load16_to_lds of the first LANES lanes (the whole wave is active around it)
     template <int LANES>
@@ -220,11 +202,11 @@ struct SmallNNIq2 {
                     uint32_t f0 = flips[b][0], f1 = flips[b][1];
 #pragma unroll
                     for (int c = 0; c < 4; c++) {  // two rows of one column side by side
-                        const uint32_t w0 = flip_signs(__builtin_amdgcn_perm(hi[b][0], lo[b][0], sel[b][0][c]), f0);
-                        const uint32_t w1 = flip_signs(__builtin_amdgcn_perm(hi[b][1], lo[b][1], sel[b][1][c]), f1);
+                        const uint32_t w0 = Iq2Signs::flip(__builtin_amdgcn_perm(hi[b][0], lo[b][0], sel[b][0][c]), f0);
+                        const uint32_t w1 = Iq2Signs::flip(__builtin_amdgcn_perm(hi[b][1], lo[b][1], sel[b][1][c]), f1);
                         o[2 * c][i2] = __builtin_amdgcn_perm(w1, w0, 0x05040100u);
                         o[2 * c + 1][i2] = __builtin_amdgcn_perm(w1, w0, 0x07060302u);
-                        if (c < 3) f0 = twice(f0), f1 = twice(f1);
+                        if (c < 3) f0 = Iq2Signs::twice(f0), f1 = Iq2Signs::twice(f1);
                     }
                     if (i2 == 1) write_records((S + 2) & 3);  // of the step after the next
                     __builtin_amdgcn_sched_barrier(0);
@@ -320,7 +302,7 @@ struct SmallNNIq2 {
         const int slot = (int)(blockIdx.x >> 3);
         const int row_tile = (slot / chunks) * 8 + (int)(blockIdx.x & 7), col_block = 2 * (slot % chunks);
         if (row_tile >= row_tiles) return;
-        for (int i = threadIdx.x; i < 1024 + 128; i += kThreadsWG) *lds<uint32_t>(4 * i) = i < 1024 ? Fmt<kIQ2_XXS>::table_word(i, d_iq2xxs_grid_mm[i >> 2]) : sign_word(i - 1024);
+        for (int i = threadIdx.x; i < 1024 + 128; i += kThreadsWG) *lds<uint32_t>(4 * i) = i < 1024 ? Fmt<kIQ2_XXS>::table_word(i, d_iq2xxs_grid_mm[i >> 2]) : Iq2Signs::word(i - 1024);
         const TileDesc t = p.tiles[row_tile];
         const int all = t.row_end - t.row_begin, parts = (all + kRows - 1) / kRows;
         if (parts <= 0) return;
