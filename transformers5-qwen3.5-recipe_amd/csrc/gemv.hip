@@ -239,8 +239,13 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
     };
     // (the barriers here order LDS traffic only: __syncthreads would also wait for the block requested ahead)
     // With a LoRA term x and the first sixteen factor rows go out ahead of the packed bytes: requests complete in order, and
-    // x A^T is formed while the packed bytes are on their way.
-    if (!LORA && block < blocks) request_block(block, 0);
+    // x A^T is formed while the packed bytes are on their way.  (Where the factor rows of all spans leave the kernel its 128
+    // registers, two workgroups per compute unit: else they come span by span.  At 4096 elements 165 registers, and 13.9 -> 16.6 us
+    // for one row and 5120 columns of Q6_K.)
+    constexpr bool kAhead = LORA && SP * TB <= 2;
+    // (a factor is always there with LORA; asked at run time, the compiler keeps to the 128 registers)
+    const bool lora = kAhead || (LORA && p.lora_a);
+    if (!kAhead && block < blocks) request_block(block, 0);
     uint4 xf[SP][TB][4];
 #pragma unroll
     for (int sp = 0; sp < SP; sp++)
@@ -253,34 +258,38 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
                 xf[sp][tb][i] = e < p.k ? *(const uint4*)(src + e) : make_uint4(0, 0, 0, 0);  // (k is a multiple of 32: eight elements are whole or absent)
             }
         }
-    uint4 a[SP][4];
-    auto load_a = [&](int r0) __attribute__((always_inline)) {
+    uint4 a[kAhead ? SP : 1][4];
+    auto load_a = [&](int r0, int sp, uint4* out) __attribute__((always_inline)) {
         const bf16_t* arow = p.lora_a + (int64_t)min(r0 + l16, p.r - 1) * p.k;
 #pragma unroll
-        for (int sp = 0; sp < SP; sp++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int e = (wave + WAVES * sp) * kSpan + span_element<QT>(q, i);
-                a[sp][i] = e < p.k && r0 + l16 < p.r ? *(const uint4*)(arow + e) : make_uint4(0, 0, 0, 0);
-            }
+        for (int i = 0; i < 4; i++) {
+            const int e = (wave + WAVES * sp) * kSpan + span_element<QT>(q, i);
+            out[i] = e < p.k && r0 + l16 < p.r ? *(const uint4*)(arow + e) : make_uint4(0, 0, 0, 0);
+        }
     };
-    if constexpr (LORA) {
-        load_a(0);
+    if constexpr (kAhead) {
+#pragma unroll
+        for (int sp = 0; sp < SP; sp++) load_a(0, sp, a[sp]);
         if (block < blocks) request_block(block, 0);
     }
     stage_tables<QT>(gemv_lds, threadIdx.x, 64 * WAVES);
-    if constexpr (LORA) {  // x A^T over this wave's spans, added over the waves, kept as bf16 rows in LDS
+    if (lora) {  // x A^T over this wave's spans, added over the waves, kept as bf16 rows in LDS
         for (int r0 = 0; r0 < p.r_pad; r0 += 16) {
             f32x4_t acc[TB];
 #pragma unroll
             for (int tb = 0; tb < TB; tb++) acc[tb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-            if (r0 > 0) load_a(r0);
+            if (kAhead && r0 > 0) {
+#pragma unroll
+                for (int sp = 0; sp < SP; sp++) load_a(r0, sp, a[sp]);
+            }
 #pragma unroll
             for (int sp = 0; sp < SP; sp++) {
+                uint4* const as = a[kAhead ? sp : 0];
+                if (!kAhead) load_a(r0, sp, as);
 #pragma unroll
                 for (int i = 0; i < 4; i++)
 #pragma unroll
-                    for (int tb = 0; tb < TB; tb++) acc[tb] = mfma16(as_operand(a[sp][i]), as_operand(xf[sp][tb][i]), acc[tb]);
+                    for (int tb = 0; tb < TB; tb++) acc[tb] = mfma16(as_operand(as[i]), as_operand(xf[sp][tb][i]), acc[tb]);
             }
 #pragma unroll
             for (int tb = 0; tb < TB; tb++) red[(wave * TB + tb) * 64 + lane] = acc[tb];
@@ -307,7 +316,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
         const bool adds = (wave + block) % WAVES < TB;
         const bf16_t* brow = p.lora_b + (int64_t)min(block * 16 + l16, p.n - 1) * p.r;
         uint4 b0 = make_uint4(0, 0, 0, 0);
-        if (LORA && adds) b0 = load_factor8(brow + 8 * q, p.r - 8 * q, b_vec);
+        if (lora && adds) b0 = load_factor8(brow + 8 * q, p.r - 8 * q, b_vec);
         f32x4_t acc[TB];
 #pragma unroll
         for (int tb = 0; tb < TB; tb++) acc[tb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
@@ -333,7 +342,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
             f32x4_t sum = red[tb * 64 + lane];
             for (int w = 1; w < WAVES; w++) sum += red[(w * TB + tb) * 64 + lane];
             const int col = block * 16 + 4 * q, xrow = tb * 16 + l16;
-            if constexpr (LORA) {
+            if (lora) {
                 f32x4_t lo = (f32x4_t){0.f, 0.f, 0.f, 0.f};
                 for (int r0 = 0; r0 < p.r_pad; r0 += 32) {
                     const int j = r0 + 8 * q;
