@@ -40,7 +40,7 @@ def kernel_name(qt: int, mode: int, epi: int, shape: int) -> str:
     if shape == 4:
         return f"mmq_mixed_kernel<{_TYPE_NAMES.get(qt, qt)}, {direction}, store>"
     if shape == 5:
-        return "mmq_small_iq2xxs_kernel (IQ2_XXS, forward)"
+        return "mmq_small_iq2xxs_kernel (IQ2_XXS, forward)" if mode == 0 else f"mmq_small_nn_{'q4k' if qt == 12 else 'iq2xxs'}_kernel ({_TYPE_NAMES.get(qt, qt)}, grad_input)"
     if shape == 6:  # (the record spans the call's decoding pass, with the rank-sized work in it, and its matmul)
         return f"decode_panel + dense_gemm_kernel<{_TYPE_NAMES.get(qt, qt)}, {direction}, {'store' if epi == 0 else 'accumulate_f32'}>"
     if shape == 7:

@@ -143,7 +143,7 @@ static int launch_direct(const MmqParams& p, hipStream_t s) {
     if (g_timing && g_timed_count < kMaxTimedLaunches) {
         t = &g_timed[g_timed_count];
         if (hipEventCreate(&t->start) != hipSuccess || hipEventCreate(&t->stop) != hipSuccess) return set_error(GGQ_ERR_RUNTIME, "mmq: event creation failed");
-        t->qt = kQ4_K, t->mode = MODE, t->epi = kEpiStore, t->shape = kShapeDirect;
+        t->qt = kQ4_K, t->mode = MODE, t->epi = kEpiStore, t->shape = few_rows ? kShapeSmall : kShapeDirect;
         g_timed_count++;
         (void)hipEventRecord(t->start, s);
     }
