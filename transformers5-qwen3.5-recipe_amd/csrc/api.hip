@@ -197,9 +197,11 @@ static int direct_tiles_per_wg(int64_t rows, int64_t groups, int col_tiles, int 
 
 // Direct shape, grad-input: groups that average at most 40 rows take the kernel that keeps decoded weights out of LDS (groups of
 // more than its 48 rows decode the weights again), where its 512-column tiles give every compute unit two workgroups.  256 experts,
-// 2048 / 512, 997 tokens, top-8 (31 rows): 139 -> 99 us for gate / up; for down, one workgroup per compute unit, both take 61 us.
+// 2048 / 512, 997 tokens, top-8 (31 rows): 139 -> 99 us for gate / up.  With one workgroup per compute unit, up to 24 rows: down of that
+// layer 64 -> 57 us at 160 tokens, 64 both at 515, 68 -> 65 at 760 (16, 24 rows), no gain beyond.
 static bool grad_input_of_few_rows(int64_t rows, int64_t groups, int64_t k) {
-    return k % 512 == 0 && rows <= 40 * groups && groups * (k / 512) >= 512;
+    const int64_t tiles = groups * (k / 512);
+    return k % 512 == 0 && ((rows <= 40 * groups && tiles >= 512) || (rows <= 24 * groups && tiles >= 256));
 }
 
 // IQ2_XXS, grad-input: groups that average at most 72 rows take the kernel that keeps decoded weights out of LDS (its tiles have 80
