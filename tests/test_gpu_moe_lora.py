@@ -209,6 +209,7 @@ def test_grouped_lora_projection_all_gradients(pkg, dev, qt, r, shape, n, force_
     ([40, 100, 128], 520, 768, 32, False),                                   # three column tiles, the last one 8 wide; rank 32
     ([5, 90], 8, 1024, 4, True),                                             # fewer columns than one wave owns; rank padded to 16
     ([128] * 3 + [1] * 5, 512, 256, 64, False),                              # rank 64
+    ([33, 20, 97, 5], 70, 768, 16, False),                                   # planes that start 4, 8 and 12 bytes past a multiple of 16
 ])
 @pytest.mark.parametrize("shape", ["", "1"])
 def test_iq2xxs_forward_of_small_groups(pkg, dev, sizes, n, k, r, pair, shape, force_grouped_shape):
