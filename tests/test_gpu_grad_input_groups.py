@@ -1,0 +1,85 @@
+"""Grad-input of expert groups of very different sizes in one call, on the kernels for groups of a few rows."""
+
+import statistics
+
+import pytest
+import torch
+
+from helpers import TYPE_NAMES
+from oracle import gguf_blocks as gb
+
+pytestmark = pytest.mark.gpu
+
+BLOCKS = {gb.Q4_K: 144, gb.IQ2_XXS: 66}
+
+
+def _payload(dev, seed, qt, experts, n, k):
+    """Arbitrary quants with block scales of about 1e-4 (and, for Q4_K, offsets of the same size), made on the device."""
+    gen = torch.Generator(device=dev).manual_seed(seed)
+    blocks = torch.randint(0, 256, (experts * n * (k // 256), BLOCKS[qt]), dtype=torch.uint8, generator=gen, device=dev)
+    scales = ((0.5 + torch.rand(blocks.shape[0], 2, generator=gen, device=dev)) * 1e-4).half().view(torch.uint8)
+    fields = 4 if qt == gb.Q4_K else 2
+    blocks[:, :fields] = scales[:, :fields]
+    return blocks.reshape(experts, n, -1)
+
+
+def _rows(dev, seed, rows, cols):
+    return torch.randn(rows, cols, generator=torch.Generator(device=dev).manual_seed(seed), device=dev).bfloat16()
+
+
+def _ends(dev, sizes):
+    return torch.tensor(sizes, device=dev).cumsum(0).int()
+
+
+def _microseconds(call, repeats=7, calls=10):
+    times = []
+    call()
+    for _ in range(repeats):
+        start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(calls):
+            call()
+        stop.record()
+        stop.synchronize()
+        times.append(start.elapsed_time(stop) * 1e3 / calls)
+    return statistics.median(times)
+
+
+@pytest.mark.parametrize("qt,n,k,even,skewed", [
+    # one workgroup per compute unit in the even grouping; six groups of 192 rows must not each be one workgroup's chain of tiles
+    (gb.Q4_K, 2048, 512, [5] * 256, [192] * 6 + [0, 1] * 64 + [0] * 122),
+    (gb.Q4_K, 768, 1024, [16] * 256, [192] * 20 + [0, 2] * 64 + [0] * 108),
+], ids=lambda v: TYPE_NAMES.get(v, str(v)) if isinstance(v, int) else f"max{max(v)}")
+def test_skewed_groups_cost_little_more_than_even_ones(pkg, dev, qt, n, k, even, skewed):
+    # measured 1.1 to 1.3 times the even grouping's time; with one workgroup per 192 rows it was 2.6 and 3.8 times
+    assert len(even) == len(skewed) == 256 and abs(sum(even) - sum(skewed)) <= 0.05 * sum(even)
+    w, ids = _payload(dev, 1, qt, 256, n, k), torch.arange(256, device=dev)
+    times = []
+    for sizes in (even, skewed):
+        dy, ends = _rows(dev, 2, sum(sizes), n), _ends(dev, sizes)
+        times.append(_microseconds(lambda: pkg.fast_moe_lora.grouped_mmq_grad_input(dy, w, ids, ends, qt, k)))
+    assert times[1] <= 1.8 * times[0], f"even {times[0]:.1f} us, skewed {times[1]:.1f} us"
+
+
+@pytest.mark.parametrize("rank", [0, 16])
+@pytest.mark.parametrize("sizes", [[49, 63, 64, 65, 0, 0, 0], [127, 128, 129, 1] + [0] * 7, [192, 193, 0, 48] + [0] * 12, [255, 0, 0, 0, 0, 0, 0, 16]])
+def test_q4k_groups_beyond_a_tile_match_the_kernel_for_larger_groups(pkg, dev, sizes, rank):
+    # the same rows with the empty groups left out average more rows than the rule takes: the eight-wave kernel, bit for bit
+    qt, n, k, groups = gb.Q4_K, 256, 4096, 64
+    ml = pkg.fast_moe_lora
+    sizes = (sizes * groups)[:groups]
+    active = [g for g, size in enumerate(sizes) if size]
+    assert sum(sizes) <= 40 * groups and sum(sizes) > 40 * len(active)
+    w = _payload(dev, 3, qt, groups, n, k)
+    dy, x = _rows(dev, 4, sum(sizes), n), _rows(dev, 5, sum(sizes), k)
+    a, b = _rows(dev, 6, groups * rank, k).view(groups, rank, k), _rows(dev, 7, groups * n, rank).view(groups, n, rank)
+    got = []
+    for ids in (list(range(groups)), active):
+        e, o = torch.tensor(ids, device=dev), _ends(dev, [sizes[g] for g in ids])
+        if rank:
+            xd = x.clone().requires_grad_(True)
+            ml.grouped_lora_mmq(xd, w, e, o, qt, n, a, b, 2.0).backward(dy)
+            got.append(xd.grad)
+        else:
+            got.append(ml.grouped_mmq_grad_input(dy, w, e, o, qt, k))
+    assert torch.isfinite(got[0]).all() and torch.equal(*got)

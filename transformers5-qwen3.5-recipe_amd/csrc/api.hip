@@ -195,13 +195,17 @@ static int direct_tiles_per_wg(int64_t rows, int64_t groups, int col_tiles, int 
     return per_wg;
 }
 
-// Direct shape, grad-input: groups that average at most 40 rows take the kernel that keeps decoded weights out of LDS (groups of
-// more than its 48 rows decode the weights again), where its 512-column tiles give every compute unit two workgroups.  256 experts,
-// 2048 / 512, 997 tokens, top-8 (31 rows): 139 -> 99 us for gate / up.  With one workgroup per compute unit, up to 24 rows: down of that
-// layer 64 -> 57 us at 160 tokens, 64 both at 515, 68 -> 65 at 760 (16, 24 rows), no gain beyond.
+// Direct shape, grad-input: groups that average at most 40 rows take the kernel that keeps decoded weights out of LDS, where its
+// 512-column tiles give every compute unit two workgroups; with one, groups of up to 24 rows in the mean.  The sizes themselves are on
+// the device, so a call goes to one kernel as a whole, and groups beyond its 64 rows are several tiles that each decode the
+// weights.  Against mmq_direct8_nn.h, 256 experts, rows drawn uniformly / by geometric weights / by Zipf weights: 2 x 512 rows of
+// W, k 2048: 16 rows in the mean 129 -> 90 / 147 -> 88 / 183 -> 100 us, 31 rows 147 -> 102 / 185 -> 114 / 226 -> 119, 40 rows 152 -> 109 /
+// 196 -> 123 / 226 -> 133; 2048 rows, k 512: 5 rows 68 -> 59 / 67 -> 63 / 93 -> 75, 24 rows 73 -> 69 / 83 -> 83 / 128 -> 86 (31 rows:
+// 81 / 93 / 125, no gain).  What loses is an eighth of the experts with all of the rows: 31 rows in the mean, 248 per active expert:
+// 4096 rows of W, k 2048: 197 -> 260 us (but 2 x 512 rows: 168 -> 80).
 static bool grad_input_of_few_rows(int64_t rows, int64_t groups, int64_t k) {
     const int64_t tiles = groups * (k / 512);
-    return k % 512 == 0 && ((rows <= 40 * groups && tiles >= 512) || (rows <= 24 * groups && tiles >= 256));
+    return k % 512 == 0 && ((rows <= kSmallNNRowsPerGroup * groups && tiles >= 512) || (rows <= 24 * groups && tiles >= 256));
 }
 
 // IQ2_XXS, grad-input: groups that average at most 72 rows take the kernel that keeps decoded weights out of LDS (its tiles have 80
@@ -317,13 +321,14 @@ int ggq_fixed_grouped_mmq_grad_input_ws(const void* dy, const void* packed_group
 }
 
 // Row-tile tables of one grouping, built once (ggq_group_tables_build) and handed to the launches that share it: the
-// main table in group order and sorted by size, the 64-row table of the LoRA side kernels, the two tile counts, the
-// per-expert row ranges.  Only the decoding-wave kernels' tile height is covered; a launch of another shape builds its own.
+// main table in group order and sorted by size, the 64-row table of the LoRA side kernels (of small groups also sorted, for
+// the grad-input kernel of 64-row tiles), the tile counts, the per-expert row ranges.  Only the decoding-wave kernels' tile
+// heights are covered; a launch of another shape builds its own.
 struct GroupTablesView {
-    TileDesc *t_main, *t_sorted, *t64, *t_few;  // (t_few: while groups are small)
+    TileDesc *t_main, *t_sorted, *t64, *t64_sorted, *t_few;  // (t64_sorted, t_few: while groups are small)
     int* counts;
     int* ranges;
-    int max_main, max64, max_few;
+    int max_main, max64, max64_sorted, max_few;
 };
 static int64_t group_tables_layout(void* base, int64_t rows, int64_t groups, int64_t experts, GroupTablesView& v) {
     Bump b{(char*)base, INT64_MAX, 0};
@@ -331,6 +336,8 @@ static int64_t group_tables_layout(void* base, int64_t rows, int64_t groups, int
     v.t_main = (TileDesc*)b.take((int64_t)v.max_main * sizeof(TileDesc));
     v.t_sorted = (TileDesc*)b.take((int64_t)v.max_main * sizeof(TileDesc));
     v.t64 = (TileDesc*)b.take((int64_t)v.max64 * sizeof(TileDesc));
+    v.max64_sorted = rows <= kSmallNNRowsPerGroup * groups ? v.max64 : 0;
+    v.t64_sorted = (TileDesc*)b.take((int64_t)v.max64_sorted * sizeof(TileDesc));
     v.max_few = rows <= kFewRowsPerGroup * groups ? (int)(rows / kFewRowsTile + groups) : 0;
     v.t_few = (TileDesc*)b.take((int64_t)v.max_few * sizeof(TileDesc));
     v.counts = (int*)b.take(16);
@@ -342,7 +349,7 @@ static RowTileTables group_tables(void* base, int64_t rows, int64_t groups, int6
     group_tables_layout(base, rows, groups, experts, v);
     RowTileTables tb{};
     tb.add(kDirectBM, 0, 0x7FFFFFFF, v.t_main, v.counts, v.t_sorted);
-    tb.add(64, 0, 0x7FFFFFFF, v.t64, v.counts + 1);
+    tb.add(64, 0, 0x7FFFFFFF, v.t64, v.counts + 1, v.max64_sorted ? v.t64_sorted : nullptr);
     if (v.max_few) tb.add(kFewRowsTile, 0, 0x7FFFFFFF, v.t_few, v.counts + 2);
     return tb;
 }
@@ -614,6 +621,14 @@ static int grouped_backward(const char* what, const void* dy1, const void* dy2, 
         }
     }
 
+    // t = dy . B, into the workspace behind the tables
+    SkinnyNtParams sp{};
+    sp.in[0] = (const bf16_t*)dy1, sp.in[1] = (const bf16_t*)dy2, sp.ld_in = n, sp.in_rows = dy_index;
+    sp.f = (const bf16_t*)lora_b, sp.ldf = r, sp.f_expert_elems = (int64_t)r * ntot, sp.f_natural = 1;
+    sp.m = (int)rows, sp.c = (int)n, sp.r = r, sp.nseg = nseg;
+    const bool transposed = lora_a && rows > 0 && !skinny_nt_takes_natural_factor(sp);
+    const int64_t product_bytes = lora_a ? align256(rows * rp * 2) + (transposed ? align256(experts * ntot * r * 2) : 0) : 0;
+
     const TileDesc* tiles64 = nullptr;
     const int* num_tiles64 = nullptr;
     const int* ranges = nullptr;
@@ -628,6 +643,7 @@ static int grouped_backward(const char* what, const void* dy1, const void* dy2, 
         group_tables_layout(const_cast<void*>(group_tables), rows, groups, experts, v);
         max_tiles64 = v.max64;
         p.expert_ids = expert_ids, p.tiles = v.t_sorted, p.num_tiles = v.counts, p.max_row_tiles = v.max_main;
+        if (p.few_rows) p.tiles = v.t64_sorted, p.num_tiles = v.counts + 1, p.max_row_tiles = v.max64_sorted;
         tiles64 = v.t64, num_tiles64 = v.counts + 1, ranges = v.ranges;
     } else if (groups > 0) {
         const bool wide = p.shape == kShapeWide;  // small groups: wide tiles; larger ones: a second, tall launch
@@ -636,10 +652,14 @@ static int grouped_backward(const char* what, const void* dy1, const void* dy2, 
         max_tall = wide ? (int)std::min<int64_t>(rows / kBM + groups, rows / (kWideBM + 1) + rows / kBM + 1) : 0;
         max_tiles64 = (int)(rows / 64 + groups);
         const bool direct = p.shape == kShapeDirect;  // its workgroups take the tiles with the most rows first
-        TileDesc* t128 = (TileDesc*)bump.take((int64_t)max128 * sizeof(TileDesc));
-        TileDesc* t_sorted = direct ? (TileDesc*)bump.take((int64_t)max128 * sizeof(TileDesc)) : nullptr;
+        const int64_t rest = align256(16) + (lora_a ? align256(experts * 2 * 4) : 0) + product_bytes;
+        p.few_rows = p.few_rows && 2 * align256((int64_t)max_tiles64 * sizeof(TileDesc)) + rest <= ws_bytes;
+        const bool few = p.few_rows;                  // in place of the direct table: 64-row tiles, the largest first
+        TileDesc* t128 = few ? nullptr : (TileDesc*)bump.take((int64_t)max128 * sizeof(TileDesc));
+        TileDesc* t_sorted = direct && !few ? (TileDesc*)bump.take((int64_t)max128 * sizeof(TileDesc)) : nullptr;
         t_tall = wide ? (TileDesc*)bump.take((int64_t)max_tall * sizeof(TileDesc)) : nullptr;
-        TileDesc* t64 = lora_a ? (TileDesc*)bump.take((int64_t)max_tiles64 * sizeof(TileDesc)) : nullptr;
+        TileDesc* t64 = lora_a || few ? (TileDesc*)bump.take((int64_t)max_tiles64 * sizeof(TileDesc)) : nullptr;
+        TileDesc* t64_sorted = few ? (TileDesc*)bump.take((int64_t)max_tiles64 * sizeof(TileDesc)) : nullptr;
         // IQ2_XXS, small groups: the groups of at most 128 rows leave the wide table for a launch of their own
         const bool small = wide && qt == 16 /* GGML IQ2_XXS */ && iq2_grad_input_of_few_rows(rows, groups, n, k) && aligned16(dy1) && (!dy2 || aligned16(dy2)) &&
                            (!lora_a || (aligned16(lora_a) && aligned16(ws))) && g_shape_override.load() != kShapeWide;
@@ -647,29 +667,25 @@ static int grouped_backward(const char* what, const void* dy1, const void* dy2, 
         TileDesc* t_small_sorted = small ? (TileDesc*)bump.take((int64_t)groups * sizeof(TileDesc)) : nullptr;  // most row blocks first
         int* counts = (int*)bump.take(16);
         int* rg = lora_a ? (int*)bump.take(experts * 2 * 4) : nullptr;
-        if (!t128 || !counts || (lora_a && (!t64 || !rg)) || (wide && !t_tall) || (direct && !t_sorted) || (small && (!t_small || !t_small_sorted))) return set_error(GGQ_ERR_WORKSPACE, "%s: workspace too small", what);
+        if ((few ? !t64_sorted : !t128) || !counts || (lora_a && (!t64 || !rg)) || (wide && !t_tall) || (direct && !few && !t_sorted) || (small && (!t_small || !t_small_sorted))) return set_error(GGQ_ERR_WORKSPACE, "%s: workspace too small", what);
         RowTileTables tb{};
-        tb.add(bm_main, small ? kSmallBM : 0, wide ? kWideBM : 0x7FFFFFFF, t128, counts, t_sorted);
+        if (!few) tb.add(bm_main, small ? kSmallBM : 0, wide ? kWideBM : 0x7FFFFFFF, t128, counts, t_sorted);
         if (direct) t128 = t_sorted;
         if (wide) tb.add(kBM, kWideBM, 0x7FFFFFFF, t_tall, counts + 2), n_tall = counts + 2;
-        if (lora_a) tb.add(64, 0, 0x7FFFFFFF, t64, counts + 1);
+        if (t64) tb.add(64, 0, 0x7FFFFFFF, t64, counts + 1, t64_sorted);
         if (small) tb.add(kSmallBM, 0, kSmallBM, t_small, counts + 3, t_small_sorted), n_small = counts + 3, t_small = t_small_sorted;
         if (int rc = build_row_tile_tables(expert_ids, end_offsets, (int)groups, tb, rg, (int)experts, s)) return rc;
         p.expert_ids = expert_ids, p.tiles = t128, p.num_tiles = counts, p.max_row_tiles = small ? 0 : max128;  // (small: the wide table stays empty)
+        if (few) p.tiles = t64_sorted, p.num_tiles = counts + 1, p.max_row_tiles = max_tiles64;
         tiles64 = t64, num_tiles64 = counts + 1, ranges = rg;
     }
     if (lora_a) {
-        // t = dy . B
         bf16_t* dyb = (bf16_t*)bump.take(rows * rp * 2);
         if (!dyb) return set_error(GGQ_ERR_WORKSPACE, "%s: workspace too small", what);
         if (rows > 0) {
-            SkinnyNtParams sp{};
-            sp.in[0] = (const bf16_t*)dy1, sp.in[1] = (const bf16_t*)dy2, sp.ld_in = n, sp.in_rows = dy_index;
-            sp.f = (const bf16_t*)lora_b, sp.ldf = r, sp.f_expert_elems = (int64_t)r * ntot, sp.f_natural = 1;
             sp.out = dyb;
-            sp.m = (int)rows, sp.c = (int)n, sp.r = r, sp.nseg = nseg;
             sp.expert_ids = groups > 0 ? expert_ids : nullptr, sp.tiles = tiles64, sp.num_tiles = num_tiles64;
-            if (!skinny_nt_takes_natural_factor(sp)) {
+            if (transposed) {
                 // B^T, so that both operands are contraction-contiguous
                 bf16_t* bt = (bf16_t*)bump.take(experts * ntot * r * 2);
                 if (!bt) return set_error(GGQ_ERR_WORKSPACE, "%s: workspace too small", what);

@@ -3,25 +3,26 @@
 //   C[m, k] = sum_seg sum_n A_seg[m, n] * W_seg[n, k]  (+ s * LA[m, :] . LB[:, k])
 //
 // The kernel of mmq_direct8_nn.h turns every decoded block through LDS (a lane decodes a weight row, an MFMA operand holds
-// eight rows of one column): 8 KB in and out per wave and step of 64 x 32 weights, which 16 to 48 activation rows cannot pay
+// eight rows of one column): 8 KB in and out per wave and step of 64 x 32 weights, which 16 to 64 activation rows cannot pay
 // for.  Here no decoded weight touches LDS.  A lane holds four adjacent packed bytes of EIGHT weight rows, so it has eight
 // contraction rows of four columns and, in the high nibbles, of four more: the two halves of an operand register are two rows
 // of one column, and one v_cvt_pk_bf16_f32 that has to be spent anyway puts them together.  The sixteen columns of a
 // 16x16x32 MFMA are then every fourth column: lane c = lane % 16 has byte column 4 c + j for operand j, a wave 128 columns
 // (half a block's 128 quant bytes, both nibbles), and the quarter lane / 16 takes contraction rows 8 q .. 8 q + 7.
 //
-// A workgroup is four waves = 512 columns = two adjacent blocks of every weight row (288 contiguous bytes), up to 48 activation
-// rows, two of them on a compute unit (168 registers, for a third, spill at 48 rows).  Per step of 32 weight rows
-//   * the packed rows and the A tile [48][32] go global -> LDS directly, two steps ahead, through a ring of three stages;
+// A workgroup is four waves = 512 columns = two adjacent blocks of every weight row (288 contiguous bytes), up to 64 activation
+// rows, two of them on a compute unit (210 registers; 168, for a third, spill).  Larger groups are several tiles, each a
+// workgroup of its own.  Per step of 32 weight rows
+//   * the packed rows and the A tile [64][32] go global -> LDS directly, two steps ahead, through a ring of three stages;
 //   * every lane works out one (sub-block scale, min) pair of pairs (one row, one quant group) for all four waves;
 //   * a wave reads its dwords and scales, forms its eight operands and issues 8 x (row blocks of 16) MFMAs.
 // The LDS layouts are permuted so that all of these reads are free of bank conflicts (raw_chunk, scale_slot, a_slot32).  Sums and
 // roundings are those of mmq_direct8_nn.h, in the same order.
 //
 // What bounds it: the packed bytes (302 MB, 50 us) and, at 32 rows and more, the instructions of a step; with all packed rows in
-// L2 74 / 87 / 102 us at 16 / 32 / 48 rows.  256 experts, 2 x 512 rows of W, k 2048: 82 / 89 / 107 / 124 us at 5 / 16 / 32 / 48
-// rows per expert, against 109 / 113 / 119 / 137 of mmq_direct8_nn.h.  2048 rows of W, k 512, where it has one workgroup per
-// compute unit: 51 / 54 / 61 / 65 against 58 / 60 / 61 / 63.
+// L2 74 / 87 / 102 us at 16 / 32 / 48 rows.  The call (with dY . B, 9 us) for 256 experts of 5 / 16 / 32 / 48 / 64 rows each: 2 x 512
+// rows of W, k 2048: 83 / 86 / 96 / 116 / 130 us, against 126 / 134 / 129 / 159 / 160 on mmq_direct8_nn.h; 2048 rows of W, k 512,
+// where it has one workgroup per compute unit: 59 / 60 / 66 / 77 / 84 against 69 / 70 / 70 / 82 / 86.
 #pragma once
 #include "mmq_direct.h"
 
@@ -29,7 +30,7 @@ namespace ggq {
 
 struct SmallNN {
     static constexpr int kWaves = 4, kThreadsWG = 64 * kWaves;
-    static constexpr int kRows = 48, kCols = 512;      // of a tile
+    static constexpr int kRows = 64, kCols = 512;      // of a tile
     static constexpr int kStages = 3;
     static constexpr int kRawBytes = 32 * 288, kABytes = kRows * 64;
     static constexpr int kScaleBase = kStages * (kRawBytes + kABytes);
@@ -105,7 +106,6 @@ struct SmallNN {
         const int grp_sh = 16 * (part & 1);
         const bool grp_hi = (part & 2) != 0;
 
-        lds_barrier();  // (a second row tile: every wave is done with the stages of the first)
         request();
         request();
         int rd = 0;
@@ -157,7 +157,7 @@ struct SmallNN {
 #pragma unroll
                         for (int rb = 0; rb < RB; rb++) acc[4 * hi + odd + 2 * u][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[rb], acc[4 * hi + odd + 2 * u][rb], 0, 0, 0);
                     }
-                    __builtin_amdgcn_sched_barrier(0);  // (one pair of operands at a time: the register need stays under three workgroups' share)
+                    __builtin_amdgcn_sched_barrier(0);  // (one pair of operands at a time: fewer registers)
                 }
             }
         }
@@ -227,7 +227,7 @@ struct SmallNN {
         }
     }
 
-    // A unit is 512 columns of one entry of the row-tile table; entries of more than 48 rows are walked 48 at a time.
+    // A unit is 512 columns of one entry of the row-tile table, of at most 64 rows.
     static __device__ __forceinline__ void run(const MmqParams& p) {
         const int chunks = p.col_tiles_per_seg / 2;
         const int row_tiles = min(*p.num_tiles, p.max_row_tiles);
@@ -235,12 +235,12 @@ struct SmallNN {
         const int row_tile = (slot / chunks) * 8 + (int)(blockIdx.x & 7), col_block = 2 * (slot % chunks);
         if (row_tile >= row_tiles) return;
         const TileDesc t = p.tiles[row_tile];
-        for (int row = t.row_begin; row < t.row_end; row += kRows) {
-            const int rows = min(kRows, t.row_end - row);
-            if (rows <= 16) work<1>(p, t.expert, row, rows, col_block);
-            else if (rows <= 32) work<2>(p, t.expert, row, rows, col_block);
-            else work<3>(p, t.expert, row, rows, col_block);
-        }
+        const int rows = min(t.row_end - t.row_begin, kRows);
+        if (rows <= 0) return;
+        if (rows <= 16) work<1>(p, t.expert, t.row_begin, rows, col_block);
+        else if (rows <= 32) work<2>(p, t.expert, t.row_begin, rows, col_block);
+        else if (rows <= 48) work<3>(p, t.expert, t.row_begin, rows, col_block);
+        else work<4>(p, t.expert, t.row_begin, rows, col_block);
     }
 };
 
