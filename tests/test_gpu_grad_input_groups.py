@@ -83,3 +83,36 @@ def test_q4k_groups_beyond_a_tile_match_the_kernel_for_larger_groups(pkg, dev, s
         else:
             got.append(ml.grouped_mmq_grad_input(dy, w, e, o, qt, k))
     assert torch.isfinite(got[0]).all() and torch.equal(*got)
+
+
+@pytest.mark.parametrize("rank", [0, 16, 40])
+@pytest.mark.parametrize("pair", [False, True], ids=["one", "pair"])
+def test_iq2xxs_groups_of_few_rows_match_the_tile_kernel(pkg, dev, pair, rank, force_grouped_shape):
+    # the same products in the same order, the LoRA term ahead of them: bit for bit
+    qt, n, k, groups = gb.IQ2_XXS, 384, 4096, 64
+    ml = pkg.fast_moe_lora
+    sizes = ([1, 15, 16, 17, 33, 48, 49, 64, 65, 80, 81, 96, 128, 0, 2, 129] * groups)[:groups]
+    assert sum(sizes) <= 72 * groups
+    ids, ends = torch.arange(groups, device=dev), _ends(dev, sizes)
+    planes = [_payload(dev, 10 + i, qt, groups, n, k) for i in range(2 if pair else 1)]
+    cotangents = [_rows(dev, 20 + i, sum(sizes), n) for i in range(len(planes))]
+    x, nt = _rows(dev, 30, sum(sizes), k), n * len(planes)
+    a, b = _rows(dev, 31, groups * rank, k).view(groups, rank, k), _rows(dev, 32, groups * nt, rank).view(groups, nt, rank)
+    got = []
+    for shape in ("", "1"):
+        force_grouped_shape(shape)
+        if rank:
+            xd = x.clone().requires_grad_(True)
+            if pair:
+                out = ml.grouped_lora_mmq_pair(xd, *planes, ids, ends, qt, n, a, b, 2.0)
+            else:
+                out = (ml.grouped_lora_mmq(xd, planes[0], ids, ends, qt, n, a, b, 2.0),)
+            torch.autograd.backward(out, cotangents)
+            got.append(xd.grad)
+        elif pair:
+            xd = x.clone().requires_grad_(True)
+            torch.autograd.backward(ml.grouped_mmq_pair(xd, *planes, ids, ends, qt, n), cotangents)
+            got.append(xd.grad)
+        else:
+            got.append(ml.grouped_mmq_grad_input(cotangents[0], planes[0], ids, ends, qt, k))
+    assert torch.isfinite(got[0]).all() and torch.equal(*got)

@@ -8,7 +8,8 @@
 // takes contraction rows 8 q .. 8 q + 7: a wave covers 128 columns, half a block.
 //
 // A workgroup is four waves = 512 columns = two adjacent blocks of every weight row (132 bytes), up to 80 activation rows, two of
-// them on a compute unit (256 registers: 160 of accumulators).  Per step of 32 weight rows
+// them on a compute unit (256 registers: 160 of accumulators).  The sums are those of the tile kernel (mmq_tile.h) in the same
+// order, the LoRA term first: bit for bit the same results (with the term last, 0.03 % of the norm apart).  Per step of 32 weight rows
 //   * the packed rows (as the 16-byte chunks that cover them) go global -> LDS four steps ahead, the A tile two steps ahead;
 //   * every lane makes two records of the step after the next, one per (row, sub-block of 32): the magnitudes 8, 25, 43 times its
 //     scale as bf16, the codebook indexes, the sign fields;
@@ -149,6 +150,41 @@ struct SmallNNIq2 {
 #pragma unroll
         for (int i = 0; i < 3; i++) request_w(cw.w + i * w_step, i);
         request_a(ca.a, 0);
+        // acc[j][rb][v]: row 16 rb + l16, column 32 v + 8 q + j of the wave's 128
+        const int col0 = col_block * 256 + 128 * wave;
+        if (p.r_pad > 0) {  // the LoRA term ahead of the products, as in the tile kernel: the same sums in the same order
+            const bf16_t* const factor = p.lb + expert * p.lb_expert_elems + col0 + 32 * (l16 & 3) + 8 * (l16 >> 2);  // [rank][k]; operand column l16 of set 0
+#pragma unroll 1
+            for (int r0 = 0; r0 < p.r_pad; r0 += 32) {
+                const int r = r0 + 8 * q;
+                bf16x8_t la[RB];
+#pragma unroll
+                for (int rb = 0; rb < RB; rb++)
+                    la[rb] = __builtin_bit_cast(bf16x8_t, r < p.r_pad ? *(const uint4*)(p.la + (int64_t)(row_begin + min(16 * rb + l16, rows_valid - 1)) * p.r_pad + r) : make_uint4(0, 0, 0, 0));
+                uint4 f[8];  // eight columns of eight ranks (zeros past the rank)
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    f[i] = *(const uint4*)(factor + (int64_t)min(r + i, p.lora_rank - 1) * p.k);
+                    if (r + i >= p.lora_rank) f[i] = make_uint4(0, 0, 0, 0);
+                }
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    uint32_t o[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const uint4 &f0 = f[2 * i], &f1 = f[2 * i + 1];
+                        const uint32_t e0 = j < 2 ? f0.x : j < 4 ? f0.y : j < 6 ? f0.z : f0.w, e1 = j < 2 ? f1.x : j < 4 ? f1.y : j < 6 ? f1.z : f1.w;
+                        o[i] = __builtin_amdgcn_perm(e1, e0, (j & 1) ? 0x07060302u : 0x05040100u);
+                    }
+#pragma unroll
+                    for (int rb = 0; rb < RB; rb++) acc[j][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Direct::as_operand(o), la[rb], acc[j][rb], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+#pragma unroll
+                for (int rb = 0; rb < RB; rb++) acc[j][rb] *= p.lora_scale;
+        }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         lds_barrier();
         read_raw(0);
@@ -238,43 +274,6 @@ struct SmallNNIq2 {
         asm volatile("" ::"v"(rec[0].x), "v"(rec[1].x));
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load may land in LDS after the workgroup has gone
 
-        // acc[j][rb][v]: row 16 rb + l16, column 32 v + 8 q + j of the wave's 128
-        const int col0 = col_block * 256 + 128 * wave;
-        if (p.r_pad > 0) {
-            const bf16_t* const factor = p.lb + expert * p.lb_expert_elems + col0 + 32 * (l16 & 3) + 8 * (l16 >> 2);  // [rank][k]; operand column l16 of set 0
-            for (int r0 = 0; r0 < p.r_pad; r0 += 32) {
-                const int r = r0 + 8 * q;
-                bf16x8_t la[RB];
-#pragma unroll
-                for (int rb = 0; rb < RB; rb++)
-                    la[rb] = __builtin_bit_cast(bf16x8_t, r < p.r_pad ? *(const uint4*)(p.la + (int64_t)(row_begin + min(16 * rb + l16, rows_valid - 1)) * p.r_pad + r) : make_uint4(0, 0, 0, 0));
-#pragma unroll
-                for (int half = 0; half < 2; half++) {
-                    uint2 f[8];  // four columns of eight ranks (zeros past the rank)
-#pragma unroll
-                    for (int i = 0; i < 8; i++) {
-                        f[i] = *(const uint2*)(factor + (int64_t)min(r + i, p.lora_rank - 1) * p.k + 4 * half);
-                        if (r + i >= p.lora_rank) f[i] = make_uint2(0, 0);
-                    }
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        uint32_t o[4];
-#pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            const uint32_t e0 = j < 2 ? f[2 * i].x : f[2 * i].y, e1 = j < 2 ? f[2 * i + 1].x : f[2 * i + 1].y;
-                            o[i] = __builtin_amdgcn_perm(e1, e0, (j & 1) ? 0x07060302u : 0x05040100u);
-                        }
-#pragma unroll
-                        for (int rb = 0; rb < RB; rb++) {
-                            const f32x4_t t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Direct::as_operand(o), la[rb], (f32x4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-                            for (int v = 0; v < 4; v++) acc[4 * half + j][rb][v] = __builtin_fmaf(p.lora_scale, t[v], acc[4 * half + j][rb][v]);
-                        }
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-        }
         bf16_t* const cbase = (bf16_t*)p.c[0];
         const bool vec = (p.ldc & 7) == 0 && (((uintptr_t)cbase) & 15) == 0;
 #pragma unroll
