@@ -61,6 +61,19 @@ def test_skewed_groups_cost_little_more_than_even_ones(pkg, dev, qt, n, k, even,
     assert times[1] <= 1.8 * times[0], f"even {times[0]:.1f} us, skewed {times[1]:.1f} us"
 
 
+@pytest.mark.parametrize("sizes", [[96] * 42 + [0] * 214, [128] * 16 + [1] * 240], ids=["96_or_none", "128_or_1"])
+def test_iq2xxs_groups_beyond_a_tile_cost_what_they_cost_on_the_tile_kernel(pkg, dev, sizes, force_grouped_shape):
+    # measured (4096 rows of W) 1.03 and 0.8 times the tile kernel's time; with groups of more than 80 rows walked in two parts the first was 1.7 times
+    qt, n, k = gb.IQ2_XXS, 2048, 2048
+    w, ids = _payload(dev, 1, qt, 256, n, k), torch.arange(256, device=dev)
+    dy, ends = _rows(dev, 2, sum(sizes), n), _ends(dev, sizes)
+    times = []
+    for shape in ("", "1"):
+        force_grouped_shape(shape)
+        times.append(_microseconds(lambda: pkg.fast_moe_lora.grouped_mmq_grad_input(dy, w, ids, ends, qt, k)))
+    assert times[0] <= 1.3 * times[1], f"{times[0]:.1f} us, tile kernel {times[1]:.1f} us"
+
+
 @pytest.mark.parametrize("rank", [0, 16])
 @pytest.mark.parametrize("sizes", [[49, 63, 64, 65, 0, 0, 0], [127, 128, 129, 1] + [0] * 7, [192, 193, 0, 48] + [0] * 12, [255, 0, 0, 0, 0, 0, 0, 16]])
 def test_q4k_groups_beyond_a_tile_match_the_kernel_for_larger_groups(pkg, dev, sizes, rank):

@@ -208,10 +208,11 @@ static bool grad_input_of_few_rows(int64_t rows, int64_t groups, int64_t k) {
     return k % 512 == 0 && ((rows <= kSmallNNRowsPerGroup * groups && tiles >= 512) || (rows <= 24 * groups && tiles >= 256));
 }
 
-// IQ2_XXS, grad-input: groups that average at most 72 rows take the kernel that keeps decoded weights out of LDS (its tiles have 80
-// rows; a group with more decodes the weights again, 1490 us against the tile kernel's 1140 if all have), where its 512-column
-// tiles give every compute unit two workgroups.  256 experts, 4096 / 2048, 2048 tokens, top-8 (64 rows): gate / up and down
-// together 1680 -> 1420 us, the training step of that layer 3390 -> 3080.
+// IQ2_XXS, grad-input: where groups average at most 72 rows, those of at most 80 take the kernel that keeps decoded weights out of
+// LDS (its tiles have 80 rows; larger groups stay on the tile kernel), and its 512-column tiles give every compute unit two
+// workgroups.  256 experts, 2048 rows of W, k 4096, uniform / geometric / Zipf routing against the tile kernel alone: 16 rows in the mean
+// 461 -> 302 / 459 -> 336 / 484 -> 354 us, 40 rows 547 -> 371 / 540 -> 433 / 588 -> 457, 72 rows 627 -> 498 / 688 -> 609 / 713 -> 600.  With
+// groups of up to 128 rows walked in two tiles, 42 groups of 96 rows (4096 rows of W, k 2048) took 232 us against 138.
 static bool iq2_grad_input_of_few_rows(int64_t rows, int64_t groups, int64_t n, int64_t k) {
     return k % 512 == 0 && n % 128 == 0 && n < (1 << 22) && k < (1 << 22) && rows <= 72 * groups && groups * (k / 512) >= 512;
 }
@@ -660,7 +661,7 @@ static int grouped_backward(const char* what, const void* dy1, const void* dy2, 
         t_tall = wide ? (TileDesc*)bump.take((int64_t)max_tall * sizeof(TileDesc)) : nullptr;
         TileDesc* t64 = lora_a || few ? (TileDesc*)bump.take((int64_t)max_tiles64 * sizeof(TileDesc)) : nullptr;
         TileDesc* t64_sorted = few ? (TileDesc*)bump.take((int64_t)max_tiles64 * sizeof(TileDesc)) : nullptr;
-        // IQ2_XXS, small groups: the groups of at most 128 rows leave the wide table for a launch of their own
+        // IQ2_XXS, small groups: the groups of one such tile leave the wide table for a launch of their own
         const bool small = wide && qt == 16 /* GGML IQ2_XXS */ && iq2_grad_input_of_few_rows(rows, groups, n, k) && aligned16(dy1) && (!dy2 || aligned16(dy2)) &&
                            (!lora_a || (aligned16(lora_a) && aligned16(ws))) && g_shape_override.load() != kShapeWide;
         t_small = small ? (TileDesc*)bump.take((int64_t)groups * sizeof(TileDesc)) : nullptr;
@@ -669,13 +670,13 @@ static int grouped_backward(const char* what, const void* dy1, const void* dy2, 
         int* rg = lora_a ? (int*)bump.take(experts * 2 * 4) : nullptr;
         if ((few ? !t64_sorted : !t128) || !counts || (lora_a && (!t64 || !rg)) || (wide && !t_tall) || (direct && !few && !t_sorted) || (small && (!t_small || !t_small_sorted))) return set_error(GGQ_ERR_WORKSPACE, "%s: workspace too small", what);
         RowTileTables tb{};
-        if (!few) tb.add(bm_main, small ? kSmallBM : 0, wide ? kWideBM : 0x7FFFFFFF, t128, counts, t_sorted);
+        if (!few) tb.add(bm_main, small ? kSmallNNIq2Rows : 0, wide ? kWideBM : 0x7FFFFFFF, t128, counts, t_sorted);
         if (direct) t128 = t_sorted;
         if (wide) tb.add(kBM, kWideBM, 0x7FFFFFFF, t_tall, counts + 2), n_tall = counts + 2;
         if (t64) tb.add(64, 0, 0x7FFFFFFF, t64, counts + 1, t64_sorted);
-        if (small) tb.add(kSmallBM, 0, kSmallBM, t_small, counts + 3, t_small_sorted), n_small = counts + 3, t_small = t_small_sorted;
+        if (small) tb.add(kSmallNNIq2Rows, 0, kSmallNNIq2Rows, t_small, counts + 3, t_small_sorted), n_small = counts + 3, t_small = t_small_sorted;
         if (int rc = build_row_tile_tables(expert_ids, end_offsets, (int)groups, tb, rg, (int)experts, s)) return rc;
-        p.expert_ids = expert_ids, p.tiles = t128, p.num_tiles = counts, p.max_row_tiles = small ? 0 : max128;  // (small: the wide table stays empty)
+        p.expert_ids = expert_ids, p.tiles = t128, p.num_tiles = counts, p.max_row_tiles = small ? (int)std::min<int64_t>(groups, rows / (kSmallNNIq2Rows + 1)) : max128;
         if (few) p.tiles = t64_sorted, p.num_tiles = counts + 1, p.max_row_tiles = max_tiles64;
         tiles64 = t64, num_tiles64 = counts + 1, ranges = rg;
     }

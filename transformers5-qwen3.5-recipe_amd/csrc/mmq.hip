@@ -213,7 +213,7 @@ int launch_mmq_small(const MmqParams& p, hipStream_t s) {
     return check_launch("mmq_small_iq2xxs_kernel");
 }
 
-// IQ2_XXS, grad-input, store epilogue: entries of up to kSmallBM rows (p.tiles).
+// IQ2_XXS, grad-input, store epilogue: entries of up to kSmallNNIq2Rows rows (p.tiles).
 int launch_mmq_small_nn(const MmqParams& p, hipStream_t s) {
     if ((p.k & 511) || (p.n & 127)) return set_error(GGQ_ERR_SHAPE, "mmq: the small-group grad-input kernel needs whole pairs of blocks and a contraction of whole groups of 128 rows");
     // row tiles are dealt round-robin over the eight XCDs; the column tiles of a row tile follow one another

@@ -66,6 +66,7 @@ constexpr int kBM = 256, kBN = 128, kBK = 64;  // the tall tile shape (dense lau
 constexpr int kWideBM = 128, kWideBN = 256;    // the wide tile shape (Q4_K expert groups of about a hundred rows)
 constexpr int kDirectBM = 192, kDirectBN = 256;  // the direct shape (Q4_K expert groups: the MFMA waves decode the weights themselves)
 constexpr int64_t kSmallNNRowsPerGroup = 40;    // Q4_K grad-input on tiles of 64 rows (mmq_small_nn.h): groups that average at most this many
+constexpr int kSmallNNIq2Rows = 80;             // IQ2_XXS grad-input (mmq_small_nn_iq2.h): groups of at most this many rows, a tile each
 constexpr int kSmallBM = 128, kSmallBN = 256;   // the small shape (IQ2_XXS forward, expert groups of at most 128 rows: decoding waves)
 constexpr int kShapeTall = 0, kShapeWide = 1, kShapeDirect = 3;
 constexpr int kShapeSmall = 5;  // (a launch beside the wide and tall tiles of a call, never the shape of a whole call)

@@ -20,7 +20,7 @@
 // doubled from pair to pair, instead of four words of a table: 650 -> 595 us at 16 rows) and, beside it, the instructions of two
 // waves per SIMD; with sixty-four columns per wave and four waves per SIMD it takes 892 us.  256 experts, 2 x 2048 rows of W,
 // k 4096: 595 / 714 / 804 / 910 us at 16 / 48 / 64 / 80 rows per expert, against 853 / 986 / 1000 / 1132 of the tile kernel; 4096
-// rows of W, k 2048: 323 / 391 / 445 / 490 against 426 / 513 / 539 / 582.  Groups of more than 80 rows decode the weights again.
+// rows of W, k 2048: 323 / 391 / 445 / 490 against 426 / 513 / 539 / 582.  Groups of more than 80 rows stay there.
 #pragma once
 #include "mmq_small_iq2.h"
 
@@ -29,6 +29,7 @@ namespace ggq {
 struct SmallNNIq2 {
     static constexpr int kWaves = 4, kThreadsWG = 64 * kWaves;
     static constexpr int kBlocks = 5, kRows = 16 * kBlocks, kCols = 512;  // of a tile
+    static_assert(kRows == kSmallNNIq2Rows, "table entries");
     static constexpr int kStages = 4;
     static constexpr int kTableBytes = 256 * 16 + 128 * 4;                         // the selectors of Fmt<kIQ2_XXS>, then a word of signs per seven-bit field
     static constexpr int kRawPitch = 144, kRawBytes = 32 * kRawPitch;             // the 16-byte chunks that cover a row's 132 bytes
@@ -146,7 +147,6 @@ struct SmallNNIq2 {
         const uint32_t a_at = opaque(kABase + a_slot32(l16, q) * 16);
 
         Cursor cw{w_plane[0], p.a[0] + a_row0, groups_per_seg, 0}, ca = cw;
-        lds_barrier();  // (a second row tile: every wave is done with the stages of the first)
 #pragma unroll
         for (int i = 0; i < 3; i++) request_w(cw.w + i * w_step, i);
         request_a(ca.a, 0);
@@ -295,7 +295,7 @@ struct SmallNNIq2 {
         }
     }
 
-    // A unit is 512 columns of one entry of the row-tile table; entries of more than 80 rows are walked in equal parts.
+    // A unit is 512 columns of one entry of the row-tile table, of at most 80 rows.
     static __device__ __forceinline__ void run(const MmqParams& p) {
         const int chunks = p.k / kCols;
         const int row_tiles = min(*p.num_tiles, p.max_row_tiles);
@@ -304,17 +304,13 @@ struct SmallNNIq2 {
         if (row_tile >= row_tiles) return;
         for (int i = threadIdx.x; i < 1024 + 128; i += kThreadsWG) *lds<uint32_t>(4 * i) = i < 1024 ? Fmt<kIQ2_XXS>::table_word(i, d_iq2xxs_grid_mm[i >> 2]) : Iq2Signs::word(i - 1024);
         const TileDesc t = p.tiles[row_tile];
-        const int all = t.row_end - t.row_begin, parts = (all + kRows - 1) / kRows;
-        if (parts <= 0) return;
-        const int part = ((all + parts - 1) / parts + 15) & ~15;  // (at most kRows, a multiple of sixteen)
-        for (int row = t.row_begin; row < t.row_end; row += part) {
-            const int rows = min(part, t.row_end - row);
-            if (rows <= 16) work<1>(p, t.expert, row, rows, col_block);
-            else if (rows <= 32) work<2>(p, t.expert, row, rows, col_block);
-            else if (rows <= 48) work<3>(p, t.expert, row, rows, col_block);
-            else if (rows <= 64) work<4>(p, t.expert, row, rows, col_block);
-            else work<5>(p, t.expert, row, rows, col_block);
-        }
+        const int rows = min(t.row_end - t.row_begin, kRows);
+        if (rows <= 0) return;
+        if (rows <= 16) work<1>(p, t.expert, t.row_begin, rows, col_block);
+        else if (rows <= 32) work<2>(p, t.expert, t.row_begin, rows, col_block);
+        else if (rows <= 48) work<3>(p, t.expert, t.row_begin, rows, col_block);
+        else if (rows <= 64) work<4>(p, t.expert, t.row_begin, rows, col_block);
+        else work<5>(p, t.expert, t.row_begin, rows, col_block);
     }
 };
 
