@@ -158,6 +158,8 @@ def _expert_layer(pkg, dev, qt, qt_down, experts, hidden, inter, r, limit=None, 
     (1, 8, 2048, 512, 16, None, torch.int64), (8, 8, 256, 256, 5, 0.25, torch.int32),   # 64 routes: past every limit of the path without a plan
     (4, 16, 512, 768, 64, None, torch.int64), (2, 16, 256, 512, 40, None, torch.int64), (3, 1, 4096, 256, 24, None, torch.int32),
     (1, 2, 256, 3584, 24, None, torch.int64),  # Q2_K, Q3_K: sixteen packed rows per wave leave no LDS for x
+    (1, 8, 4096, 512, 16, None, torch.int64),  # more than 2048 elements of x: Q2_K, Q3_K two column sets per workgroup, the others one
+    (1, 4, 3072, 1024, 40, None, torch.int64),  # and IQ2_XXS two, a rank padded to 48
 ])
 @pytest.mark.parametrize("qt", ALL_TYPES, ids=[TYPE_NAMES[q] for q in ALL_TYPES])
 def test_experts_of_a_few_routes(pkg, dev, qt, tokens, top_k, hidden, inter, r, limit, ids):

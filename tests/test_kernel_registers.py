@@ -1,0 +1,39 @@
+"""Registers of kernels whose launch counts on a number of workgroups per compute unit, as the compiler reports them.
+
+A SIMD has 512 registers per lane: a kernel of up to 128 runs four waves on it, of up to 80 six."""
+import pathlib
+import re
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = pathlib.Path(__file__).resolve().parents[1] / "transformers5-qwen3.5-recipe_amd" / "csrc"
+
+
+@pytest.fixture(scope="module")
+def resources(tmp_path_factory):
+    """{mangled kernel name: (registers, bytes of scratch per lane)} of gemv.hip."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not pathlib.Path(hipcc).exists():
+        pytest.skip("hipcc is not installed")
+    cmd = [hipcc, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-c", "--cuda-device-only",
+           "-Rpass-analysis=kernel-resource-usage", str(CSRC / "gemv.hip"), "-o", str(tmp_path_factory.mktemp("registers") / "gemv.o")]
+    done = subprocess.run(cmd, capture_output=True, text=True, timeout=600)
+    assert done.returncode == 0, done.stderr[-2000:]
+    out = {}
+    for block in done.stderr.split("Function Name: ")[1:]:
+        vgprs, agprs, scratch = (int(re.search(key + r": (\d+)", block).group(1)) for key in (r" VGPRs", r" AGPRs", r"ScratchSize \[bytes/lane\]"))
+        out[block.split()[0]] = (vgprs + agprs, scratch)
+    return out
+
+
+def _named(resources, pattern):
+    found = {name: r for name, r in resources.items() if re.search(pattern, name)}
+    assert found, pattern
+    return found
+
+
+def test_few_routes_gate_up_leaves_room_for_two_workgroups(resources):
+    for name, (registers, scratch) in _named(resources, r"few_routes_gate_up_kernelILi\d+ELi\d+ELi\d+E").items():
+        assert registers <= 128 and scratch == 0, (name, registers, scratch)
