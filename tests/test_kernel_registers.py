@@ -37,3 +37,12 @@ def _named(resources, pattern):
 def test_few_routes_gate_up_leaves_room_for_two_workgroups(resources):
     for name, (registers, scratch) in _named(resources, r"few_routes_gate_up_kernelILi\d+ELi\d+ELi\d+E").items():
         assert registers <= 128 and scratch == 0, (name, registers, scratch)
+
+
+def test_one_row_block_products_leave_room_for_the_workgroups_the_launch_asks_for(resources):
+    # gemv_kernel<type, 8 waves, 2 spans, 1 row block, no LoRA>: three workgroups of eight waves unless the rule names the type, else two
+    rule = re.search(r"static bool many_small_workgroups\(.*", (CSRC / "gemv.hip").read_text()).group(0)
+    ids = {"kQ8_0": 8, "kQ2_K": 10, "kQ3_K": 11, "kQ4_K": 12, "kQ5_K": 13, "kQ6_K": 14, "kIQ2_XXS": 16}
+    for name, qt in ids.items():
+        ((kernel, (registers, scratch)),) = _named(resources, rf"11gemv_kernelILi{qt}ELi8ELi2ELi1ELb0E").items()
+        assert registers <= (128 if f"qt != {name}" in rule else 80) and scratch == 0, (kernel, registers, scratch)

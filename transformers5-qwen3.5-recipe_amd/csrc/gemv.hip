@@ -370,14 +370,15 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
 // One row block of up to 2048 elements without a LoRA term: three workgroups per compute unit with one LDS buffer each, instead of
 // two with two.  A block's way through its workgroup (requests, decoding, two barriers) is longer than the memory's, and three
 // independent ones hide more of it than a request ahead does: 151936 x 2048 Q6_K, one row, 66.5 -> 58.0 us; Q8_0 109 -> 103.  (A
-// fourth needs 64 registers and spills: 67 us.  Sixteen waves on one block: 88 us with two to five buffers.)
-static bool many_small_workgroups(bool lora, int64_t m, int64_t k) { return !lora && m <= 16 && k <= 2048; }
+// fourth needs 64 registers and spills: 67 us.  Sixteen waves on one block: 88 us with two to five buffers.)  Six waves per SIMD need
+// the kernel within 80 registers: Q3_K takes 88 and keeps two workgroups with two buffers, 67.3 -> 65.3 us.
+static bool many_small_workgroups(int qt, bool lora, int64_t m, int64_t k) { return qt != kQ3_K && !lora && m <= 16 && k <= 2048; }
 template <int QT, int WAVES, int SP, int TB, bool LORA>
 static int launch_gemv(const GemvParams& p, hipStream_t s) {
     const int lds = kTableBytes<QT> + p.buffers * p.stage_bytes + WAVES * TB * 64 * 16 + TB * 16 * 64 * 2;
     static LdsLimit lim;
     if (int rc = raise_lds_limit(lim, (const void*)gemv_kernel<QT, WAVES, SP, TB, LORA>, 160 * 1024, "gemv")) return rc;
-    const int per_cu = std::max(1, std::min(160 * 1024 / lds, (many_small_workgroups(LORA, p.m, p.k) ? 24 : 16) / WAVES));
+    const int per_cu = std::max(1, std::min(160 * 1024 / lds, (many_small_workgroups(QT, LORA, p.m, p.k) ? 24 : 16) / WAVES));
     hipLaunchKernelGGL((gemv_kernel<QT, WAVES, SP, TB, LORA>), dim3(std::min((p.n + 15) / 16, 256 * per_cu)), dim3(64 * WAVES), lds, s, p);
     return check_launch("gemv");
 }
@@ -415,7 +416,7 @@ int gemv(int qt, const void* x, int64_t ldx, const void* w, int64_t m, int64_t n
     p.ldx = ldx, p.ldy = ldy;
     if (lora_a) p.lora_a = (const bf16_t*)lora_a, p.lora_b = (const bf16_t*)lora_b, p.r = r, p.r_pad = (r + 15) / 16 * 16, p.lora_scale = scale, p.xa_out = (bf16_t*)xa_out;
     p.stage_bytes = row_block_bytes(qt, p.head + 16 * p.row_bytes);
-    p.buffers = (p.n + 15) / 16 > 256 && p.stage_bytes <= 36 * 1024 && !many_small_workgroups(lora_a != nullptr, m, k) ? 2 : 1;  // (one block per workgroup needs one buffer)
+    p.buffers = (p.n + 15) / 16 > 256 && p.stage_bytes <= 36 * 1024 && !many_small_workgroups(qt, lora_a != nullptr, m, k) ? 2 : 1;  // (one block per workgroup needs one buffer)
     TimedScope timed(qt, kModeNT, kEpiStore, kShapeFewRows, s);
     switch (qt) {
         case kQ8_0: return launch_gemv_qt<kQ8_0>(p, s);
