@@ -69,6 +69,10 @@ int ggq_set_factor_gradient_overlap(int mode);
  * the stated tolerances whatever is chosen. */
 int ggq_debug_force_grouped_shape(int shape);
 
+/* Test aid with no counterpart in the reference: the tile (0 = 256 x 256, 1 = 128 x 128, 2 = 64 x 64, 3 = 128 x 256) and the number of
+ * contraction splits a dense call over decoded panels would run with in a workspace of ws_bytes.  Host only. */
+int ggq_debug_dense_plan(int grad_input, int64_t m, int64_t n, int64_t k, int64_t ws_bytes, int* shape, int* splits);
+
 /* fast_lora.py:24-31 (_NATIVE_MMQ_QUANT_TYPES / supports_native_mmq): 1 if this library has kernels
  * for the GGML type id. */
 int ggq_supports_quant_type(int qt);

@@ -156,3 +156,23 @@ def test_dynamic_lds_limits_are_raised_to_a_constant():
     for call in calls:
         size = call.rsplit(",", 1)[1].strip()
         assert not re.search(r"\b(?!int\b|sizeof\b|k[A-Z])[a-z]\w*", size), f"raise_lds_limit(..., {size}): a size of this call"
+
+
+@pytest.mark.parametrize("m,n,k", [(701, 32768, 2048), (256, 32768, 2048), (1021, 32768, 512), (4096, 32768, 2048)])
+def test_a_workspace_without_room_for_split_sums_gets_a_tile_for_no_splits(pkg, m, n, k):
+    """The 256-row tiles of a long contraction are chosen together with its splits; without the splits they would leave
+    most of 256 compute units idle."""
+    lib, sides = pkg._lib.load(), [(256, 256), (128, 128), (64, 64), (128, 256)]
+
+    def plan(ws_bytes):
+        shape, splits = ctypes.c_int(), ctypes.c_int()
+        pkg._lib.check(lib.ggq_debug_dense_plan(1, m, n, k, ws_bytes, ctypes.byref(shape), ctypes.byref(splits)))
+        rows, cols = sides[shape.value]
+        return -(-m // rows) * -(-k // cols), splits.value
+
+    roomy, whole = plan(1 << 40), lib.ggq_lora_workspace_bytes(m, 0, 1, n, k, 0)
+    assert roomy[1] > 1 and plan(whole) == roomy
+    panel = -(-k // 256) * 256 * (n // 64) * 128
+    tiles, splits = plan(panel)
+    assert splits == 1 and tiles >= 128, (tiles, roomy)
+    assert 1 <= plan(panel + 3 * m * k * 4)[1] <= 3  # room for three

@@ -145,6 +145,13 @@ int ggq_debug_force_grouped_shape(int shape) {
     return GGQ_OK;
 }
 
+int ggq_debug_dense_plan(int grad_input, int64_t m, int64_t n, int64_t k, int64_t ws_bytes, int* shape, int* splits) {
+    if (!shape || !splits) return set_error(GGQ_ERR_NULL, "debug_dense_plan: null pointer");
+    if (m <= 0 || n <= 0 || k <= 0) return set_error(GGQ_ERR_SHAPE, "debug_dense_plan: bad shape m=%lld n=%lld k=%lld", (long long)m, (long long)n, (long long)k);
+    dense_plan(grad_input ? kModeNN : kModeNT, m, n, k, ws_bytes, *shape, *splits);
+    return GGQ_OK;
+}
+
 int ggq_set_factor_gradient_overlap(int mode) {
     g_overlap_mode.store(mode == kOverlapCaptured ? kOverlapCaptured : mode ? kOverlapAlways : kOverlapNever, std::memory_order_relaxed);
     return GGQ_OK;

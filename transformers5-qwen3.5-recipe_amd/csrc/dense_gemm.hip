@@ -666,7 +666,9 @@ bool dense_panel_whole(int64_t n, int64_t k) { return slab_columns(n, k) >= n &&
 // A larger tile reads less per output: 256 x 256 wins where it fills the chip in whole rounds or by splits (4096 x 8192 over
 // 2048: 119 us against 128 with 128 x 128), 128 x 256 where it would leave a half of it idle (4096 x 2048 over 8192: 113 us
 // against 154, and 122 with 128 x 128), the smaller ones for short sequences.
-static void pick_tile(int64_t m, int64_t cols, int64_t steps, bool can_split, int& shape, int& splits) {
+// max_splits: what the output's alignment and the workspace allow (with none, the shape chosen for ten splits can leave most of the
+// chip idle: 701 x 2048 over 32768, 577 us against 207 with the shape for one).
+static void pick_tile(int64_t m, int64_t cols, int64_t steps, int64_t max_splits, int& shape, int& splits) {
     static const struct { int rows, cols, slots; double idle, full, fixed; } kShape[4] = {
         {256, 256, 256, 1.05, 1.40, 6.0}, {128, 128, 512, 0.36, 0.90, 2.5}, {64, 64, 512, 0.11, 0.30, 2.5}, {128, 256, 256, 0.50, 0.80, 5.0}};  // (fixed: a tile's start and end)
     double best = 1e30;
@@ -674,7 +676,7 @@ static void pick_tile(int64_t m, int64_t cols, int64_t steps, bool can_split, in
     for (int sh = 0; sh < 4; sh++) {
         const auto& t = kShape[sh];
         const int64_t tiles = ((m + t.rows - 1) / t.rows) * ((cols + t.cols - 1) / t.cols);
-        for (int sp = 1; sp <= (can_split ? kMaxSplits : 1); sp++) {
+        for (int sp = 1; sp <= max_splits; sp++) {
             const int64_t per = (steps + sp - 1) / sp;
             if (sp > 1 && (per < 4 || (sp - 1) * per >= steps)) continue;
             const int64_t units = tiles * sp, rounds = units / t.slots, rest = units % t.slots;
@@ -686,6 +688,14 @@ static void pick_tile(int64_t m, int64_t cols, int64_t steps, bool can_split, in
     }
 }
 
+static int64_t splits_with_room(int64_t bytes, int64_t m, int64_t cols) { return std::min<int64_t>(kMaxSplits, std::max<int64_t>(1, bytes / (m * cols * 4))); }
+
+void dense_plan(int mode, int64_t m, int64_t n, int64_t k, int64_t ws_bytes, int& shape, int& splits) {
+    const int64_t cols = mode == kModeNT ? n : k, contraction = mode == kModeNT ? k : n, steps = (contraction + 63) / 64;
+    const int64_t slab = slab_columns(cols, contraction), panel_bytes = (slab * steps * 128 + 255) / 256 * 256, cn = std::min(cols, slab);
+    pick_tile(m, cn, steps, cn % 4 == 0 ? splits_with_room(ws_bytes - panel_bytes, m, cn) : 1, shape, splits);
+}
+
 int64_t dense_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     if (m < kDenseMinRows || n <= 0 || k <= 0) return 0;
     const int64_t nt = slab_columns(n, k) * ((k + 63) / 64) * 128, nn = slab_columns(k, n) * ((n + 63) / 64) * 128;
@@ -694,7 +704,7 @@ int64_t dense_workspace_bytes(int64_t m, int64_t n, int64_t k) {
         const int64_t cols = mode == kModeNT ? n : k, c = mode == kModeNT ? k : n;
         const int64_t slab = std::min(cols, slab_columns(cols, c));
         int shape, splits;
-        pick_tile(m, slab, (c + 63) / 64, slab % 4 == 0, shape, splits);
+        pick_tile(m, slab, (c + 63) / 64, slab % 4 == 0 ? kMaxSplits : 1, shape, splits);
         if (splits > 1) partial = std::max(partial, (int64_t)splits * m * slab * 4);
     }
     return (std::max(nt, nn) + 255) / 256 * 256 + (partial + 255) / 256 * 256;
@@ -730,8 +740,7 @@ int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s, con
         }
         int shape, splits;
         const bool can_split = cn % 4 == 0 && q.ldc % 4 == 0 && ((uintptr_t)q.c & 7) == 0;
-        pick_tile(q.m, cn, steps, can_split, shape, splits);
-        if (splits > 1 && ws_bytes < panel_bytes + splits * q.m * cn * 4) splits = 1;
+        pick_tile(q.m, cn, steps, can_split ? splits_with_room(ws_bytes - panel_bytes, q.m, cn) : 1, shape, splits);
         p.splits = splits;
         if (splits > 1) {
             float* partial = (float*)(panel + panel_bytes);

@@ -169,6 +169,7 @@ constexpr int kDenseSideMaxRank = 32;
 bool dense_side_takes(const DenseSide& side);
 bool dense_takes(int mode, int64_t m, int64_t n, int64_t k, const void* a, int64_t lda, bool a_zero_padded = false);
 bool dense_panel_whole(int64_t n, int64_t k);
+void dense_plan(int mode, int64_t m, int64_t n, int64_t k, int64_t ws_bytes, int& shape, int& splits);  // of the first slab of columns
 int64_t dense_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s, const DenseSide* side = nullptr);
 
