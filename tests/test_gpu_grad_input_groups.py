@@ -129,3 +129,30 @@ def test_iq2xxs_groups_of_few_rows_match_the_tile_kernel(pkg, dev, pair, rank, f
         else:
             got.append(ml.grouped_mmq_grad_input(cotangents[0], planes[0], ids, ends, qt, k))
     assert torch.isfinite(got[0]).all() and torch.equal(*got)
+
+
+@pytest.mark.parametrize("rank", [0, 16])
+def test_iq2xxs_workspace_without_room_for_the_small_tables_keeps_the_tile_kernel(pkg, dev, rank):
+    # through the C ABI: what the call needed before there was a launch of its own for small groups is still enough
+    qt, n, k, groups, s = gb.IQ2_XXS, 256, 4096, 64, 2.0
+    lib, stream = pkg._lib.load(), torch.cuda.current_stream().cuda_stream
+    sizes = ([5, 33, 90, 1] * groups)[:groups]
+    rows, w, ids, ends = sum(sizes), _payload(dev, 40, qt, groups, n, k), torch.arange(groups, device=dev), _ends(dev, sizes)
+    dy, x = _rows(dev, 41, rows, n), _rows(dev, 42, rows, k)
+    a, b = _rows(dev, 43, groups * rank, k), _rows(dev, 44, groups * n, rank)
+    # tables of 16-byte entries (wide, tall, 64-row), the counts, the row ranges, dy . B, each a multiple of 256 bytes
+    up = lambda v: -(-v // 256) * 256
+    tall = min(rows // 256 + groups, rows // 129 + rows // 256 + 1)
+    small = up(16 * groups) + up(16 * tall) + 256 + ((up(16 * (rows // 64 + groups)) + up(8 * groups) + up(rows * rank * 2)) if rank else 0)
+    whole = lib.ggq_lora_workspace_bytes(rows, groups, groups, n, k, rank)
+    got = []
+    for size in (small, whole):
+        ws, dx = torch.empty(size, dtype=torch.uint8, device=dev), torch.empty(rows, k, dtype=torch.bfloat16, device=dev)
+        lora = (a.data_ptr(), b.data_ptr(), rank, s) if rank else (None, None, 0, 0.0)
+        pkg._lib.check(lib.ggq_grouped_lora_mmq_backward(dy.data_ptr(), None, w.data_ptr(), None, ids.data_ptr(), ends.data_ptr(), groups, groups, qt, rows, n, k,
+                                                         x.data_ptr(), x.data_ptr(), *lora, dx.data_ptr(), None, None, None, ws.data_ptr(), size, stream))
+        got.append(dx)
+    assert torch.equal(*got)
+    with pytest.raises(RuntimeError, match="workspace too small"):
+        pkg._lib.check(lib.ggq_grouped_lora_mmq_backward(dy.data_ptr(), None, w.data_ptr(), None, ids.data_ptr(), ends.data_ptr(), groups, groups, qt, rows, n, k,
+                                                         x.data_ptr(), x.data_ptr(), *lora, dx.data_ptr(), None, None, None, ws.data_ptr(), small - 256, stream))

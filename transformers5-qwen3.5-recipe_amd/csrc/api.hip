@@ -668,9 +668,11 @@ static int grouped_backward(const char* what, const void* dy1, const void* dy2, 
         t_tall = wide ? (TileDesc*)bump.take((int64_t)max_tall * sizeof(TileDesc)) : nullptr;
         TileDesc* t64 = lora_a || few ? (TileDesc*)bump.take((int64_t)max_tiles64 * sizeof(TileDesc)) : nullptr;
         TileDesc* t64_sorted = few ? (TileDesc*)bump.take((int64_t)max_tiles64 * sizeof(TileDesc)) : nullptr;
-        // IQ2_XXS, small groups: the groups of one such tile leave the wide table for a launch of their own
+        // IQ2_XXS, small groups: the groups of one such tile leave the wide table for a launch of their own (where the workspace has
+        // room for its tables)
         const bool small = wide && qt == 16 /* GGML IQ2_XXS */ && iq2_grad_input_of_few_rows(rows, groups, n, k) && aligned16(dy1) && (!dy2 || aligned16(dy2)) &&
-                           (!lora_a || (aligned16(lora_a) && aligned16(ws))) && g_shape_override.load() != kShapeWide;
+                           (!lora_a || (aligned16(lora_a) && aligned16(ws))) && g_shape_override.load() != kShapeWide &&
+                           bump.used + 2 * align256((int64_t)groups * sizeof(TileDesc)) + rest <= ws_bytes;
         t_small = small ? (TileDesc*)bump.take((int64_t)groups * sizeof(TileDesc)) : nullptr;
         TileDesc* t_small_sorted = small ? (TileDesc*)bump.take((int64_t)groups * sizeof(TileDesc)) : nullptr;  // most row blocks first
         int* counts = (int*)bump.take(16);
