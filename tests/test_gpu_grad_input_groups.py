@@ -74,7 +74,7 @@ def test_iq2xxs_groups_beyond_a_tile_cost_what_they_cost_on_the_tile_kernel(pkg,
     assert times[0] <= 1.3 * times[1], f"{times[0]:.1f} us, tile kernel {times[1]:.1f} us"
 
 
-@pytest.mark.parametrize("rank", [0, 16])
+@pytest.mark.parametrize("rank", [0, 16, 40, 64])
 @pytest.mark.parametrize("sizes", [[49, 63, 64, 65, 0, 0, 0], [127, 128, 129, 1] + [0] * 7, [192, 193, 0, 48] + [0] * 12, [255, 0, 0, 0, 0, 0, 0, 16]])
 def test_q4k_groups_beyond_a_tile_match_the_kernel_for_larger_groups(pkg, dev, sizes, rank):
     # the same rows with the empty groups left out average more rows than the rule takes: the eight-wave kernel, bit for bit

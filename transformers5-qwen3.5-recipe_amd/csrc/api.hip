@@ -209,10 +209,11 @@ static int direct_tiles_per_wg(int64_t rows, int64_t groups, int col_tiles, int 
 // W, k 2048: 16 rows in the mean 129 -> 90 / 147 -> 88 / 183 -> 100 us, 31 rows 147 -> 102 / 185 -> 114 / 226 -> 119, 40 rows 152 -> 109 /
 // 196 -> 123 / 226 -> 133; 2048 rows, k 512: 5 rows 68 -> 59 / 67 -> 63 / 93 -> 75, 24 rows 73 -> 69 / 83 -> 83 / 128 -> 86 (31 rows:
 // 81 / 93 / 125, no gain).  What loses is an eighth of the experts with all of the rows: 31 rows in the mean, 248 per active expert:
-// 4096 rows of W, k 2048: 197 -> 260 us (but 2 x 512 rows: 168 -> 80).
-static bool grad_input_of_few_rows(int64_t rows, int64_t groups, int64_t k) {
+// 4096 rows of W, k 2048: 197 -> 260 us (but 2 x 512 rows: 168 -> 80).  Ranks above 32 keep mmq_direct8_nn.h: it sums LA . LB over
+// all ranks before it scales, and beside 128 accumulators there are no registers for the factors of 64 ranks (they spill).
+static bool grad_input_of_few_rows(int64_t rows, int64_t groups, int64_t k, int r_pad) {
     const int64_t tiles = groups * (k / 512);
-    return k % 512 == 0 && ((rows <= kSmallNNRowsPerGroup * groups && tiles >= 512) || (rows <= 24 * groups && tiles >= 256));
+    return k % 512 == 0 && r_pad <= 32 && ((rows <= kSmallNNRowsPerGroup * groups && tiles >= 512) || (rows <= 24 * groups && tiles >= 256));
 }
 
 // IQ2_XXS, grad-input: where groups average at most 72 rows, those of at most 80 take the kernel that keeps decoded weights out of
@@ -593,7 +594,7 @@ static int grouped_backward(const char* what, const void* dy1, const void* dy2, 
     p.w[0] = (const uint8_t*)packed1, p.w[1] = (const uint8_t*)packed2;
     p.c[0] = dx, p.ldc = k;
     if (p.shape == kShapeDirect) p.col_tiles_per_wg = direct_tiles_per_wg(rows, groups, p.col_tiles_per_seg, nseg * p.steps_per_seg, kModeNN);
-    p.few_rows = p.shape == kShapeDirect && grad_input_of_few_rows(rows, groups, k);
+    p.few_rows = p.shape == kShapeDirect && grad_input_of_few_rows(rows, groups, k, rp);
 
     if (groups == 0 && !packed2 && !dy_index.on() && !x_index.on() && !row_weights && rows > 0 && lora_a && ws && aligned16(ws) && dense_takes(kModeNN, rows, n, k, dy1, n)) {
         // A dense LoRA layer: dy B and the gradient of B ride in the decoding pass's launch, the gradient of A follows the

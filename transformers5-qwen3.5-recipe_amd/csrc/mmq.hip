@@ -130,7 +130,7 @@ static int launch_direct(const MmqParams& p, hipStream_t s) {
     const int col_tiles = (MODE == kModeNT ? p.nseg : 1) * p.col_tiles_per_seg;
     if (p.col_tiles_per_wg < 1) return set_error(GGQ_ERR_SHAPE, "mmq: column tiles per workgroup must be at least 1");
     const bool few_rows = MODE == kModeNN && p.few_rows;  // 512 columns per workgroup
-    if (few_rows && (p.k & 511)) return set_error(GGQ_ERR_SHAPE, "mmq: the grad-input kernel for few rows needs whole pairs of blocks");
+    if (few_rows && ((p.k & 511) || p.r_pad > 32)) return set_error(GGQ_ERR_SHAPE, "mmq: the grad-input kernel for few rows needs whole pairs of blocks and ranks up to 32");
     // row tiles are dealt round-robin over the eight XCDs; each XCD walks its row tiles' column-tile runs
     const int per_wg = few_rows ? 2 : p.col_tiles_per_wg;
     const int64_t total = (int64_t)((p.max_row_tiles + 7) / 8) * ((col_tiles + per_wg - 1) / per_wg);

@@ -17,7 +17,7 @@
 //   * every lane works out one (sub-block scale, min) pair of pairs (one row, one quant group) for all four waves;
 //   * a wave reads its dwords and scales, forms its eight operands and issues 8 x (row blocks of 16) MFMAs.
 // The LDS layouts are permuted so that all of these reads are free of bank conflicts (raw_chunk, scale_slot, a_slot32).  Sums and
-// roundings are those of mmq_direct8_nn.h, in the same order.
+// roundings are those of mmq_direct8_nn.h, in the same order (LoRA ranks up to 32): the same bits.
 //
 // What bounds it: the packed bytes (302 MB, 50 us) and, at 32 rows and more, the instructions of a step; with all packed rows in
 // L2 74 / 87 / 102 us at 16 / 32 / 48 rows.  The call (with dY . B, 9 us) for 256 experts of 5 / 16 / 32 / 48 / 64 rows each: 2 x 512
@@ -168,34 +168,32 @@ struct SmallNN {
         if (p.r_pad > 0) {
             const bf16_t* const factor = p.lb + expert * p.lb_expert_elems;  // [rank][k]
             const int c8 = l16 >> 3, cl = (4 * l16) & 31;                     // operand column c of set (hi, j): 64 c8 + 32 hi + cl + j
-            for (int r0 = 0; r0 < p.r_pad; r0 += 32) {
-                const int r = r0 + 8 * q;
-                bf16x8_t la[RB];
+            const int r = 8 * q;  // this lane's eight ranks of 32
+            bf16x8_t la[RB];
 #pragma unroll
-                for (int rb = 0; rb < RB; rb++)
-                    la[rb] = __builtin_bit_cast(bf16x8_t, r < p.r_pad ? *(const uint4*)(p.la + (int64_t)(row_begin + min(16 * rb + l16, rows_valid - 1)) * p.r_pad + r) : make_uint4(0, 0, 0, 0));
+            for (int rb = 0; rb < RB; rb++)
+                la[rb] = __builtin_bit_cast(bf16x8_t, r < p.r_pad ? *(const uint4*)(p.la + (int64_t)(row_begin + min(16 * rb + l16, rows_valid - 1)) * p.r_pad + r) : make_uint4(0, 0, 0, 0));
 #pragma unroll
-                for (int hi = 0; hi < 2; hi++) {
-                    uint2 f[8];  // four columns of eight ranks (zeros past the rank)
+            for (int hi = 0; hi < 2; hi++) {
+                uint2 f[8];  // four columns of eight ranks (zeros past the rank)
 #pragma unroll
-                    for (int i = 0; i < 8; i++) {
-                        f[i] = *(const uint2*)(factor + (int64_t)min(r + i, p.lora_rank - 1) * p.k + col0 + 64 * c8 + 32 * hi + cl);
-                        if (r + i >= p.lora_rank) f[i] = make_uint2(0, 0);
+                for (int i = 0; i < 8; i++) {
+                    f[i] = *(const uint2*)(factor + (int64_t)min(r + i, p.lora_rank - 1) * p.k + col0 + 64 * c8 + 32 * hi + cl);
+                    if (r + i >= p.lora_rank) f[i] = make_uint2(0, 0);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    uint32_t o[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const uint32_t e0 = j < 2 ? f[2 * i].x : f[2 * i].y, e1 = j < 2 ? f[2 * i + 1].x : f[2 * i + 1].y;
+                        o[i] = (j & 1) ? (e0 >> 16) | (e1 & 0xFFFF0000u) : (e0 & 0xFFFFu) | (e1 << 16);
                     }
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        uint32_t o[4];
+                    for (int rb = 0; rb < RB; rb++) {
+                        const f32x4_t t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Direct::as_operand(o), la[rb], (f32x4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            const uint32_t e0 = j < 2 ? f[2 * i].x : f[2 * i].y, e1 = j < 2 ? f[2 * i + 1].x : f[2 * i + 1].y;
-                            o[i] = (j & 1) ? (e0 >> 16) | (e1 & 0xFFFF0000u) : (e0 & 0xFFFFu) | (e1 << 16);
-                        }
-#pragma unroll
-                        for (int rb = 0; rb < RB; rb++) {
-                            const f32x4_t t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Direct::as_operand(o), la[rb], (f32x4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-                            for (int v = 0; v < 4; v++) acc[4 * hi + j][rb][v] = __builtin_fmaf(p.lora_scale, t[v], acc[4 * hi + j][rb][v]);
-                        }
+                        for (int v = 0; v < 4; v++) acc[4 * hi + j][rb][v] = __builtin_fmaf(p.lora_scale, t[v], acc[4 * hi + j][rb][v]);
                     }
                 }
             }
