@@ -69,6 +69,11 @@ int ggq_set_factor_gradient_overlap(int mode);
  * the stated tolerances whatever is chosen. */
 int ggq_debug_force_grouped_shape(int shape);
 
+/* Test aid with no counterpart in the reference: the tile and split count of the dense calls over decoded panels that follow
+ * (shape as ggq_debug_dense_plan names it, -1 = any; splits 0 = any, else that many where the contraction, the output's alignment and
+ * the workspace allow it).  FOR TESTS ONLY, under the conditions of ggq_debug_force_grouped_shape. */
+int ggq_debug_force_dense_tile(int shape, int splits);
+
 /* Test aid with no counterpart in the reference: the tile (0 = 256 x 256, 1 = 128 x 128, 2 = 64 x 64, 3 = 128 x 256) and the number of
  * contraction splits a dense call over decoded panels would run with in a workspace of ws_bytes.  Host only. */
 int ggq_debug_dense_plan(int grad_input, int64_t m, int64_t n, int64_t k, int64_t ws_bytes, int* shape, int* splits);

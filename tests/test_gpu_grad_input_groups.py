@@ -5,7 +5,7 @@ import statistics
 import pytest
 import torch
 
-from helpers import TYPE_NAMES
+from helpers import TYPE_NAMES, assert_close_bf16
 from oracle import gguf_blocks as gb
 
 pytestmark = pytest.mark.gpu
@@ -74,7 +74,7 @@ def test_iq2xxs_groups_beyond_a_tile_cost_what_they_cost_on_the_tile_kernel(pkg,
     assert times[0] <= 1.3 * times[1], f"{times[0]:.1f} us, tile kernel {times[1]:.1f} us"
 
 
-@pytest.mark.parametrize("rank", [0, 16, 40, 64])
+@pytest.mark.parametrize("rank", [0, 16, 32, 40, 64])
 @pytest.mark.parametrize("sizes", [[49, 63, 64, 65, 0, 0, 0], [127, 128, 129, 1] + [0] * 7, [192, 193, 0, 48] + [0] * 12, [255, 0, 0, 0, 0, 0, 0, 16]])
 def test_q4k_groups_beyond_a_tile_match_the_kernel_for_larger_groups(pkg, dev, sizes, rank):
     # the same rows with the empty groups left out average more rows than the rule takes: the eight-wave kernel, bit for bit
@@ -156,3 +156,111 @@ def test_iq2xxs_workspace_without_room_for_the_small_tables_keeps_the_tile_kerne
     with pytest.raises(RuntimeError, match="workspace too small"):
         pkg._lib.check(lib.ggq_grouped_lora_mmq_backward(dy.data_ptr(), None, w.data_ptr(), None, ids.data_ptr(), ends.data_ptr(), groups, groups, qt, rows, n, k,
                                                          x.data_ptr(), x.data_ptr(), *lora, dx.data_ptr(), None, None, None, ws.data_ptr(), small - 256, stream))
+
+
+@pytest.mark.parametrize("tokens,experts,skew", [
+    (500, 256, 0.0),     # Q4_K tiles of 64 rows, the caller's tables, a cotangent read through the routing permutation
+    (700, 256, 0.25),    # and groups of several tiles among them
+    (1601, 16, 0.0),     # factor gradients of a gathered matrix of more than 6 MB: units in the order of its column blocks
+])
+def test_backward_of_a_combined_output(pkg, dev, tokens, experts, skew):
+    # against the same rows materialised with tables built by the call (bit for bit), and fp32 products of sampled experts
+    qt, n, k, top_k, rank, s = gb.Q4_K, 2048, 512, 8, 16, 2.0
+    lib, stream = pkg._lib.load(), torch.cuda.current_stream().cuda_stream
+    gen = torch.Generator(device=dev).manual_seed(60 + experts)
+    scores = torch.rand(tokens, experts, generator=gen, device=dev)
+    scores[:, 3:6] += skew
+    idx, weights = scores.topk(top_k, dim=1).indices, torch.rand(tokens, top_k, generator=gen, device=dev)
+    plan = pkg.fast_moe_routing.prepare_expert_routing(_rows(dev, 61, tokens, n), idx, weights, experts, gather=False)
+    perm, ends, rows = plan.permutation, plan.expert_end_offsets, tokens * top_k
+    w, ids = _payload(dev, 62, qt, experts, n, k), torch.arange(experts, device=dev)
+    grad_out, x, xa = _rows(dev, 63, tokens, n), _rows(dev, 64, rows, k), _rows(dev, 65, rows, rank)
+    a, b = (0.02 * _rows(dev, 66, experts * rank, k)).view(experts, rank, k), (0.02 * _rows(dev, 67, experts * n, rank)).view(experts, n, rank)
+    tables = torch.empty(lib.ggq_group_tables_bytes(rows, experts, experts), dtype=torch.uint8, device=dev)
+    pkg._lib.check(lib.ggq_group_tables_build(ids.data_ptr(), ends.data_ptr(), experts, experts, rows, tables.data_ptr(), tables.numel(), stream))
+    ws = torch.empty(lib.ggq_lora_workspace_bytes(rows, experts, experts, n, k, rank), dtype=torch.uint8, device=dev)
+    dx, dx_rows = (torch.empty(rows, k, dtype=torch.bfloat16, device=dev) for _ in range(2))
+    da, db = torch.empty_like(a), torch.empty_like(b)
+    pkg._lib.check(lib.ggq_grouped_lora_mmq_backward_routed_output(
+        grad_out.data_ptr(), tokens, perm.data_ptr(), top_k, weights.data_ptr(), 0, w.data_ptr(), ids.data_ptr(), ends.data_ptr(), experts, experts, qt, rows, n, k,
+        x.data_ptr(), xa.data_ptr(), a.data_ptr(), b.data_ptr(), rank, s, dx.data_ptr(), da.data_ptr(), db.data_ptr(), tables.data_ptr(), ws.data_ptr(), ws.numel(), stream))
+    dy = grad_out[perm // top_k].contiguous()
+    pkg._lib.check(lib.ggq_grouped_lora_mmq_backward(
+        dy.data_ptr(), None, w.data_ptr(), None, ids.data_ptr(), ends.data_ptr(), experts, experts, qt, rows, n, k,
+        x.data_ptr(), xa.data_ptr(), a.data_ptr(), b.data_ptr(), rank, s, dx_rows.data_ptr(), None, None, None, ws.data_ptr(), ws.numel(), stream))
+    assert torch.equal(dx, dx_rows)
+    bounds, route_weights = [0] + ends.tolist(), weights.reshape(-1)[perm].bfloat16().float()[:, None]  # (weights act at bf16 precision)
+    for e in {0, 3, 7, experts - 1}:
+        r = slice(bounds[e], bounds[e + 1])
+        if r.start == r.stop:
+            continue
+        d, we = dy[r].float(), pkg.gguf.dequantize_gguf_tensor(pkg.gguf.GGUFQuantizedTensor(w[e : e + 1], qt, (1, n, k)), qt, torch.float32)[0].bfloat16().float()
+        dyb = (d @ b[e].float()).bfloat16().float()
+        assert_close_bf16(dx[r], (d @ we + s * dyb @ a[e].float()).double(), f"dX of expert {e}")
+        # (dY . B may round to the neighbour, a bf16 step of each of its terms, and once more with its weight)
+        assert_close_bf16(da[e], (s * (route_weights[r] * dyb).bfloat16().float().T @ x[r].float()).double(), f"dA of expert {e}", ulps=4)
+        assert_close_bf16(db[e], (s * d.T @ (route_weights[r] * xa[r].float()).bfloat16().float()).double(), f"dB of expert {e}")
+
+
+@pytest.mark.parametrize("tokens,k", [(1601, 2048), (801, 4096), (300, 512)])
+def test_factor_gradients_of_tokens_read_in_place(pkg, dev, tokens, k):
+    # the order of the units (column blocks outer beyond 6 MB) against the gathered copy's, bit for bit
+    ml, mr = pkg.fast_moe_lora, pkg.fast_moe_routing
+    qt, n, experts, top_k, rank = gb.Q4_K, 256, 24, 8, 16
+    x, w = _rows(dev, 70, tokens, k), [_payload(dev, 71 + i, qt, experts, n, k) for i in range(2)]
+    idx = torch.rand(tokens, experts, generator=torch.Generator(device=dev).manual_seed(73), device=dev).topk(top_k, dim=1).indices
+    a, b = _rows(dev, 74, experts * rank, k).view(experts, rank, k), _rows(dev, 75, experts * 2 * n, rank).view(experts, 2 * n, rank)
+    ids, dy = torch.arange(experts, device=dev), [_rows(dev, 76 + i, tokens * top_k, n) for i in range(2)]
+    got = []
+    for in_place in (True, False):
+        plan = mr.prepare_expert_routing(x, idx, torch.full((tokens, top_k), 0.125, device=dev), experts, gather=not in_place)
+        ad, bd = a.clone().requires_grad_(True), b.clone().requires_grad_(True)
+        if in_place:
+            out = ml._RoutedGroupedLoraProjection.apply(x, plan.permutation, plan.inverse_permutation, top_k, *w, ids, plan.expert_end_offsets, qt, n, ad, bd, 2.0)
+        else:
+            rows, ends = plan.selected_hidden_states, plan.expert_end_offsets
+            out = ml._GroupedLoraProjection.apply(rows, *w, ids, ends, qt, n, ad, bd, 2.0)
+        torch.autograd.backward(out, dy)
+        got.append((ad.grad, bd.grad))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    bounds, e = [0] + ends.tolist(), 5
+    r = slice(bounds[e], bounds[e + 1])
+    d = torch.cat([t[r] for t in dy], dim=1).float()
+    dyb, xa = (d @ b[e].float()).bfloat16().float(), (rows[r].float() @ a[e].float().T).bfloat16().float()
+    assert_close_bf16(got[0][0][e], (2.0 * dyb.T @ rows[r].float()).double(), "dA")
+    assert_close_bf16(got[0][1][e], (2.0 * d.T @ xa).double(), "dB")
+
+
+@pytest.mark.parametrize("qt,n", [(gb.Q4_K, 256), (gb.IQ2_XXS, 256)], ids=lambda v: TYPE_NAMES.get(v, str(v)))
+def test_an_output_at_any_address(pkg, dev, qt, n):
+    # stores of a row that is not 16-byte aligned, element by element
+    k, groups = 4096, 64
+    lib, stream = pkg._lib.load(), torch.cuda.current_stream().cuda_stream
+    sizes = ([1, 17, 48, 66, 0] * groups)[:groups]
+    rows, w, ids, ends = sum(sizes), _payload(dev, 80, qt, groups, n, k), torch.arange(groups, device=dev), _ends(dev, sizes)
+    assert rows <= 40 * groups
+    dy, ws = _rows(dev, 81, rows, n), torch.empty(lib.ggq_lora_workspace_bytes(rows, groups, groups, n, k, 0), dtype=torch.uint8, device=dev)
+    got = []
+    for skip in (0, 1):
+        buffer = torch.zeros(rows * k + 8, dtype=torch.bfloat16, device=dev)
+        pkg._lib.check(lib.ggq_grouped_lora_mmq_backward(dy.data_ptr(), None, w.data_ptr(), None, ids.data_ptr(), ends.data_ptr(), groups, groups, qt, rows, n, k, None, None,
+                                                         None, None, 0, 0.0, buffer.data_ptr() + 2 * skip, None, None, None, ws.data_ptr(), ws.numel(), stream))
+        got.append(buffer[skip : skip + rows * k])
+        assert not buffer[:skip].any() and not buffer[skip + rows * k :].any()
+    assert torch.equal(*got) and got[0].any()
+
+
+def test_iq2xxs_pair_of_skewed_groups_beside_tall_tiles(pkg, dev, force_grouped_shape):
+    # groups of every table of one call: small, wide and tall, with a pair of matrices; bit for bit the tile kernel's results
+    qt, n, k, groups, ml = gb.IQ2_XXS, 256, 4096, 64, pkg.fast_moe_lora
+    sizes = ([300, 0, 0, 0, 81, 7, 131, 0, 512, 0, 0, 0, 0, 80, 0, 1] * groups)[:groups]
+    assert sum(sizes) <= 72 * groups
+    ids, ends = torch.arange(groups, device=dev), _ends(dev, sizes)
+    planes, cotangents, x = [_payload(dev, 90 + i, qt, groups, n, k) for i in range(2)], [_rows(dev, 92 + i, sum(sizes), n) for i in range(2)], _rows(dev, 94, sum(sizes), k)
+    got = []
+    for shape in ("", "1"):
+        force_grouped_shape(shape)
+        xd = x.clone().requires_grad_(True)
+        torch.autograd.backward(ml.grouped_mmq_pair(xd, *planes, ids, ends, qt, n), cotangents)
+        got.append(xd.grad)
+    assert torch.isfinite(got[0]).all() and torch.equal(*got)

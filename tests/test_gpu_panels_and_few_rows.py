@@ -2,6 +2,7 @@
 where they can go wrong: tile edges, split contractions, ragged rows and columns, the ends of each range."""
 
 import contextlib
+import ctypes
 
 import numpy as np
 import pytest
@@ -44,13 +45,28 @@ def _check_lora(pkg, dev, payload, qt, x, a, b, s, dy):
     (1500, 2052, 1024, 8),  # 128 x 128 tiles forward
     (3001, 5001, 256, 16),  # 256 x 256 tiles, ragged both ways; the shortest contraction
     (4096, 1028, 2048, 4),
-    (1999, 4097, 2048, 16),  # 128 x 256 tiles forward, ragged both ways
-    (4003, 4100, 2048, 24),  # and in the grad-input; a contraction that ends inside a step
+    (1999, 4097, 2048, 16),  # ragged both ways
+    (4003, 4100, 2048, 24),  # 128 x 256 tiles in the grad-input; a contraction that ends inside a step
 ])
 @pytest.mark.parametrize("qt", [gb.Q8_0, gb.Q4_K, gb.IQ2_XXS], ids=lambda q: TYPE_NAMES[q])
 def test_dense_lora_over_panels(pkg, dev, qt, m, n, k, r):
     payload, x, a, b, dy = _lora_case(7000 + m + n, m, n, k, r, qt)
     _check_lora(pkg, dev, payload, qt, x, a, b, 32.0 / r, dy)
+
+
+@pytest.mark.parametrize("n,splits", [(1301, 1), (1304, 1), (1304, 3), (1304, 4)])  # an odd column count; forward splits of 7, 7, 6 steps, grad-input of 6, 6, 6, 3
+@pytest.mark.parametrize("shape,rows", [(0, 517), (1, 515), (2, 131), (3, 389)])
+def test_every_panel_tile_at_ragged_sizes(pkg, dev, shape, rows, n, splits):
+    lib, k, qt = pkg._lib.load(), 1280, gb.Q4_K
+    payload, x, a, b, dy = _lora_case(shape + n, rows, n, k, 24, qt)
+    try:
+        pkg._lib.check(lib.ggq_debug_force_dense_tile(shape, splits))
+        got = [ctypes.c_int(), ctypes.c_int()]
+        pkg._lib.check(lib.ggq_debug_dense_plan(0, rows, n, k, 1 << 40, *map(ctypes.byref, got)))
+        assert [v.value for v in got] == [shape, splits if n % 4 == 0 else 1]
+        _check_lora(pkg, dev, payload, qt, x, a, b, 1.5, dy)
+    finally:
+        pkg._lib.check(lib.ggq_debug_force_dense_tile(-1, 0))
 
 
 def test_a_workspace_without_room_for_panels_keeps_the_tile_kernel(pkg, dev):

@@ -1,12 +1,14 @@
 """Static check of the compiled decoding-wave kernels: no instruction touches a register that an untracked load still owns.
 
-The kernels in csrc/mmq_small_iq2.h, csrc/mmq_direct8.h and csrc/mmq_direct8_nn.h request packed bytes several steps ahead
-with inline-asm loads the compiler does not track, and wait for them with exact `s_waitcnt vmcnt` counts.  The compiler
-is free to copy such a register (a loop-carried copy at the back edge, a hoisted read) while its load is still on its
-way, which copies stale data and loses the load's result: wrong numbers without any fault.  This test compiles the three
-kernels to gfx950 assembly and replays every loop body twice against the in-order queue of vector-memory operations:
-between an inline-asm load into a VGPR and the wait that retires it, no instruction may name that VGPR.  It also checks
-that the loops hold no scratch (spill) traffic, which would drain the queue through compiler-made waits.
+These kernels request packed bytes, activation rows and LoRA factor pieces several steps ahead with inline-asm loads the
+compiler does not track, most of them straight to LDS and a few into registers (a factor piece in csrc/mmq_direct8.h and
+csrc/mmq_direct8_nn.h), and wait for them with exact `s_waitcnt vmcnt` counts.  The compiler is free to copy such a
+register (a loop-carried copy at the back edge, a hoisted read) while its load is still on its way, which copies stale
+data and loses the load's result: wrong numbers without any fault.  This test compiles the kernels to gfx950 assembly and
+replays every loop body twice against the in-order queue of vector-memory operations: between an inline-asm load into a
+VGPR and the wait that retires it, no instruction may name that VGPR.  It also checks that the loops hold no scratch
+(spill) traffic, which would drain the queue through compiler-made waits; csrc/mmq_small_iq2.h and csrc/mmq_small_nn_iq2.h
+do spill, outside them.
 
 It also guards the compiler's own LDS waits.  A load through a pointer selected between LDS and global memory is a flat
 load; the compiler never sees these kernels' inline-asm `vmcnt` waits, so it takes such a load for outstanding through
@@ -26,6 +28,8 @@ KERNELS = {
     "mmq_small_iq2xxs_kernel": "mmq_small_iq2.h",
     "mmq_direct8_q4k_kernel": "mmq_direct8.h",
     "mmq_direct8_nn_q4k_kernel": "mmq_direct8_nn.h",
+    "mmq_small_nn_q4k_kernel": "mmq_small_nn.h",
+    "mmq_small_nn_iq2xxs_kernel": "mmq_small_nn_iq2.h",
 }
 VMEM = re.compile(r"^(global_load|global_store|global_atomic|buffer_load|buffer_store|scratch_load|scratch_store|flat_load|flat_store)")
 REG = re.compile(r"\bv(\d+)\b|\bv\[(\d+):(\d+)\]")

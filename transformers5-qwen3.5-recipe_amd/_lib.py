@@ -31,6 +31,7 @@ SIGNATURES: dict[str, tuple] = {
     "ggq_set_factor_gradient_overlap": (_I, [_I]),
     "ggq_measure_mfma_ceiling": (_I, [_P, _P, _L, _I, _P, _P, _P]),
     "ggq_debug_force_grouped_shape": (_I, [_I]),
+    "ggq_debug_force_dense_tile": (_I, [_I, _I]),
     "ggq_debug_dense_plan": (_I, [_I, _L, _L, _L, _L, _P, _P]),
     "ggq_supports_quant_type": (_I, [_I]),
     "ggq_row_bytes": (_L, [_I, _L]),

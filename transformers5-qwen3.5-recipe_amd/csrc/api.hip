@@ -145,6 +145,12 @@ int ggq_debug_force_grouped_shape(int shape) {
     return GGQ_OK;
 }
 
+int ggq_debug_force_dense_tile(int shape, int splits) {
+    if (shape < -1 || shape > 3 || splits < 0) return set_error(GGQ_ERR_SHAPE, "debug_force_dense_tile: unknown shape %d or splits %d", shape, splits);
+    g_dense_shape.store(shape), g_dense_splits.store(splits);
+    return GGQ_OK;
+}
+
 int ggq_debug_dense_plan(int grad_input, int64_t m, int64_t n, int64_t k, int64_t ws_bytes, int* shape, int* splits) {
     if (!shape || !splits) return set_error(GGQ_ERR_NULL, "debug_dense_plan: null pointer");
     if (m <= 0 || n <= 0 || k <= 0) return set_error(GGQ_ERR_SHAPE, "debug_dense_plan: bad shape m=%lld n=%lld k=%lld", (long long)m, (long long)n, (long long)k);
@@ -183,7 +189,7 @@ static int launch_wide_and_tall(int qt, int mode, MmqParams& p, int rows, int n,
 // tall tiles.
 static int pick_shape(int qt, int64_t rows, int64_t groups, bool direct_ok) {
     const int forced = g_shape_override.load();  // a test aid
-    const bool q4k = qt == 12;            // GGML Q4_K: the only block format with decoding-wave kernels
+    const bool q4k = qt == 12;            // GGML Q4_K (IQ2_XXS has decoding-wave kernels of its own beside the wide shape)
     if (q4k && direct_ok && (forced == kShapeDirect || (forced < 0 && groups > 0 && rows <= 256 * groups))) return kShapeDirect;
     if (forced == kShapeTall || !(groups > 0 && rows <= 192 * groups)) return kShapeTall;
     return kShapeWide;

@@ -666,19 +666,24 @@ bool dense_panel_whole(int64_t n, int64_t k) { return slab_columns(n, k) >= n &&
 // A larger tile reads less per output: 256 x 256 wins where it fills the chip in whole rounds or by splits (4096 x 8192 over
 // 2048: 119 us against 128 with 128 x 128), 128 x 256 where it would leave a half of it idle (4096 x 2048 over 8192: 113 us
 // against 154, and 122 with 128 x 128), the smaller ones for short sequences.
+std::atomic<int> g_dense_shape{-1}, g_dense_splits{0};  // ggq_debug_force_dense_tile (a test aid): the automatic choice
+
 // max_splits: what the output's alignment and the workspace allow (with none, the shape chosen for ten splits can leave most of the
 // chip idle: 701 x 2048 over 32768, 577 us against 207 with the shape for one).
 static void pick_tile(int64_t m, int64_t cols, int64_t steps, int64_t max_splits, int& shape, int& splits) {
     static const struct { int rows, cols, slots; double idle, full, fixed; } kShape[4] = {
         {256, 256, 256, 1.05, 1.40, 6.0}, {128, 128, 512, 0.36, 0.90, 2.5}, {64, 64, 512, 0.11, 0.30, 2.5}, {128, 256, 256, 0.50, 0.80, 5.0}};  // (fixed: a tile's start and end)
     double best = 1e30;
-    shape = 0, splits = 1;
+    const int only_shape = g_dense_shape.load(std::memory_order_relaxed), only_splits = g_dense_splits.load(std::memory_order_relaxed);
+    shape = std::max(only_shape, 0), splits = 1;
     for (int sh = 0; sh < 4; sh++) {
+        if (only_shape >= 0 && sh != only_shape) continue;
         const auto& t = kShape[sh];
         const int64_t tiles = ((m + t.rows - 1) / t.rows) * ((cols + t.cols - 1) / t.cols);
         for (int sp = 1; sp <= max_splits; sp++) {
             const int64_t per = (steps + sp - 1) / sp;
             if (sp > 1 && (per < 4 || (sp - 1) * per >= steps)) continue;
+            if (only_splits > 0 && sp != std::min<int64_t>(only_splits, max_splits)) continue;
             const int64_t units = tiles * sp, rounds = units / t.slots, rest = units % t.slots;
             const double load = (double)rest / t.slots, slow = sh == 0 ? load * load : load;
             double est = 3.0 + rounds * (per * t.full + t.fixed) + (rest ? per * (t.idle + (t.full - t.idle) * slow) + t.fixed : 0.0);

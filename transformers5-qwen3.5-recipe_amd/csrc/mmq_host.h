@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <atomic>
 
 namespace ggq {
 
@@ -63,7 +64,7 @@ struct FactorGradParams {
 };
 
 constexpr int kBM = 256, kBN = 128, kBK = 64;  // the tall tile shape (dense launches, large expert groups)
-constexpr int kWideBM = 128, kWideBN = 256;    // the wide tile shape (Q4_K expert groups of about a hundred rows)
+constexpr int kWideBM = 128, kWideBN = 256;    // the wide tile shape (expert groups of about a hundred rows)
 constexpr int kDirectBM = 192, kDirectBN = 256;  // the direct shape (Q4_K expert groups: the MFMA waves decode the weights themselves)
 constexpr int64_t kSmallNNRowsPerGroup = 40;    // Q4_K grad-input on tiles of 64 rows (mmq_small_nn.h): groups that average at most this many
 constexpr int kSmallNNIq2Rows = 80;             // IQ2_XXS grad-input (mmq_small_nn_iq2.h): groups of at most this many rows, a tile each
@@ -123,7 +124,7 @@ int profile_end(float* ms, int* qt, int* mode, int* epi, int* shape, int capacit
 int measure_mfma_ceiling(const void* a_samples, const void* b_samples, int64_t elems, int iters, void* sink_buffer, float* tflops_out, hipStream_t s);
 const char* last_error();
 int launch_mmq(int qt, int mode, int epi, const MmqParams& p, hipStream_t s);
-int launch_mmq_mixed(int qt, int mode, const MmqParams& p, hipStream_t s);  // Q4_K, store epilogue, tiles + tiles2
+int launch_mmq_mixed(int qt, int mode, const MmqParams& p, hipStream_t s);  // every format, store epilogue, tiles + tiles2
 int launch_mmq_small(const MmqParams& p, hipStream_t s);  // IQ2_XXS forward, store epilogue, tiles of kSmallBM rows
 int launch_mmq_small_nn(const MmqParams& p, hipStream_t s);  // its grad-input
 int init_params(MmqParams& p, int qt, int mode, int m, int n, int k, int nseg, int shape = kShapeTall);
@@ -169,6 +170,7 @@ constexpr int kDenseSideMaxRank = 32;
 bool dense_side_takes(const DenseSide& side);
 bool dense_takes(int mode, int64_t m, int64_t n, int64_t k, const void* a, int64_t lda, bool a_zero_padded = false);
 bool dense_panel_whole(int64_t n, int64_t k);
+extern std::atomic<int> g_dense_shape, g_dense_splits;  // (tests: the only tile shape and split count; -1 and 0: any)
 void dense_plan(int mode, int64_t m, int64_t n, int64_t k, int64_t ws_bytes, int& shape, int& splits);  // of the first slab of columns
 int64_t dense_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int dense_mmq(const DenseCall& q, void* ws, int64_t ws_bytes, hipStream_t s, const DenseSide* side = nullptr);
