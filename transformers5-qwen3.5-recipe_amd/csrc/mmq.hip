@@ -147,7 +147,7 @@ static int launch_direct(const MmqParams& p, hipStream_t s) {
         g_timed_count++;
         (void)hipEventRecord(t->start, s);
     }
-    if (few_rows) {  // (its 40 KB need no raised limit)
+    if (few_rows) {  // (its 43 KB need no raised limit)
         hipLaunchKernelGGL(mmq_small_nn_q4k_kernel, dim3((unsigned)grid), dim3(SmallNN::kThreadsWG), SmallNN::kLdsBytes, s, p);
         if (t) (void)hipEventRecord(t->stop, s);
         return check_launch("mmq_small_nn_q4k_kernel");

@@ -17,10 +17,10 @@
 //     order, so the lane half reads the matching 16-byte slot (4 h + i) of the A row.  No decoded weight touches LDS.
 // All requests of the loop are inline-asm loads the compiler does not track, in a fixed order, waited for with exact counts (vector
 // memory operations complete in issue order).
-// The workgroup keeps 77 KB of LDS (73 KB dynamic, the tables static) and at most 128 registers per lane, so two workgroups share a
-// compute unit and cover each other's barriers.  The weights are the MFMA's first operand, so a lane's accumulator registers hold
-// four consecutive columns of one row; a finished row block goes through a wave-private LDS block (in the ring, idle by then) and
-// leaves as 64-byte row pieces, the LoRA term added there.
+// The workgroup keeps 77 KB of LDS (73 KB dynamic, the tables static) and at most 128 registers per lane (the rest, 364 bytes per lane,
+// is spilled outside the contraction loops), so two workgroups share a compute unit and cover each other's barriers.  The weights are
+// the MFMA's first operand, so a lane's accumulator registers hold four consecutive columns of one row; a finished row block goes
+// through a wave-private LDS block (in the ring, idle by then) and leaves as 64-byte row pieces, the LoRA term added there.
 //
 // What bounds it: requests, decoding and MFMAs add up rather than overlap.  256 experts, 2 x 2048 rows of W, k 4096, 64 rows each:
 // 740 us; with eight bytes per lane and step asked for straight into registers (a request of 32 cache lines) 797, with four words
@@ -62,7 +62,7 @@ struct SmallIq2 {
     static constexpr int kPackedBase = kLaBase + kTM * 32;                          // then a block of every column per wave, as five 16-byte chunks
     static constexpr int kPackedPitch = 80, kPackedBytes = 32 * kPackedPitch;
     static constexpr int kLdsBytes = kPackedBase + kWaves * kPackedBytes + 16;      // 48 + 4 + 20 = 72 KB of dynamic LDS (a run's third dword may lie past the last block)
-    // (the decoder's tables, 6 KB, are a static array: it sits at LDS address 0, which the compiler then folds into the lookups)
+    // (the decoder's tables, 4.5 KB, are a static array: it sits at LDS address 0, which the compiler then folds into the lookups)
     static constexpr int kOutBase = 0;  // eight 2 KB staging blocks of the epilogue: over the ring, which a finished tile no longer needs
 
     using RowCtx = Direct::RowCtx;

@@ -34,7 +34,7 @@ struct SmallNN {
     static constexpr int kStages = 3;
     static constexpr int kRawBytes = 32 * 288, kABytes = kRows * 64;
     static constexpr int kScaleBase = kStages * (kRawBytes + kABytes);
-    static constexpr int kLdsBytes = kScaleBase + 32 * 8 * 16;  // 40 KB
+    static constexpr int kLdsBytes = kScaleBase + 32 * 8 * 16;  // 43 KB
 
     // Chunk (16 bytes) of a raw stage that holds piece (0..17) of weight row 8 q + i: rows 8 q + i, q = 0..3, side by side, their
     // pieces turned by two per q, so that the same piece of the four rows falls on four different quarters of the banks.

@@ -17,10 +17,11 @@
 //     sixteen rows.
 //
 // What bounds it: LDS (the codebook reads are random: 15 cycles for 64 lanes' 16 bytes, which is why a group's signs are one word,
-// doubled from pair to pair, instead of four words of a table: 650 -> 595 us at 16 rows) and, beside it, the instructions of two
-// waves per SIMD; with sixty-four columns per wave and four waves per SIMD it takes 892 us.  256 experts, 2 x 2048 rows of W,
-// k 4096: 595 / 714 / 804 / 910 us at 16 / 48 / 64 / 80 rows per expert, against 853 / 986 / 1000 / 1132 of the tile kernel; 4096
-// rows of W, k 2048: 323 / 391 / 445 / 490 against 426 / 513 / 539 / 582.  Groups of more than 80 rows stay there.
+// doubled from pair to pair, instead of four words of a table: 8 % less at 16 rows) and, beside it, the instructions of two waves per
+// SIMD; sixty-four columns per wave and four waves per SIMD take 1.4 times as long.  256 experts, 2 x 2048 rows of W, k 4096: 541 / 660 / 743 /
+// 823 us at 16 / 48 / 64 / 72 rows per expert, against 834 / 973 / 991 / 1083 of the tile kernel (with rank 16, the call with dY . B: 569 /
+// 685 / 778 / 855 against 866 / 1015 / 1037 / 1128); 4096 rows of W, k 2048: 284 / 335 / 383 / 418 against 423 / 493 / 504 / 549.  Groups of
+// more than 80 rows stay there.
 #pragma once
 #include "mmq_small_iq2.h"
 
@@ -141,7 +142,7 @@ struct SmallNNIq2 {
 #pragma unroll
             for (int rb = 0; rb < RB; rb++) acc[s][rb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
         // this lane's records: weight rows 8 q + i (+ 256 i bytes), sub-block 4 wave + l16 % 4, of it group l16 / 4 (in this order the four
-        // lanes of a row store 64 contiguous bytes: 796 -> 778 us at 64 rows, 0.6 % of a step)
+        // lanes of a row store 64 contiguous bytes: 2 % of the launch at 64 rows)
         const uint32_t rec_at = opaque(kRecBase + rec_slot(8 * q, 4 * wave + (l16 & 3)) * 16);
         const uint32_t idx_rot = (8 * (l16 >> 2) + 28) & 31, sgn_rot = (7 * (l16 >> 2) + 30) & 31;  // (the byte ends up at bit 4, the seven bits at bit 2: entries of 16 and of 4 bytes)
         const uint32_t a_at = opaque(kABase + a_slot32(l16, q) * 16);
