@@ -62,8 +62,8 @@ int ggq_set_factor_gradient_overlap(int mode);
 
 /* Test aid with no counterpart in the reference: force the kernel family of the grouped launches that follow (0 = tall
  * tiles, 1 = the wide / tall tile mix and nothing else, 3 = the Q4_K kernels whose MFMA waves decode the weights themselves,
- * 5 = the wide / tall mix with the IQ2_XXS forward of groups of up to 128 rows on its decoding-wave kernel, which is also what
- * IQ2_XXS calls get by default, each wherever its operand conditions hold; -1 = the library's own choice, the default).
+ * 5 = the wide / tall mix with the IQ2_XXS small groups on their decoding-wave kernels, which is also what IQ2_XXS calls get by
+ * default, each wherever its operand conditions hold; -1 = the library's own choice, the default).
  * FOR TESTS ONLY: a process-wide setting that stays until it is set back to -1 and changes the kernel choice of every later
  * caller in the process; not thread safe (no launch may run in another thread while it changes); results are the same to
  * the stated tolerances whatever is chosen. */
