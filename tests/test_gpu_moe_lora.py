@@ -91,11 +91,11 @@ def test_q4k_grouped_grad_input_decoding_waves(pkg, dev):
 
 
 @pytest.mark.parametrize("qt,sizes,n,r,pair", [
-    (gb.Q4_K, [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 0, 97, 5, 2], 256, 16, True),  # every count of 16-row blocks, groups walked in two and three parts
+    (gb.Q4_K, [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 0, 97, 5, 2], 256, 16, True),  # every count of 16-row blocks, a group of two tiles
     (gb.Q4_K, [1, 40, 16, 0, 3], 256, 0, False),
     (gb.Q4_K, [20, 7, 48, 33], 128, 4, True),      # four 64-row steps, the fewest; a rank padded to 16
-    (gb.Q4_K, [9, 33, 50], 320 + 64, 40, False),   # a rank padded to 48: a half-filled second factor step
-    (gb.IQ2_XXS, [1, 15, 16, 17, 33, 48, 49, 64, 65, 80, 81, 128, 129, 0, 2], 128, 16, True),  # ... groups walked in two parts, a tall tile
+    (gb.Q4_K, [9, 33, 50], 320 + 64, 40, False),   # a rank padded to 48: the kernel for larger groups
+    (gb.IQ2_XXS, [1, 15, 16, 17, 33, 48, 49, 64, 65, 80, 81, 128, 129, 0, 2], 128, 16, True),  # ... groups of wide tiles, a tall tile
     (gb.IQ2_XXS, [3, 0, 79, 64], 128, 0, False),   # one group of four steps
     (gb.IQ2_XXS, [70, 9, 96], 384, 40, False),
 ])
