@@ -54,6 +54,18 @@ def test_dense_lora_over_panels(pkg, dev, qt, m, n, k, r):
     _check_lora(pkg, dev, payload, qt, x, a, b, 32.0 / r, dy)
 
 
+@pytest.mark.parametrize("m,n,k,r", [
+    (49, 72, 256, 8),       # fewer spans of 128 than waves, the only one partial; half of the padded rank
+    (65, 136, 512, 12),     # a rank that is no multiple of eight; a second span of eight elements
+    (130, 1544, 1792, 16),  # spans beyond the ones in flight: twelve whole and a partial one over four waves
+    (100, 1096, 3072, 24),  # the same with two blocks of ranks, the second one half full
+    (64, 2048, 3328, 32),
+])
+def test_rank_sized_products_beside_the_decoding_pass(pkg, dev, m, n, k, r):
+    payload, x, a, b, dy = _lora_case(7100 + n + k, m, n, k, r, gb.Q8_0)
+    _check_lora(pkg, dev, payload, gb.Q8_0, x, a, b, 32.0 / r, dy)
+
+
 @pytest.mark.parametrize("n,splits", [(1301, 1), (1304, 1), (1304, 3), (1304, 4)])  # an odd column count; forward splits of 7, 7, 6 steps, grad-input of 6, 6, 6, 3
 @pytest.mark.parametrize("shape,rows", [(0, 517), (1, 515), (2, 131), (3, 389)])
 def test_every_panel_tile_at_ragged_sizes(pkg, dev, shape, rows, n, splits):

@@ -100,56 +100,66 @@ __global__ __launch_bounds__(256) void decode_panel_kernel(DecodeParams p) {
     decode_panel_body<QT>(p, blockIdx.x, lds);
 }
 
-// ---- out[m, 0..r_pad) = In[m, :] . F^T for sixteen rows: the four waves deal the contraction out in spans of 128, the next
-// span's loads in flight under the current one's MFMAs, and add their sums in wave order.  F is [r][ldf] (contraction
-// contiguous), or [contraction][r] (f_natural): then a span of it goes through the wave's own LDS as [128][r_pad] and the
-// operand is read back transposed.
+// ---- out[m, 0..r_pad) = In[m, :] . F^T for sixteen rows: the four waves deal the contraction out in spans of 128 and add
+// their sums in wave order.  F is [r][ldf] (contraction contiguous), or [contraction][r] (NATURAL): then a span of it goes
+// through the wave's own LDS as [128][r_pad] and the operand is read back transposed.
+// What bounds it is latency: a few dozen workgroups on part of the chip.  So DEPTH spans are in flight per wave, and no load
+// stands behind a branch (there the compiler waits for every load before it): past the end of the contraction or of the rank
+// a lane reads the last whole piece and drops it.  VEC: whole, aligned pieces of F's rows (NATURAL: r is a multiple of eight).
+// The launch with the decoding pass, rank 16, forward / backward: 512 rows, 2048 x 2048 Q8_0 13.9 / 11.6 -> 11.3 / 9.6 us; 1021
+// rows, 512 x 2048 Q6_K 9.6 / 7.0 -> 7.0 / 6.8; 4096 rows, 4096 x 2048 Q4_K 14.4 / 20.0 -> 13.6 / 18.9 (there at the memory's rate).
 template <int JB>
 struct ThinLds {
     bf16_t f[4][128][JB * 16];
     f32x4_t red[4][JB][64];
 };
-template <int JB>
+__device__ __forceinline__ uint4 kept_if(bool keep, const uint4& v) { return make_uint4(keep ? v.x : 0u, keep ? v.y : 0u, keep ? v.z : 0u, keep ? v.w : 0u); }
+template <int JB, bool NATURAL, bool VEC>
 __device__ __forceinline__ void thin_product_body(const SkinnyNtParams& p, int wg, ThinLds<JB>& lds) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int DEPTH = JB == 1 ? 3 : 2;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 15, lq = lane >> 4;
     const int m0 = wg * 16, spans = (p.c + 127) / 128;
     const bf16_t* in = p.in[0] + (int64_t)min(m0 + li, p.m - 1) * p.ld_in;
-    const bool vec = (p.r & 7) == 0;
     f32x4_t acc[JB];
 #pragma unroll
     for (int jb = 0; jb < JB; jb++) acc[jb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-    uint4 x[4], f[JB][4];
-    auto load = [&](int span) __attribute__((always_inline)) {
+    uint4 x[DEPTH][4], f[DEPTH][JB][4];
+    // NATURAL: piece (jb, i) of a span is contraction row ((4 jb + i) 64 + lane) / (2 JB), the lane's eight columns from j
+    const int nat_j = lane % (2 * JB) * 8, nat_row = lane / (2 * JB);
+    auto load = [&](int d, int span) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int e = span * 128 + 32 * i + 8 * lq;
-            x[i] = e < p.c ? *(const uint4*)(in + e) : make_uint4(0, 0, 0, 0);
-        }
+        for (int i = 0; i < 4; i++) x[d][i] = *(const uint4*)(in + min(span * 128 + 32 * i + 8 * lq, p.c - 8));
 #pragma unroll
         for (int jb = 0; jb < JB; jb++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                if (p.f_natural) {  // piece (contraction row, eight columns) of the span
-                    const int piece = (jb * 4 + i) * 64 + lane, row = span * 128 + piece / (2 * JB), j = piece % (2 * JB) * 8;
-                    f[jb][i] = load8g(p.f + (int64_t)row * p.r + j, row < p.c ? p.r - j : 0, vec);
+                if constexpr (NATURAL) {
+                    const int row = span * 128 + (4 * jb + i) * (32 / JB) + nat_row;
+                    if constexpr (VEC) f[d][jb][i] = *(const uint4*)(p.f + (int64_t)min(row, p.c - 1) * p.r + min(nat_j, p.r - 8));
+                    else f[d][jb][i] = load8g(p.f + (int64_t)row * p.r + nat_j, row < p.c ? p.r - nat_j : 0, false);
                 } else {
-                    const int j = jb * 16 + li, e = span * 128 + 32 * i + 8 * lq;
-                    f[jb][i] = j < p.r && e < p.c ? *(const uint4*)(p.f + (int64_t)j * p.ldf + e) : make_uint4(0, 0, 0, 0);
+                    f[d][jb][i] = *(const uint4*)(p.f + (int64_t)min(jb * 16 + li, p.r - 1) * p.ldf + min(span * 128 + 32 * i + 8 * lq, p.c - 8));
                 }
             }
     };
-    if (wave < spans) load(wave);
-    for (int span = wave; span < spans; span += 4) {
-        bf16x8_t a[4], b[JB][4];
+    auto multiply = [&](int d, int span) __attribute__((always_inline)) {
+        if (span * 128 + 128 > p.c) {  // the last, partial span
 #pragma unroll
-        for (int i = 0; i < 4; i++) a[i] = __builtin_bit_cast(bf16x8_t, x[i]);
-        if (p.f_natural) {
+            for (int i = 0; i < 4; i++) {
+                x[d][i] = kept_if(span * 128 + 32 * i + 8 * lq < p.c, x[d][i]);
+#pragma unroll
+                for (int jb = 0; jb < JB; jb++)
+                    f[d][jb][i] = kept_if((NATURAL ? span * 128 + (4 * jb + i) * (32 / JB) + nat_row : span * 128 + 32 * i + 8 * lq) < p.c, f[d][jb][i]);
+            }
+        }
+        bf16x8_t b[JB][4];
+        if constexpr (NATURAL) {
             uint4* dst = (uint4*)&lds.f[wave][0][0];
 #pragma unroll
             for (int jb = 0; jb < JB; jb++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) dst[(jb * 4 + i) * 64 + lane] = f[jb][i];
+                for (int i = 0; i < 4; i++) dst[(jb * 4 + i) * 64 + lane] = VEC ? kept_if(nat_j < p.r, f[d][jb][i]) : f[d][jb][i];
             // (LDS serves a wave in order, and no other wave uses this piece)
 #pragma unroll
             for (int jb = 0; jb < JB; jb++)
@@ -164,14 +174,26 @@ __device__ __forceinline__ void thin_product_body(const SkinnyNtParams& p, int w
 #pragma unroll
             for (int jb = 0; jb < JB; jb++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) b[jb][i] = __builtin_bit_cast(bf16x8_t, f[jb][i]);
+                for (int i = 0; i < 4; i++) b[jb][i] = __builtin_bit_cast(bf16x8_t, kept_if(jb * 16 + li < p.r, f[d][jb][i]));
         }
-        load(min(span + 4, spans - 1));  // (past the end: the last span again)
 #pragma unroll
         for (int jb = 0; jb < JB; jb++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc[jb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[jb][i], acc[jb], 0, 0, 0);
+            for (int i = 0; i < 4; i++) acc[jb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[d][i]), b[jb][i], acc[jb], 0, 0, 0);
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) load(d, wave + 4 * d);
+    int span = wave;
+    for (; span + 4 * (DEPTH - 1) < spans; span += 4 * DEPTH) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; d++) {
+            multiply(d, span + 4 * d);
+            load(d, span + 4 * (d + DEPTH));
+        }
     }
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; d++)
+        if (span + 4 * d < spans) multiply(d, span + 4 * d);
 #pragma unroll
     for (int jb = 0; jb < JB; jb++) lds.red[wave][jb][lane] = acc[jb];
     __syncthreads();
@@ -194,7 +216,7 @@ struct SidePassParams {
     int product_wgs, gradient_wgs;
 };
 template <int QT, int JB>
-__global__ __launch_bounds__(256) void decode_side_kernel(SidePassParams p) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void decode_side_kernel(SidePassParams p) {
     __shared__ __attribute__((aligned(16))) union {
         DecodeLds<QT> decode;
         ThinLds<JB> thin;
@@ -202,7 +224,11 @@ __global__ __launch_bounds__(256) void decode_side_kernel(SidePassParams p) {
         FactorGradLds<JB, 2> wide;
     } lds;
     int wg = blockIdx.x;
-    if (wg < p.product_wgs) return thin_product_body<JB>(p.product, wg, lds.thin);
+    if (wg < p.product_wgs) {
+        if (!p.product.f_natural) return thin_product_body<JB, false, true>(p.product, wg, lds.thin);
+        if (p.product.r % 8 == 0) return thin_product_body<JB, true, true>(p.product, wg, lds.thin);
+        return thin_product_body<JB, true, false>(p.product, wg, lds.thin);
+    }
     wg -= p.product_wgs;
     if (wg < p.gradient_wgs) {
         if (p.gradient.c % 128 == 0) factor_grad_body<JB, 2>(p.gradient, wg, lds.wide);
