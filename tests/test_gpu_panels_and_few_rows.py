@@ -60,6 +60,12 @@ def test_dense_lora_over_panels(pkg, dev, qt, m, n, k, r):
     (130, 1544, 1792, 16),  # spans beyond the ones in flight: twelve whole and a partial one over four waves
     (100, 1096, 3072, 24),  # the same with two blocks of ranks, the second one half full
     (64, 2048, 3328, 32),
+    # ranks whose rows of B are no whole pieces
+    (50, 8, 256, 1),        # one piece in all
+    (49, 1672, 256, 4),     # the spans in flight once over and a partial one of eight elements
+    (97, 1416, 512, 7),     # rows at odd elements
+    (65, 1544, 512, 20),    # two blocks of ranks
+    (100, 1096, 512, 31),
 ])
 def test_rank_sized_products_beside_the_decoding_pass(pkg, dev, m, n, k, r):
     payload, x, a, b, dy = _lora_case(7100 + n + k, m, n, k, r, gb.Q8_0)

@@ -105,18 +105,23 @@ __global__ __launch_bounds__(256) void decode_panel_kernel(DecodeParams p) {
 // through the wave's own LDS as [128][r_pad] and the operand is read back transposed.
 // What bounds it is latency: a few dozen workgroups on part of the chip.  So DEPTH spans are in flight per wave, and no load
 // stands behind a branch (there the compiler waits for every load before it): past the end of the contraction or of the rank
-// a lane reads the last whole piece and drops it.  VEC: whole, aligned pieces of F's rows (NATURAL: r is a multiple of eight).
-// The launch with the decoding pass, rank 16, forward / backward: 512 rows, 2048 x 2048 Q8_0 13.9 / 11.6 -> 11.3 / 9.6 us; 1021
-// rows, 512 x 2048 Q6_K 9.6 / 7.0 -> 7.0 / 6.8; 4096 rows, 4096 x 2048 Q4_K 14.4 / 20.0 -> 13.6 / 18.9 (there at the memory's rate).
+// a lane reads the last whole piece and drops it.  VEC: rows of F in whole pieces (NATURAL: r is a multiple of eight).  Without,
+// a span of F is one run of pieces all the same, and its elements are taken apart behind LDS; one span less is in flight there,
+// which leaves the kernel the registers of four workgroups per compute unit (three for ranks above 16).
+// The launch with the decoding pass, forward / backward, before there was more than one span in flight and now (us): 512 rows, 2048 x
+// 2048 Q8_0, rank 16 13.9 / 11.4 -> 11.0 / 9.6, rank 32 16.4 / 11.4 -> 11.8 / 9.0, rank 4 13.7 / 19.4 -> 10.2 / 9.9; 1021 rows, 512 x
+// 2048 Q6_K, rank 8 9.5 / 7.0 -> 7.0 / 7.1; 4096 rows, 4096 x 2048 Q4_K, rank 16 13.7 / 19.2 -> 12.8 / 17.8 (there at the memory's
+// rate), rank 20 17.7 / 60.4 -> 12.8 / 20.1.
 template <int JB>
 struct ThinLds {
     bf16_t f[4][128][JB * 16];
     f32x4_t red[4][JB][64];
 };
+typedef bf16_t __attribute__((may_alias)) aliasing_bf16_t;  // (read where 16-byte pieces were written)
 __device__ __forceinline__ uint4 kept_if(bool keep, const uint4& v) { return make_uint4(keep ? v.x : 0u, keep ? v.y : 0u, keep ? v.z : 0u, keep ? v.w : 0u); }
 template <int JB, bool NATURAL, bool VEC>
 __device__ __forceinline__ void thin_product_body(const SkinnyNtParams& p, int wg, ThinLds<JB>& lds) {
-    constexpr int DEPTH = JB == 1 ? 3 : 2;
+    constexpr int DEPTH = 4 - JB - (NATURAL && !VEC);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 15, lq = lane >> 4;
     const int m0 = wg * 16, spans = (p.c + 127) / 128;
@@ -125,7 +130,9 @@ __device__ __forceinline__ void thin_product_body(const SkinnyNtParams& p, int w
 #pragma unroll
     for (int jb = 0; jb < JB; jb++) acc[jb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     uint4 x[DEPTH][4], f[DEPTH][JB][4];
-    // NATURAL: piece (jb, i) of a span is contraction row ((4 jb + i) 64 + lane) / (2 JB), the lane's eight columns from j
+    // NATURAL: piece (jb, i) of a span is contraction row ((4 jb + i) 64 + lane) / (2 JB), the lane's eight columns from j.  A rank that
+    // is no multiple of eight has no such pieces: there it is the ((4 jb + i) 64 + lane)-th of the 16 r pieces of the span's rows,
+    // one run that begins on a whole piece (the base is aligned, 128 rows are 256 r bytes) and ends on one (c is in eights).
     const int nat_j = lane % (2 * JB) * 8, nat_row = lane / (2 * JB);
     auto load = [&](int d, int span) __attribute__((always_inline)) {
 #pragma unroll
@@ -137,7 +144,7 @@ __device__ __forceinline__ void thin_product_body(const SkinnyNtParams& p, int w
                 if constexpr (NATURAL) {
                     const int row = span * 128 + (4 * jb + i) * (32 / JB) + nat_row;
                     if constexpr (VEC) f[d][jb][i] = *(const uint4*)(p.f + (int64_t)min(row, p.c - 1) * p.r + min(nat_j, p.r - 8));
-                    else f[d][jb][i] = load8g(p.f + (int64_t)row * p.r + nat_j, row < p.c ? p.r - nat_j : 0, false);
+                    else f[d][jb][i] = *(const uint4*)(p.f + min((int64_t)span * 128 * p.r + 8 * min((4 * jb + i) * 64 + lane, 16 * p.r - 1), (int64_t)p.c * p.r - 8));
                 } else {
                     f[d][jb][i] = *(const uint4*)(p.f + (int64_t)min(jb * 16 + li, p.r - 1) * p.ldf + min(span * 128 + 32 * i + 8 * lq, p.c - 8));
                 }
@@ -149,7 +156,7 @@ __device__ __forceinline__ void thin_product_body(const SkinnyNtParams& p, int w
             for (int i = 0; i < 4; i++) {
                 x[d][i] = kept_if(span * 128 + 32 * i + 8 * lq < p.c, x[d][i]);
 #pragma unroll
-                for (int jb = 0; jb < JB; jb++)
+                for (int jb = 0; VEC && jb < JB; jb++)
                     f[d][jb][i] = kept_if((NATURAL ? span * 128 + (4 * jb + i) * (32 / JB) + nat_row : span * 128 + 32 * i + 8 * lq) < p.c, f[d][jb][i]);
             }
         }
@@ -165,10 +172,19 @@ __device__ __forceinline__ void thin_product_body(const SkinnyNtParams& p, int w
             for (int jb = 0; jb < JB; jb++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const bf16_t* src = &lds.f[wave][32 * i + 8 * lq + (li >> 2)][jb * 16 + (li & 3) * 4];
-                    const v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)src);
-                    const v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)(src + 4 * JB * 16));
-                    b[jb][i] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                    if constexpr (VEC) {
+                        const bf16_t* src = &lds.f[wave][32 * i + 8 * lq + (li >> 2)][jb * 16 + (li & 3) * 4];
+                        const v4i16_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)src);
+                        const v4i16_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_ptr)(src + 4 * JB * 16));
+                        b[jb][i] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                    } else {  // rows of any rank start at any element: one at a time
+                        const int row = 32 * i + 8 * lq, j = jb * 16 + li, r = (int)opaque((uint32_t)p.r);  // (else the addresses of all are kept through the loop)
+                        const aliasing_bf16_t* src = (const aliasing_bf16_t*)&lds.f[wave][0][0] + row * r + min(j, r - 1);
+                        uint32_t e[8];
+#pragma unroll
+                        for (int t = 0; t < 8; t++) e[t] = src[t * r];
+                        b[jb][i] = __builtin_bit_cast(bf16x8_t, kept_if(j < r && span * 128 + row < p.c, make_uint4(e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16)));
+                    }
                 }
         } else {
 #pragma unroll
@@ -216,7 +232,7 @@ struct SidePassParams {
     int product_wgs, gradient_wgs;
 };
 template <int QT, int JB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void decode_side_kernel(SidePassParams p) {
+__global__ __launch_bounds__(256) void decode_side_kernel(SidePassParams p) {
     __shared__ __attribute__((aligned(16))) union {
         DecodeLds<QT> decode;
         ThinLds<JB> thin;
