@@ -770,12 +770,12 @@ __device__ __forceinline__ void load_row_pieces(const bf16_t* row, int k, int la
 #pragma unroll
     for (int t = 0; t < PIECES; t++) {
         const int e = 512 * t + 8 * lane;
-        if constexpr (PIECES <= 4) {
-            // 32-bit offsets from a row that all lanes share, and no branch: past the end a lane reads the last piece and drops it.  One token, 8 of
-            // 256 Q4_K experts, 2048 / 512: gate / up 7.4 -> 7.2 us, down 9.2-9.6 -> 9.1-9.2.
+        if constexpr (PIECES == 1) {
+            // (the down kernel's) 32-bit offsets from a row that all lanes share, and no branch: past the end a lane reads the last piece and drops
+            // it.  One token, 8 of 256 Q4_K experts, 2048 / 512: 9.5 -> 9.2 us.
             const uint4 p = *(const uint4*)((const uint8_t*)row + 2u * (uint32_t)min(e, k - 8));
             v[t] = make_uint4(e < k ? p.x : 0u, e < k ? p.y : 0u, e < k ? p.z : 0u, e < k ? p.w : 0u);
-        } else {  // (eight pieces of two rows together, dropped behind the loads, would take more than 128 registers)
+        } else {  // (gate / up: without the branch 12 registers more and nothing gained, one token 7.5 and 7.5 us, four tokens 18.3 and 18.6)
             v[t] = e < k ? *(const uint4*)(row + e) : make_uint4(0, 0, 0, 0);
         }
     }
