@@ -677,7 +677,8 @@ static int decode_panel(int qt, const DecodeParams& d, const DenseSide* side, hi
     return set_error(GGQ_ERR_QTYPE, "unsupported GGML type id %d", qt);
 }
 
-// Aligned rows in eights, one segment without an index, rank up to kDenseSideMaxRank.
+// Aligned rows in eights, one segment without an index, rank up to kDenseSideMaxRank.  (A natural factor is aligned: the entry points refuse
+// others.)
 bool dense_side_takes(const DenseSide& side) {
     if (side.r_pad > kDenseSideMaxRank) return false;
     if (const SkinnyNtParams* q = side.product)

@@ -22,8 +22,9 @@ __device__ __forceinline__ uint4 load8g(const bf16_t* p, int valid, bool vec) {
 // ---- G[e][c, j] = s * sum_m In[m, c] * S[m, j] over the rows of expert e.  One workgroup per
 // (expert, 64 * CB columns); each wave owns CB blocks of 16 columns; rows are consumed 32 at a time
 // through LDS, where the operands of the contraction over m are read with transposing loads.  The loads
-// of four 32-row slices are issued together and the slices then go through two alternating LDS buffers,
-// one barrier each.  Experts without rows get zeros.
+// of four 32-row slices are issued together (of rows in place; a slice of rows behind an index waits for its
+// indices and the loads before them, one with routing weights for its weights) and the slices then go through
+// two alternating LDS buffers, one barrier each.  Experts without rows get zeros.
 template <int JB, int CB>
 struct FactorGradLds {
     static constexpr int kPitch = 64 * CB + 32, kSPitch = JB * 16 + 8;

@@ -223,7 +223,8 @@ struct GemvParams {
 
 // WAVES waves deal the spans of the contraction out (span s to wave s % WAVES, at most SP each); TB blocks of sixteen rows of x.
 // LORA is a template parameter because a load the compiler tracks may stand nowhere in the block loop of a plain product: on
-// whatever path, it makes every iteration wait for all requests, the block requested ahead among them.
+// whatever path, it makes every iteration wait for all requests, the block requested ahead among them.  (With LORA the row of B
+// is such a load: there each request waits for the one before it, and the next block has landed before the current one is multiplied.)
 template <int QT, int WAVES, int SP, int TB, bool LORA>  // TB <= WAVES
 __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t gemv_lds[];
@@ -726,7 +727,7 @@ int router_logits(const void* x, const void* w, int64_t m, int64_t n, int64_t k,
 //   act[route] = silu(gate) * up         one workgroup per (route, eight or sixteen gate rows and the up rows of the same columns)
 //   out[token] = sum w[route] * down     one workgroup per (token, sixteen output columns), one wave per route
 // The LoRA products x A^T are formed by every workgroup for itself (64 KB of factor out of the L2 at rank 16 and 2048
-// columns): cheaper than a launch.  One token, 8 of 256 Q4_K experts, 2048 / 512: 7.6 and 9.6 us; with the factor rows read
+// columns): cheaper than a launch.  One token, 8 of 256 Q4_K experts, 2048 / 512: 7.5 and 9.2 us; with the factor rows read
 // as MFMA operands and eight gate rows per workgroup 10.4 and 11.3.
 struct FewRoutesParams {
     const bf16_t* x;       // [tokens, hidden]
@@ -794,8 +795,9 @@ __device__ __forceinline__ float wave_sum(float s) {
 
 // Eight gate rows and eight up rows per set; a workgroup takes SETS sets of one route.  What bounds it is latency and the
 // vector cache's requests: every workgroup forms x A^T for itself, and as MFMA operands (16 rows x 64 bytes a request) the 64 KB
-// of A cost two workgroups of a compute unit 2.3 us.  So each wave takes whole rows of A (1 KB a request, half the time, under
-// the weights' latency), x comes to LDS once, and two sets share one x A^T where that leaves enough workgroups.
+// of A cost two workgroups of a compute unit 2.3 us.  So each wave takes whole rows of A (1 KB a request, half the time), x
+// comes to LDS once, and two sets share one x A^T where that leaves enough workgroups.  The requests of the packed rows are ahead of A's,
+// not beside them: x is unpacked in front of the loop over the ranks, and the wait for x takes the packed rows along.
 __host__ __device__ __forceinline__ int gate_up_half_lds(int qt, int row_bytes, int sets) {
     const int bytes = 8 * sets * row_bytes;
     return qt == kQ4_K ? (bytes + (bytes >> 10) * kPieceGap<kQ4_K> + 127) & ~127 : (bytes + 15) & ~15;
@@ -887,6 +889,8 @@ __global__ __launch_bounds__(512) void few_routes_gate_up_kernel(FewRoutesParams
     }
 }
 
+// What bounds it is round trips one after another: the expert's id, the route's weight, the packed rows (the compiler waits for every
+// request of request_bytes before the next, for Q4_K rows of 512 elements five), x, and the rows of A in eights.
 template <int QT>
 __global__ __launch_bounds__(512) void few_routes_down_kernel(FewRoutesParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t down_lds[];
