@@ -91,6 +91,15 @@ def test_null_and_shape_errors_come_back_before_any_launch(pkg):
     assert lib.ggq_dequantize(12, ctypes.c_void_p(16), 1, 100, ctypes.c_void_p(16), 0, None) == -2  # K not whole blocks
 
 
+@pytest.mark.parametrize("a,b", [(32, 34), (34, 32), (32, 40)])
+def test_factors_off_16_bytes_are_refused_before_any_launch(pkg, a, b):
+    # (the kernels load a factor's rows in whole 16-byte pieces)
+    lib, at = pkg._lib.load(), ctypes.c_void_p(64)
+    assert lib.ggq_lora_mmq_forward(at, at, 12, 64, 64, 256, ctypes.c_void_p(a), ctypes.c_void_p(b), 16, 1.0, at, at, at, 1 << 20, None) == -3
+    assert lib.ggq_lora_mmq_backward(at, at, 12, 64, 64, 256, at, at, ctypes.c_void_p(a), ctypes.c_void_p(b), 16, 1.0, at, at, at, at, 1 << 20, None) == -3
+    assert b"aligned" in lib.ggq_last_error()
+
+
 def test_python_mirror_guards(pkg):
     loss_mod = pkg.gguf_liger_loss
     h = torch.zeros(4, 64, dtype=torch.bfloat16)
